@@ -304,46 +304,75 @@ __global__ __launch_bounds__(256) void k_blk_scatter(const int *__restrict__ ptr
     if (DOT) blk_block_partials(acc, partials);
 }
 
-// Folds G block partials of quantity q per column (fixed order) -> out[pos].
-__device__ void blk_fold(const double *partials, int G, double *out)
+// Folds the G <= PF_BLK_MAXG block partials of FOLD_C consecutive columns
+// (positions c0 ..) of one quantity in the fixed order: part p adds blocks p,
+// p + 4, ... in turn, the four parts are added left to right.  The order is a
+// serial chain per part (512 additions at 2,048 blocks), so a fold is bound
+// by latency, not by bytes (1 MB a quantity): a workgroup brings its columns'
+// partials into LDS with 16 loads in flight per thread, then one lane per
+// (column, part) walks the chain from there, a batch of reads ahead of the
+// additions.  FOLD_T threads, PF_BLK / FOLD_C workgroups a quantity.
+// Returns the sum of column c0 + lane in lanes 0 .. FOLD_C - 1 of wave 0.
+// (20^3 hex20, 2,048 blocks: one workgroup folding all 64 columns 29 us a
+// quantity; one per column, whose strided loads use 8 bytes of a line,
+// 14.6 us; this 10 us.)
+constexpr int FOLD_T = 256, FOLD_C = 4;
+__device__ __forceinline__ double blk_fold(const double *__restrict__ partials, int G, int c0)
 {
-    __shared__ double ws[4][PF_BLK];
-    const int col = threadIdx.x & 63, part = threadIdx.x >> 6;
-    // thread (col, part) adds blocks part, part+4, ... in that order, the
-    // loads of a batch of 16 issued before the dependent additions
-    double s = 0.0;
-    for (int b0 = part; b0 < G; b0 += 64) {
-        double t[16];
+    __shared__ double sp[PF_BLK_MAXG * FOLD_C];
+    const int t = threadIdx.x, n = G * FOLD_C;
+    for (int i0 = t; i0 < n; i0 += 16 * FOLD_T) {
+        double v[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
-            const int b = b0 + 4 * u;
-            t[u] = b < G ? partials[(long)b * PF_BLK + col] : 0.0;
+            const int i = i0 + u * FOLD_T;
+            v[u] = i < n ? partials[(long)(i / FOLD_C) * PF_BLK + c0 + i % FOLD_C] : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < 16; ++u)
-            if (b0 + 4 * u < G) s = __dadd_rn(s, t[u]);
-    }
-    ws[part][col] = s;
-    __syncthreads();
-    if (threadIdx.x < PF_BLK) {
-        double t = ws[0][col];
-        for (int p = 1; p < 4; ++p) t = __dadd_rn(t, ws[p][col]);
-        out[col] = t;
+            if (i0 + u * FOLD_T < n) sp[i0 + u * FOLD_T] = v[u];
     }
     __syncthreads();
+    double s = 0.0;
+    if (t < 64) {
+        // lane 4p + c: entries (p + 4m, c) lie at lane + 16m
+        const int l = t & 15, p = l >> 2;
+        const int nm = G > p ? (G - p + 3) / 4 : 0, full = G / 64 * 16;   // every part has G/4 entries or one more
+        double v[16];
+        if (full) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = sp[l + 16 * u];
+        }
+        for (int m = 0; m < full; m += 16) {
+            double w[16];
+            const int mn = m + 16 < full ? m + 16 : 0;   // the last batch reads the first again, unused
+#pragma unroll
+            for (int u = 0; u < 16; ++u) w[u] = sp[l + 16 * (mn + u)];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s = __dadd_rn(s, v[u]);
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = w[u];
+        }
+        for (int m = full; m < nm; ++m) s = __dadd_rn(s, sp[l + 16 * m]);
+        const double s1 = __shfl(s, (l & 3) + 4, 64), s2 = __shfl(s, (l & 3) + 8, 64), s3 = __shfl(s, (l & 3) + 12, 64);
+        s = __dadd_rn(__dadd_rn(__dadd_rn(s, s1), s2), s3);   // lanes 0..3 hold part 0
+    }
+    return s;
 }
 
-__global__ __launch_bounds__(256) void k_blk_fold_alpha(const double *partials, int G, pf_blk_state *st)
+// Workgroup b: columns FOLD_C b ...
+__global__ __launch_bounds__(FOLD_T) void k_blk_fold_alpha(const double *__restrict__ partials, int G,
+                                                          pf_blk_state *st)
 {
+    const int c0 = blockIdx.x * FOLD_C;
     if (st->done) {
-        if (threadIdx.x == 0) st->xlast = 0;   // the last p update has run
+        if (c0 == 0 && threadIdx.x == 0) st->xlast = 0;   // the last p update has run
         return;
     }
-    __shared__ double pu[PF_BLK];
-    blk_fold(partials, G, pu);
-    if (threadIdx.x < PF_BLK) {
-        const int c = threadIdx.x;
-        const double a = st->frozen[c] || pu[c] == 0.0 ? 0.0 : st->up[c] / pu[c];
+    const double pu = blk_fold(partials, G, c0);
+    if (threadIdx.x < FOLD_C) {
+        const int c = c0 + threadIdx.x;
+        const double a = st->frozen[c] || pu == 0.0 ? 0.0 : st->up[c] / pu;
         st->alpha[c] = isfinite(a) ? a : 0.0;
     }
 }
@@ -381,37 +410,41 @@ __global__ __launch_bounds__(256) void k_blk_update(float *__restrict__ R, const
     blk_block_partials(rr, partials + (long)PF_BLK_MAXG * PF_BLK);
 }
 
-// beta = (r,d)/up per active column; a column whose recurrence residual fell
-// by delta since its last replacement, or below tol ||f||, asks for a
-// residual replacement (trig); done at the iteration limit.
-__global__ __launch_bounds__(256) void k_blk_fold_update(const double *partials, int G, pf_blk_state *st)
+// beta = (r,d)/up per active column (blockIdx.y 0); a column whose recurrence
+// residual fell by delta since its last replacement, or below tol ||f||, asks
+// for a residual replacement (blockIdx.y 1: trig); done at the iteration
+// limit.  The first workgroup counts the iteration.  One that starts after
+// it has set done leaves its columns as they are (one thread reads the flag
+// for all): past the limit only alpha is read (the last x update), and the
+// replacement that follows sets up, rr and beta anew.
+__global__ __launch_bounds__(FOLD_T) void k_blk_fold_update(const double *__restrict__ partials, int G,
+                                                           pf_blk_state *st)
 {
-    if (st->done) return;
-    __shared__ double rd[PF_BLK], rr[PF_BLK];
-    __shared__ int trig;
-    blk_fold(partials, G, rd);
-    blk_fold(partials + (long)PF_BLK_MAXG * PF_BLK, G, rr);
-    if (threadIdx.x == 0) trig = 0;
+    __shared__ int stop;
+    if (threadIdx.x == 0) stop = st->done;
     __syncthreads();
-    if (threadIdx.x < PF_BLK) {
-        const int c = threadIdx.x;
+    if (stop) return;
+    const int c0 = blockIdx.x * FOLD_C;
+    const double v = blk_fold(partials + (long)blockIdx.y * PF_BLK_MAXG * PF_BLK, G, c0);
+    if (threadIdx.x >= FOLD_C) return;
+    const int c = c0 + threadIdx.x;
+    if (blockIdx.y == 0) {
         if (!st->frozen[c]) {
-            const double b = st->up[c] == 0.0 ? 0.0 : rd[c] / st->up[c];
+            const double b = st->up[c] == 0.0 ? 0.0 : v / st->up[c];
             st->beta[c] = isfinite(b) ? b : 0.0;
-            st->up[c] = rd[c];
-            st->rr[c] = rr[c];
-            if (!(rr[c] > st->delta2 * st->rr_ref[c]) || !(rr[c] > st->tol2 * st->ff[c])) atomicAdd(&trig, 1);
+            st->up[c] = v;
         } else {
             st->beta[c] = 0.0;
         }
+    } else if (!st->frozen[c]) {
+        st->rr[c] = v;
+        if (!(v > st->delta2 * st->rr_ref[c]) || !(v > st->tol2 * st->ff[c])) st->trig = 1;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
+    if (c == 0 && blockIdx.y == 0) {
         st->iters += 1;
-        if (trig) st->trig = 1;
         if (st->iters >= st->limit) {
-            st->done = 1;
             st->xlast = 1;
+            st->done = 1;
         }
     }
 }
@@ -483,19 +516,21 @@ __global__ __launch_bounds__(256) void k_blk_inner_init(float *__restrict__ X, f
 
 // After a start or a replacement: up = (r,d), rr = rr_ref = (r,r), no
 // pending request.  Frozen flags and the tolerances are set by the host.
-__global__ __launch_bounds__(256) void k_blk_fold_init(const double *partials, int G, pf_blk_state *st)
+__global__ __launch_bounds__(FOLD_T) void k_blk_fold_init(const double *__restrict__ partials, int G,
+                                                         pf_blk_state *st)
 {
-    __shared__ double rd[PF_BLK], rr[PF_BLK];
-    blk_fold(partials, G, rd);
-    blk_fold(partials + (long)PF_BLK_MAXG * PF_BLK, G, rr);
-    if (threadIdx.x < PF_BLK) {
-        const int c = threadIdx.x;
-        st->up[c] = rd[c];
-        st->rr[c] = rr[c];
-        st->rr_ref[c] = rr[c];
+    const int c0 = blockIdx.x * FOLD_C;
+    const double v = blk_fold(partials + (long)blockIdx.y * PF_BLK_MAXG * PF_BLK, G, c0);
+    if (threadIdx.x >= FOLD_C) return;
+    const int c = c0 + threadIdx.x;
+    if (blockIdx.y == 0) {
+        st->up[c] = v;
         st->alpha[c] = st->beta[c] = 0.0;
+        if (c == 0) st->trig = 0;
+    } else {
+        st->rr[c] = v;
+        st->rr_ref[c] = v;
     }
-    if (threadIdx.x == 0) st->trig = 0;
 }
 
 // X64 += X (FP32 correction), then X = 0 when CLEAR.
@@ -527,11 +562,11 @@ __global__ __launch_bounds__(256) void k_blk_residual(double *__restrict__ R64, 
     blk_block_partials(rr, partials);
 }
 
-__global__ __launch_bounds__(256) void k_blk_fold_out(const double *partials, int G, double *out)
+__global__ __launch_bounds__(FOLD_T) void k_blk_fold_out(const double *__restrict__ partials, int G,
+                                                        double *__restrict__ out)
 {
-    __shared__ double v[PF_BLK];
-    blk_fold(partials, G, v);
-    if (threadIdx.x < PF_BLK) out[threadIdx.x] = v[threadIdx.x];
+    const double v = blk_fold(partials, G, blockIdx.x * FOLD_C);
+    if (threadIdx.x < FOLD_C) out[blockIdx.x * FOLD_C + threadIdx.x] = v;
 }
 
 // host order (neq x k, column-major) <-> block order ((neq+1) x 64, row 0 = 0)
@@ -711,7 +746,7 @@ int blk_true_residual(pf_ctx *c, double *rr_host)
                        b->Ut64, (const double *)nullptr, b->U64, c->neq, (double *)nullptr,
                        (const pf_blk_state *)nullptr);
     hipLaunchKernelGGL(k_blk_residual, dim3(G), dim3(256), 0, c->stream, b->R64, b->F64, b->U64, c->neq, b->partials);
-    hipLaunchKernelGGL(k_blk_fold_out, dim3(1), dim3(256), 0, c->stream, b->partials, G,
+    hipLaunchKernelGGL(k_blk_fold_out, dim3(PF_BLK / FOLD_C), dim3(FOLD_T), 0, c->stream, b->partials, G,
                        b->partials + (long)2 * PF_BLK_MAXG * PF_BLK);
     PF_HIP(hipGetLastError());
     PF_HIP(hipMemcpyAsync(rr_host, b->partials + (long)2 * PF_BLK_MAXG * PF_BLK, PF_BLK * sizeof(double),
@@ -849,7 +884,7 @@ int pf_block_solve(pf_ctx *c, int k, const double *f, double *x, const pf_block_
     // Start: x = 0 in FP32, p = d = dinv fl32(r).
     hipLaunchKernelGGL(k_blk_inner_init<true>, dim3(G), dim3(256), 0, c->stream, b->X, b->R, b->P, b->R64, b->dinv,
                        c->neq, b->partials);
-    hipLaunchKernelGGL(k_blk_fold_init, dim3(1), dim3(256), 0, c->stream, b->partials, G, b->st);
+    hipLaunchKernelGGL(k_blk_fold_init, dim3(PF_BLK / FOLD_C, 2), dim3(FOLD_T), 0, c->stream, b->partials, G, b->st);
     PF_HIP(hipGetLastError());
     bool first = true;
     for (;;) {
@@ -899,13 +934,13 @@ int pf_block_solve(pf_ctx *c, int k, const double *f, double *x, const pf_block_
                 if (tm) PF_HIP(hipEventRecord(t0, c->stream));
                 hipLaunchKernelGGL((k_blk_scatter<float, true>), dim3(G), dim3(256), 0, c->stream, c->csr_ptr,
                                    c->csr_slot, b->Ut32, b->P, b->U, c->neq, b->partials, b->st);
-                hipLaunchKernelGGL(k_blk_fold_alpha, dim3(1), dim3(256), 0, c->stream, b->partials, G, b->st);
+                hipLaunchKernelGGL(k_blk_fold_alpha, dim3(PF_BLK / FOLD_C), dim3(FOLD_T), 0, c->stream, b->partials, G, b->st);
                 if (tm) PF_HIP(hipEventRecord(t1, c->stream));
                 tm = pf_timing_begin(c, PF_K_UPDATE, &t0, &t1);
                 if (tm) PF_HIP(hipEventRecord(t0, c->stream));
                 hipLaunchKernelGGL(k_blk_update, dim3(G), dim3(256), 0, c->stream, b->R, b->U, b->dinv, c->neq,
                                    b->partials, b->st);
-                hipLaunchKernelGGL(k_blk_fold_update, dim3(1), dim3(256), 0, c->stream, b->partials, G, b->st);
+                hipLaunchKernelGGL(k_blk_fold_update, dim3(PF_BLK / FOLD_C, 2), dim3(FOLD_T), 0, c->stream, b->partials, G, b->st);
                 if (tm) PF_HIP(hipEventRecord(t1, c->stream));
                 tm = pf_timing_begin(c, PF_K_PUPDATE, &t0, &t1);
                 if (tm) PF_HIP(hipEventRecord(t0, c->stream));
@@ -942,7 +977,7 @@ int pf_block_solve(pf_ctx *c, int k, const double *f, double *x, const pf_block_
         else
             hipLaunchKernelGGL(k_blk_inner_init<false>, dim3(G), dim3(256), 0, c->stream, b->X, b->R, b->P, b->R64,
                                b->dinv, c->neq, b->partials);
-        hipLaunchKernelGGL(k_blk_fold_init, dim3(1), dim3(256), 0, c->stream, b->partials, G, b->st);
+        hipLaunchKernelGGL(k_blk_fold_init, dim3(PF_BLK / FOLD_C, 2), dim3(FOLD_T), 0, c->stream, b->partials, G, b->st);
         PF_HIP(hipGetLastError());
         R.outer += 1;
     }
