@@ -172,6 +172,7 @@ static void reset_problem(pf_ctx *c)
     free_arr(c, c->csr_ptr, (size_t)c->neq + 1);
     free_arr(c, c->csr_slot, (size_t)c->nnz);
     free_arr(c, c->csr_slot_t, (size_t)c->nnz);
+    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
     free_arr(c, c->utemp, (size_t)c->ntot * c->nels);
     free_arr(c, c->utemp32, (size_t)c->ntot * c->nels);
     c->nod = c->nels = c->ntot = c->neq = 0;
@@ -196,6 +197,7 @@ int pf_steer_install(pf_ctx *c, int ntot, int nels, int neq)
     free_arr(c, c->csr_ptr, (size_t)c->neq + 1);
     free_arr(c, c->csr_slot, (size_t)c->nnz);
     free_arr(c, c->csr_slot_t, (size_t)c->nnz);
+    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
     free_arr(c, c->utemp, (size_t)c->ntot * c->nels);
     free_arr(c, c->utemp32, (size_t)c->ntot * c->nels);
     c->ntot = ntot;
@@ -227,6 +229,7 @@ void pf_steer_drop(pf_ctx *c)
     free_arr(c, c->csr_ptr, (size_t)c->neq + 1);
     free_arr(c, c->csr_slot, (size_t)c->nnz);
     free_arr(c, c->csr_slot_t, (size_t)c->nnz);
+    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
     free_arr(c, c->utemp, (size_t)c->ntot * c->nels);
     free_arr(c, c->utemp32, (size_t)c->ntot * c->nels);
     c->ntot = c->neq = 0;
@@ -277,14 +280,14 @@ int pf_create(int device, pf_ctx **out)
     }
     c->stream = c->own_stream;
     int rc = pf_scratch_init(device);   // device address of the allocation-free scratch
-    if (!rc) rc = pf_alloc(c, (void **)&c->state, sizeof(pf_state));
+    if (!rc) rc = pf_alloc(c, (void **)&c->state, 2 * sizeof(pf_state));
     if (!rc) rc = pf_alloc(c, (void **)&c->partials, sizeof(double) * kPartials);
     if (!rc && hipHostMalloc((void **)&c->state_host, sizeof(pf_state), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
     if (!rc && hipHostMalloc((void **)&c->scalar_host, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
     if (!rc && hipHostMalloc((void **)&c->state_query, sizeof(pf_state), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
     if (!rc && hipEventCreateWithFlags(&c->ev_query, hipEventDisableTiming) != hipSuccess) rc = PF_ERR_HIP;
     if (!rc) {
-        hipError_t z = hipMemsetAsync(c->state, 0, sizeof(pf_state), c->stream);
+        hipError_t z = hipMemsetAsync(c->state, 0, 2 * sizeof(pf_state), c->stream);
         if (z == hipSuccess) z = hipStreamSynchronize(c->stream);
         if (z != hipSuccess) rc = pf_set_hip_error(z, "init state", __FILE__, __LINE__);
     }
@@ -303,7 +306,7 @@ int pf_destroy(pf_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     reset_problem(c);
     free_arr(c, c->partials, kPartials);
-    pf_free(c, c->state, sizeof(pf_state));
+    pf_free(c, c->state, 2 * sizeof(pf_state));
     if (c->state_host) (void)hipHostFree(c->state_host);
     if (c->scalar_host) (void)hipHostFree(c->scalar_host);
     if (c->state_query) (void)hipHostFree(c->state_query);

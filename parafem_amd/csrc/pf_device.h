@@ -19,18 +19,45 @@ __device__ __forceinline__ bool skip(const pf_state *st, int gate)
     return gate == RUN_REFINE && !st->refine;
 }
 
+// v of lane l + OFF, in the lanes below OFF (the others' values are not used):
+// the halves of the wavefront through the permlane swaps, lanes of one row of
+// 16 through DPP.  These stay in the vector pipe; a shuffle goes through the
+// LDS unit, and the twelve of a wavefront's sum, each waiting for the one
+// before, took 0.4 us of the small kernels' 3.
+template <int OFF> __device__ __forceinline__ unsigned lane_down32(unsigned v)
+{
+    if constexpr (OFF == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+    else if constexpr (OFF == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 | OFF, 0xf, 0xf, true);   // row_shl:OFF
+}
+
+template <int OFF> __device__ __forceinline__ double lane_down(double v)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = lane_down32<OFF>((unsigned)b), hi = lane_down32<OFF>((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Lane 0: the wavefront's sum (maximum), v[l] = v[l] + v[l + off] for off =
+// 32, 16, 8, 4, 2, 1.  Every lane must be active.
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = __dadd_rn(v, __shfl_down(v, off, 64));
-    return v;
+    v = __dadd_rn(v, lane_down<32>(v));
+    v = __dadd_rn(v, lane_down<16>(v));
+    v = __dadd_rn(v, lane_down<8>(v));
+    v = __dadd_rn(v, lane_down<4>(v));
+    v = __dadd_rn(v, lane_down<2>(v));
+    return __dadd_rn(v, lane_down<1>(v));
 }
 
 __device__ __forceinline__ double wave_max(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
-    return v;
+    v = fmax(v, lane_down<32>(v));
+    v = fmax(v, lane_down<16>(v));
+    v = fmax(v, lane_down<8>(v));
+    v = fmax(v, lane_down<4>(v));
+    v = fmax(v, lane_down<2>(v));
+    return fmax(v, lane_down<1>(v));
 }
 
 // Folds NQ per-thread values of this block (sum or max per quantity) and
@@ -92,6 +119,47 @@ __device__ void fold_partials(double (&out)[NQ], const int (&qid)[NQ], const boo
             for (int w = 1; w < PF_BLOCK / 64; ++w) s = ismax[k] ? fmax(s, ws[k][w]) : __dadd_rn(s, ws[k][w]);
             out[k] = s;
         }
+    }
+}
+
+// fold_partials for every thread of any workgroup: each folds all G block
+// results itself, in the same order, and has them in out[].  Meant for small
+// G (a few entries per thread): it replaces a launch of the one-block fold.
+template <int NQ>
+__device__ __forceinline__ void fold_everywhere(double (&out)[NQ], const int (&qid)[NQ], const bool (&ismax)[NQ],
+                                                const double *__restrict__ partials, int G)
+{
+    __shared__ double ws[NQ][PF_BLOCK / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double s[NQ];
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) s[k] = 0.0;
+    for (int b0 = threadIdx.x; b0 < G; b0 += 4 * PF_BLOCK) {
+        double t[NQ][4];
+#pragma unroll
+        for (int k = 0; k < NQ; ++k)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int b = b0 + u * PF_BLOCK;
+                t[k][u] = b < G ? partials[qid[k] * MAXG + b] : 0.0;
+            }
+#pragma unroll
+        for (int k = 0; k < NQ; ++k)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (b0 + u * PF_BLOCK < G) s[k] = ismax[k] ? fmax(s[k], t[k][u]) : __dadd_rn(s[k], t[k][u]);
+    }
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+        s[k] = ismax[k] ? wave_max(s[k]) : wave_sum(s[k]);
+        if (lane == 0) ws[k][wave] = s[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+        double v = ws[k][0];
+        for (int w = 1; w < PF_BLOCK / 64; ++w) v = ismax[k] ? fmax(v, ws[k][w]) : __dadd_rn(v, ws[k][w]);
+        out[k] = v;
     }
 }
 

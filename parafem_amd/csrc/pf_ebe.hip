@@ -21,6 +21,10 @@
 //   k_fold_update (one block) beta, the stopping rule, the iteration count
 //                 and the freeze flag;
 //   k_pupdate     p = d + p*beta (and, for the mixed solver, p32 = fl32(p)).
+// A problem of few reduction blocks is bound by its launches (about 3 us each,
+// whether enqueued one by one or replayed from a graph) and runs the same
+// iteration without the folds' launches (see "iterations without fold
+// launches" below), with the same bits.
 // The mixed solver adds a true-residual replacement (reliable update) on
 // the iterations its fold kernel flags: k_ebe over hi+lo in FP64 with x,
 // k_scatter_res (r = f - K x, d = dinv*r) and k_fold_refine.
@@ -42,6 +46,99 @@
 #include "pf_device.h"
 
 namespace {
+
+// End of an iteration: beta = rd/up, the stopping rule, the count.
+__device__ void finish_iteration(pf_state *st, double rd, double rr, double maxx, double maxdx)
+{
+    const double beta = rd / st->up;
+    const double crit = st->stop_mode == PF_STOP_CHECON ? maxdx / maxx : sqrt(rr / st->rr0);
+    st->beta = beta;
+    st->up = rd;
+    st->rr = rr;
+    st->crit = crit;
+    st->iters += 1;
+    st->pfresh = 0;
+    st->converged = crit <= st->tol;
+    if (!isfinite(beta) || !isfinite(rd)) st->breakdown = 1;
+    if (st->converged || st->iters >= st->limit || st->breakdown) st->frozen = 1;
+}
+
+// ------------------------------------ iterations without fold launches
+// Up to PF_FOLD_MAXG reduction blocks the folds cost no launch: every workgroup
+// of the kernel that needs alpha or beta folds the block partials itself (the
+// fixed order, so the same bits), and the first workgroup also writes the
+// state.  Two copies of the state keep a kernel's readers apart from its
+// writer: `live` is written by the kernel that ends an iteration and read by
+// the ones after it; the scatter's first workgroup, which runs when live is
+// settled, copies it to `work`, from which the update, the replacement and
+// the end of the iteration read.
+//   k_ebe, k_scatter_copy, k_update_fold (alpha), [k_ebe_due, k_scatter_res,]
+//   k_pupdate_fold (beta, the stopping rule)
+// and up to FORM_MAXG, where even the p update's launch is worth saving, the
+// products of the next iteration end this one and form p = d + p*beta as they
+// gather it; the scatter then stores p (the last iteration of a run ends with
+// k_pupdate_fold, so that p is complete between runs).
+// Measured, us per iteration with the folds' launches / without / with p
+// formed in the products (the launches 6 / 4 / 3, mixed 9 / 6 / 5): FP64 hex20
+// 4^3 20.1 / 13.1 / 12.2, 20^3 58 / 51 / 51, mixed 39 / 30 / 30; Laplace 25^3
+// 20.3 / 15.3 / 13.2.
+
+// Work state of a running solve: a breakdown stops the iteration it occurs in.
+__device__ __forceinline__ bool stopped(const pf_state *work) { return work->frozen || work->breakdown; }
+
+// Folds the update's partials (or the replacement's) and ends the iteration
+// of `work`; the lead workgroup writes the new state to *live.  Returns
+// whether the solve has stopped (before or now); *beta is valid otherwise.
+// The state is looked at after the fold's barrier, so that its load, the
+// partials' and the caller's are in flight together: in these small kernels a
+// dependent load is worth 0.7 us.
+template <bool CHECON>
+__device__ __forceinline__ bool end_iteration(const double *__restrict__ partials, int G, const pf_state *work,
+                                              pf_state *live, bool lead, double *beta)
+{
+    const bool ref = !CHECON && work->refine;
+    double rd, rr = 0.0, maxx = 0.0, maxdx = 0.0;
+    if constexpr (CHECON) {
+        constexpr int qid[3] = {PF_Q_RD, PF_Q_MAXX, PF_Q_MAXDX};
+        constexpr bool mx[3] = {false, true, true};
+        double o[3];
+        fold_everywhere<3>(o, qid, mx, partials, G);
+        rd = o[0];
+        maxx = o[1];
+        maxdx = o[2];
+    } else {
+        const int qid[2] = {ref ? PF_Q_RD2 : PF_Q_RD, ref ? PF_Q_RR2 : PF_Q_RR};
+        constexpr bool mx[2] = {false, false};
+        double o[2];
+        fold_everywhere<2>(o, qid, mx, partials, G);
+        rd = o[0];
+        rr = o[1];
+    }
+    pf_state s = *work;
+    if (s.frozen || s.breakdown) return true;
+    if (s.precision == PF_PREC_MIXED || s.precision == PF_PREC_MIXED64) s.since_refine += 1;
+    if (ref) {
+        s.refine = 0;
+        s.refinements += 1;
+        s.since_refine = 0;
+        s.rr_ref = rr;
+    }
+    finish_iteration(&s, rd, rr, maxx, maxdx);
+    if (lead && threadIdx.x == 0) *live = s;
+    *beta = s.beta;
+    return s.frozen != 0;
+}
+
+// What the products need to end the previous iteration and form p.
+struct pf_form {
+    const double *d;
+    const double *partials;
+    int G;
+    const pf_state *work;
+    pf_state *live;
+    bool lead;
+};
+enum { FORM_NONE = 0, FORM_CHECON = 1, FORM_RELRES = 2 };
 
 // Element products.  GATHER: src is a neq+1 vector with src[0] = 0 and the
 // element vector is src[g_g]; otherwise src is pmul (ntot,nels).  Lane i of
@@ -67,11 +164,19 @@ namespace {
 // scatter, not by this kernel): 2% faster FP64 products, 0.5-1% FP32.
 // ebe_block forms the products of logical block lb (PF_BLOCK/64 * EPW * EPL
 // consecutive elements); the kernels below choose lb.
-template <int NT, int KIND, bool GATHER, typename OUT, int EPL>
+// FORM: the previous iteration ends here and the gathered vector is
+// p = d + p*beta, with every load (matrix, p, d, partials) in flight before
+// the fold's barrier.
+// stop: the solve has stopped.  With FORM it is looked at with the steering
+// (whose entries are never negative), so that one load latency covers both;
+// otherwise before anything else, so that the matrix loads do not wait for
+// the steering (waiting cost the 100^3 mixed product 2%).
+template <int NT, int KIND, bool GATHER, typename OUT, int EPL, int FORM = FORM_NONE>
 __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K64, const float *__restrict__ Khi,
                                           const float *__restrict__ Klo, const int *__restrict__ gg,
                                           const double *__restrict__ src, const float *__restrict__ src32,
-                                          OUT *__restrict__ out, int nels, long kstride, int rowmajor)
+                                          OUT *__restrict__ out, int nels, long kstride, int rowmajor,
+                                          bool stop, const pf_form &fm = pf_form{})
 {
     using L = Lanes<NT, KIND>;
     // packed layout: Q quads and R more full diagonals, then the half one (d = H)
@@ -87,12 +192,31 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
     const long ebase = (lb * (PF_BLOCK / 64) + wave) * L::EPW * EPL;
     long ev[EPL], ec[EPL];
     int g[EPL];
+    if (FORM == FORM_NONE && stop) return;
 #pragma unroll
     for (int t = 0; t < EPL; ++t) {
         ev[t] = ebase + t * L::EPW + sub;
         ec[t] = ev[t] < nels ? ev[t] : (long)nels - 1;
         g[t] = GATHER ? __builtin_nontemporal_load(&gg[ec[t] * NT + i]) : 0;   // read once per product
     }
+    if (FORM != FORM_NONE && (stop | (__builtin_amdgcn_readfirstlane(g[0]) < 0))) return;
+    // the gathered entry of slot t, after the matrix loads
+    double fp[EPL], fd[EPL], beta = 0.0;
+    auto form = [&]() {
+        if constexpr (FORM != FORM_NONE) {
+#pragma unroll
+            for (int t = 0; t < EPL; ++t) {
+                fp[t] = src[g[t]];
+                fd[t] = fm.d[g[t]];
+            }
+            return end_iteration<FORM == FORM_CHECON>(fm.partials, fm.G, fm.work, fm.live, fm.lead, &beta);
+        }
+        return false;
+    };
+    auto entry = [&](int t) -> double {
+        if constexpr (FORM != FORM_NONE) return __dadd_rn(fd[t], __dmul_rn(fp[t], beta));
+        return GATHER ? src[g[t]] : src[ec[t] * NT + i];
+    };
     if constexpr (KIND == KIND_F64) {
         // Every column pair of K_e is in flight before the dependent gather.
         d2_t kc[EPL][NT / 2];
@@ -102,8 +226,9 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
 #pragma unroll
             for (int j = 0; j < NT / 2; ++j) kc[t][j] = __builtin_nontemporal_load(&Kp[j * NT]);
         }
+        if (form()) return;
 #pragma unroll
-        for (int t = 0; t < EPL; ++t) ps[wave][t][lane] = GATHER ? src[g[t]] : src[ec[t] * NT + i];
+        for (int t = 0; t < EPL; ++t) ps[wave][t][lane] = entry(t);
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
@@ -136,13 +261,14 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
             for (int r = 0; r < R; ++r) kd[t][4 * Q + r] = __builtin_nontemporal_load(Ke + 4 * Q * NT + R * i + r);
             kd[t][H] = __builtin_nontemporal_load(Ke + H * NT + i % H);
         }
+        if (form()) return;
         float pv[EPL];
 #pragma unroll
         for (int t = 0; t < EPL; ++t) {
-            if constexpr (GATHER)
+            if constexpr (GATHER && FORM == FORM_NONE)
                 pv[t] = src32 ? src32[g[t]] : (float)src[g[t]];
             else
-                pv[t] = (float)src[ec[t] * NT + i];
+                pv[t] = (float)entry(t);
             float *pg = reinterpret_cast<float *>(&ps[wave][t][0]) + 2 * gb;
             if (li < NT) {
                 pg[li] = pv[t];
@@ -204,10 +330,11 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
                                 (double)__builtin_nontemporal_load(Kl + H * NT + i % H)
                           : (double)__builtin_nontemporal_load(Kh + H * NT + i % H);
         }
+        if (form()) return;
         double pv[EPL];
 #pragma unroll
         for (int t = 0; t < EPL; ++t) {
-            pv[t] = GATHER ? src[g[t]] : src[ec[t] * NT + i];
+            pv[t] = entry(t);
             double *pg = &ps[wave][t][0] + 2 * gb;
             if (li < NT) {
                 pg[li] = pv[t];
@@ -249,15 +376,17 @@ __global__ __launch_bounds__(PF_BLOCK) void k_ebe(const double *__restrict__ K64
                                                  OUT *__restrict__ out, int nels, long kstride,
                                                  const pf_state *__restrict__ st, int gate, long nlb, int rowmajor)
 {
-    if (skip(st, gate)) return;
+    const bool stop = skip(st, gate);
     const long lb0 = xcd_block(blockIdx.x, gridDim.x);
     if constexpr (LOOP) {
+        if (stop) return;
         for (long lb = lb0; lb < nlb; lb += gridDim.x) {
-            ebe_block<NT, KIND, GATHER, OUT, EPLT>(lb, K64, Khi, Klo, gg, src, src32, out, nels, kstride, rowmajor);
+            ebe_block<NT, KIND, GATHER, OUT, EPLT>(lb, K64, Khi, Klo, gg, src, src32, out, nels, kstride, rowmajor,
+                                                   false);
             __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
         }
     } else {
-        ebe_block<NT, KIND, GATHER, OUT, EPLT>(lb0, K64, Khi, Klo, gg, src, src32, out, nels, kstride, rowmajor);
+        ebe_block<NT, KIND, GATHER, OUT, EPLT>(lb0, K64, Khi, Klo, gg, src, src32, out, nels, kstride, rowmajor, stop);
     }
 }
 
@@ -444,22 +573,6 @@ __global__ __launch_bounds__(PF_BLOCK) void k_update(double *__restrict__ x, dou
     update_block<CHECON>(blockIdx.x, gridDim.x, x, r, d, p, u, dinv, neq, partials, st);
 }
 
-// End of an iteration: beta = rd/up, the stopping rule, the count.
-__device__ void finish_iteration(pf_state *st, double rd, double rr, double maxx, double maxdx)
-{
-    const double beta = rd / st->up;
-    const double crit = st->stop_mode == PF_STOP_CHECON ? maxdx / maxx : sqrt(rr / st->rr0);
-    st->beta = beta;
-    st->up = rd;
-    st->rr = rr;
-    st->crit = crit;
-    st->iters += 1;
-    st->pfresh = 0;
-    st->converged = crit <= st->tol;
-    if (!isfinite(beta) || !isfinite(rd)) st->breakdown = 1;
-    if (st->converged || st->iters >= st->limit || st->breakdown) st->frozen = 1;
-}
-
 template <bool CHECON>
 __device__ __forceinline__ void fold_update_block(const double *partials, int G, pf_state *st)
 {
@@ -512,7 +625,7 @@ __device__ __forceinline__ void scatter_res_block(int lb, int G, const int *__re
                                                   const double *__restrict__ fixstore, const double *__restrict__ x,
                                                   const double *__restrict__ f, double *__restrict__ r,
                                                   double *__restrict__ d, const double *__restrict__ dinv, int neq,
-                                                  double *partials)
+                                                  double *partials, bool second = false)
 {
     double v[2] = {0.0, 0.0};
     const int stride = G * PF_BLOCK;
@@ -529,7 +642,7 @@ __device__ __forceinline__ void scatter_res_block(int lb, int G, const int *__re
         v[0] = __dadd_rn(v[0], __dmul_rn(rq, dq));
         v[1] = __dadd_rn(v[1], __dmul_rn(rq, rq));
     }
-    constexpr int qid[2] = {PF_Q_RD, PF_Q_RR};
+    const int qid[2] = {second ? PF_Q_RD2 : PF_Q_RD, second ? PF_Q_RR2 : PF_Q_RR};
     constexpr bool mx[2] = {false, false};
     block_to_partials<2>(v, qid, mx, partials, lb);
 }
@@ -540,10 +653,11 @@ __global__ __launch_bounds__(PF_BLOCK) void k_scatter_res(const int *__restrict_
                                                          const double *__restrict__ x, const double *__restrict__ f,
                                                          double *__restrict__ r, double *__restrict__ d,
                                                          const double *__restrict__ dinv, int neq, double *partials,
-                                                         const pf_state *st)
+                                                         const pf_state *st, int second)
 {
-    if (skip(st, RUN_REFINE)) return;
-    scatter_res_block(blockIdx.x, gridDim.x, ptr, slot, utemp, fixstore, x, f, r, d, dinv, neq, partials);
+    // second: an iteration without fold launches (the working state decides)
+    if (second ? stopped(st + 1) || !st[1].refine : skip(st, RUN_REFINE)) return;
+    scatter_res_block(blockIdx.x, gridDim.x, ptr, slot, utemp, fixstore, x, f, r, d, dinv, neq, partials, second != 0);
 }
 
 __device__ __forceinline__ void fold_refine_block(const double *partials, int G, pf_state *st)
@@ -589,6 +703,210 @@ __global__ __launch_bounds__(PF_BLOCK) void k_pupdate(double *__restrict__ p, fl
 {
     if (skip(st, RUN_LIVE)) return;
     pupdate_block(blockIdx.x, gridDim.x, p, p32, d, neq, st);
+}
+
+// ---- kernels of an iteration without fold launches (see above)
+
+// The products of the next iteration: end this one, form p as it is gathered.
+template <int NT, int KIND, typename OUT, int FORM>
+__global__ __launch_bounds__(PF_BLOCK) void k_ebe_form(const double *__restrict__ K64, const float *__restrict__ Khi,
+                                                      const float *__restrict__ Klo, const int *__restrict__ gg,
+                                                      const double *__restrict__ p, OUT *__restrict__ out, int nels,
+                                                      long kstride, int rowmajor, const double *__restrict__ d,
+                                                      const double *__restrict__ partials, int G, pf_state *st)
+{
+    const pf_form fm{d, partials, G, st + 1, st, blockIdx.x == 0};
+    ebe_block<NT, KIND, true, OUT, Lanes<NT, KIND>::EPL, FORM>(xcd_block(blockIdx.x, gridDim.x), K64, Khi, Klo, gg, p,
+                                                              nullptr, out, nels, kstride, rowmajor,
+                                                              stopped(st + 1), fm);
+}
+
+// SCATTER with p.u of thread lb*PF_BLOCK + t's one equation, from the padded
+// slot table (plane j holds slot j of every equation, -1 past its last): no
+// offsets to wait for before the slots.  The first workgroup copies the
+// settled live state to the working copy.  With d: p = d + p*beta is formed
+// and stored.  rowmajor: an 8-node mesh's products as [row][element].
+template <typename UT>
+__device__ __forceinline__ void scatter_copy_block(int lb, const int *__restrict__ slot8,
+                                                   const UT *__restrict__ utemp, const double *__restrict__ fixstore,
+                                                   double *__restrict__ p, double *__restrict__ u, int neq,
+                                                   int fix_zero, double *partials, pf_state *st,
+                                                   const double *__restrict__ d, int rowmajor, int nels)
+{
+    const int q = lb * PF_BLOCK + threadIdx.x;
+    const bool live = q < neq;
+    int sl[PF_SLOT8];
+#pragma unroll
+    for (int j = 0; j < PF_SLOT8; ++j) sl[j] = live ? slot8[(long)j * neq + q] : -1;
+    const bool stop = skip(st, RUN_LIVE);
+    if (lb == 0 && threadIdx.x == 0) st[1] = st[0];
+    if (stop | (__builtin_amdgcn_readfirstlane(sl[0]) < -1)) return;   // with the slots: one load latency
+    double pq = live ? p[q + 1] : 0.0;
+    if (d) pq = __dadd_rn(live ? d[q + 1] : 0.0, __dmul_rn(pq, st->beta));
+    const double fs = fixstore && live ? fixstore[q + 1] : 0.0;
+    double v[PF_SLOT8];
+#pragma unroll
+    for (int j = 0; j < PF_SLOT8; ++j) {
+        const int k = rowmajor ? (sl[j] & 7) * nels + (sl[j] >> 3) : sl[j];
+        v[j] = sl[j] >= 0 ? (double)utemp[k] : 0.0;
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < PF_SLOT8; ++j)
+        if (sl[j] >= 0) s = __dadd_rn(s, v[j]);
+    double acc[1] = {0.0};
+    if (live) {
+        if (fs != 0.0) s = fix_zero ? 0.0 : __dmul_rn(pq, fs);
+        if (d) p[q + 1] = pq;
+        u[q + 1] = s;
+        acc[0] = __dadd_rn(acc[0], __dmul_rn(pq, s));
+    }
+    constexpr int qid[1] = {PF_Q_PU};
+    constexpr bool mx[1] = {false};
+    block_to_partials<1>(acc, qid, mx, partials, lb);
+}
+
+template <typename UT>
+__global__ __launch_bounds__(PF_BLOCK) void k_scatter_copy(const int *__restrict__ slot8,
+                                                          const UT *__restrict__ utemp,
+                                                          const double *__restrict__ fixstore, double *__restrict__ p,
+                                                          double *__restrict__ u, int neq, int fix_zero,
+                                                          double *partials, pf_state *st,
+                                                          const double *__restrict__ d, int rowmajor, int nels)
+{
+    scatter_copy_block<UT>(blockIdx.x, slot8, utemp, fixstore, p, u, neq, fix_zero, partials, st, d, rowmajor, nels);
+}
+
+// alpha, folded by every workgroup, then the x/r/d update of thread
+// lb*PF_BLOCK + t's one equation (G < PF_REDUCE_MAX_GRID: no second one),
+// loaded before the fold.
+template <bool CHECON>
+__device__ __forceinline__ void update_fold_block(int lb, int G, double *__restrict__ x, double *__restrict__ r,
+                                                  double *__restrict__ d, const double *__restrict__ p,
+                                                  const double *__restrict__ u, const double *__restrict__ dinv,
+                                                  int neq, double *partials, pf_state *st)
+{
+    pf_state *work = st + 1;
+    const int q = lb * PF_BLOCK + threadIdx.x + 1;
+    const bool live = q <= neq;
+    const double xo = live ? x[q] : 0.0, pq = live ? p[q] : 0.0, ro = live ? r[q] : 0.0;
+    const double uq = live ? u[q] : 0.0, di = live ? dinv[q] : 0.0;
+    constexpr int qpu[1] = {PF_Q_PU};
+    constexpr bool mpu[1] = {false};
+    double pu[1];
+    fold_everywhere<1>(pu, qpu, mpu, partials, G);
+    if (work->frozen) return;
+    const double alpha = work->up / pu[0];
+    const bool lead = lb == 0 && threadIdx.x == 0;
+    if (lead) work->alpha = alpha;
+    if (!isfinite(alpha)) {
+        if (lead) {
+            work->breakdown = 1;
+            st->alpha = alpha;
+            st->breakdown = 1;
+            st->frozen = 1;
+        }
+        return;
+    }
+    constexpr int NQ = CHECON ? 3 : 2;
+    double v[NQ];
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) v[k] = 0.0;
+    if (live) {
+        const double xn = __dadd_rn(xo, __dmul_rn(pq, alpha));
+        const double rq = __dsub_rn(ro, __dmul_rn(uq, alpha));
+        const double dq = __dmul_rn(di, rq);
+        x[q] = xn;
+        r[q] = rq;
+        d[q] = dq;
+        v[0] = __dadd_rn(v[0], __dmul_rn(rq, dq));
+        if constexpr (CHECON) {
+            v[1] = fmax(v[1], fabs(xn));
+            v[2] = fmax(v[2], fabs(__dsub_rn(xn, xo)));
+        } else {
+            v[1] = __dadd_rn(v[1], __dmul_rn(rq, rq));
+        }
+    }
+    if constexpr (CHECON) {
+        constexpr int qid[3] = {PF_Q_RD, PF_Q_MAXX, PF_Q_MAXDX};
+        constexpr bool mx[3] = {false, true, true};
+        block_to_partials<3>(v, qid, mx, partials, lb);
+    } else {
+        constexpr int qid[2] = {PF_Q_RD, PF_Q_RR};
+        constexpr bool mx[2] = {false, false};
+        block_to_partials<2>(v, qid, mx, partials, lb);
+    }
+}
+
+template <bool CHECON>
+__global__ __launch_bounds__(PF_BLOCK) void k_update_fold(double *__restrict__ x, double *__restrict__ r,
+                                                         double *__restrict__ d, const double *__restrict__ p,
+                                                         const double *__restrict__ u,
+                                                         const double *__restrict__ dinv, int neq, double *partials,
+                                                         pf_state *st)
+{
+    update_fold_block<CHECON>(blockIdx.x, gridDim.x, x, r, d, p, u, dinv, neq, partials, st);
+}
+
+// Whether a true-residual replacement is due, folded from the update's
+// partials by every workgroup (the rule of fold_update_block); the lead one
+// notes it for the kernels that follow.
+__device__ __forceinline__ bool refine_due(const double *__restrict__ partials, int G, pf_state *work, bool lead)
+{
+    constexpr int qid[1] = {PF_Q_RR};
+    constexpr bool mx[1] = {false};
+    double rr[1];
+    fold_everywhere<1>(rr, qid, mx, partials, G);
+    if (stopped(work)) return false;
+    const bool trig = rr[0] <= work->delta2 * work->rr_ref || sqrt(rr[0] / work->rr0) <= work->tol ||
+                      (work->refine_every > 0 && work->since_refine + 1 >= work->refine_every);
+    const bool due = trig && isfinite(rr[0]);
+    if (due && lead && threadIdx.x == 0) work->refine = 1;   // cleared by the next scatter's copy
+    return due;
+}
+
+// The true-residual products, in few workgroups that loop: on most
+// iterations they only find that nothing is due.
+template <int NT>
+__global__ __launch_bounds__(PF_BLOCK) void k_ebe_due(const double *__restrict__ K64, const float *__restrict__ Khi,
+                                                     const float *__restrict__ Klo, const int *__restrict__ gg,
+                                                     const double *__restrict__ x, double *__restrict__ out, int nels,
+                                                     long kstride, int rowmajor, long nlb,
+                                                     const double *__restrict__ partials, int G, pf_state *st)
+{
+    if (!refine_due(partials, G, st + 1, blockIdx.x == 0)) return;
+    for (long lb = xcd_block(blockIdx.x, gridDim.x); lb < nlb; lb += gridDim.x) {
+        ebe_block<NT, KIND_ACC, true, double, Lanes<NT, KIND_ACC>::EPL>(lb, K64, Khi, Klo, gg, x, nullptr, out, nels,
+                                                                       kstride, rowmajor, false);
+        __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
+    }
+}
+
+// beta and the stopping rule, folded by every workgroup, then p = d + p*beta
+// of thread lb*PF_BLOCK + t's one equation.
+template <bool CHECON>
+__device__ __forceinline__ void pupdate_fold_block(int lb, int G, double *__restrict__ p, float *__restrict__ p32,
+                                                   const double *__restrict__ d, int neq,
+                                                   const double *__restrict__ partials, pf_state *st)
+{
+    const int q = lb * PF_BLOCK + threadIdx.x + 1;
+    const bool live = q <= neq;
+    const double dq = live ? d[q] : 0.0, pq = live ? p[q] : 0.0;
+    double beta;
+    if (end_iteration<CHECON>(partials, G, st + 1, st, lb == 0, &beta)) return;
+    if (live) {
+        const double pn = __dadd_rn(dq, __dmul_rn(pq, beta));
+        p[q] = pn;
+        if (p32) p32[q] = (float)pn;
+    }
+}
+
+template <bool CHECON>
+__global__ __launch_bounds__(PF_BLOCK) void k_pupdate_fold(double *__restrict__ p, float *__restrict__ p32,
+                                                          const double *__restrict__ d, int neq,
+                                                          const double *__restrict__ partials, pf_state *st)
+{
+    pupdate_fold_block<CHECON>(blockIdx.x, gridDim.x, p, p32, d, neq, partials, st);
 }
 
 // PCG start: dinv = 1/diag, d = dinv*r, p = d, x = x0 (or 0), f = r; partial
@@ -1032,17 +1350,17 @@ __device__ __forceinline__ void bs_ebe(const pf_bslot *__restrict__ T, const lon
     constexpr int EPL = Lanes<NT, KIND>::EPL;
     const int s = bslot_find(est, ns, gb);
     const pf_bslot S = slot_of(T, s);
-    if (skip(S.st, gate)) return;
+    const bool stop = skip(S.st, gate);
     const long lb = gb - est[s];
     if constexpr (REF)
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.x, nullptr, (OUT *)S.utemp, S.nels,
-                                            S.kstride, S.rowmajor);
+                                            S.kstride, S.rowmajor, stop);
     else if constexpr (KIND == KIND_F32)
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, S.p32, (OUT *)S.utemp32, S.nels,
-                                            S.kstride, S.rowmajor);
+                                            S.kstride, S.rowmajor, stop);
     else
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
-                                            S.kstride, S.rowmajor);
+                                            S.kstride, S.rowmajor, stop);
 }
 
 // The true-residual products of the solves due for a replacement, solve by
@@ -1489,6 +1807,141 @@ int pf_pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const pf_pcg_opt
     return pcg_begin(c, r0, r0_on_device, nullptr, opts);
 }
 
+}  // extern "C"
+
+// Up to PF_FOLD_MAXG reduction blocks (and 8 slots an equation, for the padded
+// slot table): an iteration without fold launches; up to FORM_MAXG the
+// products also form p.  Every workgroup then reads all partials, which grows
+// with the square of the block count, and the gather reads d beside p: at
+// 1,925 blocks (34^3 hex20) 225 / 91.6 us FP64 / mixed against 227 / 95 with
+// the folds' launches, at 4,025 (100^3 Laplace) 165 / 123 against 155 / 115;
+// forming p at 404 (20^3) 50.9 / 30.1 against 50.9 / 30.3, at 690 (24^3) 82.2 /
+// 41.3 against 81.9 / 40.3, at 270 (40^3 Laplace) 18.7 against 20.7.
+constexpr int FORM_MAXG = 512;
+
+template <int NT, int KIND, typename OUT>
+static void launch_ebe_form(pf_ctx *c, OUT *out, int rm, int G)
+{
+    constexpr int EPB = Lanes<NT, KIND>::EPB;
+    const dim3 grid((c->nels + EPB - 1) / EPB), blk(PF_BLOCK);
+    if (c->opts.stop_mode == PF_STOP_CHECON)
+        hipLaunchKernelGGL((k_ebe_form<NT, KIND, OUT, FORM_CHECON>), grid, blk, 0, c->stream, c->K64, c->K32hi,
+                           c->K32lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
+    else
+        hipLaunchKernelGGL((k_ebe_form<NT, KIND, OUT, FORM_RELRES>), grid, blk, 0, c->stream, c->K64, c->K32hi,
+                           c->K32lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
+}
+
+template <int NT>
+static void launch_form_due(pf_ctx *c, bool due, int rm, int G)
+{
+    if (due) {
+        constexpr int EPB = Lanes<NT, KIND_ACC>::EPB;
+        const long nlb = (c->nels + EPB - 1) / EPB;
+        const int grid = (int)std::min<long>(nlb, 768);   // three workgroups per CU
+        hipLaunchKernelGGL(k_ebe_due<NT>, dim3(grid), dim3(PF_BLOCK), 0, c->stream, c->K64, c->K32hi, c->K32lo, c->g_g,
+                           c->x, c->utemp, c->nels, pf_k64_estride(c), rm, nlb, c->partials, G, c->state);
+        return;
+    }
+    switch (c->opts.precision) {
+    case PF_PREC_MIXED: launch_ebe_form<NT, KIND_F32, float>(c, c->utemp32, rm, G); break;
+    case PF_PREC_MIXED64: launch_ebe_form<NT, KIND_WIDE, double>(c, c->utemp, rm, G); break;
+    case PF_PREC_SPLIT: launch_ebe_form<NT, KIND_ACC, double>(c, c->utemp, rm, G); break;
+    default: launch_ebe_form<NT, KIND_F64, double>(c, c->utemp, rm, G); break;
+    }
+}
+
+// The products that form p (due = false), or the true-residual products of
+// the iterations that ask for them.
+static int launch_small(pf_ctx *c, bool due, int rm, int G)
+{
+    switch (c->ntot) {
+    case 60: launch_form_due<60>(c, due, rm, G); break;
+    case 24: launch_form_due<24>(c, due, rm, G); break;
+    case 8: launch_form_due<8>(c, due, rm, G); break;
+    default: return PF_ERR_ARG;
+    }
+    return PF_OK;
+}
+
+// The iteration's product of p as it stands.
+static int launch_products(pf_ctx *c, float *p32, int rm)
+{
+    switch (c->opts.precision) {
+    case PF_PREC_MIXED:
+        return launch_ebe<KIND_F32, true, float>(c, c->p, c->utemp32, c->state, RUN_LIVE, nullptr, p32, rm);
+    case PF_PREC_MIXED64:
+        return launch_ebe<KIND_WIDE, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
+    case PF_PREC_SPLIT:
+        return launch_ebe<KIND_ACC, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
+    default:
+        return launch_ebe<KIND_F64, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
+    }
+}
+
+// pf_pcg_run without fold launches (the conditions are the caller's).
+static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *slot)
+{
+    const bool checon = c->opts.stop_mode == PF_STOP_CHECON, mixed = c->opts.precision == PF_PREC_MIXED;
+    const bool refines = mixed || c->opts.precision == PF_PREC_MIXED64;
+    const bool form = G <= FORM_MAXG;
+    const dim3 grid(G), blk(PF_BLOCK);
+    const int fz = c->fix_zero ? 1 : 0;
+    hipEvent_t t0, t1;
+    for (int it = 0; it < n; ++it) {
+        const bool formed = form && it > 0;   // the products end the previous iteration and form p
+        int rc;
+        bool tm = pf_timing_begin(c, PF_K_EBE, &t0, &t1);
+        if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+        rc = formed ? launch_small(c, false, rm, G) : launch_products(c, p32, rm);
+        if (rc) return rc;
+        if (tm) PF_HIP(hipEventRecord(t1, c->stream));
+        tm = pf_timing_begin(c, PF_K_SCATTER, &t0, &t1);
+        if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+        const double *fd = formed ? c->d : nullptr;
+        if (mixed)
+            hipLaunchKernelGGL(k_scatter_copy<float>, grid, blk, 0, c->stream, c->csr_slot8, c->utemp32, c->fixstore,
+                               c->p, c->u, c->neq, fz, c->partials, c->state, fd, rm, c->nels);
+        else
+            hipLaunchKernelGGL(k_scatter_copy<double>, grid, blk, 0, c->stream, c->csr_slot8, c->utemp, c->fixstore,
+                               c->p, c->u, c->neq, fz, c->partials, c->state, fd, rm, c->nels);
+        if (tm) PF_HIP(hipEventRecord(t1, c->stream));
+        tm = pf_timing_begin(c, PF_K_UPDATE, &t0, &t1);
+        if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+        if (checon)
+            hipLaunchKernelGGL(k_update_fold<true>, grid, blk, 0, c->stream, c->x, c->r, c->d, c->p, c->u, c->dinv,
+                               c->neq, c->partials, c->state);
+        else
+            hipLaunchKernelGGL(k_update_fold<false>, grid, blk, 0, c->stream, c->x, c->r, c->d, c->p, c->u, c->dinv,
+                               c->neq, c->partials, c->state);
+        if (tm) PF_HIP(hipEventRecord(t1, c->stream));
+        if (refines) {
+            tm = pf_timing_begin(c, PF_K_REFINE, &t0, &t1);
+            if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+            rc = launch_small(c, true, rm, G);
+            if (rc) return rc;
+            hipLaunchKernelGGL(k_scatter_res, grid, blk, 0, c->stream, c->csr_ptr, slot, c->utemp, c->fixstore, c->x,
+                               c->f, c->r, c->d, c->dinv, c->neq, c->partials, c->state, 1);
+            if (tm) PF_HIP(hipEventRecord(t1, c->stream));
+        }
+        if (!form || it + 1 == n) {
+            tm = pf_timing_begin(c, PF_K_PUPDATE, &t0, &t1);
+            if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+            if (checon)
+                hipLaunchKernelGGL(k_pupdate_fold<true>, grid, blk, 0, c->stream, c->p, p32, c->d, c->neq, c->partials,
+                                   c->state);
+            else
+                hipLaunchKernelGGL(k_pupdate_fold<false>, grid, blk, 0, c->stream, c->p, p32, c->d, c->neq,
+                                   c->partials, c->state);
+            if (tm) PF_HIP(hipEventRecord(t1, c->stream));
+        }
+        PF_HIP(hipGetLastError());
+    }
+    return PF_OK;
+}
+
+extern "C" {
+
 int pf_pcg_run(pf_ctx *c, int n)
 {
     if (!c || n < 0) return PF_ERR_ARG;
@@ -1496,7 +1949,6 @@ int pf_pcg_run(pf_ctx *c, int n)
     const int G = pf_grid_for(c->neq);
     const bool mixed = c->opts.precision == PF_PREC_MIXED;
     const bool wide = c->opts.precision == PF_PREC_MIXED64;
-    const bool split = c->opts.precision == PF_PREC_SPLIT;
     float *p32 = mixed && c->ntot <= 24 ? c->p32 : nullptr;
     // hex8 with FP64 products: row-major (row i of every element side by
     // side, read back through the matching slot list; the scatter's reads of
@@ -1507,6 +1959,7 @@ int pf_pcg_run(pf_ctx *c, int n)
     const int *slot = rm ? c->csr_slot_t : c->csr_slot;
     const bool ranges = mixed && c->scatter_mode == PF_SCATTER_RANGES;
     if (ranges && !c->rng) return PF_ERR_STATE;   // pf_pcg_begin builds them
+    if (c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE) return run_foldless(c, n, G, p32, rm, slot);
     hipEvent_t t0, t1;
     for (int it = 0; it < n; ++it) {
         int rc;
@@ -1514,14 +1967,8 @@ int pf_pcg_run(pf_ctx *c, int n)
         if (tm) PF_HIP(hipEventRecord(t0, c->stream));
         if (ranges)
             rc = pf_ranges_iteration(c);   // p, the products, their sums into u, p.u per range
-        else if (mixed)
-            rc = launch_ebe<KIND_F32, true, float>(c, c->p, c->utemp32, c->state, RUN_LIVE, nullptr, p32, rm);
-        else if (wide)
-            rc = launch_ebe<KIND_WIDE, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
-        else if (split)
-            rc = launch_ebe<KIND_ACC, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
         else
-            rc = launch_ebe<KIND_F64, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
+            rc = launch_products(c, p32, rm);
         if (rc) return rc;
         if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         tm = pf_timing_begin(c, PF_K_SCATTER, &t0, &t1);
@@ -1570,7 +2017,7 @@ int pf_pcg_run(pf_ctx *c, int n)
             if (rc) return rc;
             hipLaunchKernelGGL(k_scatter_res, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->csr_ptr, slot,
                                c->utemp, c->fixstore, c->x, c->f, c->r, c->d, c->dinv, c->neq, c->partials,
-                               c->state);
+                               c->state, 0);
             const int Gr = seq_reduce(c, G, c->r + 1, c->d + 1, PF_Q_RD, c->r + 1, c->r + 1, PF_Q_RR, false,
                                       c->neq, c->state, RUN_REFINE);
             hipLaunchKernelGGL(k_fold_refine, dim3(1), dim3(PF_BLOCK), 0, c->stream, c->partials, Gr, c->state);

@@ -13,6 +13,8 @@
 
 #define PF_BLOCK 256                 // threads per block of the vector kernels
 #define PF_REDUCE_MAX_GRID 16384     // upper bound on reduction grid size G
+#define PF_FOLD_MAXG 2048            // reduction blocks up to which an iteration has no fold launches
+#define PF_SLOT8 8                   // slots per equation the padded slot table holds
 
 // Kernels of one PCG iteration, in launch order (pf_pcg_timing_get indices):
 // element products, scatter + p.u (and its fold), x/r/d update (and its
@@ -21,7 +23,9 @@
 enum { PF_K_EBE = 0, PF_K_SCATTER = 1, PF_K_UPDATE = 2, PF_K_PUPDATE = 3, PF_K_REFINE = 4, PF_NKERNELS = 5 };
 
 // Per-block partial quantities kept in the partials buffer.
-enum { PF_Q_PU = 0, PF_Q_RD = 1, PF_Q_RR = 2, PF_Q_MAXX = 3, PF_Q_MAXDX = 4, PF_NQ = 5 };
+// RD2, RR2: those of a true-residual replacement in an iteration without
+// fold launches (RD and RR stay readable beside them).
+enum { PF_Q_PU = 0, PF_Q_RD = 1, PF_Q_RR = 2, PF_Q_MAXX = 3, PF_Q_MAXDX = 4, PF_Q_RD2 = 5, PF_Q_RR2 = 6, PF_NQ = 7 };
 
 // Internal element-matrix layouts (the C ABI speaks storkm_pp's column-major
 // order; pf_storkm_set/get convert).  For element e, row i, column j of an
@@ -63,8 +67,12 @@ __host__ __device__ inline long pf_idx_sym_ij(long e, int nt, int i, int j)
     return d <= nt / 2 ? pf_idx_sym(e, nt, i, d) : pf_idx_sym(e, nt, j, nt - d);
 }
 
-// Device-resident PCG scalars.  Written only by the one-block fold kernels;
-// read at the start of the following kernels.
+// Device-resident PCG scalars.  Written only by the one-block fold kernels,
+// or, in an iteration without fold launches, by the first workgroup of the
+// kernel that ends the iteration; read at the start of the following kernels.
+// A context holds two: the live state ([0]: what polls and snapshots see),
+// and the working copy ([1]) that the kernels of an iteration without fold
+// launches read while the live one is being written.
 struct pf_state {
     double up;        // (r,d) of the current iterate (the reference's "up")
     double alpha;
@@ -157,6 +165,7 @@ struct pf_ctx {
     int *g_g = nullptr;                // (ntot,nels), 1-based, 0 = restrained
     int *csr_ptr = nullptr;            // (neq+1) offsets into csr_slot
     int *csr_slot = nullptr;           // element slots e*ntot+i, ascending
+    int *csr_slot8 = nullptr;          // small problems: the list as PF_SLOT8 planes of neq entries, -1 padded
     int *csr_slot_t = nullptr;         // hex8: the same list as i*nels+e (row-major iteration products)
     int64_t nnz = 0;
     // element matrices (internal layouts above)
@@ -181,7 +190,7 @@ struct pf_ctx {
     double *utemp = nullptr;           // (ntot,nels) element products, FP64
     float *utemp32 = nullptr;          // (ntot,nels) element products, FP32
     double *partials = nullptr;        // PF_NQ * PF_REDUCE_MAX_GRID (+ spare)
-    pf_state *state = nullptr;         // device
+    pf_state *state = nullptr;         // device: live state and working copy (2)
     pf_state *state_host = nullptr;    // pinned mirror for polling
     double *scalar_host = nullptr;     // pinned scratch for primitive results
     pf_pcg_opts opts{};

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(1024) void k_scan_top(int *__restrict__ bsum, int n
 }
 
 // ptr[q + 1] = sum of cnt[0..q] (ptr[0] = 0 is set by the caller); flags an
-// equation that no slot touches.
+// equation that no slot touches (2) or more than PF_SLOT8 do (4).
 __global__ __launch_bounds__(256) void k_scan_apply(const int *__restrict__ cnt, int n, const int *__restrict__ boff,
                                                    int *__restrict__ ptr, int *__restrict__ err)
 {
@@ -86,14 +86,16 @@ __global__ __launch_bounds__(256) void k_scan_apply(const int *__restrict__ cnt,
     const long base = (long)blockIdx.x * SCAN_CHUNK + (long)threadIdx.x * SCAN_ITEMS;
     int v[SCAN_ITEMS];
     int s = 0;
+    bool many = false;
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; ++j) {
         v[j] = base + j < n ? cnt[base + j] : 0;
         if (base + j < n && v[j] == 0) atomicOr(err, 2);
+        if (v[j] > PF_SLOT8) many = true;
         s += v[j];
     }
     ts[threadIdx.x] = s;
-    __syncthreads();
+    if (__syncthreads_or(many) && threadIdx.x == 0) atomicOr(err, 4);
     // inclusive scan of the 256 thread sums (Hillis-Steele)
     for (int off = 1; off < 256; off <<= 1) {
         const int add = threadIdx.x >= off ? ts[threadIdx.x - off] : 0;
@@ -118,8 +120,10 @@ __global__ __launch_bounds__(256) void k_csr_fill(const int *__restrict__ gg, lo
     }
 }
 
-// Each equation's slots in ascending order (insertion sort of a short list).
-__global__ __launch_bounds__(256) void k_csr_sort(const int *__restrict__ ptr, int *__restrict__ slot, int neq)
+// Each equation's slots in ascending order (insertion sort of a short list),
+// and, with slot8, their copy in the padded table.
+__global__ __launch_bounds__(256) void k_csr_sort(const int *__restrict__ ptr, int *__restrict__ slot, int neq,
+                                                 int *__restrict__ slot8)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= neq) return;
@@ -133,6 +137,8 @@ __global__ __launch_bounds__(256) void k_csr_sort(const int *__restrict__ ptr, i
         }
         slot[j + 1] = v;
     }
+    if (slot8)
+        for (int j = 0; j < PF_SLOT8; ++j) slot8[(long)j * neq + q] = a + j < b ? slot[a + j] : -1;
 }
 
 // slot_t[s] = i*nels + e for slot[s] = e*ntot + i: where the iteration's
@@ -212,7 +218,7 @@ int pf_csr_build(pf_ctx *c)
         release();
         return pf_set_hip_error(he, "transposed steering", __FILE__, __LINE__);
     }
-    if (host[0]) {
+    if (host[0] & 3) {
         release();
         return PF_ERR_ARG;
     }
@@ -220,6 +226,8 @@ int pf_csr_build(pf_ctx *c)
     rc = pf_alloc(c, (void **)&c->csr_slot, (size_t)std::max<int64_t>(c->nnz, 1) * sizeof(int));
     if (!rc && c->ntot == 8)
         rc = pf_alloc(c, (void **)&c->csr_slot_t, (size_t)std::max<int64_t>(c->nnz, 1) * sizeof(int));
+    if (!rc && !(host[0] & 4) && pf_grid_for(neq) <= PF_FOLD_MAXG)
+        rc = pf_alloc(c, (void **)&c->csr_slot8, (size_t)PF_SLOT8 * neq * sizeof(int));
     if (rc) {
         release();
         return rc;
@@ -230,7 +238,7 @@ int pf_csr_build(pf_ctx *c)
         hipLaunchKernelGGL(k_csr_fill, dim3(grid_for_stride(nslot)), dim3(256), 0, c->stream, c->g_g, nslot, cnt,
                            c->csr_slot);
         hipLaunchKernelGGL(k_csr_sort, dim3((neq + 255) / 256), dim3(256), 0, c->stream, c->csr_ptr, c->csr_slot,
-                           neq);
+                           neq, c->csr_slot8);
         if (c->csr_slot_t)
             hipLaunchKernelGGL(k_csr_transpose, dim3(grid_for_stride(c->nnz)), dim3(256), 0, c->stream, c->csr_slot,
                                (long)c->nnz, c->ntot, c->nels, c->csr_slot_t);

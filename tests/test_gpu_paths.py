@@ -8,6 +8,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import oracle as O
 from parafem_amd import Context, problems as P
 from parafem_amd.api import BlockOpts, BlockResult, lib
 
@@ -38,3 +39,59 @@ def test_block_fold_sizes(box):
             p = dinv * F[:, c]
             x = (F[:, c] @ p) / (p @ ctx.apply(p)) * p
             assert np.abs(X[:, c] - x).max() <= 1e-4 * np.abs(x).max()
+
+
+def _oracle_iterates(pr, stop, iters):
+    """x after `iters` iterations of the oracle in the device's order."""
+    gc = pr.g_coord()
+    K = (O.assemble_elastic(gc, pr.e, pr.v, pr.e_elem, nthreads=8) if pr.kind == "elastic"
+         else O.assemble_laplace(gc, pr.kx, pr.ky, pr.kz, pr.k_elem, nthreads=8))
+    dg = O.diag(pr.g_g, K, pr.neq)
+    kw = {}
+    r = pr.r0.copy()
+    if pr.fix_eq is not None:
+        store = dg[pr.fix_eq - 1] + P.PENALTY
+        dg[pr.fix_eq - 1] = store
+        r[pr.fix_eq - 1] = store * pr.fix_val
+        kw = {"no_f": pr.fix_eq, "store": store}
+    return O.pcg(pr.g_g, K, r, dg, 0.0, iters, stop=O.STOP_CHECON if stop == "checon" else O.STOP_RELRES,
+                 dot_order=O.DOT_DEVICE, nthreads=8, **kw)[0]
+
+
+# Reduction blocks (256 equations) at the edges of the rules: one; 512 | 513
+# (p formed in the products | not); 2,048 | 2,049 (no fold launches | folds)
+@pytest.mark.parametrize("box", [(5, 5, 5), (31, 63, 63), (32, 63, 63), (63, 63, 127), (64, 63, 127)])
+@pytest.mark.parametrize("stop", ["checon", "relres"])
+def test_iteration_tiers_bitexact(box, stop):
+    pr = P.laplace_cube(1, nels_xyz=box)
+    print(f"[gpu-test] tiers {box} neq={pr.neq} {stop}", flush=True)
+    with Context(0) as ctx:
+        r = P.setup(ctx, pr)
+        ctx.pcg_begin(r, 7, 0.0, stop=stop)
+        ctx.pcg_run(3)          # p is complete between runs
+        ctx.pcg_run(1)
+        ctx.pcg_run(5)          # three iterations to the limit, then nothing
+        assert ctx.pcg_poll().iters == 7
+        assert np.array_equal(ctx.pcg_x(), _oracle_iterates(pr, stop, 7))
+
+
+def test_more_slots_than_the_padded_table_holds():
+    """Equations that more than eight elements list (freedoms tied together)
+    take the iteration that reads the slot list itself: the oracle's bits."""
+    pr = P.elastic_cube(3)
+    g = pr.g_g.copy()
+    # the z freedoms of the top face become one equation
+    top = np.nonzero(np.abs(pr.mesh.coords[:, 2]) < 1e-12)[0]
+    tied = pr.nf[top, 2]
+    g[np.isin(g, tied)] = tied[0]
+    keep = np.unique(g[g > 0])
+    new = np.zeros(pr.neq + 1, dtype=np.int32)
+    new[keep] = np.arange(1, keep.size + 1)
+    r = np.zeros(keep.size)
+    np.add.at(r, new[np.where(np.isin(np.arange(1, pr.neq + 1), tied), tied[0], np.arange(1, pr.neq + 1))] - 1, pr.r0)
+    tp = P.Problem("elastic", pr.mesh, new[g], keep.size, r, pr.nf, e=pr.e, v=pr.v)
+    assert np.bincount(tp.g_g.ravel())[1:].max() > 8
+    with Context(0) as ctx:
+        P.setup(ctx, tp)
+        x, res = ctx.pcg_solve(r, 40, 0.0, stop="relres")
+        assert res.iters == 40 and np.array_equal(x, _oracle_iterates(tp, "relres", 40))
