@@ -43,11 +43,14 @@ def log(msg):
 
 def ebe_bytes(ntot, store, precision="mixed"):
     """Algorithmic HBM bytes of one element product: the element matrix once
-    (full FP64, or the FP32 hi part packed symmetric: the ntot(ntot+1)/2
-    entries of one triangle padded to a multiple of 4, hi and lo for the
-    split precision) and the int32 steering once."""
+    (the FP64 packed triangle as assembled: ntot/2 (ntot/2 + 1) column pairs
+    and, but for the Laplace elements, the 2-byte differences of the entries
+    below them and a word for their unit; or the FP32 hi part packed
+    symmetric: the ntot(ntot+1)/2 entries of one triangle padded to a multiple
+    of 4, hi and lo for the split precision) and the int32 steering once."""
     if store == "fp64":
-        return ntot * ntot * 8 + ntot * 4
+        h = ntot // 2
+        return 16 * h * (h + 1) + (4 * h * (h - 1) + 4 if ntot != 8 else 0) + ntot * 4
     parts = 2 if precision == "split" else 1
     packed = (ntot * (ntot + 1) // 2 + 3) // 4 * 4
     return parts * packed * 4 + ntot * 4
@@ -61,8 +64,9 @@ def iteration_bytes(nels, ntot, neq, store, precision="mixed"):
 
 def ebe_kernel_name(ntot, precision, epl):
     """The iteration's element-product kernel as rocprofv3 names it."""
-    kind, out = {"fp64": (0, "double"), "mixed": (1, "float"), "split": (2, "double"),
-                 "mixed64": (3, "double")}[precision]
+    if precision == "fp64":              # the packed triangle's products have one shape
+        return f"k_ebe<{ntot}, {4 if ntot == 8 else 5}, true, double, false, {2 if ntot == 8 else 1}>"
+    kind, out = {"mixed": (1, "float"), "split": (2, "double"), "mixed64": (3, "double")}[precision]
     return f"k_ebe<{ntot}, {kind}, true, {out}, false, {epl}>"
 
 

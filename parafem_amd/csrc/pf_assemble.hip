@@ -2,11 +2,12 @@
 //
 // One 64-lane wavefront builds one element: SAMPLE's 2x2x2 Gauss points,
 // SHAPE_DER at each point, the jacobian, its determinant and inverse, global
-// derivatives, then the element matrix, written once to HBM: in the
-// library's FP64 column-pair layout (pf_internal.h), or -- for FP32 storage
-// -- straight into the packed symmetric hi/lo layout (hi = fl32(K), lo =
-// fl32(K - hi) of the upper triangle) together with the element's FP64
-// diagonal, so an FP32-stored problem never holds the FP64 matrices.
+// derivatives, then the element matrix, written once to HBM: as the FP64
+// packed triangle (pf_internal.h; column pairs where it does not hold), or --
+// for FP32 storage -- straight into the packed symmetric hi/lo layout (hi =
+// fl32(K), lo = fl32(K - hi) of the upper triangle) together with the
+// element's FP64 diagonal, so an FP32-stored problem never holds the FP64
+// matrices.
 // Nothing but the element coordinates is read and nothing but the matrix is
 // written.
 //
@@ -23,82 +24,94 @@
 // a sequential evaluation of p121's MATMUL(MATMUL(TRANSPOSE(bee),dee),bee)
 // *det*weights(i) gives, bit for bit.
 #include "pf_internal.h"
+#include "pf_device.h"
 #include "pf_element.h"
 
 namespace {
 
 constexpr int WAVES = 4;   // elements per block
 
+// SAMPLE hexahedron nip=8 (new_library.f90:1406-1433): the signs of
+// (xi,eta,zeta) at point g, in the reference's order, and 1/sqrt(3).
+constexpr int gauss_sign[8][3] = {{1, 1, 1}, {1, 1, -1}, {1, -1, 1}, {1, -1, -1},
+                                  {-1, 1, 1}, {-1, -1, 1}, {-1, 1, -1}, {-1, -1, -1}};
+constexpr double gauss_r3 = 0.57735026918962584;   // the double 1.0 / sqrt(3.0)
+
+// SHAPE_DER at every Gauss point: the same for every element, so evaluated
+// once, by the compiler, with the operations of shape_der3 in their order.
+template <int NOD> struct DerTable {
+    double v[8][3][NOD];
+    constexpr DerTable() : v()
+    {
+        for (int g = 0; g < 8; ++g)
+            for (int l = 0; l < NOD; ++l) {
+                double d[3] = {0.0, 0.0, 0.0};
+                shape_der3<NOD>(gauss_sign[g][0] * gauss_r3, gauss_sign[g][1] * gauss_r3, gauss_sign[g][2] * gauss_r3, l,
+                                d);
+                for (int a = 0; a < 3; ++a) v[g][a][l] = d[a];
+            }
+    }
+};
+__device__ constexpr DerTable<8> der_table8{};
+__device__ constexpr DerTable<20> der_table20{};
+template <int NOD> __device__ __forceinline__ const double *der_at(int g, int a)
+{
+    if constexpr (NOD == 8) return der_table8.v[g][a];
+    else return der_table20.v[g][a];
+}
+
 // Per-wave LDS scratch for one element.
 template <int NOD>
 struct ElemLds {
     double coord[NOD * 3];      // (nod,3) column-major, as g_coord_pp(:,:,iel)
-    double der[8][3][NOD];      // local derivatives per Gauss point
-    double jac[8][9];           // jacobian (3x3 column-major), then its inverse
+    double jac[8][9];           // jacobian (3x3 column-major)
+    double inv[8][9];           // its inverse
     double dw[8];               // det * weight
     double deriv[8][3][NOD];    // global derivatives
 };
 
-// Stages shared by both element types: Gauss points, local derivatives,
-// jacobian, DETERMINANT/INVERT, global derivatives.  All four waves of the
-// block call it (block-uniform barriers); `valid` masks elements past nels.
+// Stages shared by the element types: jacobian, DETERMINANT/INVERT, global
+// derivatives.  All waves of the block call it (block-uniform barriers);
+// `valid` masks elements past the last.
 template <int NOD>
 __device__ __forceinline__ void element_geometry(ElemLds<NOD> &L, const double *__restrict__ gc, int lane, bool valid)
 {
-    const double r3 = 1.0 / sqrt(3.0);
     if (valid)
         for (int k = lane; k < NOD * 3; k += 64) L.coord[k] = gc[k];
-    // SAMPLE hexahedron nip=8 (new_library.f90:1406-1433): the signs of
-    // (xi,eta,zeta) at point g, in the reference's order.
-    constexpr int gs[8][3] = {{1, 1, 1}, {1, 1, -1}, {1, -1, 1}, {1, -1, -1},
-                              {-1, 1, 1}, {-1, -1, 1}, {-1, 1, -1}, {-1, -1, -1}};
-    for (int k = lane; k < 8 * NOD; k += 64) {
-        const int g = k / NOD, l = k % NOD;
-        const double xi = gs[g][0] > 0 ? r3 : -r3;
-        const double eta = gs[g][1] > 0 ? r3 : -r3;
-        const double zeta = gs[g][2] > 0 ? r3 : -r3;
-        double d3[3];
-        shape_der3<NOD>(xi, eta, zeta, l, d3);
-        L.der[g][0][l] = d3[0];
-        L.der[g][1][l] = d3[1];
-        L.der[g][2][l] = d3[2];
-    }
     __syncthreads();
     // jac = MATMUL(der, coord): 72 entries (8 points x 3 x 3).
     for (int k = lane; k < 72; k += 64) {
         const int g = k / 9, ab = k % 9, a = ab % 3, b = ab / 3;
+        const double *der = der_at<NOD>(g, a);
         double s = 0.0;
-        for (int l = 0; l < NOD; ++l) s += L.der[g][a][l] * L.coord[l + NOD * b];
+#pragma unroll
+        for (int l = 0; l < NOD; ++l) s += der[l] * L.coord[l + NOD * b];
         L.jac[g][a + 3 * b] = s;
     }
     __syncthreads();
-    if (lane < 8) {
-        double *m = L.jac[lane];
+    // DETERMINANT (maths.f90:615-619) and INVERT (maths.f90:525-547), an entry
+    // per lane: entry (r,c) of the inverse is P - Q with P = M(c+1,r+1)
+    // M(c+2,r+2) and Q = M(c+2,r+1) M(c+1,r+2), indices cyclic -- INVERT's nine
+    // statements, whose -A + B and B - A round alike -- over the determinant.
+    for (int k = lane; k < 72; k += 64) {
+        const int g = k / 9, rc = k % 9, r = rc % 3, c = rc / 3;
+        const double *m = L.jac[g];
 #define M(a, b) m[((a)-1) + 3 * ((b)-1)]
         double det = M(1, 1) * (M(2, 2) * M(3, 3) - M(3, 2) * M(2, 3));
         det = det - M(1, 2) * (M(2, 1) * M(3, 3) - M(3, 1) * M(2, 3));
         det = det + M(1, 3) * (M(2, 1) * M(3, 2) - M(3, 1) * M(2, 2));
-        const double j11 = M(2, 2) * M(3, 3) - M(3, 2) * M(2, 3);
-        const double j21 = -M(2, 1) * M(3, 3) + M(3, 1) * M(2, 3);
-        const double j31 = M(2, 1) * M(3, 2) - M(3, 1) * M(2, 2);
-        const double j12 = -M(1, 2) * M(3, 3) + M(3, 2) * M(1, 3);
-        const double j22 = M(1, 1) * M(3, 3) - M(3, 1) * M(1, 3);
-        const double j32 = -M(1, 1) * M(3, 2) + M(3, 1) * M(1, 2);
-        const double j13 = M(1, 2) * M(2, 3) - M(2, 2) * M(1, 3);
-        const double j23 = -M(1, 1) * M(2, 3) + M(2, 1) * M(1, 3);
-        const double j33 = M(1, 1) * M(2, 2) - M(2, 1) * M(1, 2);
-        M(1, 1) = j11 / det; M(1, 2) = j12 / det; M(1, 3) = j13 / det;
-        M(2, 1) = j21 / det; M(2, 2) = j22 / det; M(2, 3) = j23 / det;
-        M(3, 1) = j31 / det; M(3, 2) = j32 / det; M(3, 3) = j33 / det;
 #undef M
-        L.dw[lane] = det;   // SAMPLE weights are 1 for nip = 8
+        const int r1 = r == 2 ? 0 : r + 1, r2 = r == 0 ? 2 : r - 1, c1 = c == 2 ? 0 : c + 1, c2 = c == 0 ? 2 : c - 1;
+        const double P = m[c1 + 3 * r1] * m[c2 + 3 * r2], Q = m[c2 + 3 * r1] * m[c1 + 3 * r2];
+        L.inv[g][r + 3 * c] = (P - Q) / det;
+        if (rc == 0) L.dw[g] = det;   // SAMPLE weights are 1 for nip = 8
     }
     __syncthreads();
     // deriv = MATMUL(jac^-1, der)
     for (int k = lane; k < 8 * NOD; k += 64) {
         const int g = k / NOD, l = k % NOD;
-        const double *ji = L.jac[g];
-        const double d0 = L.der[g][0][l], d1 = L.der[g][1][l], d2 = L.der[g][2][l];
+        const double *ji = L.inv[g];
+        const double d0 = der_at<NOD>(g, 0)[l], d1 = der_at<NOD>(g, 1)[l], d2 = der_at<NOD>(g, 2)[l];
         for (int a = 0; a < 3; ++a) L.deriv[g][a][l] = ji[a] * d0 + ji[a + 3] * d1 + ji[a + 6] * d2;
     }
     __syncthreads();
@@ -139,82 +152,208 @@ __device__ __forceinline__ void zero_padding(long e, int lane, float *__restrict
     }
 }
 
-template <int NOD, bool S32>
-__global__ __launch_bounds__(64 * WAVES) void k_assemble_elastic(
-    const double *__restrict__ g_coord, const double *__restrict__ e_elem, double v2, double vv,
-    double den, double e0, double *__restrict__ K, float *__restrict__ hi, float *__restrict__ lo,
-    double *__restrict__ dg, int nels)
+// Difference K(i,j) - K(j,i) as an FP16 multiple of the element's unit (inv =
+// 1/unit, a power of two: both scalings are exact), and whether it brings the
+// entry back exactly as the product will form it.
+__device__ __forceinline__ _Float16 tri_code(double low, double up, double inv, double unit, bool &fail)
 {
-    constexpr int NTOT = 3 * NOD;
-    __shared__ ElemLds<NOD> lds[WAVES];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long e = (long)blockIdx.x * WAVES + wave;
-    const bool valid = e < nels;
-    ElemLds<NOD> &L = lds[wave];
-    element_geometry<NOD>(L, g_coord + (valid ? e : 0) * (NOD * 3), lane, valid);
-    if (!valid) return;
-    if constexpr (S32) zero_padding<NTOT>(e, lane, hi, lo);
-    if (lane >= NTOT) return;
+    const _Float16 h = (_Float16)(float)(__dsub_rn(low, up) * inv);
+    fail |= __fma_rn((double)h, unit, up) != low;
+    return h;
+}
+
+// The unit (its high word; inv its reciprocal) that puts an element's largest
+// difference dm at [2^14, 2^15) units; false where there is none.
+__device__ __forceinline__ bool tri_unit(double dm, unsigned &uh, double &unit, double &inv)
+{
+    const int ex = (int)((__double_as_longlong(dm) >> 52) & 0x7FF);   // dm >= 0
+    const bool ok = dm == 0.0 || (ex > 14 && ex < 2046 - 14);
+    uh = dm == 0.0 || !ok ? 1023u << 20 : (unsigned)(ex - 14) << 20;
+    unit = __hiloint2double((int)uh, 0);
+    inv = __hiloint2double((int)((2046u << 20) - uh), 0);
+    return ok;
+}
+
+// Where the elastic assembly writes.
+enum { AS_PAIRS = 0, AS_PACK32 = 1, AS_TRI = 2 };
+struct as_out {
+    double *K;                   // AS_PAIRS: column pairs; AS_TRI: the triangle
+    unsigned *diff, *unit;       // AS_TRI
+    int *bad;                    // AS_TRI: set where an entry does not come back exactly
+    float *hi, *lo;              // AS_PACK32
+    double *dg;                  // AS_PACK32, AS_TRI: element diagonals
+};
+
+// One wavefront per workgroup and element.  The row's NT entries are
+// accumulated in registers, Gauss point by Gauss point: a point costs its 3 NOD
+// global derivatives, read from LDS as broadcasts, once for all columns (a
+// column-by-column evaluation read every derivative for every entry and kept
+// B^T D of all 8 points in registers instead).  Bound by the FP64 products
+// and sums, which the reference's rounding keeps apart: 21 per node and point,
+// 5.5 ms for 1M hex20 elements.  The LDS of the geometry is reused to hand the
+// upper triangle from the lanes that hold it to those that write it.
+template <int NOD, int MODE>
+__global__ __launch_bounds__(64, NOD == 20 ? 2 : 4) void k_assemble_elastic(
+    const double *__restrict__ g_coord, const double *__restrict__ e_elem, double v2, double vv,
+    double den, double e0, as_out O)
+{
+    constexpr int NT = 3 * NOD, H = NT / 2, LOW = H * (H - 1), PAIRS = H * (H + 1);
+    constexpr size_t XCH = sizeof(double2) * (MODE == AS_TRI ? LOW : MODE == AS_PACK32 ? PAIRS : 1);
+    constexpr size_t GEO = sizeof(ElemLds<NOD>);
+    __shared__ __attribute__((aligned(16))) unsigned char raw[GEO > XCH ? GEO : XCH];
+    ElemLds<NOD> &L = *reinterpret_cast<ElemLds<NOD> *>(raw);
+    const int lane = threadIdx.x;
+    const long e = blockIdx.x;
+    element_geometry<NOD>(L, g_coord + e * (NOD * 3), lane, true);
     // DEEMAT: dee = dee0 * (e / (2(1+v)vv)) with dee0 = 1 on the normal
     // diagonal, v2 off it, vv on the shear diagonal.
     const double f = (e_elem ? e_elem[e] : e0) / den;
     const double D11 = 1.0 * f, D12 = v2 * f, D44 = vv * f;
-    const int a = lane / 3, ci = lane - 3 * (lane / 3);
-    double bt[8][6];
+    const int i = lane < NT ? lane : NT - 1;
+    const bool on = lane < NT;
+    const int a = i / 3, ci = i - 3 * a;
+    double k[NT];
 #pragma unroll
+    for (int j = 0; j < NT; ++j) k[j] = 0.0;
+#pragma unroll 1
     for (int g = 0; g < 8; ++g) {
-        const double dx = L.deriv[g][0][a], dy = L.deriv[g][1][a], dz = L.deriv[g][2][a];
-        if (ci == 0) {
-            bt[g][0] = dx * D11; bt[g][1] = dx * D12; bt[g][2] = dx * D12;
-            bt[g][3] = dy * D44; bt[g][4] = 0.0;      bt[g][5] = dz * D44;
-        } else if (ci == 1) {
-            bt[g][0] = dy * D12; bt[g][1] = dy * D11; bt[g][2] = dy * D12;
-            bt[g][3] = dx * D44; bt[g][4] = dz * D44; bt[g][5] = 0.0;
-        } else {
-            bt[g][0] = dz * D12; bt[g][1] = dz * D12; bt[g][2] = dz * D11;
-            bt[g][3] = 0.0;      bt[g][4] = dy * D44; bt[g][5] = dx * D44;
+        const double ax = L.deriv[g][0][a], ay = L.deriv[g][1][a], az = L.deriv[g][2][a];
+        const double det = L.dw[g];
+        // row i of B^T D at this point
+        const double an = ci == 0 ? ax : ci == 1 ? ay : az;
+        const double t0 = an * (ci == 0 ? D11 : D12), t1 = an * (ci == 1 ? D11 : D12), t2 = an * (ci == 2 ? D11 : D12);
+        const double t3 = ci == 0 ? ay * D44 : ci == 1 ? ax * D44 : 0.0;
+        const double t4 = ci == 0 ? 0.0 : ci == 1 ? az * D44 : ay * D44;
+        const double t5 = ci == 0 ? az * D44 : ci == 1 ? 0.0 : ax * D44;
+#pragma unroll
+        for (int b = 0; b < NOD; ++b) {
+            const double dx = L.deriv[g][0][b], dy = L.deriv[g][1][b], dz = L.deriv[g][2][b];
+            const double sx = (t0 * dx + t3 * dy) + t5 * dz;   // column x dof of node b
+            const double sy = (t1 * dy + t3 * dx) + t4 * dz;   // column y dof
+            const double sz = (t2 * dz + t4 * dy) + t5 * dx;   // column z dof
+            k[3 * b] = k[3 * b] + sx * det;
+            k[3 * b + 1] = k[3 * b + 1] + sy * det;
+            k[3 * b + 2] = k[3 * b + 2] + sz * det;
         }
     }
-    // Two nodes (6 columns = 3 column pairs) per step so that every store
-    // is one 16-byte column pair of the FP64 pair layout.
-    double2 *Kp = reinterpret_cast<double2 *>(K + e * (long)(NTOT * NTOT)) + lane;
-    for (int bb = 0; bb < NOD / 2; ++bb) {
-        double o[6];
+    __syncthreads();   // the derivatives' LDS is free
+    if constexpr (MODE == AS_PAIRS) {
+        double2 *Kp = reinterpret_cast<double2 *>(O.K + e * (long)(NT * NT)) + i;
+        if (on)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int b = 2 * bb + h;
-            double o0 = 0.0, o1 = 0.0, o2 = 0.0;
+            for (int s = 0; s < H; ++s) Kp[s * NT] = make_double2(k[2 * s], k[2 * s + 1]);
+    } else if constexpr (MODE == AS_PACK32) {
+        // the upper triangle through LDS (as column pairs), so that every lane
+        // writes its row's packed entries K(i, i+d mod NT) as whole quads
+        double2 *X = reinterpret_cast<double2 *>(raw);
 #pragma unroll
-            for (int g = 0; g < 8; ++g) {
-                const double dx = L.deriv[g][0][b], dy = L.deriv[g][1][b], dz = L.deriv[g][2][b];
-                const double det = L.dw[g];
-                const double *t = bt[g];
-                const double sx = (t[0] * dx + t[3] * dy) + t[5] * dz;   // column x dof of node b
-                const double sy = (t[1] * dy + t[3] * dx) + t[4] * dz;   // column y dof
-                const double sz = (t[2] * dz + t[4] * dy) + t[5] * dx;   // column z dof
-                o0 = o0 + sx * det;
-                o1 = o1 + sy * det;
-                o2 = o2 + sz * det;
+        for (int s = 0; s < H; ++s)
+            if (on && i <= 2 * s + 1) X[pf_tri_pair(s, i)] = make_double2(k[2 * s], k[2 * s + 1]);
+        __syncthreads();
+        const double *x = reinterpret_cast<const double *>(raw);
+        auto entry = [&](int d) {   // K(i, i + d mod NT) from the upper triangle
+            int j = i + d;
+            if (j >= NT) j -= NT;
+            const int r = i < j ? i : j, q = i < j ? j : i;
+            return x[2 * pf_tri_pair(q >> 1, r) + (q & 1)];
+        };
+        constexpr int Q = pf_sym_quads(NT), RM = pf_sym_rem(NT);
+        float *hi = O.hi + e * pf_sym_per(NT), *lo = O.lo + e * pf_sym_per(NT);
+        if (on) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                float4 h, l;
+                float *hp = &h.x, *lp = &l.x;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const double v = entry(4 * q + c);
+                    hp[c] = (float)v;
+                    lp[c] = (float)(v - (double)hp[c]);
+                }
+                reinterpret_cast<float4 *>(hi)[q * NT + i] = h;
+                reinterpret_cast<float4 *>(lo)[q * NT + i] = l;
             }
-            o[3 * h + 0] = o0;
-            o[3 * h + 1] = o1;
-            o[3 * h + 2] = o2;
-        }
-        if constexpr (S32) {
 #pragma unroll
-            for (int q = 0; q < 6; ++q) store_packed<NTOT>(e, lane, 6 * bb + q, o[q], hi, lo, dg);
-        } else {
-#pragma unroll
-            for (int q = 0; q < 3; ++q) Kp[(3 * bb + q) * NTOT] = make_double2(o[2 * q], o[2 * q + 1]);
+            for (int c = 0; c < RM; ++c) {
+                const double v = entry(4 * Q + c);
+                const float h = (float)v;
+                hi[4 * Q * NT + RM * i + c] = h;
+                lo[4 * Q * NT + RM * i + c] = (float)(v - (double)h);
+            }
+            if (i < H) {
+                const double v = entry(H);
+                const float h = (float)v;
+                hi[H * NT + i] = h;
+                lo[H * NT + i] = (float)(v - (double)h);
+            }
+            O.dg[e * NT + i] = entry(0);
         }
+        zero_padding<NT>(e, lane, O.hi, O.lo);
+    } else {
+        // the triangle and its differences: lane j > 2t+1 receives the row
+        // pair t's entries of column j (the product's exchange)
+        double2 *Te = reinterpret_cast<double2 *>(O.K) + e * PAIRS;
+        double *lw = reinterpret_cast<double *>(raw);
+        const int t = i >> 1, o = 2 * (t * (NT - 3 - t) - 2) + (i & 1);
+        bool fail = false;
+        double diag = 0.0;
+#pragma unroll
+        for (int s = 0; s < H; ++s) {
+            double own = i & 1 ? k[2 * s + 1] : k[2 * s];
+            asm volatile("" : "+v"(own));   // a select per pair: not an indexed read of k, which would move it to memory
+            diag = t == s ? own : diag;
+            if (on && i <= 2 * s + 1) {
+                Te[pf_tri_pair(s, i)] = make_double2(k[2 * s], k[2 * s + 1]);
+            }
+            if (s && on && i < 2 * s) {
+                lw[o + 4 * s] = k[2 * s];
+                lw[o + 4 * s + 2] = k[2 * s + 1];
+            }
+        }
+        if (on) O.dg[e * NT + i] = diag;
+        __syncthreads();
+        const double2 *lr = reinterpret_cast<const double2 *>(raw);
+        double dm = 0.0;
+#pragma unroll
+        for (int s = 0; s < H - 1; ++s) {
+            if (!(on && i > 2 * s + 1)) continue;
+            const double2 w = lr[s * (NT - 3 - s) + i - 2];
+            const double d0 = __dsub_rn(k[2 * s], w.x), d1 = __dsub_rn(k[2 * s + 1], w.y);
+            // with the check of the code below: the entry comes back exactly
+            // (an infinite or undefined one does not)
+            fail |= __dadd_rn(w.x, d0) != k[2 * s] || __dadd_rn(w.y, d1) != k[2 * s + 1];
+            k[2 * s] = d0;
+            k[2 * s + 1] = d1;
+            dm = fmax(dm, fmax(fabs(d0), fabs(d1)));
+        }
+        dm = wave_max(dm);
+        dm = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(dm)),
+                              __builtin_amdgcn_readfirstlane(__double2loint(dm)));
+        unsigned uh;
+        double unit, inv;
+        fail |= !tri_unit(dm, uh, unit, inv);
+        unsigned *De = O.diff + e * LOW + i;
+#pragma unroll
+        for (int s = 0; s < H - 1; ++s) {
+            if (!(on && i > 2 * s + 1)) continue;
+            union { unsigned u; _Float16 h[2]; } c;
+            c.h[0] = (_Float16)(float)(k[2 * s] * inv);
+            c.h[1] = (_Float16)(float)(k[2 * s + 1] * inv);
+            fail |= (double)c.h[0] * unit != k[2 * s] || (double)c.h[1] * unit != k[2 * s + 1];
+            De[pf_tri_diff(NT, s, 0)] = c.u;
+        }
+        if (lane == 0) O.unit[e] = uh;
+        if (fail) *O.bad = 1;
     }
 }
 
 // p123: kc{x,y,z} = sum_g d{x,y,z}_a d{x,y,z}_b det w; storkc = kx*kcx + ky*kcy + kz*kcz.
+// Rows and columns enter every product alike, so K(a,b) = K(b,a) bit for bit
+// and FP64 storage is the packed triangle without differences.
 template <bool S32>
 __global__ __launch_bounds__(64 * WAVES) void k_assemble_laplace8(
     const double *__restrict__ g_coord, const double *__restrict__ k_elem, double kx, double ky,
-    double kz, double *__restrict__ K, float *__restrict__ hi, float *__restrict__ lo, double *__restrict__ dg,
+    double kz, double *__restrict__ T, float *__restrict__ hi, float *__restrict__ lo, double *__restrict__ dg,
     int nels)
 {
     __shared__ ElemLds<8> lds[WAVES];
@@ -236,7 +375,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_assemble_laplace8(
     const double s = k_elem ? k_elem[e] : 1.0;
     const double k = cx * (kx * s) + cy * (ky * s) + cz * (kz * s);
     if constexpr (S32) store_packed<8>(e, a, b, k, hi, lo, dg);
-    else K[pf_idx_pair(e, 8, a, b)] = k;
+    else if (a <= (b | 1)) T[2 * (e * pf_tri_pairs(8) + pf_tri_pair(b >> 1, a)) + (b & 1)] = k;
 }
 
 // p124's element loop (src/programs/5th_ed/p124/p124.f90:73-86) on an
@@ -250,12 +389,12 @@ __global__ __launch_bounds__(64 * WAVES) void k_assemble_laplace8(
 // others add exact zeros), the weights of SAMPLE are 1.
 __global__ __launch_bounds__(64 * WAVES) void k_assemble_transient8(
     const double *__restrict__ g_coord, const double *__restrict__ prop, const int *__restrict__ etype,
-    double theta, double dtim, double *__restrict__ Ka, double *__restrict__ Kb, int nels)
+    double theta, double dtim, double *__restrict__ Ka, double *__restrict__ Kb, long first, long end)
 {
     __shared__ ElemLds<8> lds[WAVES];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long e = (long)blockIdx.x * WAVES + wave;
-    const bool valid = e < nels;
+    const long e = first + (long)blockIdx.x * WAVES + wave;
+    const bool valid = e < end;
     ElemLds<8> &L = lds[wave];
     element_geometry<8>(L, g_coord + (valid ? e : 0) * 24, lane, valid);
     if (!valid) return;
@@ -267,13 +406,12 @@ __global__ __launch_bounds__(64 * WAVES) void k_assemble_transient8(
     constexpr int sx[8] = {-1, -1, 1, 1, -1, -1, 1, 1};
     constexpr int sy[8] = {-1, -1, -1, -1, 1, 1, 1, 1};
     constexpr int sz[8] = {-1, 1, 1, -1, -1, 1, 1, -1};
-    constexpr int gs[8][3] = {{1, 1, 1}, {1, 1, -1}, {1, -1, 1}, {1, -1, -1},
-                              {-1, 1, 1}, {-1, -1, 1}, {-1, 1, -1}, {-1, -1, -1}};
-    const double r3 = 1.0 / sqrt(3.0);
+    constexpr double r3 = gauss_r3;
     double kc = 0.0, pm = 0.0;
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
-        const double xi = gs[g][0] > 0 ? r3 : -r3, eta = gs[g][1] > 0 ? r3 : -r3, zeta = gs[g][2] > 0 ? r3 : -r3;
+        const double xi = gauss_sign[g][0] > 0 ? r3 : -r3, eta = gauss_sign[g][1] > 0 ? r3 : -r3,
+                     zeta = gauss_sign[g][2] > 0 ? r3 : -r3;
         const double xim = 1.0 - xi, etam = 1.0 - eta, zetam = 1.0 - zeta;
         const double xip = xi + 1.0, etap = eta + 1.0, zetap = zeta + 1.0;
         const double fa = 0.125 * (sx[a] < 0 ? xim : xip) * (sy[a] < 0 ? etam : etap) * (sz[a] < 0 ? zetam : zetap);
@@ -285,7 +423,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_assemble_transient8(
         kc = kc + t * det * 1.0;
         pm = pm + fa * fb * det * 1.0 * rho * cp;
     }
-    Ka[pf_idx_pair(e, 8, a, b)] = pm + kc * theta * dtim;
+    Ka[pf_idx_pair(e - first, 8, a, b)] = pm + kc * theta * dtim;
     Kb[pf_idx_pair(e, 8, a, b)] = pm - kc * (1.0 - theta) * dtim;
 }
 
@@ -336,17 +474,75 @@ __global__ void k_from_colmajor(const double *__restrict__ src, double *__restri
     }
 }
 
-// internal layout -> storkm_pp chunk (FP64 pairs, or packed symmetric hi + lo).
-__global__ void k_to_colmajor(const double *__restrict__ K, const float *__restrict__ hi,
-                              const float *__restrict__ lo, double *__restrict__ dst, int nt, long e0, long nel,
-                              long kstride)
+// FP64 matrices (column pairs, or column-major) -> packed triangle.  One lane
+// group per element (lane = row), the whole matrix in LDS; every entry below
+// the diagonal is reconstructed as the product will and compared.  Bound by
+// the reads of src, which a bounded chunk leaves in the last-level cache.
+template <int NT, bool COLMAJOR>
+__global__ __launch_bounds__(64) void k_tri_pack(const double *__restrict__ src, double *__restrict__ T,
+                                                unsigned *__restrict__ diff, unsigned *__restrict__ unit, long e0,
+                                                long nel, int *__restrict__ bad)
+{
+    constexpr int W = NT > 32 ? 64 : (NT > 16 ? 32 : 8), EPW = 64 / W, H = NT / 2, PITCH = NT + 1;
+    __shared__ double m[EPW][NT * PITCH];
+    const int lane = threadIdx.x & 63, sub = lane / W, i = lane % W;
+    const long el = (long)blockIdx.x * EPW + sub;
+    const bool on = el < nel && i < NT;
+    double *M = m[sub];
+    const double *S = src + (el < nel ? el : 0) * (long)(NT * NT);
+    if (on) {
+#pragma unroll
+        for (int s = 0; s < H; ++s) {
+            if constexpr (COLMAJOR) {
+                M[i * PITCH + 2 * s] = S[2 * s * NT + i];
+                M[i * PITCH + 2 * s + 1] = S[(2 * s + 1) * NT + i];
+            } else {
+                const double2 v = reinterpret_cast<const double2 *>(S)[s * NT + i];
+                M[i * PITCH + 2 * s] = v.x;
+                M[i * PITCH + 2 * s + 1] = v.y;
+            }
+        }
+    }
+    __syncthreads();
+    // the largest difference of the element
+    double dm = 0.0;
+    if (on)
+        for (int j = 0; j < (i & ~1); ++j) dm = fmax(dm, fabs(__dsub_rn(M[i * PITCH + j], M[j * PITCH + i])));
+    for (int off = W / 2; off > 0; off >>= 1) dm = fmax(dm, __shfl_xor(dm, off, 64));
+    unsigned uh;
+    double un, inv;
+    bool fail = !tri_unit(dm, uh, un, inv) && on;
+    const long e = e0 + el;
+    if (on) {
+        double2 *Te = reinterpret_cast<double2 *>(T) + e * pf_tri_pairs(NT);
+        unsigned *De = diff + e * pf_tri_diffs(NT);
+        for (int s = 0; s < H; ++s) {
+            const double a = M[i * PITCH + 2 * s], b = M[i * PITCH + 2 * s + 1];
+            if (i <= 2 * s + 1) {
+                Te[pf_tri_pair(s, i)] = make_double2(a, b);
+                continue;
+            }
+            const double ua = M[2 * s * PITCH + i], ub = M[(2 * s + 1) * PITCH + i];
+            union { unsigned u; _Float16 h[2]; } w;
+            w.h[0] = tri_code(a, ua, inv, un, fail);
+            w.h[1] = tri_code(b, ub, inv, un, fail);
+            De[pf_tri_diff(NT, s, i)] = w.u;
+        }
+        if (i == 0) unit[e] = uh;
+    }
+    if (fail) *bad = 1;
+}
+
+// internal layout -> storkm_pp chunk (FP64, or packed symmetric hi + lo).
+__global__ void k_to_colmajor(pf_f64_view V, const float *__restrict__ hi, const float *__restrict__ lo,
+                              double *__restrict__ dst, int nt, long e0, long nel)
 {
     const long nn = (long)nt * nt, n = nel * nn;
     for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
         const long el = q / nn, w = q - el * nn;
         const int j = (int)(w / nt), i = (int)(w - (long)j * nt);
-        if (K) {
-            dst[q] = K[pf_idx_pair((e0 + el) * kstride, nt, i, j)];
+        if (V.K || V.T) {
+            dst[q] = pf_f64_entry(V, e0 + el, nt, i, j);
         } else {
             const long t = pf_idx_sym_ij(e0 + el, nt, i, j);
             dst[q] = (double)hi[t] + (double)lo[t];
@@ -356,8 +552,8 @@ __global__ void k_to_colmajor(const double *__restrict__ K, const float *__restr
 
 // Assembled diagonal: diag(q) = sum over the slots of q, ascending element,
 // of storkm(i,i,e) (p121.f90:65-69 then SCATTER).  diag has a leading 0 slot.
-__global__ void k_diag(const int *__restrict__ ptr, const int *__restrict__ slot, const double *__restrict__ K,
-                       int ntot, long kstride, double *__restrict__ diag, int neq)
+__global__ void k_diag(const int *__restrict__ ptr, const int *__restrict__ slot, pf_f64_view V, int ntot,
+                       double *__restrict__ diag, int neq)
 {
     for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < neq; q += gridDim.x * blockDim.x) {
         double s = 0.0;
@@ -365,7 +561,7 @@ __global__ void k_diag(const int *__restrict__ ptr, const int *__restrict__ slot
             const long sl = slot[k];
             const long e = sl / ntot;
             const int i = (int)(sl - e * ntot);
-            s = __dadd_rn(s, K[pf_idx_pair(e * kstride, ntot, i, i)]);
+            s = __dadd_rn(s, pf_f64_entry(V, e, ntot, i, i));
         }
         diag[q + 1] = s;
     }
@@ -387,30 +583,30 @@ __global__ void k_diag_elem(const int *__restrict__ ptr, const int *__restrict__
 
 }  // namespace
 
-// FP64 storage writes K64; FP32 storage writes K32hi/K32lo and the element
-// diagonals into dg (ntot*nels doubles).
-int pf_launch_assemble_elastic(pf_ctx *c, double v2, double vv, double den, double e0, const double *e_elem,
-                               double *dg)
+// FP32 storage writes K32hi/K32lo, FP64 storage the triangle (*bad set where
+// it does not hold), both with the element diagonals in dg (ntot*nels
+// doubles); FP64 storage without a triangle writes K64.
+int pf_launch_assemble_elastic(pf_ctx *c, double v2, double vv, double den, double e, const double *e_elem,
+                               double *dg, int *bad)
 {
-    const int grid = (c->nels + WAVES - 1) / WAVES;
-    const bool s32 = c->store == PF_STORE_FP32;
-    if (s32 && (!c->K32hi || !c->K32lo || !dg)) return PF_ERR_STATE;
-    if (c->nod == 20 && s32)
-        hipLaunchKernelGGL((k_assemble_elastic<20, true>), dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord,
-                           e_elem, v2, vv, den, e0, (double *)nullptr, c->K32hi, c->K32lo, dg, c->nels);
-    else if (c->nod == 20)
-        hipLaunchKernelGGL((k_assemble_elastic<20, false>), dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord,
-                           e_elem, v2, vv, den, e0, c->K64, (float *)nullptr, (float *)nullptr, (double *)nullptr,
-                           c->nels);
-    else if (c->nod == 8 && s32)
-        hipLaunchKernelGGL((k_assemble_elastic<8, true>), dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord,
-                           e_elem, v2, vv, den, e0, (double *)nullptr, c->K32hi, c->K32lo, dg, c->nels);
-    else if (c->nod == 8)
-        hipLaunchKernelGGL((k_assemble_elastic<8, false>), dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord,
-                           e_elem, v2, vv, den, e0, c->K64, (float *)nullptr, (float *)nullptr, (double *)nullptr,
-                           c->nels);
-    else
+    const bool s32 = c->store == PF_STORE_FP32, tri = !s32 && c->T64;
+    if (s32 ? !c->K32hi || !c->K32lo || !dg : tri ? !c->T64d || !c->T64u || !bad || !dg : !c->K64) return PF_ERR_STATE;
+    const as_out O{tri ? c->T64 : c->K64, c->T64d, c->T64u, bad, c->K32hi, c->K32lo, dg};
+    const dim3 grid(c->nels), blk(64);
+#define PF_AS(NOD, MODE)                                                                                           \
+    hipLaunchKernelGGL((k_assemble_elastic<NOD, MODE>), grid, blk, 0, c->stream, c->g_coord, e_elem, v2, vv, den, e, O)
+    if (c->nod == 20) {
+        if (s32) PF_AS(20, AS_PACK32);
+        else if (tri) PF_AS(20, AS_TRI);
+        else PF_AS(20, AS_PAIRS);
+    } else if (c->nod == 8) {
+        if (s32) PF_AS(8, AS_PACK32);
+        else if (tri) PF_AS(8, AS_TRI);
+        else PF_AS(8, AS_PAIRS);
+    } else {
         return PF_ERR_ARG;
+    }
+#undef PF_AS
     PF_HIP(hipGetLastError());
     return PF_OK;
 }
@@ -424,9 +620,34 @@ int pf_launch_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const
         hipLaunchKernelGGL(k_assemble_laplace8<true>, dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord,
                            k_elem, kx, ky, kz, (double *)nullptr, c->K32hi, c->K32lo, dg, c->nels);
     } else {
+        if (!c->T64) return PF_ERR_STATE;
         hipLaunchKernelGGL(k_assemble_laplace8<false>, dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord,
-                           k_elem, kx, ky, kz, c->K64, (float *)nullptr, (float *)nullptr, (double *)nullptr,
+                           k_elem, kx, ky, kz, c->T64, (float *)nullptr, (float *)nullptr, (double *)nullptr,
                            c->nels);
+    }
+    PF_HIP(hipGetLastError());
+    return PF_OK;
+}
+
+template <int NT>
+static void launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad)
+{
+    constexpr int EPW = NT > 32 ? 1 : (NT > 16 ? 2 : 8);
+    const dim3 grid((unsigned)((nel + EPW - 1) / EPW)), blk(64);
+    if (colmajor)
+        hipLaunchKernelGGL((k_tri_pack<NT, true>), grid, blk, 0, c->stream, src, c->T64, c->T64d, c->T64u, e0, nel, bad);
+    else
+        hipLaunchKernelGGL((k_tri_pack<NT, false>), grid, blk, 0, c->stream, src, c->T64, c->T64d, c->T64u, e0, nel, bad);
+}
+
+int pf_launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad)
+{
+    if (!c->T64 || !c->T64d || !c->T64u) return PF_ERR_STATE;
+    switch (c->ntot) {
+    case 60: launch_tri_pack<60>(c, src, colmajor, e0, nel, bad); break;
+    case 24: launch_tri_pack<24>(c, src, colmajor, e0, nel, bad); break;
+    case 8: launch_tri_pack<8>(c, src, colmajor, e0, nel, bad); break;
+    default: return PF_ERR_ARG;
     }
     PF_HIP(hipGetLastError());
     return PF_OK;
@@ -440,12 +661,12 @@ int pf_launch_diag_elem(pf_ctx *c, const double *dg, double *diag)
     return PF_OK;
 }
 
-int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const double *prop, const int *etype)
+int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const double *prop, const int *etype,
+                                 double *Ka, long e0, long nel)
 {
     if (c->nod != 8) return PF_ERR_ARG;
-    const int grid = (c->nels + WAVES - 1) / WAVES;
-    hipLaunchKernelGGL(k_assemble_transient8, dim3(grid), dim3(64 * WAVES), 0, c->stream, c->g_coord, prop, etype,
-                       theta, dtim, c->K64, c->K64b, c->nels);
+    hipLaunchKernelGGL(k_assemble_transient8, dim3((unsigned)((nel + WAVES - 1) / WAVES)), dim3(64 * WAVES), 0,
+                       c->stream, c->g_coord, prop, etype, theta, dtim, Ka, c->K64b, e0, e0 + nel);
     PF_HIP(hipGetLastError());
     return PF_OK;
 }
@@ -467,8 +688,8 @@ int pf_launch_from_colmajor(pf_ctx *c, const double *src, long e0, long nel)
 
 int pf_launch_to_colmajor(pf_ctx *c, double *dst, long e0, long nel)
 {
-    hipLaunchKernelGGL(k_to_colmajor, dim3(8192), dim3(256), 0, c->stream, c->K64, c->K32hi, c->K32lo, dst,
-                       c->ntot, e0, nel, pf_k64_estride(c));
+    hipLaunchKernelGGL(k_to_colmajor, dim3(8192), dim3(256), 0, c->stream, pf_f64(c), c->K32hi, c->K32lo, dst,
+                       c->ntot, e0, nel);
     PF_HIP(hipGetLastError());
     return PF_OK;
 }
@@ -476,8 +697,8 @@ int pf_launch_to_colmajor(pf_ctx *c, double *dst, long e0, long nel)
 int pf_launch_diag(pf_ctx *c, double *diag)
 {
     const int grid = (c->neq + 255) / 256 < 8192 ? (c->neq + 255) / 256 : 8192;
-    hipLaunchKernelGGL(k_diag, dim3(grid), dim3(256), 0, c->stream, c->csr_ptr, c->csr_slot, c->K64, c->ntot,
-                       pf_k64_estride(c), diag, c->neq);
+    hipLaunchKernelGGL(k_diag, dim3(grid), dim3(256), 0, c->stream, c->csr_ptr, c->csr_slot, pf_f64(c), c->ntot,
+                       diag, c->neq);
     PF_HIP(hipGetLastError());
     return PF_OK;
 }

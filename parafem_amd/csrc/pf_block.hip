@@ -62,9 +62,9 @@ template <int NT> struct Tiles {
     static constexpr int PER = MT * KQ * 256;      // stored values per element
 };
 
-// K64 (column pairs) -> A-operand tiles [e][mt][kq][lane][j], zero padded.
+// FP64 matrices -> A-operand tiles [e][mt][kq][lane][j], zero padded.
 template <int NT, typename T>
-__global__ void k_blk_pack(const double *__restrict__ K, long kstride, T *__restrict__ Kt, long nels)
+__global__ void k_blk_pack(pf_f64_view V, T *__restrict__ Kt, long nels)
 {
     using TL = Tiles<NT>;
     const long n = nels * TL::PER;
@@ -73,7 +73,7 @@ __global__ void k_blk_pack(const double *__restrict__ K, long kstride, T *__rest
         const int w = (int)(q - e * TL::PER);
         const int j = w & 3, l = (w >> 2) & 63, kq = (w >> 8) % TL::KQ, mt = (w >> 8) / TL::KQ;
         const int row = 16 * mt + (l & 15), col = 4 * (4 * kq + j) + (l >> 4);
-        Kt[q] = (row < NT && col < NT) ? (T)K[pf_idx_pair(e * kstride, NT, row, col)] : (T)0;
+        Kt[q] = (row < NT && col < NT) ? (T)pf_f64_entry(V, e, NT, row, col) : (T)0;
     }
 }
 
@@ -145,7 +145,7 @@ template <int NT> struct SymTiles {
 };
 
 template <int NT>
-__global__ void k_blk_pack_sym(const double *__restrict__ K, long kstride, float *__restrict__ Ks, long nels)
+__global__ void k_blk_pack_sym(pf_f64_view V, float *__restrict__ Ks, long nels)
 {
     using ST = SymTiles<NT>;
     const long n = nels * ST::PER;
@@ -161,7 +161,7 @@ __global__ void k_blk_pack_sym(const double *__restrict__ K, long kstride, float
         const int b = a + t;
         const int row = 16 * a + (l & 15), col = 16 * b + 4 * j + (l >> 4);
         const int lo = row < col ? row : col, hi = row < col ? col : row;
-        Ks[q] = (hi < NT) ? (float)K[pf_idx_pair(e * kstride, NT, lo, hi)] : 0.0f;
+        Ks[q] = (hi < NT) ? (float)pf_f64_entry(V, e, NT, lo, hi) : 0.0f;
     }
 }
 
@@ -638,31 +638,30 @@ int blk_sym_per(int nt)
 // Allocate (once per problem) and pack the element matrices.
 int blk_setup(pf_ctx *c, bool need32)
 {
-    if (!c->K64) return PF_ERR_ARG;            // needs FP64 element matrices
+    if (!pf_has_f64(c)) return PF_ERR_ARG;     // needs FP64 element matrices
     if (!c->blk) c->blk = new pf_block();
     pf_block *b = c->blk;
     const size_t nv = (size_t)(c->neq + 1) * PF_BLK;
     const size_t ns = (size_t)c->nels * c->ntot * PF_BLK;
     const long ke = c->k_shared ? 1 : c->nels;
     const size_t nt = (size_t)ke * blk_tiles_per(c->ntot);
-    const long ks = pf_k64_estride(c);
     int rc = PF_OK;
     if (!b->Kt64) {
         rc = blk_alloc(c, b->Kt64, nt);
         if (rc) return rc;
         switch (c->ntot) {
-        case 60: hipLaunchKernelGGL((k_blk_pack<60, double>), dim3(4096), dim3(256), 0, c->stream, c->K64, ks, b->Kt64, ke); break;
-        case 24: hipLaunchKernelGGL((k_blk_pack<24, double>), dim3(4096), dim3(256), 0, c->stream, c->K64, ks, b->Kt64, ke); break;
-        default: hipLaunchKernelGGL((k_blk_pack<8, double>), dim3(4096), dim3(256), 0, c->stream, c->K64, ks, b->Kt64, ke); break;
+        case 60: hipLaunchKernelGGL((k_blk_pack<60, double>), dim3(4096), dim3(256), 0, c->stream, pf_f64(c), b->Kt64, ke); break;
+        case 24: hipLaunchKernelGGL((k_blk_pack<24, double>), dim3(4096), dim3(256), 0, c->stream, pf_f64(c), b->Kt64, ke); break;
+        default: hipLaunchKernelGGL((k_blk_pack<8, double>), dim3(4096), dim3(256), 0, c->stream, pf_f64(c), b->Kt64, ke); break;
         }
     }
     if (need32 && !b->Kt32) {
         rc = blk_alloc(c, b->Kt32, (size_t)ke * blk_sym_per(c->ntot));
         if (rc) return rc;
         switch (c->ntot) {
-        case 60: hipLaunchKernelGGL(k_blk_pack_sym<60>, dim3(4096), dim3(256), 0, c->stream, c->K64, ks, b->Kt32, ke); break;
-        case 24: hipLaunchKernelGGL(k_blk_pack_sym<24>, dim3(4096), dim3(256), 0, c->stream, c->K64, ks, b->Kt32, ke); break;
-        default: hipLaunchKernelGGL(k_blk_pack_sym<8>, dim3(4096), dim3(256), 0, c->stream, c->K64, ks, b->Kt32, ke); break;
+        case 60: hipLaunchKernelGGL(k_blk_pack_sym<60>, dim3(4096), dim3(256), 0, c->stream, pf_f64(c), b->Kt32, ke); break;
+        case 24: hipLaunchKernelGGL(k_blk_pack_sym<24>, dim3(4096), dim3(256), 0, c->stream, pf_f64(c), b->Kt32, ke); break;
+        default: hipLaunchKernelGGL(k_blk_pack_sym<8>, dim3(4096), dim3(256), 0, c->stream, pf_f64(c), b->Kt32, ke); break;
         }
     }
     PF_HIP(hipGetLastError());

@@ -152,6 +152,9 @@ static void free_matrices(pf_ctx *c)
     pf_block_free(c);
     const size_t ns = (size_t)pf_sym_per(c->ntot) * c->nels;
     free_arr(c, c->K64, pf_k64_count(c));
+    free_arr(c, c->T64, (size_t)2 * pf_tri_pairs(c->ntot) * c->nels);
+    free_arr(c, c->T64d, (size_t)pf_tri_diffs(c->ntot) * c->nels);
+    free_arr(c, c->T64u, (size_t)c->nels);
     free_arr(c, c->K64b, (size_t)c->ntot * c->ntot * c->nels);
     free_arr(c, c->K32hi, ns);
     free_arr(c, c->K32lo, ns);
@@ -473,15 +476,73 @@ static int alloc_k64(pf_ctx *c, int store, bool shared = false)
     return pf_alloc(c, (void **)&c->K64, pf_k64_count(c) * sizeof(double));
 }
 
-// Storage for an assembly on the device: K64 for FP64, the packed hi/lo
-// matrices (and the FP32 products' utemp32) for FP32 -- the FP32 assembly
-// writes them directly, with no FP64 copy.
-static int alloc_assembly(pf_ctx *c, int store)
+// FP64 storage as the packed triangle, with or without differences.
+static int alloc_tri(pf_ctx *c, bool diffs)
 {
-    if (store == PF_STORE_FP64) return alloc_k64(c, store);
-    if (store != PF_STORE_FP32) return PF_ERR_ARG;
     free_matrices(c);
-    c->store = store;
+    c->store = PF_STORE_FP64;
+    c->k_shared = false;
+    int rc = pf_alloc(c, (void **)&c->T64, (size_t)2 * pf_tri_pairs(c->ntot) * c->nels * sizeof(double));
+    if (!rc && diffs) rc = pf_alloc(c, (void **)&c->T64d, (size_t)pf_tri_diffs(c->ntot) * c->nels * sizeof(unsigned));
+    if (!rc && diffs) rc = pf_alloc(c, (void **)&c->T64u, (size_t)c->nels * sizeof(unsigned));
+    return rc;
+}
+
+// Elements formed and packed at a time: a chunk of whole matrices of 128 MB
+// stays in the last-level cache (256 MB) between the two kernels.
+static long pack_elems(const pf_ctx *c)
+{
+    const long per = (long)c->ntot * c->ntot * (long)sizeof(double), n = (128L << 20) / per;
+    return n < c->nels ? n : c->nels;
+}
+
+// The flag a packing kernel sets where an entry does not come back exactly: a
+// word of pinned memory, cleared here (nothing of the context is in flight
+// during set-up), so that it costs neither a fill nor a copy.
+static int *tri_flag(pf_ctx *c)
+{
+    int *bad = reinterpret_cast<int *>(c->scalar_host + 63);
+    *bad = 0;
+    return bad;
+}
+
+}  // extern "C"
+
+// FP64 matrices formed chunk by chunk by form(stage, e0, nel) -- into a
+// bounded staging buffer, as column pairs or column-major -- and packed into
+// the triangle.  *whole is set, and nothing kept, where an entry does not
+// come back exactly: the caller then stores whole matrices.
+template <class F>
+static int form_and_pack(pf_ctx *c, bool colmajor, bool *whole, F form)
+{
+    *whole = false;
+    int rc = alloc_tri(c, true);
+    const long chunk = pack_elems(c);
+    const size_t sb = (size_t)chunk * c->ntot * c->ntot * sizeof(double);
+    double *stage = nullptr;
+    int *bad = tri_flag(c);
+    if (!rc) rc = pf_alloc(c, (void **)&stage, sb);
+    for (long e0 = 0; !rc && e0 < c->nels; e0 += chunk) {
+        const long nel = std::min(chunk, (long)c->nels - e0);
+        rc = form(stage, e0, nel);
+        if (!rc) rc = pf_launch_tri_pack(c, stage, colmajor, e0, nel, bad);
+    }
+    const hipError_t he = hipStreamSynchronize(c->stream);
+    if (!rc && he != hipSuccess) rc = pf_set_hip_error(he, "packing", __FILE__, __LINE__);
+    pf_free(c, stage, sb);
+    *whole = !rc && *bad;
+    if (rc || *whole) free_matrices(c);
+    return rc;
+}
+
+extern "C" {
+
+// Storage for an assembly straight into the packed FP32 hi/lo matrices (and
+// the FP32 products' utemp32), with no FP64 copy.
+static int alloc_direct32(pf_ctx *c)
+{
+    free_matrices(c);
+    c->store = PF_STORE_FP32;
     c->k_shared = false;
     const size_t ns = (size_t)pf_sym_per(c->ntot) * c->nels;
     int rc = pf_alloc(c, (void **)&c->K32hi, ns * sizeof(float));
@@ -490,9 +551,10 @@ static int alloc_assembly(pf_ctx *c, int store)
     return rc;
 }
 
-// After a direct FP32 assembly: the assembled diagonal from the element
-// diagonals dg the assembly wrote (the same sums as from FP64 matrices).
-static int finish_direct32(pf_ctx *c, const double *dg)
+// After an assembly that wrote the element diagonals into dg: the assembled
+// diagonal from them (the same sums as from the matrices, 8 bytes an entry
+// instead of a cache line: 100^3 hex20 0.1 ms against 0.9).
+static int finish_direct(pf_ctx *c, const double *dg)
 {
     const size_t nv = (size_t)c->neq + 1;
     int rc = pf_launch_diag_elem(c, dg, c->diag0);
@@ -507,7 +569,7 @@ static int finish_direct32(pf_ctx *c, const double *dg)
     return PF_OK;
 }
 
-// After a FP64 assembly or upload into K64: the assembled diagonal
+// After a FP64 assembly or upload: the assembled diagonal
 // (ascending element order, as SCATTER adds it) and, for FP32 storage, the
 // hi/lo split, after which the FP64 copy is released.
 static int finish_matrices(pf_ctx *c)
@@ -542,9 +604,9 @@ int pf_assemble_elastic(pf_ctx *c, double e, double v, const double *e_elem, int
     if (!c->g_coord || !c->g_g) return PF_ERR_STATE;
     if (c->ntot != 3 * c->nod) return PF_ERR_ARG;
     if (!(v > -1.0 && v < 0.5)) return PF_ERR_ARG;
+    if (store != PF_STORE_FP64 && store != PF_STORE_FP32) return PF_ERR_ARG;
     PF_HIP(hipSetDevice(c->device));
-    int rc = alloc_assembly(c, store);
-    if (rc) return rc;
+    int rc = PF_OK;
     double *ee = nullptr;
     if (e_elem) {
         rc = pf_alloc(c, (void **)&ee, sizeof(double) * c->nels);
@@ -556,15 +618,31 @@ int pf_assemble_elastic(pf_ctx *c, double e, double v, const double *e_elem, int
     const double v2 = v / (1.0 - v);
     const double vv = (1.0 - 2.0 * v) / (1.0 - v) * 0.5;
     const double den = 2.0 * (1.0 + v) * vv;
-    // FP32 storage: the element diagonals go to utemp (ntot*nels doubles,
-    // free until the PCG runs)
-    rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp);
+    // the element diagonals go to utemp (ntot*nels doubles, free until the PCG
+    // runs)
+    if (store == PF_STORE_FP32) {
+        rc = alloc_direct32(c);
+        if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp, nullptr);
+    } else {
+        rc = alloc_tri(c, true);
+        int *bad = tri_flag(c);
+        if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp, bad);
+        if (!rc) {
+            const hipError_t he = hipStreamSynchronize(c->stream);
+            if (he != hipSuccess) rc = pf_set_hip_error(he, "assembly", __FILE__, __LINE__);
+        }
+        if (!rc && *bad) {   // whole matrices
+            rc = alloc_k64(c, store);
+            if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, nullptr, nullptr);
+        }
+    }
     if (ee) {
         (void)hipStreamSynchronize(c->stream);
         pf_free(c, ee, sizeof(double) * c->nels);
     }
     if (rc) return rc;
-    return store == PF_STORE_FP32 ? finish_direct32(c, c->utemp) : finish_matrices(c);
+    // the element diagonals are in utemp; whole matrices hold their own
+    return c->K64 ? finish_matrices(c) : finish_direct(c, c->utemp);
 }
 
 int pf_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double *k_elem, int store)
@@ -573,7 +651,8 @@ int pf_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double
     if (!c->g_coord || !c->g_g) return PF_ERR_STATE;
     if (c->ntot != c->nod || c->nod != 8) return PF_ERR_ARG;
     PF_HIP(hipSetDevice(c->device));
-    int rc = alloc_assembly(c, store);
+    if (store != PF_STORE_FP64 && store != PF_STORE_FP32) return PF_ERR_ARG;
+    int rc = store == PF_STORE_FP32 ? alloc_direct32(c) : alloc_tri(c, false);
     if (rc) return rc;
     double *kk = nullptr;
     if (k_elem) {
@@ -587,7 +666,7 @@ int pf_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double
         pf_free(c, kk, sizeof(double) * c->nels);
     }
     if (rc) return rc;
-    return store == PF_STORE_FP32 ? finish_direct32(c, c->utemp) : finish_matrices(c);
+    return store == PF_STORE_FP32 ? finish_direct(c, c->utemp) : finish_matrices(c);
 }
 
 int pf_assemble_transient(pf_ctx *c, double theta, double dtim, int np_types, const double *prop,
@@ -599,12 +678,10 @@ int pf_assemble_transient(pf_ctx *c, double theta, double dtim, int np_types, co
     for (int e = 0; e < c->nels; ++e)
         if (etype[e] < 1 || etype[e] > np_types) return PF_ERR_ARG;
     PF_HIP(hipSetDevice(c->device));
-    int rc = alloc_k64(c, store);
-    if (!rc) rc = pf_alloc(c, (void **)&c->K64b, (size_t)64 * c->nels * sizeof(double));
-    if (rc) return rc;
+    if (store != PF_STORE_FP64 && store != PF_STORE_FP32) return PF_ERR_ARG;
     double *dprop = nullptr;
     int *dtype = nullptr;
-    rc = pf_alloc(c, (void **)&dprop, sizeof(double) * 5 * np_types);
+    int rc = pf_alloc(c, (void **)&dprop, sizeof(double) * 5 * np_types);
     if (!rc) rc = pf_alloc(c, (void **)&dtype, sizeof(int) * c->nels);
     if (!rc) {
         hipError_t he = hipMemcpyAsync(dprop, prop, sizeof(double) * 5 * np_types, hipMemcpyHostToDevice, c->stream);
@@ -612,7 +689,20 @@ int pf_assemble_transient(pf_ctx *c, double theta, double dtim, int np_types, co
             he = hipMemcpyAsync(dtype, etype, sizeof(int) * c->nels, hipMemcpyHostToDevice, c->stream);
         if (he != hipSuccess) rc = pf_set_hip_error(he, "transient upload", __FILE__, __LINE__);
     }
-    if (!rc) rc = pf_launch_assemble_transient(c, theta, dtim, dprop, dtype);
+    auto alloc_b = [&]() {
+        return c->K64b ? PF_OK : pf_alloc(c, (void **)&c->K64b, (size_t)64 * c->nels * sizeof(double));
+    };
+    bool whole = store == PF_STORE_FP32;   // the hi/lo split reads whole matrices
+    if (!rc && !whole)
+        rc = form_and_pack(c, false, &whole, [&](double *Ka, long e0, long nel) {
+            const int r = alloc_b();
+            return r ? r : pf_launch_assemble_transient(c, theta, dtim, dprop, dtype, Ka, e0, nel);
+        });
+    if (!rc && whole) {
+        rc = alloc_k64(c, store);
+        if (!rc) rc = alloc_b();
+        if (!rc) rc = pf_launch_assemble_transient(c, theta, dtim, dprop, dtype, c->K64, 0, c->nels);
+    }
     (void)hipStreamSynchronize(c->stream);
     pf_free(c, dprop, sizeof(double) * 5 * np_types);
     pf_free(c, dtype, sizeof(int) * c->nels);
@@ -634,9 +724,21 @@ int pf_storkm_set(pf_ctx *c, const double *storkm, int store)
     if (!c || !storkm) return PF_ERR_ARG;
     if (!c->g_g) return PF_ERR_STATE;
     PF_HIP(hipSetDevice(c->device));
+    if (store != PF_STORE_FP64 && store != PF_STORE_FP32) return PF_ERR_ARG;
+    const long nn = (long)c->ntot * c->ntot;
+    if (store == PF_STORE_FP64) {
+        bool whole = false;
+        const int rp = form_and_pack(c, true, &whole, [&](double *dst, long e0, long nel) {
+            const hipError_t he = hipMemcpyAsync(dst, storkm + e0 * nn, (size_t)nel * nn * sizeof(double),
+                                                 hipMemcpyHostToDevice, c->stream);
+            return he == hipSuccess ? PF_OK : pf_set_hip_error(he, "storkm upload", __FILE__, __LINE__);
+        });
+        if (rp) return rp;
+        if (!whole) return finish_matrices(c);
+    }
     int rc = alloc_k64(c, store);
     if (rc) return rc;
-    const long chunk = staging_elems(c), nn = (long)c->ntot * c->ntot;
+    const long chunk = staging_elems(c);
     double *stage = nullptr;
     rc = pf_alloc(c, (void **)&stage, (size_t)chunk * nn * sizeof(double));
     for (long e0 = 0; !rc && e0 < c->nels; e0 += chunk) {

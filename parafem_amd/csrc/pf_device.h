@@ -9,7 +9,8 @@ namespace {
 
 constexpr int MAXG = PF_REDUCE_MAX_GRID;
 
-enum { KIND_F64 = 0, KIND_F32 = 1, KIND_ACC = 2, KIND_WIDE = 3 };   // K_e storage / arithmetic
+// K_e storage / arithmetic (TRI, TRID: FP64 packed triangle without and with differences)
+enum { KIND_F64 = 0, KIND_F32 = 1, KIND_ACC = 2, KIND_WIDE = 3, KIND_TRI = 4, KIND_TRID = 5 };
 enum { RUN_ALWAYS = 0, RUN_LIVE = 1, RUN_REFINE = 2 };  // state gating
 
 __device__ __forceinline__ bool skip(const pf_state *st, int gate)
@@ -169,7 +170,8 @@ __device__ __forceinline__ void fold_everywhere(double (&out)[NQ], const int (&q
 template <int NT, int KIND> struct Lanes {
     static constexpr int W = NT > 32 ? 64 : (NT > 16 ? 32 : (NT > 8 ? 16 : 8));
     static constexpr int EPW = 64 / W;
-    static constexpr int EPL = NT > 32 ? 1 : NT > 8 ? (KIND == 1 ? 2 : 1) : (KIND == 1 ? 8 : KIND == 0 ? 1 : 4);
+    static constexpr int EPL = NT > 32 ? 1 : NT > 8 ? (KIND == 1 ? 2 : 1)
+                                                    : (KIND == 1 ? 8 : KIND == 0 ? 1 : KIND >= 4 ? 2 : 4);
     static constexpr int EPB = EPW * EPL * (PF_BLOCK / 64);   // elements per block
 };
 

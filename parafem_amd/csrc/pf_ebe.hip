@@ -154,7 +154,16 @@ enum { FORM_NONE = 0, FORM_CHECON = 1, FORM_RELRES = 2 };
 //   KIND_ACC: packed symmetric (double)hi + (double)lo, FP64 arithmetic ->
 //             out (double);
 //   KIND_WIDE: packed symmetric (double)hi, FP64 arithmetic on the FP64 p ->
-//             out (double).
+//             out (double);
+//   KIND_TRI, KIND_TRID: the FP64 packed triangle (K64, with the differences
+//             in Khi and their units in Klo for TRID), the chain of KIND_F64
+//             on the same entries -> out (double).  Lane i loads the column
+//             pairs that hold its row's entries on and right of the diagonal,
+//             and hands its entry (i, j), j beyond its own pair, to lane j
+//             through LDS (row pair t of the triangle, 16 bytes per lane
+//             j > 2t+1, read back without conflicts); lane j adds the
+//             difference.  Bound by the reads of K_e: 18,364 bytes an element
+//             (hex20) against 28,800 whole.
 // Packed symmetric rows: lane i holds K(i, i+d mod NT) for d = 0..NT/2 and
 // forms sum_d K(i,i+d) p(i+d) from p staged twice in LDS, then receives
 // K(i-d,i) p(i) from lane i-d (mod NT) for d = 1..NT/2-1 by ds_bpermute,
@@ -171,7 +180,7 @@ enum { FORM_NONE = 0, FORM_CHECON = 1, FORM_RELRES = 2 };
 // (whose entries are never negative), so that one load latency covers both;
 // otherwise before anything else, so that the matrix loads do not wait for
 // the steering (waiting cost the 100^3 mixed product 2%).
-template <int NT, int KIND, bool GATHER, typename OUT, int EPL, int FORM = FORM_NONE>
+template <int NT, int KIND, bool GATHER, typename OUT, int EPL, int FORM = FORM_NONE, int WPB = PF_BLOCK / 64>
 __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K64, const float *__restrict__ Khi,
                                           const float *__restrict__ Klo, const int *__restrict__ gg,
                                           const double *__restrict__ src, const float *__restrict__ src32,
@@ -184,12 +193,13 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
     constexpr long PER = pf_sym_per(NT);
     static_assert(D == 4 * Q + R + 1, "packed layout");
     // Per wave and element slot: p_e (FP64), or p_e twice (packed kinds).
-    __shared__ __attribute__((aligned(16))) double ps[PF_BLOCK / 64][EPL][KIND == KIND_F32 ? 64 : 128];
+    constexpr bool ONCE = KIND == KIND_F32 || KIND == KIND_TRI || KIND == KIND_TRID;   // (F32: 64 doubles, 128 floats)
+    __shared__ __attribute__((aligned(16))) double ps[WPB][EPL][ONCE ? 64 : 128];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane / L::W, li = lane % L::W;
     const int i = li < NT ? li : NT - 1;
     const int gb = sub * L::W;   // first lane of the element's group
-    const long ebase = (lb * (PF_BLOCK / 64) + wave) * L::EPW * EPL;
+    const long ebase = (lb * WPB + wave) * L::EPW * EPL;
     long ev[EPL], ec[EPL];
     int g[EPL];
     if (FORM == FORM_NONE && stop) return;
@@ -247,6 +257,125 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
                     __builtin_nontemporal_store((OUT)acc, &out[ev[t] * NT + li]);
             }
         }
+    } else if constexpr (NT == 8 && (KIND == KIND_TRI || KIND == KIND_TRID)) {
+        // 20 column pairs an element: the wavefront's elements are one
+        // contiguous run, copied into LDS with whole-line loads, and every
+        // lane reads its row from there (its own pairs, or the mirrored
+        // entries of row pair s).  Rows loaded pair by pair, as below, touch
+        // each line in several instructions (200^3: 0.81 ms against 0.60; whole matrices 0.86).
+        constexpr bool DIFF = KIND == KIND_TRID;
+        constexpr int PW = L::EPW * EPL * pf_tri_pairs(8), PL = (PW + 63) / 64;
+        __shared__ __attribute__((aligned(16))) d2_t xs[WPB][PW];
+        const d2_t *Kp = reinterpret_cast<const d2_t *>(K64);
+        const long last = (long)nels * pf_tri_pairs(8) - 1;
+        d2_t kc[PL];
+#pragma unroll
+        for (int u = 0; u < PL; ++u) {
+            const long k = ebase * pf_tri_pairs(8) + u * 64 + lane;
+            kc[u] = __builtin_nontemporal_load(&Kp[k < last ? k : last]);
+        }
+        unsigned df[EPL][H];
+        double unit[EPL];
+        if constexpr (DIFF) {
+#pragma unroll
+            for (int t = 0; t < EPL; ++t) {
+                const unsigned *Dp = reinterpret_cast<const unsigned *>(Khi) + ec[t] * pf_tri_diffs(NT);
+#pragma unroll
+                for (int s = 0; s < H - 1; ++s)
+                    df[t][s] = __builtin_nontemporal_load(&Dp[pf_tri_diff(NT, s, i > 2 * s + 2 ? i : 2 * s + 2)]);
+                unit[t] = __hiloint2double(
+                    (int)__builtin_nontemporal_load(reinterpret_cast<const unsigned *>(Klo) + ec[t]), 0);
+            }
+        }
+        if (form()) return;
+#pragma unroll
+        for (int t = 0; t < EPL; ++t) ps[wave][t][lane] = entry(t);
+#pragma unroll
+        for (int u = 0; u < PL; ++u)
+            if (u * 64 + lane < PW) xs[wave][u * 64 + lane] = kc[u];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int q = i >> 1;
+#pragma unroll
+        for (int t = 0; t < EPL; ++t) {
+            const double *x = reinterpret_cast<const double *>(&xs[wave][(t * L::EPW + sub) * pf_tri_pairs(8)]);
+            const double *pw = &ps[wave][t][gb];
+            double acc = 0.0;
+#pragma unroll
+            for (int s = 0; s < H; ++s) {
+                const bool own = i <= 2 * s + 1;
+                const int o = own ? 2 * pf_tri_pair(s, i) : 2 * (q * (q + 1) + 2 * s) + (i & 1);
+                double v0 = x[o], v1 = x[own ? o + 1 : o + 2];
+                if (DIFF && s < H - 1) {
+                    union { unsigned u; _Float16 h[2]; } c;
+                    c.u = df[t][s];
+                    v0 = own ? v0 : __fma_rn((double)c.h[0], unit[t], v0);
+                    v1 = own ? v1 : __fma_rn((double)c.h[1], unit[t], v1);
+                }
+                acc = __fma_rn(v0, pw[2 * s], acc);
+                acc = __fma_rn(v1, pw[2 * s + 1], acc);
+            }
+            if (ev[t] < nels) {
+                if (rowmajor)
+                    out[(long)li * nels + ev[t]] = (OUT)acc;
+                else
+                    __builtin_nontemporal_store((OUT)acc, &out[ev[t] * NT + li]);
+            }
+        }
+    } else if constexpr (KIND == KIND_TRI || KIND == KIND_TRID) {
+        static_assert(EPL == 1, "one element per lane group");
+        constexpr bool DIFF = KIND == KIND_TRID;
+        constexpr int LOW = H * (H - 1);   // entries (row pair t, lane j > 2t+1): t(NT-3-t) + j-2
+        __shared__ __attribute__((aligned(16))) d2_t low[WPB][L::EPW * LOW];
+        d2_t kc[H];
+        unsigned df[H];
+        const d2_t *Kp = reinterpret_cast<const d2_t *>(K64) + ec[0] * pf_tri_pairs(NT);
+#pragma unroll
+        for (int s = 0; s < H; ++s)   // lanes past the pair's rows read its last entry (unused)
+            kc[s] = __builtin_nontemporal_load(&Kp[pf_tri_pair(s, i < 2 * s + 1 ? i : 2 * s + 1)]);
+        double unit = 0.0;
+        if constexpr (DIFF) {
+            const unsigned *Dp = reinterpret_cast<const unsigned *>(Khi) + ec[0] * pf_tri_diffs(NT);
+#pragma unroll
+            for (int s = 0; s < H - 1; ++s)
+                df[s] = __builtin_nontemporal_load(&Dp[pf_tri_diff(NT, s, i > 2 * s + 2 ? i : 2 * s + 2)]);
+            unit = __hiloint2double((int)__builtin_nontemporal_load(reinterpret_cast<const unsigned *>(Klo) + ec[0]), 0);
+        }
+        if (form()) return;
+        ps[wave][0][lane] = entry(0);
+        double *lw = reinterpret_cast<double *>(&low[wave][sub * LOW]);
+        {
+            const int t = i >> 1, o = 2 * (t * (NT - 3 - t) - 2) + (i & 1);
+#pragma unroll
+            for (int s = 1; s < H; ++s)
+                if (i < 2 * s && li < NT) {
+                    lw[o + 4 * s] = kc[s].x;
+                    lw[o + 4 * s + 2] = kc[s].y;
+                }
+        }
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const d2_t *lr = &low[wave][sub * LOW];
+        const double *pw = &ps[wave][0][gb];
+        double acc = 0.0;
+#pragma unroll
+        for (int s = 0; s < H; ++s) {
+            d2_t v = kc[s];
+            if (s < H - 1) {
+                d2_t w = lr[s * (NT - 3 - s) + (i > 2 * s + 2 ? i : 2 * s + 2) - 2];
+                if constexpr (DIFF) {
+                    union { unsigned u; _Float16 h[2]; } x;
+                    x.u = df[s];
+                    w.x = __fma_rn((double)x.h[0], unit, w.x);
+                    w.y = __fma_rn((double)x.h[1], unit, w.y);
+                }
+                v.x = i > 2 * s + 1 ? w.x : v.x;
+                v.y = i > 2 * s + 1 ? w.y : v.y;
+            }
+            acc = __fma_rn(v.x, pw[2 * s], acc);
+            acc = __fma_rn(v.y, pw[2 * s + 1], acc);
+        }
+        if (ev[0] < nels && li < NT) __builtin_nontemporal_store((OUT)acc, &out[ev[0] * NT + li]);
     } else if constexpr (KIND == KIND_F32) {
         float kd[EPL][D];
 #pragma unroll
@@ -366,11 +495,18 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
     }
 }
 
+constexpr int TRI_WPB = 1, TRI_MINW = 2;
+
 // nlb logical blocks; with LOOP a grid smaller than nlb (the gated
 // true-residual products) loops over them, otherwise every workgroup takes
 // one.
+// wavefronts per workgroup of the plain products: the hex20 triangle's hold
+// 14 KB of LDS each, so that they come one to a workgroup (TRI_WPB)
+template <int NT, int KIND> constexpr int ebe_wpb() { return NT == 60 && KIND >= KIND_TRI ? TRI_WPB : PF_BLOCK / 64; }
+template <int NT, int KIND> constexpr int ebe_minw() { return NT == 60 && KIND >= KIND_TRI ? TRI_MINW : 1; }
+
 template <int NT, int KIND, bool GATHER, typename OUT, bool LOOP = false, int EPLT = Lanes<NT, KIND>::EPL>
-__global__ __launch_bounds__(PF_BLOCK) void k_ebe(const double *__restrict__ K64, const float *__restrict__ Khi,
+__global__ __launch_bounds__((64 * ebe_wpb<NT, KIND>()), (ebe_minw<NT, KIND>())) void k_ebe(const double *__restrict__ K64, const float *__restrict__ Khi,
                                                  const float *__restrict__ Klo, const int *__restrict__ gg,
                                                  const double *__restrict__ src, const float *__restrict__ src32,
                                                  OUT *__restrict__ out, int nels, long kstride,
@@ -386,7 +522,7 @@ __global__ __launch_bounds__(PF_BLOCK) void k_ebe(const double *__restrict__ K64
             __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
         }
     } else {
-        ebe_block<NT, KIND, GATHER, OUT, EPLT>(lb0, K64, Khi, Klo, gg, src, src32, out, nels, kstride, rowmajor, stop);
+        ebe_block<NT, KIND, GATHER, OUT, EPLT, FORM_NONE, ebe_wpb<NT, KIND>()>(lb0, K64, Khi, Klo, gg, src, src32, out, nels, kstride, rowmajor, stop);
     }
 }
 
@@ -1177,14 +1313,27 @@ __global__ void k_scatter_fix(const int *__restrict__ ptr, const int *__restrict
     }
 }
 
+// The three matrix arguments of a product kernel.
+struct k_args {
+    const double *K64;
+    const float *hi, *lo;
+};
+template <int KIND> k_args matrix_args(const pf_ctx *c, const double *K64)
+{
+    if constexpr (KIND == KIND_TRI || KIND == KIND_TRID)
+        return {c->T64, reinterpret_cast<const float *>(c->T64d), reinterpret_cast<const float *>(c->T64u)};
+    return {K64, c->K32hi, c->K32lo};
+}
+
 template <int NT, int KIND, bool GATHER, typename OUT, int EPL>
 void launch_ebe_epl(pf_ctx *c, const double *src, OUT *out, const pf_state *st, int gate, const double *K64,
                     const float *src32, int rowmajor)
 {
-    constexpr int EPB = Lanes<NT, KIND>::EPW * EPL * (PF_BLOCK / 64);
+    constexpr int WPB = ebe_wpb<NT, KIND>(), EPB = Lanes<NT, KIND>::EPW * EPL * WPB;
     const long nlb = (c->nels + EPB - 1) / EPB;
-    hipLaunchKernelGGL((k_ebe<NT, KIND, GATHER, OUT, false, EPL>), dim3((int)nlb), dim3(PF_BLOCK), 0, c->stream,
-                       K64, c->K32hi, c->K32lo, c->g_g, src, src32, out, c->nels, pf_k64_estride(c), st, gate,
+    const k_args A = matrix_args<KIND>(c, K64);
+    hipLaunchKernelGGL((k_ebe<NT, KIND, GATHER, OUT, false, EPL>), dim3((int)nlb), dim3(64 * WPB), 0, c->stream,
+                       A.K64, A.hi, A.lo, c->g_g, src, src32, out, c->nels, pf_k64_estride(c), st, gate,
                        nlb, rowmajor);
 }
 
@@ -1194,18 +1343,22 @@ int launch_ebe_nt(pf_ctx *c, const double *src, OUT *out, const pf_state *st, in
 {
     const double *K64 = Kalt ? Kalt : c->K64;
     if (gate == RUN_REFINE) {
-        // usually does nothing: dispatch few workgroups that loop
-        const long nlb = (c->nels + Lanes<NT, KIND>::EPB - 1) / Lanes<NT, KIND>::EPB;
-        const int grid = (int)std::min<long>(nlb, 2048);
-        hipLaunchKernelGGL((k_ebe<NT, KIND, GATHER, OUT, true>), dim3(grid), dim3(PF_BLOCK), 0, c->stream, K64,
-                           c->K32hi, c->K32lo, c->g_g, src, src32, out, c->nels, pf_k64_estride(c), st, gate,
-                           nlb, rowmajor);
+        if constexpr (KIND == KIND_ACC) {
+            // usually does nothing: dispatch few workgroups that loop
+            const long nlb = (c->nels + Lanes<NT, KIND>::EPB - 1) / Lanes<NT, KIND>::EPB;
+            const int grid = (int)std::min<long>(nlb, 2048);
+            hipLaunchKernelGGL((k_ebe<NT, KIND, GATHER, OUT, true>), dim3(grid), dim3(PF_BLOCK), 0, c->stream, K64,
+                               c->K32hi, c->K32lo, c->g_g, src, src32, out, c->nels, pf_k64_estride(c), st, gate,
+                               nlb, rowmajor);
+        } else {
+            return PF_ERR_ARG;   // residual replacements use hi + lo
+        }
     } else {
         // the tuned shape of the iteration's product (an out-of-range value,
         // e.g. from before the mesh changed, keeps the built-in one)
         constexpr int E0 = Lanes<NT, KIND>::EPL;
         const int e = GATHER && c->tune_epl <= pf_epl_max(NT) ? c->tune_epl : 0;
-        if constexpr (GATHER) {
+        if constexpr (GATHER && KIND < KIND_TRI) {   // the triangle's products have one shape
             if (e == 1) launch_ebe_epl<NT, KIND, GATHER, OUT, 1>(c, src, out, st, gate, K64, src32, rowmajor);
             else if (e == 2) launch_ebe_epl<NT, KIND, GATHER, OUT, 2>(c, src, out, st, gate, K64, src32, rowmajor);
             else if (e == 4) launch_ebe_epl<NT, KIND, GATHER, OUT, (NT <= 24 ? 4 : E0)>(c, src, out, st, gate, K64, src32, rowmajor);
@@ -1231,12 +1384,21 @@ int launch_ebe(pf_ctx *c, const double *src, OUT *out, const pf_state *st, int g
     }
 }
 
-// FP64 element products of the stored matrices (K64, or hi+lo for FP32
+// Products of the FP64 matrices as they are stored.
+template <bool GATHER>
+int launch_ebe_f64(pf_ctx *c, const double *src, double *out, const pf_state *st, int gate, int rowmajor = 0)
+{
+    if (!c->T64) return launch_ebe<KIND_F64, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
+    if (c->T64d) return launch_ebe<KIND_TRID, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
+    return launch_ebe<KIND_TRI, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
+}
+
+// FP64 element products of the stored matrices (FP64, or hi+lo for FP32
 // storage), without state gating: the drop-in primitive and pf_apply.
 template <bool GATHER>
 int launch_ebe_exact(pf_ctx *c, const double *src, double *out)
 {
-    if (c->K64) return launch_ebe<KIND_F64, GATHER, double>(c, src, out, nullptr, RUN_ALWAYS);
+    if (pf_has_f64(c)) return launch_ebe_f64<GATHER>(c, src, out, nullptr, RUN_ALWAYS);
     return launch_ebe<KIND_ACC, GATHER, double>(c, src, out, nullptr, RUN_ALWAYS);
 }
 
@@ -1300,6 +1462,7 @@ struct pf_bslot {
     pf_state *st;
     long kstride;
     int nels, neq, G, fix_zero, rowmajor;
+    int tri;    // FP64: 0 column pairs, 1 packed triangle (K64), 2 with differences (Khi, Klo)
     int solo;   // runs its own launches inside the batch's run: no blocks here
 };
 
@@ -1358,6 +1521,12 @@ __device__ __forceinline__ void bs_ebe(const pf_bslot *__restrict__ T, const lon
     else if constexpr (KIND == KIND_F32)
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, S.p32, (OUT *)S.utemp32, S.nels,
                                             S.kstride, S.rowmajor, stop);
+    else if (KIND == KIND_F64 && S.tri == 2)
+        ebe_block<NT, KIND_TRID, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
+                                               S.kstride, S.rowmajor, stop);
+    else if (KIND == KIND_F64 && S.tri == 1)
+        ebe_block<NT, KIND_TRI, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
+                                              S.kstride, S.rowmajor, stop);
     else
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
                                             S.kstride, S.rowmajor, stop);
@@ -1748,7 +1917,7 @@ static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double
     if (opts->limit < 1 || !(opts->tol >= 0.0)) return PF_ERR_ARG;
     if (opts->stop_mode != PF_STOP_CHECON && opts->stop_mode != PF_STOP_RELRES) return PF_ERR_ARG;
     if (opts->precision == PF_PREC_FP64) {
-        if (!c->K64) return PF_ERR_ARG;   // FP64 iterations need FP64 storage
+        if (!pf_has_f64(c)) return PF_ERR_ARG;   // FP64 iterations need FP64 storage
     } else if (opts->precision == PF_PREC_SPLIT) {
         if (!c->K32hi) return PF_ERR_ARG;
     } else if (opts->precision == PF_PREC_MIXED || opts->precision == PF_PREC_MIXED64) {
@@ -1824,12 +1993,13 @@ static void launch_ebe_form(pf_ctx *c, OUT *out, int rm, int G)
 {
     constexpr int EPB = Lanes<NT, KIND>::EPB;
     const dim3 grid((c->nels + EPB - 1) / EPB), blk(PF_BLOCK);
+    const k_args A = matrix_args<KIND>(c, c->K64);
     if (c->opts.stop_mode == PF_STOP_CHECON)
-        hipLaunchKernelGGL((k_ebe_form<NT, KIND, OUT, FORM_CHECON>), grid, blk, 0, c->stream, c->K64, c->K32hi,
-                           c->K32lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
+        hipLaunchKernelGGL((k_ebe_form<NT, KIND, OUT, FORM_CHECON>), grid, blk, 0, c->stream, A.K64, A.hi,
+                           A.lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
     else
-        hipLaunchKernelGGL((k_ebe_form<NT, KIND, OUT, FORM_RELRES>), grid, blk, 0, c->stream, c->K64, c->K32hi,
-                           c->K32lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
+        hipLaunchKernelGGL((k_ebe_form<NT, KIND, OUT, FORM_RELRES>), grid, blk, 0, c->stream, A.K64, A.hi,
+                           A.lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
 }
 
 template <int NT>
@@ -1847,7 +2017,11 @@ static void launch_form_due(pf_ctx *c, bool due, int rm, int G)
     case PF_PREC_MIXED: launch_ebe_form<NT, KIND_F32, float>(c, c->utemp32, rm, G); break;
     case PF_PREC_MIXED64: launch_ebe_form<NT, KIND_WIDE, double>(c, c->utemp, rm, G); break;
     case PF_PREC_SPLIT: launch_ebe_form<NT, KIND_ACC, double>(c, c->utemp, rm, G); break;
-    default: launch_ebe_form<NT, KIND_F64, double>(c, c->utemp, rm, G); break;
+    default:
+        if (!c->T64) launch_ebe_form<NT, KIND_F64, double>(c, c->utemp, rm, G);
+        else if (c->T64d) launch_ebe_form<NT, KIND_TRID, double>(c, c->utemp, rm, G);
+        else launch_ebe_form<NT, KIND_TRI, double>(c, c->utemp, rm, G);
+        break;
     }
 }
 
@@ -1875,7 +2049,7 @@ static int launch_products(pf_ctx *c, float *p32, int rm)
     case PF_PREC_SPLIT:
         return launch_ebe<KIND_ACC, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
     default:
-        return launch_ebe<KIND_F64, true, double>(c, c->p, c->utemp, c->state, RUN_LIVE, nullptr, nullptr, rm);
+        return launch_ebe_f64<true>(c, c->p, c->utemp, c->state, RUN_LIVE, rm);
     }
 }
 
@@ -2366,9 +2540,11 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool allow_
         const bool mixed = c->opts.precision == PF_PREC_MIXED;
         const int rm = c->csr_slot_t && !mixed ? 1 : 0;
         pf_bslot &S = T[k];
-        S.K64 = c->K64;
-        S.Khi = c->K32hi;
-        S.Klo = c->K32lo;
+        S.tri = c->opts.precision == PF_PREC_FP64 && c->T64 ? (c->T64d ? 2 : 1) : 0;
+        const k_args A = S.tri ? matrix_args<KIND_TRID>(c, nullptr) : matrix_args<KIND_F64>(c, c->K64);
+        S.K64 = A.K64;
+        S.Khi = A.hi;
+        S.Klo = A.lo;
         S.g_g = c->g_g;
         S.csr_ptr = c->csr_ptr;
         S.slot = rm ? c->csr_slot_t : c->csr_slot;

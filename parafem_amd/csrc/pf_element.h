@@ -7,7 +7,7 @@
 // SHAPE_DER for hex8 (nod = 8) and hex20 (nod = 20) at (xi, eta, zeta):
 // derivative k (0..2) of shape function l (0-based).
 template <int NOD>
-static __device__ __forceinline__ void shape_der3(double xi, double eta, double zeta, int l, double out[3])
+static __host__ __device__ constexpr inline void shape_der3(double xi, double eta, double zeta, int l, double out[3])
 {
     if constexpr (NOD == 8) {
         const double etam = 1.0 - eta, xim = 1.0 - xi, zetam = 1.0 - zeta;

@@ -67,6 +67,45 @@ __host__ __device__ inline long pf_idx_sym_ij(long e, int nt, int i, int j)
     return d <= nt / 2 ? pf_idx_sym(e, nt, i, d) : pf_idx_sym(e, nt, j, nt - d);
 }
 
+// FP64 "packed triangle", bit for bit the matrix it was packed from.  An
+// assembled K_e is symmetric up to the rounding of its evaluation order, so
+// the entries above the diagonal are stored whole and those below it as their
+// difference from the mirrored entry: h = nt/2 column pairs, pair s holding
+// (K(i,2s), K(i,2s+1)) of the rows i <= 2s+1 (16-byte loads, lane = row); and
+// for the rows i > 2s+1 the two differences K(i,2s+c) - K(2s+c,i) as FP16
+// multiples of a power of two per element (its high word in `unit`).  A
+// difference is a few units in the last place of the products summed, 4 to 11
+// significant bits within 15 binades on cubes, stretched bricks and distorted
+// meshes; the packing checks that every entry comes back exactly and the
+// matrices stay whole where one does not.  Without differences (hex8
+// Laplace, whose evaluation is symmetric) diff and unit are null.  hex20:
+// 18,364 bytes an element against 28,800.
+__host__ __device__ constexpr int pf_tri_pairs(int nt) { return nt / 2 * (nt / 2 + 1); }
+__host__ __device__ constexpr int pf_tri_diffs(int nt) { return nt / 2 * (nt / 2 - 1); }
+__host__ __device__ constexpr int pf_tri_pair(int s, int i) { return s * (s + 1) + i; }                // i <= 2s+1
+__host__ __device__ constexpr int pf_tri_diff(int nt, int s, int i) { return s * (nt - s - 1) + i - 2 * s - 2; }   // i > 2s+1
+
+// FP64 element matrices for readers of single entries: column pairs (K) or
+// the packed triangle (T).
+struct pf_f64_view {
+    const double *K;
+    const double *T;
+    const unsigned *diff;   // two FP16 a word
+    const unsigned *unit;
+    long kstride;           // 0: one matrix for every element
+};
+__device__ inline double pf_f64_entry(const pf_f64_view &V, long e, int nt, int i, int j)
+{
+    if (!V.T) return V.K[pf_idx_pair(e * V.kstride, nt, i, j)];
+    const double *T = V.T + 2 * e * pf_tri_pairs(nt);
+    if (i <= (j | 1)) return T[2 * pf_tri_pair(j >> 1, i) + (j & 1)];
+    const double up = T[2 * pf_tri_pair(i >> 1, j) + (i & 1)];
+    if (!V.diff) return up;
+    union { unsigned u; _Float16 h[2]; } w;
+    w.u = V.diff[e * pf_tri_diffs(nt) + pf_tri_diff(nt, j >> 1, i)];
+    return __fma_rn((double)w.h[j & 1], __hiloint2double((int)V.unit[e], 0), up);
+}
+
 // Device-resident PCG scalars.  Written only by the one-block fold kernels,
 // or, in an iteration without fold launches, by the first workgroup of the
 // kernel that ends the iteration; read at the start of the following kernels.
@@ -170,7 +209,9 @@ struct pf_ctx {
     int64_t nnz = 0;
     // element matrices (internal layouts above)
     int store = PF_STORE_FP64;
-    double *K64 = nullptr;             // FP64 column pairs (PF_STORE_FP64)
+    double *K64 = nullptr;             // FP64 column pairs (PF_STORE_FP64 where the triangle below does not hold)
+    double *T64 = nullptr;             // FP64 packed triangle (PF_STORE_FP64), its differences and their units
+    unsigned *T64d = nullptr, *T64u = nullptr;
     double *K64b = nullptr;            // p124's second matrix set (storkb_pp), FP64 column pairs
     bool k_shared = false;             // K64 holds one matrix used by every element
     float *K32hi = nullptr;            // packed symmetric FP32, hi = fl32(K)
@@ -245,7 +286,9 @@ void pf_scan_launch(pf_ctx *c, const int *cnt, int n, int *bsum, int *ptr, int *
 int pf_scratch_init(int device);
 
 // p124's transient element matrices into K64 (storka) and K64b (storkb).
-int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const double *prop, const int *etype);
+// Elements e0 .. e0 + nel - 1 of storka into Ka (element e0 first).
+int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const double *prop, const int *etype,
+                                 double *Ka, long e0, long nel);
 
 // Steering set-up (pf_context.hip, pf_setup.hip).
 int pf_steer_install(pf_ctx *c, int ntot, int nels, int neq);
@@ -277,6 +320,8 @@ inline size_t pf_k64_count(const pf_ctx *c)
     return (size_t)c->ntot * c->ntot * (c->k_shared ? 1 : (size_t)c->nels);
 }
 inline long pf_k64_estride(const pf_ctx *c) { return c->k_shared ? 0 : 1; }
+inline bool pf_has_f64(const pf_ctx *c) { return c->K64 || c->T64; }
+inline pf_f64_view pf_f64(const pf_ctx *c) { return {c->K64, c->T64, c->T64d, c->T64u, pf_k64_estride(c)}; }
 
 int pf_set_hip_error(hipError_t e, const char *what, const char *file, int line);
 int pf_alloc(pf_ctx *c, void **p, size_t bytes);
@@ -285,11 +330,16 @@ void pf_cache_release(pf_ctx *c);
 int pf_grid_for(int64_t n);
 
 // kernels launched across translation units ---------------------------------
-// Element assembly into K64 (FP64 storage) or, for FP32 storage, straight
-// into K32hi/K32lo with the FP64 element diagonals in dg (ntot*nels).
-int pf_launch_assemble_elastic(pf_ctx *c, double v2, double vv, double den, double e0, const double *e_elem_dev,
-                               double *dg);
+// Element assembly into T64 or K64 (FP64 storage) or, for FP32 storage, straight
+// into K32hi/K32lo with the FP64 element diagonals in dg (ntot*nels).  bad:
+// set where an entry of the triangle does not come back exactly.
+int pf_launch_assemble_elastic(pf_ctx *c, double v2, double vv, double den, double e, const double *e_elem_dev,
+                               double *dg, int *bad);
 int pf_launch_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double *k_elem_dev, double *dg);
+// Packs elements e0 .. e0 + nel - 1 (element e0 first in src: column pairs or
+// column-major) into the triangle; *bad is set where an entry does not come
+// back exactly.
+int pf_launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad);
 // Assembled diagonal (leading 0 slot) from element diagonals dg(ntot,nels).
 int pf_launch_diag_elem(pf_ctx *c, const double *dg, double *diag);
 int pf_launch_split_fp32(pf_ctx *c);

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from parafem_amd import Context, problems as P
+from parafem_amd import Batch, Context, DeviceArray, mesh as M, problems as P
 from parafem_amd.api import BlockOpts, BlockResult, lib
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +95,113 @@ def test_more_slots_than_the_padded_table_holds():
         P.setup(ctx, tp)
         x, res = ctx.pcg_solve(r, 40, 0.0, stop="relres")
         assert res.iters == 40 and np.array_equal(x, _oracle_iterates(tp, "relres", 40))
+
+
+def _mesh_problem(ntot, box):
+    if ntot == 60:
+        return P.elastic_cube(1, nels_xyz=box, lognormal_e=True)
+    if ntot == 8:
+        pr = P.laplace_cube(1, nels_xyz=box)
+        pr.fix_eq = pr.fix_val = None
+        return pr
+    m = M.box_hex8(*box)
+    nf, neq = M.steering(m.nn, 3, M.base_fixed_rest(m))
+    r = np.random.default_rng(1).standard_normal(neq)
+    return P.Problem("elastic", m, M.g_g_from(nf, m.g_num), neq, r, nf)
+
+
+def _matrices(kind, nels, nt, seed=3):
+    """Element matrices (element, column, row): symmetric but for the rounding
+    the packed triangle keeps ("ulps"), exactly symmetric, with one
+    difference of more bits than it keeps in the last element ("wide"),
+    without symmetry, or with a whole range of magnitudes ("ranges")."""
+    rng = np.random.default_rng(seed)
+    a = rng.standard_normal((nels, nt, nt))
+    if kind == "general":
+        return a
+    K = np.matmul(a, a.transpose(0, 2, 1)) + nt * np.eye(nt)
+    K = (K + K.transpose(0, 2, 1)) / 2
+    if kind == "ranges":
+        d = 2.0 ** rng.integers(-300, 300, (nels, 1, 1))
+        K = K * d
+    low = np.tril(np.ones((nt, nt), dtype=bool), -1)
+    if kind != "symmetric":
+        K[:, low] += np.ldexp(rng.integers(-900, 900, (nels, low.sum())), -48 + np.frexp(np.abs(K).max((1, 2)))[1][:, None] - 6)
+    if kind == "wide":
+        K[-1, 3, 1] = K[-1, 1, 3] * (1 + 2.0 ** -12 + 2.0 ** -40)
+    return K
+
+
+# FP64 matrices as the packed triangle (the first three kinds) and whole (the
+# others): entries, products and iterates bit for bit.  Element counts around
+# the lane groups: 16 elements a wavefront for ntot 8, 2 for 24, 1 for 60.
+@pytest.mark.parametrize("ntot,box", [(60, (1, 1, 1)), (60, (3, 1, 2)), (24, (1, 1, 1)), (24, (3, 3, 1)),
+                                      (8, (1, 1, 1)), (8, (5, 3, 1)), (8, (4, 2, 2)), (8, (17, 1, 1)), (8, (11, 3, 2))])
+@pytest.mark.parametrize("kind", ["ulps", "symmetric", "ranges", "wide", "general"])
+def test_fp64_storage_bitexact(ntot, box, kind):
+    pr = _mesh_problem(ntot, box)
+    print(f"[gpu-test] fp64 storage {ntot} {box} {kind}", flush=True)
+    K = _matrices(kind, pr.nels, ntot)
+    rng = np.random.default_rng(7)
+    with Context(0) as ctx:
+        ctx.mesh_set(pr.g_coord())
+        ctx.steer_set(pr.g_g, pr.neq)
+        before = ctx.mem_used()
+        ctx.storkm_set(K)
+        assert np.array_equal(ctx.storkm_get(), K)
+        assert np.array_equal(ctx.diag_get(), O.diag(pr.g_g, K, pr.neq))
+        x = rng.standard_normal(pr.neq)
+        assert np.array_equal(ctx.apply(x), O.apply(pr.g_g, K, x))
+        pm = rng.standard_normal((pr.nels, ntot))
+        d, u = DeviceArray.from_host(ctx, pm), DeviceArray(ctx, pm.size)
+        ctx.elem_matvec(d, u)
+        assert np.array_equal(u.download().reshape(pm.shape), O.elem_matvec(K, pm))
+        assert ctx.mem_used() > before
+        if kind in ("ulps", "symmetric"):      # positive definite: whole iterations
+            dg = O.diag(pr.g_g, K, pr.neq)
+            r = rng.standard_normal(pr.neq)
+            xg, res = ctx.pcg_solve(r, 5, 0.0, stop="relres")
+            xo = O.pcg(pr.g_g, K, r, dg, 0.0, 5, stop=O.STOP_RELRES, dot_order=O.DOT_DEVICE)[0]
+            assert np.array_equal(xg, xo)
+
+
+def test_batch_of_whole_and_packed_matrices():
+    """FP64 contexts that hold whole matrices and ones that hold the triangle
+    advance in one batch, each as alone."""
+    pr = P.elastic_cube(3)
+    Ks = [_matrices(k, pr.nels, 60, seed) for k, seed in (("wide", 1), ("ulps", 2), ("symmetric", 3))]
+    ctxs, ref = [], []
+    for K in Ks:
+        ctx = Context(0)
+        ctx.mesh_set(pr.g_coord())
+        ctx.steer_set(pr.g_g, pr.neq)
+        ctx.storkm_set(K)
+        ref.append(ctx.pcg_solve(pr.r0, 9, 0.0, stop="relres")[0])
+        ctx.pcg_begin(pr.r0, 9, 0.0, stop="relres")
+        ctxs.append(ctx)
+    for persistent in (False, True):
+        with Batch(0) as b:
+            for ctx in ctxs:
+                ctx.pcg_begin(pr.r0, 9, 0.0, stop="relres")
+            b.run(ctxs, 12, persistent=persistent)
+            for ctx, x in zip(ctxs, ref):
+                ctx.sync()
+                assert np.array_equal(ctx.pcg_x(), x)
+    for ctx in ctxs:
+        ctx.close()
+
+
+def test_assembly_that_the_triangle_cannot_hold():
+    """A degenerate element (zero determinant: undefined entries) is stored
+    whole, as the evaluation gives it."""
+    pr = P.elastic_cube(2)
+    gc = pr.g_coord().copy()
+    gc[3] = 0.0
+    with Context(0) as ctx:
+        ctx.mesh_set(gc)
+        ctx.steer_set(pr.g_g, pr.neq)
+        ctx.assemble_elastic(pr.e, pr.v)
+        K = ctx.storkm_get()
+    assert np.isnan(K[3]).all()
+    ok = [e for e in range(pr.nels) if e != 3]
+    assert np.array_equal(K[ok], O.assemble_elastic(gc, pr.e, pr.v)[ok])
