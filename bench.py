@@ -43,14 +43,13 @@ def log(msg):
 
 def ebe_bytes(ntot, store, precision="mixed"):
     """Algorithmic HBM bytes of one element product: the element matrix once
-    (the FP64 packed triangle as assembled: ntot/2 (ntot/2 + 1) column pairs
-    and, but for the Laplace elements, the 2-byte differences of the entries
-    below them and a word for their unit; or the FP32 hi part packed
-    symmetric: the ntot(ntot+1)/2 entries of one triangle padded to a multiple
-    of 4, hi and lo for the split precision) and the int32 steering once."""
+    (full FP64, or the FP32 hi part packed symmetric: the ntot(ntot+1)/2
+    entries of one triangle padded to a multiple of 4, hi and lo for the
+    split precision) and the int32 steering once.  (FP64 matrices are held as
+    a packed triangle where that is exact -- 18,364 bytes a hex20 element --
+    so the FP64 rate by these bytes exceeds what is moved.)"""
     if store == "fp64":
-        h = ntot // 2
-        return 16 * h * (h + 1) + (4 * h * (h - 1) + 4 if ntot != 8 else 0) + ntot * 4
+        return ntot * ntot * 8 + ntot * 4
     parts = 2 if precision == "split" else 1
     packed = (ntot * (ntot + 1) // 2 + 3) // 4 * 4
     return parts * packed * 4 + ntot * 4

@@ -116,8 +116,9 @@ def device_bytes(n: int, precision: str) -> int:
     steering (240), transposed steering (240 + 4 per equation), FP64
     element products (480) and the PCG vectors (12 per equation), plus the
     element matrices as stored -- FP64 (28,800 B per element where they are
-    kept whole; the packed triangle takes 18,364) or the packed symmetric FP32 hi and lo (2 x 7,328) with FP32 products (240); FP32
-    storage is assembled straight into hi/lo, with no FP64 copy."""
+    kept whole; the packed triangle takes 18,364) or the packed symmetric
+    FP32 hi and lo (2 x 7,328) with FP32 products (240); FP32 storage is
+    assembled straight into hi/lo, with no FP64 copy."""
     nels = n ** 3
     neq = 3 * ((2 * n + 1) * (n + 1) * (n + 1) + (n + 1) * (n + 1) * n)   # upper bound
     per_el = 480 + 240 + 240 + 480
