@@ -1450,11 +1450,16 @@ int reduce_prim(pf_ctx *c, const double *a, double *b, int64_t n, int mode, doub
 // launches, G blocks per solve as its own launches use), and every block
 // runs the same body with the same local block index and grid size as the
 // solve's own launch would: the results are those of the solve alone, bit
-// for bit.
+// for bit.  Solves with a padded slot table fold for themselves (as in
+// iterations without fold launches, p formed by kb_pupdate); the folds are
+// launched only for the others, so a batch of small solves runs 4 launches an
+// iteration (mixed: 6) instead of 6 (9): sixteen solves of n = 6 to 18 in
+// mixed64 83 -> 64 ms.
 struct pf_bslot {
     const double *K64;
     const float *Khi, *Klo;
     const int *g_g, *csr_ptr, *slot;   // slot: the list matching the products' layout
+    const int *slot8;                  // the padded slot table of a solve without fold launches, or null
     double *x, *r, *p, *d, *u, *dinv, *f, *utemp;
     float *p32, *utemp32;
     const double *fixstore;
@@ -1485,6 +1490,7 @@ __device__ __forceinline__ pf_bslot slot_of(const pf_bslot *__restrict__ T, int 
     pf_bslot S = R;
     S.K64 = as_global(R.K64); S.Khi = as_global(R.Khi); S.Klo = as_global(R.Klo);
     S.g_g = as_global(R.g_g); S.csr_ptr = as_global(R.csr_ptr); S.slot = as_global(R.slot);
+    S.slot8 = as_global(R.slot8);
     S.x = as_global(R.x); S.r = as_global(R.r); S.p = as_global(R.p); S.d = as_global(R.d);
     S.u = as_global(R.u); S.dinv = as_global(R.dinv); S.f = as_global(R.f); S.utemp = as_global(R.utemp);
     S.p32 = as_global(R.p32); S.utemp32 = as_global(R.utemp32); S.fixstore = as_global(R.fixstore);
@@ -1555,10 +1561,15 @@ __device__ __forceinline__ void bs_scatter_pu(const pf_bslot *__restrict__ T, co
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
-    if (skip(S.st, RUN_LIVE)) return;
     const UT *ut;
     if constexpr (sizeof(UT) == 4) ut = (const UT *)S.utemp32;
     else ut = (const UT *)S.utemp;
+    if (S.slot8) {
+        scatter_copy_block<UT>(b - qst[s], S.slot8, ut, S.fixstore, S.p, S.u, S.neq, S.fix_zero, S.partials, S.st,
+                               nullptr, S.rowmajor, S.nels);
+        return;
+    }
+    if (skip(S.st, RUN_LIVE)) return;
     scatter_pu_block<UT>(b - qst[s], S.G, S.csr_ptr, S.slot, ut, S.fixstore, S.p, S.u, S.neq, S.fix_zero,
                          S.partials);
 }
@@ -1568,6 +1579,10 @@ __device__ __forceinline__ void bs_update(const pf_bslot *__restrict__ T, const 
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
+    if (S.slot8) {
+        update_fold_block<CHECON>(b - qst[s], S.G, S.x, S.r, S.d, S.p, S.u, S.dinv, S.neq, S.partials, S.st);
+        return;
+    }
     if (skip(S.st, RUN_LIVE)) return;
     update_block<CHECON>(b - qst[s], S.G, S.x, S.r, S.d, S.p, S.u, S.dinv, S.neq, S.partials, S.st);
 }
@@ -1577,15 +1592,20 @@ __device__ __forceinline__ void bs_scatter_res(const pf_bslot *__restrict__ T, c
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
-    if (skip(S.st, RUN_REFINE)) return;
+    if (S.slot8 ? stopped(S.st + 1) || !S.st[1].refine : skip(S.st, RUN_REFINE)) return;
     scatter_res_block(b - qst[s], S.G, S.csr_ptr, S.slot, S.utemp, S.fixstore, S.x, S.f, S.r, S.d, S.dinv, S.neq,
-                      S.partials);
+                      S.partials, S.slot8 != nullptr);
 }
 
+template <bool CHECON>
 __device__ __forceinline__ void bs_pupdate(const pf_bslot *__restrict__ T, const int *__restrict__ qst, int ns, int b)
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
+    if (S.slot8) {
+        pupdate_fold_block<CHECON>(b - qst[s], S.G, S.p, S.p32, S.d, S.neq, S.partials, S.st);
+        return;
+    }
     if (skip(S.st, RUN_LIVE)) return;
     pupdate_block(b - qst[s], S.G, S.p, S.p32, S.d, S.neq, S.st);
 }
@@ -1596,7 +1616,7 @@ template <int WHICH>
 __device__ __forceinline__ void bs_fold(const pf_bslot *__restrict__ T, int s)
 {
     const pf_bslot S = slot_of(T, s);
-    if (S.solo || skip(S.st, WHICH == 3 ? RUN_REFINE : RUN_LIVE)) return;
+    if (S.solo || S.slot8 || skip(S.st, WHICH == 3 ? RUN_REFINE : RUN_LIVE)) return;
     if constexpr (WHICH == 0) fold_alpha_block(S.partials, S.G, S.st);
     else if constexpr (WHICH == 1) fold_update_block<true>(S.partials, S.G, S.st);
     else if constexpr (WHICH == 2) fold_update_block<false>(S.partials, S.G, S.st);
@@ -1610,11 +1630,26 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_ebe(const pf_bslot *__restrict__ 
     bs_ebe<NT, KIND, OUT, false>(T, est, ns, xcd_block(blockIdx.x, gridDim.x), RUN_LIVE);
 }
 
+// The true-residual products: few workgroups, dealt to the solves by their
+// size (rst: first workgroup of each solve, total in all), that loop over
+// their solve's blocks where a replacement is due.  Workgroups that each
+// looked at every solve took 15.8 us of a 98 us iteration (16 solves, n = 6
+// to 18) to find nothing due; these take 8.2.
 template <int NT>
-__global__ __launch_bounds__(PF_BLOCK) void kb_ebe_refine(const pf_bslot *__restrict__ T, const long *__restrict__ est,
-                                                         int ns, long total)
+__global__ __launch_bounds__(PF_BLOCK) void kb_ebe_refine(const pf_bslot *__restrict__ T, const int *__restrict__ rst,
+                                                         int ns, int total)
 {
-    bs_ebe_refine<NT>(T, est, ns, total, blockIdx.x, gridDim.x);
+    const int b = blockIdx.x, s = bslot_find(rst, ns, b);
+    const pf_bslot S = slot_of(T, s);
+    const int b0 = b - rst[s], nb = (s + 1 < ns ? rst[s + 1] : total) - rst[s];
+    if (S.slot8 ? !refine_due(S.partials, S.G, S.st + 1, b0 == 0) : skip(S.st, RUN_REFINE)) return;
+    constexpr int EPB = Lanes<NT, KIND_ACC>::EPB;
+    const long nlb = (S.nels + EPB - 1) / EPB;
+    for (long lb = b0; lb < nlb; lb += nb) {
+        ebe_block<NT, KIND_ACC, true, double, Lanes<NT, KIND_ACC>::EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.x, nullptr,
+                                                                       S.utemp, S.nels, S.kstride, S.rowmajor, false);
+        __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
+    }
 }
 
 template <typename UT>
@@ -1637,10 +1672,11 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_scatter_res(const pf_bslot *__res
     bs_scatter_res(T, qst, ns, blockIdx.x);
 }
 
+template <bool CHECON>
 __global__ __launch_bounds__(PF_BLOCK) void kb_pupdate(const pf_bslot *__restrict__ T, const int *__restrict__ qst,
                                                       int ns)
 {
-    bs_pupdate(T, qst, ns, blockIdx.x);
+    bs_pupdate<CHECON>(T, qst, ns, blockIdx.x);
 }
 
 template <int WHICH>
@@ -1739,7 +1775,7 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
                 if (!grid_barrier(bar, nb)) return;
             }
         }
-        for (int b = blockIdx.x; b < total_qb; b += nb) bs_pupdate(T, qst, ns, b);
+        for (int b = blockIdx.x; b < total_qb; b += nb) bs_pupdate<CHECON>(T, qst, ns, b);
         if (!grid_barrier(bar, nb)) return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) bar->iters = it;
@@ -2474,15 +2510,17 @@ struct pf_batch {
     long *est = nullptr;                           // device: first element block per solve (iteration
                                                    // kind), then the same for the FP64 hi+lo products
     int *qst = nullptr;                            // device: first equation block per solve
+    int *rst = nullptr;                            // device: first workgroup per solve of the replacement's products
     pf_bslot *T_host = nullptr;                    // pinned staging of the three (one allocation)
     long *est_host = nullptr;
-    int *qst_host = nullptr;
+    int *qst_host = nullptr, *rst_host = nullptr;
     std::vector<pf_bslot> cur;                     // the table on the device
     std::vector<long> cur_est;                     // iteration-kind starts, then ACC-kind starts
-    std::vector<int> cur_qst;
+    std::vector<int> cur_qst, cur_rst;
     int ns = 0, ntot = 0, precision = -1, stop = -1;
     long total_eb = 0, total_ebr = 0;              // element blocks: iteration kind, true-residual kind
-    int total_qb = 0;
+    int total_qb = 0, total_rb = 0;
+    bool folds = false;   // some batched solve needs the folds' launches
     pf_state *snap = nullptr, *snap_host = nullptr;
     int snap_n = 0;
     bool snap_pending = false;
@@ -2504,7 +2542,7 @@ struct pf_batch {
 };
 
 static const size_t kBatchTable = sizeof(pf_bslot) * PF_BATCH_MAX + 2 * sizeof(long) * PF_BATCH_MAX +
-                                  sizeof(int) * PF_BATCH_MAX;
+                                  2 * sizeof(int) * PF_BATCH_MAX;
 
 static void batch_graph_drop(pf_batch *b)
 {
@@ -2517,16 +2555,18 @@ static void batch_graph_drop(pf_batch *b)
 
 // Builds the table of the given contexts, uploads it when it changed and
 // orders the batch stream after each context's stream.
-static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool allow_solo = true)
+// persistent: every solve in the one kernel, with its folds as phases.
+static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persistent = false)
 {
     if (!b || nctx < 1 || nctx > PF_BATCH_MAX || !ctxs) return PF_ERR_ARG;
     const pf_ctx *c0 = ctxs[0];
     if (!c0) return PF_ERR_ARG;
     std::vector<pf_bslot> T(nctx);
     std::vector<long> est(2 * (size_t)nctx);
-    std::vector<int> qst(nctx);
+    std::vector<int> qst(nctx), rst(nctx);
     long eb = 0;
     int qb = 0;
+    bool folds = false;
     for (int k = 0; k < nctx; ++k) {
         pf_ctx *c = ctxs[k];
         if (!c || c->device != b->device) return PF_ERR_ARG;
@@ -2561,7 +2601,9 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool allow_
         S.G = pf_grid_for(c->neq);
         S.fix_zero = c->fix_zero ? 1 : 0;
         S.rowmajor = rm;
-        S.solo = allow_solo && b->solo_elems > 0 && c->nels >= b->solo_elems ? 1 : 0;
+        S.solo = !persistent && b->solo_elems > 0 && c->nels >= b->solo_elems ? 1 : 0;
+        S.slot8 = persistent || S.solo ? nullptr : c->csr_slot8;
+        if (!S.solo && !S.slot8) folds = true;
         qst[k] = qb;
         if (!S.solo) qb += S.G;
         if (mixed && !c->utemp32) return PF_ERR_STATE;
@@ -2595,21 +2637,29 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool allow_
         eb += (T[k].nels + EPB - 1) / EPB;
         ebr += (T[k].nels + EPBR - 1) / EPBR;
     }
+    // about 1,024 workgroups for the replacement's products, at least one a solve
+    int rb = 0;
+    for (int k = 0; k < nctx; ++k) {
+        rst[k] = rb;
+        if (!T[k].solo) rb += 1 + (int)(((T[k].nels + EPBR - 1) / EPBR - 1) * std::min<long>(1024, ebr) / ebr);
+    }
     PF_HIP(hipSetDevice(b->device));
     const bool same = !b->stale && nctx == b->ns &&
                       std::memcmp(T.data(), b->cur.data(), sizeof(pf_bslot) * nctx) == 0 &&
-                      est == b->cur_est && qst == b->cur_qst;
+                      est == b->cur_est && qst == b->cur_qst && rst == b->cur_rst;
     if (!same) {
         PF_HIP(hipEventSynchronize(b->ev_table));   // the staging buffer is free again
         std::memcpy(b->T_host, T.data(), sizeof(pf_bslot) * nctx);
         std::memcpy(b->est_host, est.data(), sizeof(long) * nctx);
         std::memcpy(b->est_host + PF_BATCH_MAX, est.data() + nctx, sizeof(long) * nctx);
         std::memcpy(b->qst_host, qst.data(), sizeof(int) * nctx);
+        std::memcpy(b->rst_host, rst.data(), sizeof(int) * nctx);
         PF_HIP(hipMemcpyAsync(b->T, b->T_host, kBatchTable, hipMemcpyHostToDevice, b->stream));
         PF_HIP(hipEventRecord(b->ev_table, b->stream));
         // a captured graph reads the batched solves from the table, but
         // holds the solo solves' launches with their own buffers
-        if (eb != b->total_eb || ebr != b->total_ebr || qb != b->total_qb || nctx != b->ns || c0->ntot != b->ntot ||
+        if (eb != b->total_eb || ebr != b->total_ebr || qb != b->total_qb || rb != b->total_rb ||
+            folds != b->folds || nctx != b->ns || c0->ntot != b->ntot ||
             c0->opts.precision != b->precision || c0->opts.stop_mode != b->stop || !solo.empty() ||
             !b->solo.empty() || b->stale)
             batch_graph_drop(b);
@@ -2618,6 +2668,9 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool allow_
         b->cur = T;
         b->cur_est = est;
         b->cur_qst = qst;
+        b->cur_rst = rst;
+        b->total_rb = rb;
+        b->folds = folds;
         b->ns = nctx;
         b->total_eb = eb;
         b->total_ebr = ebr;
@@ -2654,15 +2707,6 @@ static void batch_launch_ebe(pf_batch *b)
 }
 
 template <int NT>
-static void batch_launch_refine(pf_batch *b)
-{
-    // usually does nothing: few workgroups that loop over every solve's blocks
-    const int grid = (int)std::min<long>(b->total_ebr, 2048);
-    hipLaunchKernelGGL(kb_ebe_refine<NT>, dim3(grid), dim3(PF_BLOCK), 0, b->stream, b->T, b->est + PF_BATCH_MAX,
-                       b->ns, b->total_ebr);
-}
-
-template <int NT>
 static void batch_iteration_nt(pf_batch *b)
 {
     const int prec = b->precision;
@@ -2675,20 +2719,24 @@ static void batch_iteration_nt(pf_batch *b)
         hipLaunchKernelGGL(kb_scatter_pu<float>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
     else
         hipLaunchKernelGGL(kb_scatter_pu<double>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
-    hipLaunchKernelGGL(kb_fold<0>, gs, blk, 0, b->stream, b->T);
+    if (b->folds) hipLaunchKernelGGL(kb_fold<0>, gs, blk, 0, b->stream, b->T);
     if (b->stop == PF_STOP_CHECON) {
         hipLaunchKernelGGL(kb_update<true>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
-        hipLaunchKernelGGL(kb_fold<1>, gs, blk, 0, b->stream, b->T);
+        if (b->folds) hipLaunchKernelGGL(kb_fold<1>, gs, blk, 0, b->stream, b->T);
     } else {
         hipLaunchKernelGGL(kb_update<false>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
-        hipLaunchKernelGGL(kb_fold<2>, gs, blk, 0, b->stream, b->T);
+        if (b->folds) hipLaunchKernelGGL(kb_fold<2>, gs, blk, 0, b->stream, b->T);
     }
     if (prec == PF_PREC_MIXED || prec == PF_PREC_MIXED64) {
-        batch_launch_refine<NT>(b);
+        hipLaunchKernelGGL(kb_ebe_refine<NT>, dim3((unsigned)b->total_rb), blk, 0, b->stream, b->T, b->rst, b->ns,
+                           b->total_rb);
         hipLaunchKernelGGL(kb_scatter_res, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
-        hipLaunchKernelGGL(kb_fold<3>, gs, blk, 0, b->stream, b->T);
+        if (b->folds) hipLaunchKernelGGL(kb_fold<3>, gs, blk, 0, b->stream, b->T);
     }
-    hipLaunchKernelGGL(kb_pupdate, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
+    if (b->stop == PF_STOP_CHECON)
+        hipLaunchKernelGGL(kb_pupdate<true>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
+    else
+        hipLaunchKernelGGL(kb_pupdate<false>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
 }
 
 template <int NT, int KIND, typename OUT, bool CHECON, bool REF>
@@ -2796,11 +2844,13 @@ int pf_batch_create(int device, pf_batch **out)
         b->T = (pf_bslot *)dt;
         b->est = (long *)((char *)dt + sizeof(pf_bslot) * PF_BATCH_MAX);
         b->qst = (int *)((char *)b->est + 2 * sizeof(long) * PF_BATCH_MAX);
+        b->rst = b->qst + PF_BATCH_MAX;
     }
     if (ht) {
         b->T_host = (pf_bslot *)ht;
         b->est_host = (long *)((char *)ht + sizeof(pf_bslot) * PF_BATCH_MAX);
         b->qst_host = (int *)((char *)b->est_host + 2 * sizeof(long) * PF_BATCH_MAX);
+        b->rst_host = b->qst_host + PF_BATCH_MAX;
     }
     if (e != hipSuccess) {
         const int rc = pf_set_hip_error(e, "pf_batch_create", __FILE__, __LINE__);
@@ -2885,7 +2935,7 @@ int pf_batch_run_persistent(pf_batch *b, int nctx, pf_ctx *const *ctxs, int max_
 {
     if (!b || max_iters < 1) return PF_ERR_ARG;
     if (!b->coop) return PF_ERR_ARG;   // the device cannot guarantee a resident grid
-    int rc = batch_prepare(b, nctx, ctxs, false);   // every solve in the one kernel
+    int rc = batch_prepare(b, nctx, ctxs, true);
     if (rc) return rc;
     switch (b->ntot) {
     case 60: rc = batch_persistent_nt<60>(b, max_iters); break;
