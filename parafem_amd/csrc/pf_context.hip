@@ -288,6 +288,9 @@ int pf_create(int device, pf_ctx **out)
     if (!rc && hipHostMalloc((void **)&c->state_host, sizeof(pf_state), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
     if (!rc && hipHostMalloc((void **)&c->scalar_host, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
     if (!rc && hipHostMalloc((void **)&c->state_query, sizeof(pf_state), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
+    if (!rc && hipHostMalloc((void **)&c->stop_host, sizeof(int), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
+    for (hipEvent_t &e : c->ev_pace)
+        if (!rc && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) rc = PF_ERR_HIP;
     if (!rc && hipEventCreateWithFlags(&c->ev_query, hipEventDisableTiming) != hipSuccess) rc = PF_ERR_HIP;
     if (!rc) {
         hipError_t z = hipMemsetAsync(c->state, 0, 2 * sizeof(pf_state), c->stream);
@@ -311,6 +314,9 @@ int pf_destroy(pf_ctx *c)
     free_arr(c, c->partials, kPartials);
     pf_free(c, c->state, 2 * sizeof(pf_state));
     if (c->state_host) (void)hipHostFree(c->state_host);
+    if (c->stop_host) (void)hipHostFree(c->stop_host);
+    for (hipEvent_t e : c->ev_pace)
+        if (e) (void)hipEventDestroy(e);
     if (c->scalar_host) (void)hipHostFree(c->scalar_host);
     if (c->state_query) (void)hipHostFree(c->state_query);
     if (c->ev_query) (void)hipEventDestroy(c->ev_query);

@@ -20,6 +20,12 @@ __device__ __forceinline__ bool skip(const pf_state *st, int gate)
     return gate == RUN_REFINE && !st->refine;
 }
 
+// Tells the host that the solve has stopped (one thread, after frozen is set).
+__device__ __forceinline__ void tell_stop(const pf_state *st)
+{
+    if (st->frozen && st->stop) __hip_atomic_store(st->stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // v of lane l + OFF, in the lanes below OFF (the others' values are not used):
 // the halves of the wavefront through the permlane swaps, lanes of one row of
 // 16 through DPP.  These stay in the vector pipe; a shuffle goes through the

@@ -124,7 +124,10 @@ __device__ __forceinline__ bool end_iteration(const double *__restrict__ partial
         s.rr_ref = rr;
     }
     finish_iteration(&s, rd, rr, maxx, maxdx);
-    if (lead && threadIdx.x == 0) *live = s;
+    if (lead && threadIdx.x == 0) {
+        *live = s;
+        tell_stop(&s);
+    }
     *beta = s.beta;
     return s.frozen != 0;
 }
@@ -644,6 +647,7 @@ __device__ __forceinline__ void fold_alpha_block(const double *partials, int G, 
         if (!isfinite(alpha)) {
             st->breakdown = 1;
             st->frozen = 1;
+            tell_stop(st);
         }
     }
 }
@@ -744,6 +748,7 @@ __device__ __forceinline__ void fold_update_block(const double *partials, int G,
             }
         }
         finish_iteration(st, out[0], out[1], out[2], out[3]);
+        tell_stop(st);
     }
 }
 
@@ -808,6 +813,7 @@ __device__ __forceinline__ void fold_refine_block(const double *partials, int G,
         st->since_refine = 0;
         st->rr_ref = out[1];
         finish_iteration(st, out[0], out[1], 0.0, 0.0);
+        tell_stop(st);
     }
 }
 
@@ -941,6 +947,7 @@ __device__ __forceinline__ void update_fold_block(int lb, int G, double *__restr
             st->alpha = alpha;
             st->breakdown = 1;
             st->frozen = 1;
+            tell_stop(st);
         }
         return;
     }
@@ -1078,23 +1085,25 @@ __global__ __launch_bounds__(PF_BLOCK) void k_pcg_init(double *__restrict__ x, c
     block_to_partials<2>(v, qid, mx, partials, blockIdx.x);
 }
 
-__global__ __launch_bounds__(PF_BLOCK) void k_fold_init(const double *partials, int G, pf_state *st)
+// The start state: `s` with the sums of the start residual.
+__global__ __launch_bounds__(PF_BLOCK) void k_fold_init(const double *partials, int G, pf_state s, pf_state *st)
 {
     constexpr int qid[2] = {PF_Q_RD, PF_Q_RR};
     constexpr bool mx[2] = {false, false};
     double out[2];
     fold_partials<2>(out, qid, mx, partials, G);
     if (threadIdx.x == 0) {
-        st->up = out[0];
-        st->rr0 = out[1];
-        st->rr = out[1];
-        st->rr_ref = out[1];
-        st->iters = 0;
-        st->breakdown = !isfinite(out[0]) || !isfinite(out[1]);
+        s.up = out[0];
+        s.rr0 = out[1];
+        s.rr = out[1];
+        s.rr_ref = out[1];
+        s.breakdown = !isfinite(out[0]) || !isfinite(out[1]);
         // A zero right-hand side is already solved by x = 0.
-        st->converged = out[1] == 0.0;
-        st->frozen = st->converged || st->breakdown;
-        st->crit = 0.0;
+        s.converged = out[1] == 0.0;
+        s.frozen = s.converged || s.breakdown;
+        *st = s;
+        // also clears the word where an earlier solve set it
+        __hip_atomic_store(s.stop, s.frozen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1945,7 +1954,8 @@ int pf_checon_par(pf_ctx *c, const double *xnew, double tol, int *converged, dou
     return rc;
 }
 
-// pf_pcg_begin, with x starting at x0 (device, neq) when x0 is given.
+// pf_pcg_begin, with x starting at x0 (device, neq) when x0 is given; r0 is
+// read until the stream has passed the copy.
 static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double *x0, const pf_pcg_opts *opts)
 {
     if (!c || !r0 || !opts) return PF_ERR_ARG;
@@ -1989,19 +1999,16 @@ static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double
     s.delta2 = delta * delta;
     s.refine_every = opts->refine_every;
     s.pfresh = 1;
-    *c->state_host = s;
-    PF_HIP(hipMemcpyAsync(c->state, c->state_host, sizeof(pf_state), hipMemcpyHostToDevice, c->stream));
+    s.stop = c->stop_host;
+    __atomic_store_n(c->stop_host, 0, __ATOMIC_RELAXED);
     const int G = pf_grid_for(c->neq);
     float *p32 = opts->precision == PF_PREC_MIXED && c->ntot <= 24 ? c->p32 : nullptr;
     hipLaunchKernelGGL(k_pcg_init, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->x, c->r, c->d, c->p, p32, c->dinv, c->diag,
                        c->f, x0, c->neq, c->precon_given ? 1 : 0, c->partials);
     const int Gi = seq_reduce(c, G, c->r + 1, c->d + 1, PF_Q_RD, c->r + 1, c->r + 1, PF_Q_RR, false, c->neq,
                               nullptr, RUN_ALWAYS);
-    hipLaunchKernelGGL(k_fold_init, dim3(1), dim3(PF_BLOCK), 0, c->stream, c->partials, Gi, c->state);
+    hipLaunchKernelGGL(k_fold_init, dim3(1), dim3(PF_BLOCK), 0, c->stream, c->partials, Gi, s, c->state);
     PF_HIP(hipGetLastError());
-    // The host mirror is read back by pf_pcg_poll; wait so it is not reused
-    // while the copy above is still in flight.
-    PF_HIP(hipStreamSynchronize(c->stream));
     c->pcg_ready = true;
     c->query_pending = false;
     return PF_OK;
@@ -2009,7 +2016,10 @@ static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double
 
 int pf_pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const pf_pcg_opts *opts)
 {
-    return pcg_begin(c, r0, r0_on_device, nullptr, opts);
+    const int rc = pcg_begin(c, r0, r0_on_device, nullptr, opts);
+    if (rc) return rc;
+    PF_HIP(hipStreamSynchronize(c->stream));   // r0 is the caller's again
+    return PF_OK;
 }
 
 }  // extern "C"
@@ -2089,8 +2099,16 @@ static int launch_products(pf_ctx *c, float *p32, int rm)
     }
 }
 
+// Whether the solve has stopped as far as the host knows: the rest of a
+// run's launches would do nothing.  (An earlier solve of the stream may still
+// set the word: pcg_finish looks at the state before it believes it.)
+static bool stop_seen(const pf_ctx *c, bool watch)
+{
+    return watch && __atomic_load_n(c->stop_host, __ATOMIC_RELAXED);
+}
+
 // pf_pcg_run without fold launches (the conditions are the caller's).
-static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *slot)
+static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *slot, bool watch)
 {
     const bool checon = c->opts.stop_mode == PF_STOP_CHECON, mixed = c->opts.precision == PF_PREC_MIXED;
     const bool refines = mixed || c->opts.precision == PF_PREC_MIXED64;
@@ -2098,7 +2116,8 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
     const dim3 grid(G), blk(PF_BLOCK);
     const int fz = c->fix_zero ? 1 : 0;
     hipEvent_t t0, t1;
-    for (int it = 0; it < n; ++it) {
+    bool last = n < 1 || stop_seen(c, watch);
+    for (int it = 0; !last; ++it) {
         const bool formed = form && it > 0;   // the products end the previous iteration and form p
         int rc;
         bool tm = pf_timing_begin(c, PF_K_EBE, &t0, &t1);
@@ -2134,7 +2153,8 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
                                c->f, c->r, c->d, c->dinv, c->neq, c->partials, c->state, 1);
             if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         }
-        if (!form || it + 1 == n) {
+        last = it + 1 >= n || stop_seen(c, watch);
+        if (!form || last) {   // a run ends with its last iteration ended and p formed
             tm = pf_timing_begin(c, PF_K_PUPDATE, &t0, &t1);
             if (tm) PF_HIP(hipEventRecord(t0, c->stream));
             if (checon)
@@ -2152,7 +2172,9 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
 
 extern "C" {
 
-int pf_pcg_run(pf_ctx *c, int n)
+// pf_pcg_run; with watch, no further iterations are enqueued once the host
+// sees that the solve has stopped.
+static int pcg_run(pf_ctx *c, int n, bool watch)
 {
     if (!c || n < 0) return PF_ERR_ARG;
     if (!c->pcg_ready) return PF_ERR_STATE;
@@ -2169,9 +2191,9 @@ int pf_pcg_run(pf_ctx *c, int n)
     const int *slot = rm ? c->csr_slot_t : c->csr_slot;
     const bool ranges = mixed && c->scatter_mode == PF_SCATTER_RANGES;
     if (ranges && !c->rng) return PF_ERR_STATE;   // pf_pcg_begin builds them
-    if (c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE) return run_foldless(c, n, G, p32, rm, slot);
+    if (c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE) return run_foldless(c, n, G, p32, rm, slot, watch);
     hipEvent_t t0, t1;
-    for (int it = 0; it < n; ++it) {
+    for (int it = 0; it < n && !stop_seen(c, watch); ++it) {
         int rc;
         bool tm = pf_timing_begin(c, PF_K_EBE, &t0, &t1);
         if (tm) PF_HIP(hipEventRecord(t0, c->stream));
@@ -2243,6 +2265,8 @@ int pf_pcg_run(pf_ctx *c, int n)
     }
     return PF_OK;
 }
+
+int pf_pcg_run(pf_ctx *c, int n) { return pcg_run(c, n, false); }
 
 int pf_pcg_run_graph(pf_ctx *c, int n)
 {
@@ -2364,26 +2388,39 @@ int pf_pcg_r(pf_ctx *c, double *r, int on_device)
     return PF_OK;
 }
 
-// Iterations in chunks of check_every (default 16) until the state freezes.
+// Iterations until the state freezes.  They are enqueued in chunks of
+// check_every (at most PACE), one chunk ahead of the device and never waiting
+// for a copy of the state: the device sets the stop word in pinned memory, and
+// an event behind each chunk keeps the launches from running further ahead.
+// A poll per 32 iterations left the device idle for about 25 us each and
+// then ran up to 31 iterations' empty launches: 182 iterations of 125 hex20
+// elements 3.08 -> PACE5_MS ms, twenty of 25^3 bricks (p124) 0.57 -> PACE25_MS.
+constexpr int PACE = 16;
 static int pcg_finish(pf_ctx *c, const pf_pcg_opts *opts, pf_pcg_result *R)
 {
-    const int chunk = opts->check_every > 0 ? opts->check_every : 16;
-    int rc = pf_pcg_poll(c, R);
-    while (!rc && !c->state_host->frozen) {
-        int n = chunk;
-        const int left = opts->limit - R->iters;
-        if (n > left) n = left;
-        if (n < 1) n = 1;
-        rc = pf_pcg_run(c, n);
-        if (!rc) rc = pf_pcg_poll(c, R);
+    const int chunk = opts->check_every > 0 && opts->check_every < PACE ? opts->check_every : PACE;
+    for (int done = 0;;) {
+        for (int k = 0; done < opts->limit && !stop_seen(c, true); ++k) {
+            const int n = std::min(chunk, opts->limit - done);
+            const int rc = pcg_run(c, n, true);
+            if (rc) return rc;
+            done += n;
+            PF_HIP(hipEventRecord(c->ev_pace[k & 1], c->stream));
+            if (k) PF_HIP(hipEventSynchronize(c->ev_pace[(k - 1) & 1]));
+        }
+        const int rc = pf_pcg_poll(c, R);
+        if (rc || c->state_host->frozen) return rc;
+        // the word was an earlier solve's, set before this one's start
+        // cleared it; nothing is in flight now
+        __atomic_store_n(c->stop_host, 0, __ATOMIC_RELAXED);
+        done = R->iters;
     }
-    return rc;
 }
 
 int pf_pcg_solve(pf_ctx *c, const double *r0, double *x, const pf_pcg_opts *opts, pf_pcg_result *res)
 {
     if (!c || !r0 || !x || !opts) return PF_ERR_ARG;
-    int rc = pf_pcg_begin(c, r0, 0, opts);
+    int rc = pcg_begin(c, r0, 0, nullptr, opts);
     if (rc) return rc;
     pf_pcg_result tmp{};
     pf_pcg_result *R = res ? res : &tmp;

@@ -189,6 +189,7 @@ __global__ __launch_bounds__(PF_BLOCK) void k_fold_alpha_ranges(const double *fp
         if (!isfinite(alpha)) {
             st->breakdown = 1;
             st->frozen = 1;
+            tell_stop(st);
         }
     }
 }

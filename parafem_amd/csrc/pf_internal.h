@@ -133,6 +133,7 @@ struct pf_state {
     int    refinements;
     int    refine_every;
     int    since_refine;
+    int   *stop;      // the context's stop word in pinned memory (below)
     int    pfresh;    // p holds this iteration's direction (the start); otherwise the
                       // range-fused products of hex8 meshes form p = d + beta p
 };
@@ -233,6 +234,9 @@ struct pf_ctx {
     double *partials = nullptr;        // PF_NQ * PF_REDUCE_MAX_GRID (+ spare)
     pf_state *state = nullptr;         // device: live state and working copy (2)
     pf_state *state_host = nullptr;    // pinned mirror for polling
+    int *stop_host = nullptr;          // pinned: set by the device when the solve stops, so that the host can end a
+                                       // solve's launches without waiting for a copy of the state
+    hipEvent_t ev_pace[2] = {nullptr, nullptr};   // bound how far a solve's launches run ahead of the device
     double *scalar_host = nullptr;     // pinned scratch for primitive results
     pf_pcg_opts opts{};
     bool pcg_ready = false;
