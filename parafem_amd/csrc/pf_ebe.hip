@@ -2032,7 +2032,15 @@ int pf_pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const pf_pcg_opt
 // the folds' launches, at 4,025 (100^3 Laplace) 165 / 123 against 155 / 115;
 // forming p at 404 (20^3) 50.9 / 30.1 against 50.9 / 30.3, at 690 (24^3) 82.2 /
 // 41.3 against 81.9 / 40.3, at 270 (40^3 Laplace) 18.7 against 20.7.
+// The products of a triangle with differences do not form p: their LDS
+// exchange leaves two workgroups of 256 threads a CU (the fold needs them),
+// against eleven of one wavefront (18^3 hex20 35.7 us an iteration with p
+// formed, 33.3 without; 12^3 18.5 either way).
 constexpr int FORM_MAXG = 512;
+static bool forms_p(const pf_ctx *c, int G)
+{
+    return G <= FORM_MAXG && !(c->opts.precision == PF_PREC_FP64 && c->T64d);
+}
 
 template <int NT, int KIND, typename OUT>
 static void launch_ebe_form(pf_ctx *c, OUT *out, int rm, int G)
@@ -2065,7 +2073,6 @@ static void launch_form_due(pf_ctx *c, bool due, int rm, int G)
     case PF_PREC_SPLIT: launch_ebe_form<NT, KIND_ACC, double>(c, c->utemp, rm, G); break;
     default:
         if (!c->T64) launch_ebe_form<NT, KIND_F64, double>(c, c->utemp, rm, G);
-        else if (c->T64d) launch_ebe_form<NT, KIND_TRID, double>(c, c->utemp, rm, G);
         else launch_ebe_form<NT, KIND_TRI, double>(c, c->utemp, rm, G);
         break;
     }
@@ -2112,7 +2119,7 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
 {
     const bool checon = c->opts.stop_mode == PF_STOP_CHECON, mixed = c->opts.precision == PF_PREC_MIXED;
     const bool refines = mixed || c->opts.precision == PF_PREC_MIXED64;
-    const bool form = G <= FORM_MAXG;
+    const bool form = forms_p(c, G);
     const dim3 grid(G), blk(PF_BLOCK);
     const int fz = c->fix_zero ? 1 : 0;
     hipEvent_t t0, t1;
@@ -2394,7 +2401,7 @@ int pf_pcg_r(pf_ctx *c, double *r, int on_device)
 // an event behind each chunk keeps the launches from running further ahead.
 // A poll per 32 iterations left the device idle for about 25 us each and
 // then ran up to 31 iterations' empty launches: 182 iterations of 125 hex20
-// elements 3.08 -> PACE5_MS ms, twenty of 25^3 bricks (p124) 0.57 -> PACE25_MS.
+// elements 3.08 -> 2.7 ms, twenty of 25^3 bricks (p124) 0.57 -> PACE25_MS.
 constexpr int PACE = 16;
 static int pcg_finish(pf_ctx *c, const pf_pcg_opts *opts, pf_pcg_result *R)
 {
