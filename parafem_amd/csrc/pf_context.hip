@@ -60,6 +60,13 @@ int pf_alloc(pf_ctx *c, void **p, size_t bytes)
     return PF_OK;
 }
 
+int *pf_flag_word(pf_ctx *c)
+{
+    int *w = reinterpret_cast<int *>(c->scalar_host + 63);
+    *w = 0;
+    return w;
+}
+
 void pf_free(pf_ctx *c, void *p, size_t bytes)
 {
     (void)bytes;
@@ -512,16 +519,6 @@ static long pack_elems(const pf_ctx *c)
     return n < c->nels ? n : c->nels;
 }
 
-// The flag a packing kernel sets where an entry does not come back exactly: a
-// word of pinned memory, cleared here (nothing of the context is in flight
-// during set-up), so that it costs neither a fill nor a copy.
-static int *tri_flag(pf_ctx *c)
-{
-    int *bad = reinterpret_cast<int *>(c->scalar_host + 63);
-    *bad = 0;
-    return bad;
-}
-
 }  // extern "C"
 
 // FP64 matrices formed chunk by chunk by form(stage, e0, nel) -- into a
@@ -537,7 +534,7 @@ static int form_and_pack(pf_ctx *c, bool colmajor, bool *whole, F form)
     const long chunk = pack_elems(c);
     const size_t sb = (size_t)chunk * c->ntot * c->ntot * sizeof(double);
     double *stage = nullptr;
-    int *bad = tri_flag(c);
+    int *bad = pf_flag_word(c);
     if (!rc) rc = pf_alloc(c, (void **)&stage, sb);
     for (long e0 = 0; !rc && e0 < c->nels; e0 += chunk) {
         const long nel = std::min(chunk, (long)c->nels - e0);
@@ -644,7 +641,7 @@ int pf_assemble_elastic(pf_ctx *c, double e, double v, const double *e_elem, int
         bool whole = keep_whole(c);
         if (!whole) {
             rc = alloc_tri(c, true);
-            int *bad = tri_flag(c);
+            int *bad = pf_flag_word(c);
             if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp, bad);
             if (!rc) {
                 const hipError_t he = hipStreamSynchronize(c->stream);

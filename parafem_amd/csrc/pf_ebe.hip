@@ -2401,7 +2401,7 @@ int pf_pcg_r(pf_ctx *c, double *r, int on_device)
 // an event behind each chunk keeps the launches from running further ahead.
 // A poll per 32 iterations left the device idle for about 25 us each and
 // then ran up to 31 iterations' empty launches: 182 iterations of 125 hex20
-// elements 3.08 -> 2.7 ms, twenty of 25^3 bricks (p124) 0.57 -> PACE25_MS.
+// elements 3.08 -> 2.7 ms, twenty of 25^3 bricks (p124) 0.57 -> 0.44.
 constexpr int PACE = 16;
 static int pcg_finish(pf_ctx *c, const pf_pcg_opts *opts, pf_pcg_result *R)
 {

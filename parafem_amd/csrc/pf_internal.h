@@ -285,6 +285,20 @@ bool pf_ranges_form_p(const pf_ctx *c);   // the range kernels form p (no p pass
 int pf_scan_blocks(long n);
 void pf_scan_launch(pf_ctx *c, const int *cnt, int n, int *bsum, int *ptr, int *total, int *zero_flag);
 
+// A word of pinned memory, cleared, for a set-up kernel to write 1 into (nothing
+// else of the context uses it, and its callers wait for the stream): a flag
+// that costs neither a fill nor a copy.
+int *pf_flag_word(pf_ctx *c);
+
+// The (element, element node) slots of every node in ascending order, built on
+// the device from g_num (device, ns entries; entries outside 1..nn are
+// skipped): ptr (nn + 1), slot (ns).  work: pf_node_work(nn) ints.  *many is
+// set to 1 where a node has more than PF_NODE_SORT slots, whose lists are then
+// not sorted.
+constexpr int PF_NODE_SORT = 64;
+size_t pf_node_work(int nn);
+void pf_node_slots(pf_ctx *c, const int *g_num, int ns, int nn, int *work, int *ptr, int *slot, int *many);
+
 // Looks up, once per device (the device current), the address of the
 // allocation-free entry points' scratch array (pf_ebe.hip).
 int pf_scratch_init(int device);

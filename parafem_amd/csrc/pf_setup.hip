@@ -120,14 +120,9 @@ __global__ __launch_bounds__(256) void k_csr_fill(const int *__restrict__ gg, lo
     }
 }
 
-// Each equation's slots in ascending order (insertion sort of a short list),
-// and, with slot8, their copy in the padded table.
-__global__ __launch_bounds__(256) void k_csr_sort(const int *__restrict__ ptr, int *__restrict__ slot, int neq,
-                                                 int *__restrict__ slot8)
+// slot[a..b) in ascending order: insertion sort of a short list.
+__device__ __forceinline__ void sort_slots(int *__restrict__ slot, int a, int b)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= neq) return;
-    const int a = ptr[q], b = ptr[q + 1];
     for (int i = a + 1; i < b; ++i) {
         const int v = slot[i];
         int j = i - 1;
@@ -137,6 +132,17 @@ __global__ __launch_bounds__(256) void k_csr_sort(const int *__restrict__ ptr, i
         }
         slot[j + 1] = v;
     }
+}
+
+// Each equation's slots in ascending order, and, with slot8, their copy in the
+// padded table.
+__global__ __launch_bounds__(256) void k_csr_sort(const int *__restrict__ ptr, int *__restrict__ slot, int neq,
+                                                 int *__restrict__ slot8)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= neq) return;
+    const int a = ptr[q], b = ptr[q + 1];
+    sort_slots(slot, a, b);
     if (slot8)
         for (int j = 0; j < PF_SLOT8; ++j) slot8[(long)j * neq + q] = a + j < b ? slot[a + j] : -1;
 }
@@ -166,6 +172,36 @@ __global__ __launch_bounds__(256) void k_steer_gather(const int *__restrict__ g_
     }
 }
 
+// Slots per node; *many is set where a node has more than the sort takes.
+__global__ __launch_bounds__(256) void k_node_count(const int *__restrict__ g_num, int ns, int nn,
+                                                   int *__restrict__ cnt, int *__restrict__ many)
+{
+    for (long s = (long)blockIdx.x * blockDim.x + threadIdx.x; s < ns; s += (long)gridDim.x * blockDim.x) {
+        const int g = g_num[s];
+        if (g >= 1 && g <= nn && atomicAdd(&cnt[g - 1], 1) == PF_NODE_SORT) *many = 1;
+    }
+}
+
+// Every slot into its node's list, the counts used up as cursors.
+__global__ __launch_bounds__(256) void k_node_fill(const int *__restrict__ g_num, int ns, int nn,
+                                                  const int *__restrict__ ptr, int *__restrict__ cnt,
+                                                  int *__restrict__ slot)
+{
+    for (long s = (long)blockIdx.x * blockDim.x + threadIdx.x; s < ns; s += (long)gridDim.x * blockDim.x) {
+        const int g = g_num[s];
+        if (g >= 1 && g <= nn) slot[ptr[g - 1] + atomicSub(&cnt[g - 1], 1) - 1] = (int)s;
+    }
+}
+
+// Ascending order of the lists the sort takes (it is quadratic in the length).
+__global__ __launch_bounds__(256) void k_node_sort(const int *__restrict__ ptr, int *__restrict__ slot, int nn)
+{
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= nn) return;
+    const int a = ptr[n], b = ptr[n + 1];
+    if (b - a <= PF_NODE_SORT) sort_slots(slot, a, b);
+}
+
 int grid_for_stride(long n) { return (int)std::max<long>(1, std::min<long>((n + 255) / 256, 16384)); }
 
 }  // namespace
@@ -178,6 +214,21 @@ void pf_scan_launch(pf_ctx *c, const int *cnt, int n, int *bsum, int *ptr, int *
     hipLaunchKernelGGL(k_scan_sums, dim3(nb), dim3(256), 0, c->stream, cnt, n, bsum);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, c->stream, bsum, nb, total);
     hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, c->stream, cnt, n, bsum, ptr, zero_flag);
+}
+
+// work: nn counts, the block sums of the scan, its total and its flags (unused)
+size_t pf_node_work(int nn) { return (size_t)nn + pf_scan_blocks(nn) + 2; }
+
+void pf_node_slots(pf_ctx *c, const int *g_num, int ns, int nn, int *work, int *ptr, int *slot, int *many)
+{
+    int *cnt = work, *bsum = cnt + nn, *total = bsum + pf_scan_blocks(nn);
+    (void)hipMemsetAsync(cnt, 0, (size_t)nn * sizeof(int), c->stream);
+    (void)hipMemsetAsync(ptr, 0, sizeof(int), c->stream);
+    const dim3 gs(grid_for_stride(ns));
+    hipLaunchKernelGGL(k_node_count, gs, dim3(256), 0, c->stream, g_num, ns, nn, cnt, many);
+    pf_scan_launch(c, cnt, nn, bsum, ptr, total, total + 1);
+    hipLaunchKernelGGL(k_node_fill, gs, dim3(256), 0, c->stream, g_num, ns, nn, ptr, cnt, slot);
+    hipLaunchKernelGGL(k_node_sort, dim3((nn + 255) / 256), dim3(256), 0, c->stream, ptr, slot, nn);
 }
 
 // Transposed steering of c->g_g (already on the device, c->neq and c->ntot,

@@ -232,3 +232,25 @@ def test_assembled_triangle_bitexact(nod, box):
         for stop in ("checon", "relres"):
             x, _ = ctx.pcg_solve(pr.r0, 8, 0.0, stop=stop)
             assert np.array_equal(x, _oracle_iterates(pr, stop, 8))
+
+
+# Node maps on both sides of the device's rule (65,536 slots and nodes), with a
+# node of as many elements as the sort takes (64) and of one more, node numbers
+# outside the mesh and a node without elements.
+@pytest.mark.parametrize("nels", [2048, 7281, 7282, 20000])
+@pytest.mark.parametrize("star", [0, 64, 65])
+def test_node_maps(nels, star):
+    rng = np.random.default_rng(nels + star)
+    nod, nn = 8, 7287
+    g = np.empty((nels, nod), dtype=np.int32)
+    # every node but the last in at most 32 elements
+    g[:] = np.resize(rng.permutation(nn - 1) + 1, (nels, nod))
+    if star:
+        g[g == 5] = 6
+        g[rng.choice(nels, star, replace=False), 3] = 5
+    g[1, 1], g[2, 2], g[3, 4] = 0, nn + 1, -3
+    print(f"[gpu-test] node map nels={nels} star={star}", flush=True)
+    with Context(0) as ctx:
+        for numvar, flag in ((1, 1), (3, 0)):
+            c = rng.standard_normal((nels, nod, numvar))
+            assert np.array_equal(ctx.scatter_nodes(g, c, nn, flag), O.scatter_nodes(g, c, nn, flag), equal_nan=True)
