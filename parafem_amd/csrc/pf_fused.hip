@@ -50,15 +50,21 @@ template <int NT> struct RangeShape {
 // the pass 0.058 ms.
 __host__ __device__ constexpr bool range_forms_p(int nt) { return nt <= 24; }
 
-// One workgroup per range of this colour (ranges[blockIdx.x]).
+// One workgroup per range of this colour (desc[blockIdx.x]: range, first entry
+// and length of its equation list, in flight with the state).  A colour is 10
+// workgroups a CU, each a chain of dependent loads: 120x90x75 Laplace bricks
+// 69.4 ms a solve with the range and its offsets looked up one after the
+// other, 66.6 so; two or more ranges side by side in a workgroup are slower
+// (71 and more).
 template <int NT>
 __global__ __launch_bounds__(PF_BLOCK) void k_ebe_range(
     const float *__restrict__ Khi, const unsigned short *__restrict__ lmap, const unsigned char *__restrict__ lround,
-    int nround, const int *__restrict__ rptr, const unsigned *__restrict__ ue, const int *__restrict__ ranges,
+    int nround, const unsigned *__restrict__ ue, const int4 *__restrict__ desc,
     double *__restrict__ p, const double *__restrict__ d, double *__restrict__ u,
     const double *__restrict__ fixstore, int fix_zero, double *__restrict__ rpart, int nels,
     const pf_state *__restrict__ st)
 {
+    const int4 ds = desc[blockIdx.x];
     if (skip(st, RUN_LIVE)) return;
     const double beta = st->beta;
     const bool pnew = range_forms_p(NT) && !st->pfresh;
@@ -69,8 +75,7 @@ __global__ __launch_bounds__(PF_BLOCK) void k_ebe_range(
     __shared__ float pl[PF_BLOCK];                     // fl32(p) per distinct equation
     __shared__ double pacc[PF_BLOCK];                  // sums per distinct equation
     __shared__ __attribute__((aligned(16))) float ps[PF_BLOCK / 64][128];   // p_e twice per element
-    const int r = ranges[blockIdx.x];
-    const int u0 = rptr[r], nu = rptr[r + 1] - u0;
+    const int r = ds.x, u0 = ds.y, nu = ds.z;
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
     const int sub = lane / L::W, li = lane % L::W;
@@ -202,7 +207,7 @@ void launch_ranges_nt(pf_ctx *c)
         const int nb = F.cstart[col + 1] - F.cstart[col];
         if (nb <= 0) continue;
         hipLaunchKernelGGL(k_ebe_range<NT>, dim3(nb), dim3(PF_BLOCK), 0, c->stream, c->K32hi, F.lmap, F.lround,
-                           F.nround, F.rptr, F.ue, F.cperm + F.cstart[col], c->p, c->d, c->u, c->fixstore,
+                           F.nround, F.ue, F.cdesc + F.cstart[col], c->p, c->d, c->u, c->fixstore,
                            c->fix_zero ? 1 : 0, F.rpart, c->nels, c->state);
     }
 }
@@ -375,7 +380,7 @@ void pf_ranges_drop(pf_ctx *c)
     free_dev(c, F.lround, (size_t)F.nels);
     free_dev(c, F.rptr, (size_t)F.nrange + 1);
     free_dev(c, F.ue, (size_t)F.nue);
-    free_dev(c, F.cperm, (size_t)F.nrange);
+    free_dev(c, F.cdesc, (size_t)F.nrange);
     free_dev(c, F.rpart, (size_t)F.nrange + NF);
     delete c->rng;
     c->rng = nullptr;
@@ -450,7 +455,7 @@ int pf_ranges_build(pf_ctx *c)
     rc = pf_alloc(c, (void **)&F.ue, (size_t)std::max<long>(F.nue, 1) * sizeof(unsigned));
     if (!rc) rc = pf_alloc(c, (void **)&rcol, (size_t)nrange * sizeof(int));
     if (!rc) rc = pf_alloc(c, (void **)&mask, ((size_t)c->neq + 1) * sizeof(unsigned));
-    if (!rc) rc = pf_alloc(c, (void **)&F.cperm, (size_t)nrange * sizeof(int));
+    if (!rc) rc = pf_alloc(c, (void **)&F.cdesc, (size_t)nrange * sizeof(int4));
     if (!rc) rc = pf_alloc(c, (void **)&F.rpart, ((size_t)nrange + NF) * sizeof(double));
     if (rc) return fail(rc);
     switch (NT) {
@@ -485,18 +490,19 @@ int pf_ranges_build(pf_ctx *c)
         for (int a = rptr[r]; a < rptr[r + 1]; ++a) used_by[ue[a]] |= 1u << k;
     }
     // ranges by colour, ascending range order inside a colour
-    std::vector<int> cstart(ncol + 1, 0), cperm(nrange);
+    std::vector<int> cstart(ncol + 1, 0);
+    std::vector<int4> cdesc(nrange);
     for (long r = 0; r < nrange; ++r) cstart[col[r] + 1]++;
     for (int k = 0; k < ncol; ++k) cstart[k + 1] += cstart[k];
     {
         std::vector<int> fill(cstart.begin(), cstart.end() - 1);
-        for (long r = 0; r < nrange; ++r) cperm[fill[col[r]]++] = (int)r;
+        for (long r = 0; r < nrange; ++r) cdesc[fill[col[r]]++] = make_int4((int)r, rptr[r], rptr[r + 1] - rptr[r], 0);
     }
     F.ncol = ncol;
     F.cstart = cstart;
     he = hipMemcpyAsync(rcol, col.data(), nrange * sizeof(int), hipMemcpyHostToDevice, c->stream);
     if (he == hipSuccess)
-        he = hipMemcpyAsync(F.cperm, cperm.data(), nrange * sizeof(int), hipMemcpyHostToDevice, c->stream);
+        he = hipMemcpyAsync(F.cdesc, cdesc.data(), nrange * sizeof(int4), hipMemcpyHostToDevice, c->stream);
     if (he == hipSuccess) he = hipMemsetAsync(mask, 0, ((size_t)c->neq + 1) * sizeof(unsigned), c->stream);
     if (he == hipSuccess) {
         hipLaunchKernelGGL(k_rng_mask, dim3(nrange), dim3(PF_BLOCK), 0, c->stream, F.rptr, F.ue, rcol, mask);

@@ -178,11 +178,11 @@ struct pf_ranges {
     unsigned char *lround = nullptr;   // (nels) round of the element inside its range
     int *rptr = nullptr;               // (nrange+1) offsets into ue
     unsigned *ue = nullptr;            // distinct equations per range, ascending, flag bits on top
-    int *cperm = nullptr;              // ranges by colour
+    int4 *cdesc = nullptr;             // by colour: range, first entry and length of its list
     double *rpart = nullptr;           // (nrange) p.u per range
     long nslot = 0, nels = 0, nrange = 0, nue = 0;
     int nround = 1, ncol = 1;
-    std::vector<int> cstart;           // (ncol+1) colour offsets into cperm
+    std::vector<int> cstart;           // (ncol+1) colour offsets into cdesc
 };
 
 struct pf_ctx {
