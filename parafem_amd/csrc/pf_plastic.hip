@@ -1,6 +1,6 @@
 // p122's viscoplastic stress update (src/programs/5th_ed/p122/p122.f90:
-// 164-199) for every element of an 8-node brick mesh, one element per
-// thread, its Gauss points in SAMPLE's order:
+// 164-199) for every element of an 8-node brick mesh, one Gauss point per
+// lane, an element's eight side by side in SAMPLE's order:
 //   eps = MATMUL(bee, eld) - evpt;  sigma = MATMUL(dee, eps);
 //   stress = sigma + tensor;  INVAR;  MOCOUF -> f
 //   final:  devp = stress
@@ -105,30 +105,41 @@ __device__ void formm6(const double s[6], double m1[6][6], double m2[6][6], doub
         }
 }
 
+// Eight elements per wavefront.  A point is one long chain of dependent FP64
+// operations (the invariants, asin, sin, cos, tan), so the points run side by
+// side; their body loads meet in LDS, where the lanes of an element add them
+// in the points' order (a point below yield adds zero, which changes no bit).
+// With an element per lane, which left 18 wavefronts for 1,152 bricks: 1,152
+// bricks at phi = 20 54 -> 8.9 us a call, 8,000 51 -> 9.5, 64,000 61 -> 47,
+// 512,000 467 -> 313.
+constexpr int PL_ELEMS = 64 / 8, PL_PITCH = 25;   // odd pitch: the lanes' entries fall on different banks
 __global__ __launch_bounds__(64) void k_plastic(const double *__restrict__ gc, const int *__restrict__ gg,
                                                const double *__restrict__ x, double *__restrict__ evpt,
                                                double *__restrict__ tensor, double *__restrict__ bload_out, Mc mc,
                                                int nels, int final_pass)
 {
-    const long iel = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (iel >= nels) return;
-    const double *coord = gc + iel * 24;
-    double eld[24];
-    for (int i = 0; i < 24; ++i) {
-        const int g = gg[iel * 24 + i];
-        eld[i] = g ? x[g - 1] : 0.0;
-    }
-    double bload[24];
-    for (int i = 0; i < 24; ++i) bload[i] = 0.0;
-    constexpr int gs[8][3] = {{1, 1, 1}, {1, 1, -1}, {1, -1, 1}, {1, -1, -1},
-                              {-1, 1, 1}, {-1, -1, 1}, {-1, 1, -1}, {-1, -1, -1}};
-    const double r3 = 1.0 / sqrt(3.0);
-    for (int ip = 0; ip < 8; ++ip) {
+    __shared__ double sc[PL_ELEMS][24], se[PL_ELEMS][24], sb[64][PL_PITCH];
+    const int lane = threadIdx.x, sub = lane >> 3, ip = lane & 7;
+    const long iel = (long)blockIdx.x * PL_ELEMS + sub;
+    const bool on = iel < nels;
+    if (on)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int i = ip + 8 * k, g = gg[iel * 24 + i];
+            sc[sub][i] = gc[iel * 24 + i];
+            se[sub][i] = g ? x[g - 1] : 0.0;
+        }
+    __syncthreads();
+    if (on) {
+        const double *eld = se[sub];
+        // SAMPLE's signs: (+++)(++-)(+-+)(+--)(-++)(--+)(-+-)(---)
+        const double r3 = 1.0 / sqrt(3.0);
+        const double xi = ip < 4 ? r3 : -r3, eta = (0x53 >> ip) & 1 ? r3 : -r3, zeta = (0x35 >> ip) & 1 ? r3 : -r3;
         double deriv[3][8];
-        const double det = hex8_deriv(coord, gs[ip][0] > 0 ? r3 : -r3, gs[ip][1] > 0 ? r3 : -r3,
-                                      gs[ip][2] > 0 ? r3 : -r3, deriv);
+        const double det = hex8_deriv(sc[sub], xi, eta, zeta, deriv);
         // eps = MATMUL(bee, eld), BEEMAT's entries in column order
         double eps[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
         for (int m = 0; m < 8; ++m) {
             const double dx = deriv[0][m], dy = deriv[1][m], dz = deriv[2][m];
             const double ux = eld[3 * m], uy = eld[3 * m + 1], uz = eld[3 * m + 2];
@@ -178,22 +189,30 @@ __global__ __launch_bounds__(64) void k_plastic(const double *__restrict__ gc, c
                 devp[a] = s;
             }
         }
-        if (f >= 0.0) {
-            // eload = MATMUL(TRANSPOSE(bee), devp); bload += eload*det*weights(i)
-            for (int m = 0; m < 8; ++m) {
-                const double dx = deriv[0][m], dy = deriv[1][m], dz = deriv[2][m];
-                const double ex = (dx * devp[0] + dy * devp[3]) + dz * devp[5];
-                const double ey = (dy * devp[1] + dx * devp[3]) + dz * devp[4];
-                const double ez = (dz * devp[2] + dy * devp[4]) + dx * devp[5];
-                bload[3 * m] = bload[3 * m] + ex * det * 1.0;
-                bload[3 * m + 1] = bload[3 * m + 1] + ey * det * 1.0;
-                bload[3 * m + 2] = bload[3 * m + 2] + ez * det * 1.0;
-            }
+        // eload = MATMUL(TRANSPOSE(bee), devp); bload += eload*det*weights(i)
+        const bool yields = f >= 0.0;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const double dx = deriv[0][m], dy = deriv[1][m], dz = deriv[2][m];
+            const double ex = (dx * devp[0] + dy * devp[3]) + dz * devp[5];
+            const double ey = (dy * devp[1] + dx * devp[3]) + dz * devp[4];
+            const double ez = (dz * devp[2] + dy * devp[4]) + dx * devp[5];
+            sb[lane][3 * m] = yields ? ex * det * 1.0 : 0.0;
+            sb[lane][3 * m + 1] = yields ? ey * det * 1.0 : 0.0;
+            sb[lane][3 * m + 2] = yields ? ez * det * 1.0 : 0.0;
         }
         if (final_pass)
             for (int r = 0; r < 6; ++r) te[r] = stress[r];
     }
-    for (int i = 0; i < 24; ++i) bload_out[iel * 24 + i] = bload[i];
+    __syncthreads();
+    if (on)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int i = ip + 8 * k;
+            double s = 0.0;
+            for (int q = 0; q < 8; ++q) s = s + sb[(sub << 3) + q][i];
+            bload_out[iel * 24 + i] = s;
+        }
 }
 
 }  // namespace
@@ -218,7 +237,7 @@ extern "C" int pf_plastic_update(pf_ctx *c, const double *x_dev, double *evpt_de
     mc.c = coh;
     mc.psi = psi;
     mc.dt = dt;
-    hipLaunchKernelGGL(k_plastic, dim3((c->nels + 63) / 64), dim3(64), 0, c->stream, c->g_coord, c->g_g, x_dev,
+    hipLaunchKernelGGL(k_plastic, dim3((c->nels + PL_ELEMS - 1) / PL_ELEMS), dim3(64), 0, c->stream, c->g_coord, c->g_g, x_dev,
                        evpt_dev, tensor_dev, utemp_dev, mc, c->nels, final_pass);
     PF_HIP(hipGetLastError());
     return PF_OK;

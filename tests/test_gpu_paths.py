@@ -254,3 +254,32 @@ def test_node_maps(nels, star):
         for numvar, flag in ((1, 1), (3, 0)):
             c = rng.standard_normal((nels, nod, numvar))
             assert np.array_equal(ctx.scatter_nodes(g, c, nn, flag), O.scatter_nodes(g, c, nn, flag), equal_nan=True)
+
+
+# Elements of p122's stress update around the eight of a wavefront.
+@pytest.mark.parametrize("nels", [1, 7, 8, 9, 67])
+@pytest.mark.parametrize("phi", [0.0, 20.0])
+def test_plastic_update_sizes(nels, phi):
+    """Body loads, strains and stresses against the oracle to rounding
+    (trigonometric functions: 1e-11 of each array's scale)."""
+    m = M.box_hex8(nels, 1, 1, 0.5, 0.5, 0.5)
+    rng = np.random.default_rng(nels)
+    m.coords = m.coords + rng.uniform(-0.05, 0.05, m.coords.shape)
+    nf, neq = M.steering(m.nn, 3, M.base_fixed_rest(m))
+    g_g, gc = M.g_g_from(nf, m.g_num), m.g_coord()
+    print(f"[gpu-test] plastic {nels} phi={phi}", flush=True)
+    x = 1e-3 * rng.standard_normal(neq)
+    evpt = 1e-5 * rng.standard_normal((nels, 8, 6))
+    tensor = 20.0 * rng.standard_normal((nels, 8, 6))
+    args = (1e4, 0.3, phi, 15.0, phi / 4, 5e-4)   # some points below yield
+    with Context(0) as ctx:
+        ctx.mesh_set(gc)
+        ctx.steer_set(g_g, neq)
+        dx, dev, dte = DeviceArray.from_host(ctx, x), DeviceArray.from_host(ctx, evpt), DeviceArray.from_host(ctx, tensor)
+        dut = DeviceArray(ctx, nels * 24)
+        for final in (False, True):
+            ctx.plastic_update(dx, dev, dte, dut, *args, final)
+            bl = O.plastic_update(gc, g_g, x, evpt, tensor, *args, final)
+            got = dut.download().reshape(nels, 24)
+            for a, b in ((got, bl), (dev.download().reshape(evpt.shape), evpt), (dte.download().reshape(tensor.shape), tensor)):
+                assert np.abs(b).max() > 0 and np.abs(a - b).max() <= 1e-11 * np.abs(b).max(), final
