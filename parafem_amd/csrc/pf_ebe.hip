@@ -78,6 +78,16 @@ __device__ void finish_iteration(pf_state *st, double rd, double rr, double maxx
 // products of the next iteration end this one and form p = d + p*beta as they
 // gather it; the scatter then stores p (the last iteration of a run ends with
 // k_pupdate_fold, so that p is complete between runs).
+// The mixed solvers' replacement, which five or ten iterations of a solve ask
+// for, costs every iteration of pf_pcg_run its two launches (7 us with their
+// gaps).  A solve, which need not know how many iterations a run of launches
+// completes, parks instead: the end of an iteration that asks for a
+// replacement freezes the state (PF_PARKED), so that what is enqueued behind
+// it does nothing, and the replacement's kernels come only behind every
+// PARK_RUN iterations:
+//   PARK_RUN x {k_ebe, k_scatter_copy, k_update_fold, k_pupdate_fold},
+//   k_ebe_due, k_scatter_res, k_pupdate_fold (resume)
+// The arithmetic is the same, bit for bit.
 // Measured, us per iteration with the folds' launches / without / with p
 // formed in the products (the launches 6 / 4 / 3, mixed 9 / 6 / 5): FP64 hex20
 // 4^3 20.1 / 13.1 / 12.2, 20^3 58 / 51 / 51, mixed 39 / 30 / 30; Laplace 25^3
@@ -86,16 +96,28 @@ __device__ void finish_iteration(pf_state *st, double rd, double rr, double maxx
 // Work state of a running solve: a breakdown stops the iteration it occurs in.
 __device__ __forceinline__ bool stopped(const pf_state *work) { return work->frozen || work->breakdown; }
 
+// Whether the residual (r,r) asks for a true-residual replacement (the rule of
+// fold_update_block).
+__device__ __forceinline__ bool asks_refine(const pf_state &s, double rr)
+{
+    const bool trig = rr <= s.delta2 * s.rr_ref || sqrt(rr / s.rr0) <= s.tol ||
+                      (s.refine_every > 0 && s.since_refine + 1 >= s.refine_every);
+    return trig && isfinite(rr);
+}
+
 // Folds the update's partials (or the replacement's) and ends the iteration
 // of `work`; the lead workgroup writes the new state to *live.  Returns
 // whether the solve has stopped (before or now); *beta is valid otherwise.
 // The state is looked at after the fold's barrier, so that its load, the
 // partials' and the caller's are in flight together: in these small kernels a
-// dependent load is worth 0.7 us.
+// dependent load is worth 0.7 us.  With parks, an iteration that asks for a
+// replacement is left unended and the solve parked; resume ends it behind the
+// replacement, and does nothing otherwise.
 template <bool CHECON>
 __device__ __forceinline__ bool end_iteration(const double *__restrict__ partials, int G, const pf_state *work,
-                                              pf_state *live, bool lead, double *beta)
+                                              pf_state *live, bool lead, double *beta, bool resume = false)
 {
+    if (resume && work->frozen != PF_PARKED) return true;
     const bool ref = !CHECON && work->refine;
     double rd, rr = 0.0, maxx = 0.0, maxdx = 0.0;
     if constexpr (CHECON) {
@@ -115,7 +137,14 @@ __device__ __forceinline__ bool end_iteration(const double *__restrict__ partial
         rr = o[1];
     }
     pf_state s = *work;
+    if (resume) s.frozen = 0;
     if (s.frozen || s.breakdown) return true;
+    if (!CHECON && s.parks && !ref && asks_refine(s, rr)) {
+        s.refine = 1;
+        s.frozen = PF_PARKED;
+        if (lead && threadIdx.x == 0) *live = s;
+        return true;
+    }
     if (s.precision == PF_PREC_MIXED || s.precision == PF_PREC_MIXED64) s.since_refine += 1;
     if (ref) {
         s.refine = 0;
@@ -796,8 +825,12 @@ __global__ __launch_bounds__(PF_BLOCK) void k_scatter_res(const int *__restrict_
                                                          const double *__restrict__ dinv, int neq, double *partials,
                                                          const pf_state *st, int second)
 {
-    // second: an iteration without fold launches (the working state decides)
-    if (second ? stopped(st + 1) || !st[1].refine : skip(st, RUN_REFINE)) return;
+    // second: 1, an iteration without fold launches (the working state
+    // decides); 2, a parked solve
+    if (second == 2   ? st->frozen != PF_PARKED
+        : second == 1 ? stopped(st + 1) || !st[1].refine
+                      : skip(st, RUN_REFINE))
+        return;
     scatter_res_block(blockIdx.x, gridDim.x, ptr, slot, utemp, fixstore, x, f, r, d, dinv, neq, partials, second != 0);
 }
 
@@ -1001,23 +1034,25 @@ __device__ __forceinline__ bool refine_due(const double *__restrict__ partials, 
     double rr[1];
     fold_everywhere<1>(rr, qid, mx, partials, G);
     if (stopped(work)) return false;
-    const bool trig = rr[0] <= work->delta2 * work->rr_ref || sqrt(rr[0] / work->rr0) <= work->tol ||
-                      (work->refine_every > 0 && work->since_refine + 1 >= work->refine_every);
-    const bool due = trig && isfinite(rr[0]);
+    const bool due = asks_refine(*work, rr[0]);
     if (due && lead && threadIdx.x == 0) work->refine = 1;   // cleared by the next scatter's copy
     return due;
 }
 
 // The true-residual products, in few workgroups that loop: on most
-// iterations they only find that nothing is due.
+// iterations they only find that nothing is due.  parked: of a solve that parks
+// (the first workgroup then also copies the settled live state to the working
+// copy, for the end of the iteration).
 template <int NT>
 __global__ __launch_bounds__(PF_BLOCK) void k_ebe_due(const double *__restrict__ K64, const float *__restrict__ Khi,
                                                      const float *__restrict__ Klo, const int *__restrict__ gg,
                                                      const double *__restrict__ x, double *__restrict__ out, int nels,
                                                      long kstride, int rowmajor, long nlb,
-                                                     const double *__restrict__ partials, int G, pf_state *st)
+                                                     const double *__restrict__ partials, int G, pf_state *st,
+                                                     int parked)
 {
-    if (!refine_due(partials, G, st + 1, blockIdx.x == 0)) return;
+    if (parked && blockIdx.x == 0 && threadIdx.x == 0) st[1] = st[0];
+    if (parked ? st->frozen != PF_PARKED : !refine_due(partials, G, st + 1, blockIdx.x == 0)) return;
     for (long lb = xcd_block(blockIdx.x, gridDim.x); lb < nlb; lb += gridDim.x) {
         ebe_block<NT, KIND_ACC, true, double, Lanes<NT, KIND_ACC>::EPL>(lb, K64, Khi, Klo, gg, x, nullptr, out, nels,
                                                                        kstride, rowmajor, false);
@@ -1030,13 +1065,14 @@ __global__ __launch_bounds__(PF_BLOCK) void k_ebe_due(const double *__restrict__
 template <bool CHECON>
 __device__ __forceinline__ void pupdate_fold_block(int lb, int G, double *__restrict__ p, float *__restrict__ p32,
                                                    const double *__restrict__ d, int neq,
-                                                   const double *__restrict__ partials, pf_state *st)
+                                                   const double *__restrict__ partials, pf_state *st,
+                                                   bool resume = false)
 {
     const int q = lb * PF_BLOCK + threadIdx.x + 1;
     const bool live = q <= neq;
     const double dq = live ? d[q] : 0.0, pq = live ? p[q] : 0.0;
     double beta;
-    if (end_iteration<CHECON>(partials, G, st + 1, st, lb == 0, &beta)) return;
+    if (end_iteration<CHECON>(partials, G, st + 1, st, lb == 0, &beta, resume)) return;
     if (live) {
         const double pn = __dadd_rn(dq, __dmul_rn(pq, beta));
         p[q] = pn;
@@ -1047,9 +1083,10 @@ __device__ __forceinline__ void pupdate_fold_block(int lb, int G, double *__rest
 template <bool CHECON>
 __global__ __launch_bounds__(PF_BLOCK) void k_pupdate_fold(double *__restrict__ p, float *__restrict__ p32,
                                                           const double *__restrict__ d, int neq,
-                                                          const double *__restrict__ partials, pf_state *st)
+                                                          const double *__restrict__ partials, pf_state *st,
+                                                          int resume)
 {
-    pupdate_fold_block<CHECON>(blockIdx.x, gridDim.x, p, p32, d, neq, partials, st);
+    pupdate_fold_block<CHECON>(blockIdx.x, gridDim.x, p, p32, d, neq, partials, st, resume != 0);
 }
 
 // PCG start: dinv = 1/diag, d = dinv*r, p = d, x = x0 (or 0), f = r; partial
@@ -1956,7 +1993,27 @@ int pf_checon_par(pf_ctx *c, const double *xnew, double tol, int *converged, dou
 
 // pf_pcg_begin, with x starting at x0 (device, neq) when x0 is given; r0 is
 // read until the stream has passed the copy.
-static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double *x0, const pf_pcg_opts *opts)
+// Iterations of a solve that parks between two looks for a replacement: three
+// launches every PARK_RUN iterations, against half of PARK_RUN empty iterations
+// at every replacement (four launches of 2.2 to 3.3 us each).  Five
+// replacements in 200 to 3,400 iterations (refine_delta 0.01) or ten in 130 to
+// 1,300 (0.1) are usual; replacements that the caller asks for more often keep
+// their launches in every iteration.  Whole solves, ms, with the launches in
+// every iteration and parked for runs of 4 / 6 / 8 / 12 iterations: 12^3 hex20
+// mixed 11.8, 10.4 / 9.5 / 9.5 / 9.5, mixed64 7.8, 7.2 / 6.4 / 6.7 / 7.3; 4^3
+// mixed64 (ten in 126) 2.25, 2.16 / 2.08 / 2.2 / 2.2; 31x17x43 mixed 134.8,
+// 131.3 / 130.6 / 130.0 / 129.1; 40^3 Laplace mixed 6.5, 5.7 / 5.7 / 5.7 / 5.6.
+constexpr int PARK_RUN = 6;
+static bool solve_parks(const pf_ctx *c, const pf_pcg_opts *o)
+{
+    return (o->precision == PF_PREC_MIXED64 ||
+            (o->precision == PF_PREC_MIXED && c->scatter_mode != PF_SCATTER_RANGES)) &&
+           c->csr_slot8 && c->dot_order == PF_DOT_TREE && (o->refine_every == 0 || o->refine_every >= PARK_RUN);
+}
+
+// solve: the run is pcg_finish's, which enqueues iterations until it stops.
+static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double *x0, const pf_pcg_opts *opts,
+                     bool solve)
 {
     if (!c || !r0 || !opts) return PF_ERR_ARG;
     if (!c->have_K) return PF_ERR_STATE;
@@ -1998,6 +2055,7 @@ static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double
     const double delta = opts->refine_delta > 0.0 ? opts->refine_delta : 1e-2;
     s.delta2 = delta * delta;
     s.refine_every = opts->refine_every;
+    s.parks = solve && solve_parks(c, opts);
     s.pfresh = 1;
     s.stop = c->stop_host;
     __atomic_store_n(c->stop_host, 0, __ATOMIC_RELAXED);
@@ -2016,7 +2074,7 @@ static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double
 
 int pf_pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const pf_pcg_opts *opts)
 {
-    const int rc = pcg_begin(c, r0, r0_on_device, nullptr, opts);
+    const int rc = pcg_begin(c, r0, r0_on_device, nullptr, opts, false);
     if (rc) return rc;
     PF_HIP(hipStreamSynchronize(c->stream));   // r0 is the caller's again
     return PF_OK;
@@ -2056,15 +2114,17 @@ static void launch_ebe_form(pf_ctx *c, OUT *out, int rm, int G)
                            A.lo, c->g_g, c->p, out, c->nels, pf_k64_estride(c), rm, c->d, c->partials, G, c->state);
 }
 
+enum { SMALL_FORM = 0, SMALL_DUE = 1, SMALL_PARKED = 2 };
 template <int NT>
-static void launch_form_due(pf_ctx *c, bool due, int rm, int G)
+static void launch_form_due(pf_ctx *c, int what, int rm, int G)
 {
-    if (due) {
+    if (what != SMALL_FORM) {
         constexpr int EPB = Lanes<NT, KIND_ACC>::EPB;
         const long nlb = (c->nels + EPB - 1) / EPB;
         const int grid = (int)std::min<long>(nlb, 768);   // three workgroups per CU
         hipLaunchKernelGGL(k_ebe_due<NT>, dim3(grid), dim3(PF_BLOCK), 0, c->stream, c->K64, c->K32hi, c->K32lo, c->g_g,
-                           c->x, c->utemp, c->nels, pf_k64_estride(c), rm, nlb, c->partials, G, c->state);
+                           c->x, c->utemp, c->nels, pf_k64_estride(c), rm, nlb, c->partials, G, c->state,
+                           what == SMALL_PARKED ? 1 : 0);
         return;
     }
     switch (c->opts.precision) {
@@ -2078,14 +2138,14 @@ static void launch_form_due(pf_ctx *c, bool due, int rm, int G)
     }
 }
 
-// The products that form p (due = false), or the true-residual products of
-// the iterations that ask for them.
-static int launch_small(pf_ctx *c, bool due, int rm, int G)
+// The products that form p, or the true-residual products of an iteration that
+// asks for them, or of a parked solve.
+static int launch_small(pf_ctx *c, int what, int rm, int G)
 {
     switch (c->ntot) {
-    case 60: launch_form_due<60>(c, due, rm, G); break;
-    case 24: launch_form_due<24>(c, due, rm, G); break;
-    case 8: launch_form_due<8>(c, due, rm, G); break;
+    case 60: launch_form_due<60>(c, what, rm, G); break;
+    case 24: launch_form_due<24>(c, what, rm, G); break;
+    case 8: launch_form_due<8>(c, what, rm, G); break;
     default: return PF_ERR_ARG;
     }
     return PF_OK;
@@ -2115,10 +2175,10 @@ static bool stop_seen(const pf_ctx *c, bool watch)
 }
 
 // pf_pcg_run without fold launches (the conditions are the caller's).
-static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *slot, bool watch)
+static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *slot, bool watch, bool parks)
 {
     const bool checon = c->opts.stop_mode == PF_STOP_CHECON, mixed = c->opts.precision == PF_PREC_MIXED;
-    const bool refines = mixed || c->opts.precision == PF_PREC_MIXED64;
+    const bool refines = !parks && (mixed || c->opts.precision == PF_PREC_MIXED64);
     const bool form = forms_p(c, G);
     const dim3 grid(G), blk(PF_BLOCK);
     const int fz = c->fix_zero ? 1 : 0;
@@ -2129,7 +2189,7 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
         int rc;
         bool tm = pf_timing_begin(c, PF_K_EBE, &t0, &t1);
         if (tm) PF_HIP(hipEventRecord(t0, c->stream));
-        rc = formed ? launch_small(c, false, rm, G) : launch_products(c, p32, rm);
+        rc = formed ? launch_small(c, SMALL_FORM, rm, G) : launch_products(c, p32, rm);
         if (rc) return rc;
         if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         tm = pf_timing_begin(c, PF_K_SCATTER, &t0, &t1);
@@ -2154,7 +2214,7 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
         if (refines) {
             tm = pf_timing_begin(c, PF_K_REFINE, &t0, &t1);
             if (tm) PF_HIP(hipEventRecord(t0, c->stream));
-            rc = launch_small(c, true, rm, G);
+            rc = launch_small(c, SMALL_DUE, rm, G);
             if (rc) return rc;
             hipLaunchKernelGGL(k_scatter_res, grid, blk, 0, c->stream, c->csr_ptr, slot, c->utemp, c->fixstore, c->x,
                                c->f, c->r, c->d, c->dinv, c->neq, c->partials, c->state, 1);
@@ -2166,12 +2226,24 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
             if (tm) PF_HIP(hipEventRecord(t0, c->stream));
             if (checon)
                 hipLaunchKernelGGL(k_pupdate_fold<true>, grid, blk, 0, c->stream, c->p, p32, c->d, c->neq, c->partials,
-                                   c->state);
+                                   c->state, 0);
             else
                 hipLaunchKernelGGL(k_pupdate_fold<false>, grid, blk, 0, c->stream, c->p, p32, c->d, c->neq,
-                                   c->partials, c->state);
+                                   c->partials, c->state, 0);
             if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         }
+        PF_HIP(hipGetLastError());
+    }
+    if (parks) {
+        const bool tm = pf_timing_begin(c, PF_K_REFINE, &t0, &t1);
+        if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+        const int rc = launch_small(c, SMALL_PARKED, rm, G);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_scatter_res, grid, blk, 0, c->stream, c->csr_ptr, slot, c->utemp, c->fixstore, c->x, c->f,
+                           c->r, c->d, c->dinv, c->neq, c->partials, c->state, 2);
+        hipLaunchKernelGGL(k_pupdate_fold<false>, grid, blk, 0, c->stream, c->p, p32, c->d, c->neq, c->partials,
+                           c->state, 1);
+        if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         PF_HIP(hipGetLastError());
     }
     return PF_OK;
@@ -2198,7 +2270,14 @@ static int pcg_run(pf_ctx *c, int n, bool watch)
     const int *slot = rm ? c->csr_slot_t : c->csr_slot;
     const bool ranges = mixed && c->scatter_mode == PF_SCATTER_RANGES;
     if (ranges && !c->rng) return PF_ERR_STATE;   // pf_pcg_begin builds them
-    if (c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE) return run_foldless(c, n, G, p32, rm, slot, watch);
+    if (c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE) {
+        if (!watch || !solve_parks(c, &c->opts)) return run_foldless(c, n, G, p32, rm, slot, watch, false);
+        for (int done = 0; done < n && !stop_seen(c, watch); done += PARK_RUN) {
+            const int rc = run_foldless(c, std::min(PARK_RUN, n - done), G, p32, rm, slot, watch, true);
+            if (rc) return rc;
+        }
+        return PF_OK;
+    }
     hipEvent_t t0, t1;
     for (int it = 0; it < n && !stop_seen(c, watch); ++it) {
         int rc;
@@ -2427,7 +2506,7 @@ static int pcg_finish(pf_ctx *c, const pf_pcg_opts *opts, pf_pcg_result *R)
 int pf_pcg_solve(pf_ctx *c, const double *r0, double *x, const pf_pcg_opts *opts, pf_pcg_result *res)
 {
     if (!c || !r0 || !x || !opts) return PF_ERR_ARG;
-    int rc = pcg_begin(c, r0, 0, nullptr, opts);
+    int rc = pcg_begin(c, r0, 0, nullptr, opts, true);
     if (rc) return rc;
     pf_pcg_result tmp{};
     pf_pcg_result *R = res ? res : &tmp;
@@ -2445,7 +2524,7 @@ int pf_pcg_solve_warm(pf_ctx *c, const double *r0, const double *x0, double *xne
     // no residual replacement: its true residual would apply the fixed rows
     // that the caller's r0 = loads - K x0 leaves out
     if (opts->precision != PF_PREC_FP64 && opts->precision != PF_PREC_SPLIT) return PF_ERR_ARG;
-    int rc = pcg_begin(c, r0, 1, x0, opts);
+    int rc = pcg_begin(c, r0, 1, x0, opts, true);
     if (rc) return rc;
     pf_pcg_result tmp{};
     pf_pcg_result *R = res ? res : &tmp;

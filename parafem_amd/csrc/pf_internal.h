@@ -127,16 +127,21 @@ struct pf_state {
     int    stop_mode;
     int    precision;
     int    converged;
-    int    frozen;    // 1 once converged, at the limit, or broken down
+    int    frozen;    // 1 once converged, at the limit, or broken down; PF_PARKED: see below
     int    breakdown;
     int    refine;    // mixed: a true-residual replacement is due this iteration
     int    refinements;
     int    refine_every;
     int    since_refine;
     int   *stop;      // the context's stop word in pinned memory (below)
+    int    parks;     // this solve's replacements wait for the end of a short run
     int    pfresh;    // p holds this iteration's direction (the start); otherwise the
                       // range-fused products of hex8 meshes form p = d + beta p
 };
+
+// frozen while a true-residual replacement is due and its kernels have not run:
+// the iterations enqueued before them do nothing.
+#define PF_PARKED 2
 
 // Multi-RHS block solve (pf_block_solve): up to PF_BLK right-hand sides as
 // the columns of row-major (neq+1) x PF_BLK block vectors.  Column c is kept

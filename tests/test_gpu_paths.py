@@ -283,3 +283,33 @@ def test_plastic_update_sizes(nels, phi):
             got = dut.download().reshape(nels, 24)
             for a, b in ((got, bl), (dev.download().reshape(evpt.shape), evpt), (dte.download().reshape(tensor.shape), tensor)):
                 assert np.abs(b).max() > 0 and np.abs(a - b).max() <= 1e-11 * np.abs(b).max(), final
+
+
+# Solves whose replacements wait for the end of a run of six iterations, and
+# the same iterations run one call at a time: p formed in the products or not
+# (512 | 513 blocks), replacements between, on and right behind a run's end,
+# limits that fall into a run, on its end and on a replacement.
+@pytest.mark.parametrize("el,box", [(20, (4, 4, 4)), (24, (6, 5, 7)), (8, (31, 63, 63)), (8, (32, 63, 63))])
+@pytest.mark.parametrize("precision,every,delta,limit",
+                         [("mixed", 0, 0.0, 20000), ("mixed64", 0, 0.1, 20000), ("mixed64", 0, 0.9, 40),
+                          ("mixed", 6, 0.1, 60), ("mixed64", 7, 0.1, 61), ("mixed", 5, 0.1, 30), ("mixed64", 1, 0.5, 13)])
+def test_parked_replacements(el, box, precision, every, delta, limit):
+    if el == 20:
+        pr = P.elastic_cube(1, nels_xyz=box, lognormal_e=True)
+    elif el == 24:
+        pr = _mesh_problem(24, box)
+    else:
+        pr = P.laplace_cube(1, nels_xyz=box)
+    print(f"[gpu-test] parked {el} {box} {precision} {every} {delta} {limit}", flush=True)
+    kw = dict(stop="relres", precision=precision, refine_delta=delta, refine_every=every)
+    with Context(0) as ctx:
+        r = P.setup(ctx, pr, store="fp32")
+        x, res = ctx.pcg_solve(r, limit, 1e-9, **kw)
+        ctx.pcg_begin(r, limit, 1e-9, **kw)
+        while True:
+            ctx.pcg_run(50)
+            one = ctx.pcg_poll()
+            if one.converged or one.iters >= limit:
+                break
+        assert (res.iters, res.refinements, res.converged) == (one.iters, one.refinements, one.converged)
+        assert res.refinements > 0 and np.array_equal(x, ctx.pcg_x())
