@@ -292,10 +292,13 @@ int pf_create(int device, pf_ctx **out)
     int rc = pf_scratch_init(device);   // device address of the allocation-free scratch
     if (!rc) rc = pf_alloc(c, (void **)&c->state, 2 * sizeof(pf_state));
     if (!rc) rc = pf_alloc(c, (void **)&c->partials, sizeof(double) * kPartials);
-    if (!rc && hipHostMalloc((void **)&c->state_host, sizeof(pf_state), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
-    if (!rc && hipHostMalloc((void **)&c->scalar_host, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
-    if (!rc && hipHostMalloc((void **)&c->state_query, sizeof(pf_state), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
-    if (!rc && hipHostMalloc((void **)&c->stop_host, sizeof(int), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
+    if (!rc && hipHostMalloc((void **)&c->pinned, sizeof(pf_pinned), hipHostMallocDefault) != hipSuccess) rc = PF_ERR_OOM;
+    if (!rc) {
+        c->state_host = &c->pinned->state;
+        c->state_query = &c->pinned->query;
+        c->scalar_host = c->pinned->scalar;
+        c->stop_host = &c->pinned->stop;
+    }
     for (hipEvent_t &e : c->ev_pace)
         if (!rc && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) rc = PF_ERR_HIP;
     if (!rc && hipEventCreateWithFlags(&c->ev_query, hipEventDisableTiming) != hipSuccess) rc = PF_ERR_HIP;
@@ -320,12 +323,9 @@ int pf_destroy(pf_ctx *c)
     reset_problem(c);
     free_arr(c, c->partials, kPartials);
     pf_free(c, c->state, 2 * sizeof(pf_state));
-    if (c->state_host) (void)hipHostFree(c->state_host);
-    if (c->stop_host) (void)hipHostFree(c->stop_host);
+    if (c->pinned) (void)hipHostFree(c->pinned);
     for (hipEvent_t e : c->ev_pace)
         if (e) (void)hipEventDestroy(e);
-    if (c->scalar_host) (void)hipHostFree(c->scalar_host);
-    if (c->state_query) (void)hipHostFree(c->state_query);
     if (c->ev_query) (void)hipEventDestroy(c->ev_query);
     pf_graph_drop(c);
     pf_cache_release(c);

@@ -190,6 +190,13 @@ struct pf_ranges {
     std::vector<int> cstart;           // (ncol+1) colour offsets into cdesc
 };
 
+// The pinned words of a context, in one allocation (each costs about 40 us).
+struct pf_pinned {
+    pf_state state, query;
+    alignas(64) double scalar[64];
+    alignas(64) int stop;
+};
+
 struct pf_ctx {
     int device = 0;
     hipStream_t stream = nullptr;      // stream in use
@@ -238,6 +245,7 @@ struct pf_ctx {
     float *utemp32 = nullptr;          // (ntot,nels) element products, FP32
     double *partials = nullptr;        // PF_NQ * PF_REDUCE_MAX_GRID (+ spare)
     pf_state *state = nullptr;         // device: live state and working copy (2)
+    pf_pinned *pinned = nullptr;       // the four below point into it
     pf_state *state_host = nullptr;    // pinned mirror for polling
     int *stop_host = nullptr;          // pinned: set by the device when the solve stops, so that the host can end a
                                        // solve's launches without waiting for a copy of the state
