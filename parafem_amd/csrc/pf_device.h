@@ -11,13 +11,16 @@ constexpr int MAXG = PF_REDUCE_MAX_GRID;
 
 // K_e storage / arithmetic (TRI, TRID: FP64 packed triangle without and with differences)
 enum { KIND_F64 = 0, KIND_F32 = 1, KIND_ACC = 2, KIND_WIDE = 3, KIND_TRI = 4, KIND_TRID = 5 };
-enum { RUN_ALWAYS = 0, RUN_LIVE = 1, RUN_REFINE = 2 };  // state gating
+enum { RUN_ALWAYS = 0, RUN_LIVE = 1, RUN_REFINE = 2,
+       // a solve that parks: its replacement, and the p update behind it
+       RUN_PARKED = 3, RUN_RESUMED = 4 };  // state gating
 
 __device__ __forceinline__ bool skip(const pf_state *st, int gate)
 {
     if (!st || gate == RUN_ALWAYS) return false;
+    if (gate == RUN_PARKED) return st->frozen != PF_PARKED;
     if (st->frozen) return true;
-    return gate == RUN_REFINE && !st->refine;
+    return (gate == RUN_REFINE && !st->refine) || (gate == RUN_RESUMED && !st->resumed);
 }
 
 // Tells the host that the solve has stopped (one thread, after frozen is set).

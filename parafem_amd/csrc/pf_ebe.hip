@@ -87,7 +87,8 @@ __device__ void finish_iteration(pf_state *st, double rd, double rr, double maxx
 // PARK_RUN iterations:
 //   PARK_RUN x {k_ebe, k_scatter_copy, k_update_fold, k_pupdate_fold},
 //   k_ebe_due, k_scatter_res, k_pupdate_fold (resume)
-// The arithmetic is the same, bit for bit.
+// The arithmetic is the same, bit for bit.  Solves with fold launches park in
+// the same way (k_fold_update parks, k_fold_refine ends the iteration).
 // Measured, us per iteration with the folds' launches / without / with p
 // formed in the products (the launches 6 / 4 / 3, mixed 9 / 6 / 5): FP64 hex20
 // 4^3 20.1 / 13.1 / 12.2, 20^3 58 / 51 / 51, mixed 39 / 30 / 30; Laplace 25^3
@@ -773,6 +774,7 @@ __device__ __forceinline__ void fold_update_block(const double *partials, int G,
                               (st->refine_every > 0 && st->since_refine >= st->refine_every);
             if (trig && isfinite(rr)) {
                 st->refine = 1;
+                if (st->parks) st->frozen = PF_PARKED;
                 return;   // finish_iteration runs after the replacement
             }
         }
@@ -823,14 +825,11 @@ __global__ __launch_bounds__(PF_BLOCK) void k_scatter_res(const int *__restrict_
                                                          const double *__restrict__ x, const double *__restrict__ f,
                                                          double *__restrict__ r, double *__restrict__ d,
                                                          const double *__restrict__ dinv, int neq, double *partials,
-                                                         const pf_state *st, int second)
+                                                         const pf_state *st, int second, int gate)
 {
-    // second: 1, an iteration without fold launches (the working state
-    // decides); 2, a parked solve
-    if (second == 2   ? st->frozen != PF_PARKED
-        : second == 1 ? stopped(st + 1) || !st[1].refine
-                      : skip(st, RUN_REFINE))
-        return;
+    // second: an iteration without fold launches (the working state decides,
+    // unless the solve parks)
+    if (gate == RUN_REFINE && second ? stopped(st + 1) || !st[1].refine : skip(st, gate)) return;
     scatter_res_block(blockIdx.x, gridDim.x, ptr, slot, utemp, fixstore, x, f, r, d, dinv, neq, partials, second != 0);
 }
 
@@ -850,9 +849,18 @@ __device__ __forceinline__ void fold_refine_block(const double *partials, int G,
     }
 }
 
-__global__ __launch_bounds__(PF_BLOCK) void k_fold_refine(const double *partials, int G, pf_state *st)
+// parked: of a solve that parks (the p update behind it asks for resumed).
+__global__ __launch_bounds__(PF_BLOCK) void k_fold_refine(const double *partials, int G, pf_state *st, int parked)
 {
-    if (skip(st, RUN_REFINE)) return;
+    const bool none = skip(st, parked ? RUN_PARKED : RUN_REFINE);
+    if (parked) {
+        __syncthreads();   // every thread has looked at the state
+        if (threadIdx.x == 0) {
+            st->resumed = !none;
+            if (!none) st->frozen = 0;
+        }
+    }
+    if (none) return;
     fold_refine_block(partials, G, st);
 }
 
@@ -874,9 +882,9 @@ __device__ __forceinline__ void pupdate_block(int lb, int G, double *__restrict_
 
 __global__ __launch_bounds__(PF_BLOCK) void k_pupdate(double *__restrict__ p, float *__restrict__ p32,
                                                      const double *__restrict__ d, int neq,
-                                                     const pf_state *__restrict__ st)
+                                                     const pf_state *__restrict__ st, int gate)
 {
-    if (skip(st, RUN_LIVE)) return;
+    if (skip(st, gate)) return;
     pupdate_block(blockIdx.x, gridDim.x, p, p32, d, neq, st);
 }
 
@@ -1388,7 +1396,7 @@ int launch_ebe_nt(pf_ctx *c, const double *src, OUT *out, const pf_state *st, in
                   const float *src32, int rowmajor)
 {
     const double *K64 = Kalt ? Kalt : c->K64;
-    if (gate == RUN_REFINE) {
+    if (gate == RUN_REFINE || gate == RUN_PARKED) {
         if constexpr (KIND == KIND_ACC) {
             // usually does nothing: dispatch few workgroups that loop
             const long nlb = (c->nels + Lanes<NT, KIND>::EPB - 1) / Lanes<NT, KIND>::EPB;
@@ -2003,12 +2011,15 @@ int pf_checon_par(pf_ctx *c, const double *xnew, double tol, int *converged, dou
 // mixed 11.8, 10.4 / 9.5 / 9.5 / 9.5, mixed64 7.8, 7.2 / 6.4 / 6.7 / 7.3; 4^3
 // mixed64 (ten in 126) 2.25, 2.16 / 2.08 / 2.2 / 2.2; 31x17x43 mixed 134.8,
 // 131.3 / 130.6 / 130.0 / 129.1; 40^3 Laplace mixed 6.5, 5.7 / 5.7 / 5.7 / 5.6.
+// With fold launches the replacement's three empty launches are 9 us with their
+// gaps: 82^3 Laplace mixed 43.8 -> 42.2, 120^3 147.8 -> 145.2, 40^3 hex20
+// 270 -> 262, range-fused 120x90x75 Laplace 66.6 -> 63.1; 100^3 hex20, where an
+// empty iteration's 250,000 workgroups cost as much as it saves, 280 either way.
 constexpr int PARK_RUN = 6;
 static bool solve_parks(const pf_ctx *c, const pf_pcg_opts *o)
 {
-    return (o->precision == PF_PREC_MIXED64 ||
-            (o->precision == PF_PREC_MIXED && c->scatter_mode != PF_SCATTER_RANGES)) &&
-           c->csr_slot8 && c->dot_order == PF_DOT_TREE && (o->refine_every == 0 || o->refine_every >= PARK_RUN);
+    return (o->precision == PF_PREC_MIXED64 || o->precision == PF_PREC_MIXED) && c->dot_order == PF_DOT_TREE &&
+           (o->refine_every == 0 || o->refine_every >= PARK_RUN);
 }
 
 // solve: the run is pcg_finish's, which enqueues iterations until it stops.
@@ -2217,7 +2228,7 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
             rc = launch_small(c, SMALL_DUE, rm, G);
             if (rc) return rc;
             hipLaunchKernelGGL(k_scatter_res, grid, blk, 0, c->stream, c->csr_ptr, slot, c->utemp, c->fixstore, c->x,
-                               c->f, c->r, c->d, c->dinv, c->neq, c->partials, c->state, 1);
+                               c->f, c->r, c->d, c->dinv, c->neq, c->partials, c->state, 1, RUN_REFINE);
             if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         }
         last = it + 1 >= n || stop_seen(c, watch);
@@ -2240,7 +2251,7 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
         const int rc = launch_small(c, SMALL_PARKED, rm, G);
         if (rc) return rc;
         hipLaunchKernelGGL(k_scatter_res, grid, blk, 0, c->stream, c->csr_ptr, slot, c->utemp, c->fixstore, c->x, c->f,
-                           c->r, c->d, c->dinv, c->neq, c->partials, c->state, 2);
+                           c->r, c->d, c->dinv, c->neq, c->partials, c->state, 1, RUN_PARKED);
         hipLaunchKernelGGL(k_pupdate_fold<false>, grid, blk, 0, c->stream, c->p, p32, c->d, c->neq, c->partials,
                            c->state, 1);
         if (tm) PF_HIP(hipEventRecord(t1, c->stream));
@@ -2249,35 +2260,10 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
     return PF_OK;
 }
 
-extern "C" {
-
-// pf_pcg_run; with watch, no further iterations are enqueued once the host
-// sees that the solve has stopped.
-static int pcg_run(pf_ctx *c, int n, bool watch)
+// pf_pcg_run with fold launches, or the range-fused products.
+static int run_folds(pf_ctx *c, int n, int G, float *p32, int rm, const int *slot, bool watch, bool parks, bool ranges)
 {
-    if (!c || n < 0) return PF_ERR_ARG;
-    if (!c->pcg_ready) return PF_ERR_STATE;
-    const int G = pf_grid_for(c->neq);
-    const bool mixed = c->opts.precision == PF_PREC_MIXED;
-    const bool wide = c->opts.precision == PF_PREC_MIXED64;
-    float *p32 = mixed && c->ntot <= 24 ? c->p32 : nullptr;
-    // hex8 with FP64 products: row-major (row i of every element side by
-    // side, read back through the matching slot list; the scatter's reads of
-    // consecutive equations then fall on consecutive words).  The FP32
-    // products of the mixed path stay in element order: their 4-byte
-    // row-major writes cost the product more than the scatter saves.
-    const int rm = c->csr_slot_t && !mixed ? 1 : 0;
-    const int *slot = rm ? c->csr_slot_t : c->csr_slot;
-    const bool ranges = mixed && c->scatter_mode == PF_SCATTER_RANGES;
-    if (ranges && !c->rng) return PF_ERR_STATE;   // pf_pcg_begin builds them
-    if (c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE) {
-        if (!watch || !solve_parks(c, &c->opts)) return run_foldless(c, n, G, p32, rm, slot, watch, false);
-        for (int done = 0; done < n && !stop_seen(c, watch); done += PARK_RUN) {
-            const int rc = run_foldless(c, std::min(PARK_RUN, n - done), G, p32, rm, slot, watch, true);
-            if (rc) return rc;
-        }
-        return PF_OK;
-    }
+    const bool mixed = c->opts.precision == PF_PREC_MIXED, wide = c->opts.precision == PF_PREC_MIXED64;
     hipEvent_t t0, t1;
     for (int it = 0; it < n && !stop_seen(c, watch); ++it) {
         int rc;
@@ -2326,7 +2312,7 @@ static int pcg_run(pf_ctx *c, int n, bool watch)
                                c->state);
         }
         if (tm) PF_HIP(hipEventRecord(t1, c->stream));
-        if (mixed || wide) {
+        if ((mixed || wide) && !parks) {
             // True-residual replacement; the kernels do nothing unless the
             // fold above flagged this iteration.
             tm = pf_timing_begin(c, PF_K_REFINE, &t0, &t1);
@@ -2335,19 +2321,65 @@ static int pcg_run(pf_ctx *c, int n, bool watch)
             if (rc) return rc;
             hipLaunchKernelGGL(k_scatter_res, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->csr_ptr, slot,
                                c->utemp, c->fixstore, c->x, c->f, c->r, c->d, c->dinv, c->neq, c->partials,
-                               c->state, 0);
+                               c->state, 0, RUN_REFINE);
             const int Gr = seq_reduce(c, G, c->r + 1, c->d + 1, PF_Q_RD, c->r + 1, c->r + 1, PF_Q_RR, false,
                                       c->neq, c->state, RUN_REFINE);
-            hipLaunchKernelGGL(k_fold_refine, dim3(1), dim3(PF_BLOCK), 0, c->stream, c->partials, Gr, c->state);
+            hipLaunchKernelGGL(k_fold_refine, dim3(1), dim3(PF_BLOCK), 0, c->stream, c->partials, Gr, c->state, 0);
             if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         }
         if (!ranges || !pf_ranges_form_p(c)) {   // else the next range kernels form p
             tm = pf_timing_begin(c, PF_K_PUPDATE, &t0, &t1);
             if (tm) PF_HIP(hipEventRecord(t0, c->stream));
-            hipLaunchKernelGGL(k_pupdate, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->p, p32, c->d, c->neq, c->state);
+            hipLaunchKernelGGL(k_pupdate, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->p, p32, c->d, c->neq, c->state, RUN_LIVE);
             if (tm) PF_HIP(hipEventRecord(t1, c->stream));
         }
         PF_HIP(hipGetLastError());
+    }
+    if (parks) {
+        const bool tm = pf_timing_begin(c, PF_K_REFINE, &t0, &t1);
+        if (tm) PF_HIP(hipEventRecord(t0, c->stream));
+        const int rc =
+            launch_ebe<KIND_ACC, true, double>(c, c->x, c->utemp, c->state, RUN_PARKED, nullptr, nullptr, rm);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_scatter_res, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->csr_ptr, slot, c->utemp, c->fixstore,
+                           c->x, c->f, c->r, c->d, c->dinv, c->neq, c->partials, c->state, 0, RUN_PARKED);
+        hipLaunchKernelGGL(k_fold_refine, dim3(1), dim3(PF_BLOCK), 0, c->stream, c->partials, G, c->state, 1);
+        if (!ranges || !pf_ranges_form_p(c))
+            hipLaunchKernelGGL(k_pupdate, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->p, p32, c->d, c->neq, c->state,
+                               RUN_RESUMED);
+        if (tm) PF_HIP(hipEventRecord(t1, c->stream));
+        PF_HIP(hipGetLastError());
+    }
+    return PF_OK;
+}
+
+extern "C" {
+
+// pf_pcg_run; with watch, no further iterations are enqueued once the host
+// sees that the solve has stopped.
+static int pcg_run(pf_ctx *c, int n, bool watch)
+{
+    if (!c || n < 0) return PF_ERR_ARG;
+    if (!c->pcg_ready) return PF_ERR_STATE;
+    const int G = pf_grid_for(c->neq);
+    const bool mixed = c->opts.precision == PF_PREC_MIXED;
+    float *p32 = mixed && c->ntot <= 24 ? c->p32 : nullptr;
+    // hex8 with FP64 products: row-major (row i of every element side by
+    // side, read back through the matching slot list; the scatter's reads of
+    // consecutive equations then fall on consecutive words).  The FP32
+    // products of the mixed path stay in element order: their 4-byte
+    // row-major writes cost the product more than the scatter saves.
+    const int rm = c->csr_slot_t && !mixed ? 1 : 0;
+    const int *slot = rm ? c->csr_slot_t : c->csr_slot;
+    const bool ranges = mixed && c->scatter_mode == PF_SCATTER_RANGES;
+    if (ranges && !c->rng) return PF_ERR_STATE;   // pf_pcg_begin builds them
+    const bool foldless = c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE;
+    const bool parks = watch && solve_parks(c, &c->opts);
+    for (int done = 0, m; done < n && !(done && stop_seen(c, watch)); done += m) {
+        m = parks ? std::min(PARK_RUN, n - done) : n;
+        const int rc = foldless ? run_foldless(c, m, G, p32, rm, slot, watch, parks)
+                                : run_folds(c, m, G, p32, rm, slot, watch, parks, ranges);
+        if (rc) return rc;
     }
     return PF_OK;
 }

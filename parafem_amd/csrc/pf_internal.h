@@ -135,6 +135,7 @@ struct pf_state {
     int    since_refine;
     int   *stop;      // the context's stop word in pinned memory (below)
     int    parks;     // this solve's replacements wait for the end of a short run
+    int    resumed;   // the last replacement's kernels ended a parked iteration (runs with fold launches)
     int    pfresh;    // p holds this iteration's direction (the start); otherwise the
                       // range-fused products of hex8 meshes form p = d + beta p
 };

@@ -287,13 +287,18 @@ def test_plastic_update_sizes(nels, phi):
 
 # Solves whose replacements wait for the end of a run of six iterations, and
 # the same iterations run one call at a time: p formed in the products or not
-# (512 | 513 blocks), replacements between, on and right behind a run's end,
-# limits that fall into a run, on its end and on a replacement.
-@pytest.mark.parametrize("el,box", [(20, (4, 4, 4)), (24, (6, 5, 7)), (8, (31, 63, 63)), (8, (32, 63, 63))])
+# (512 | 513 blocks), with fold launches (2,049 blocks) and with range-fused
+# products (p formed in them and not), replacements between, on and right behind
+# a run's end, limits that fall into a run, on its end and on a replacement.
+@pytest.mark.parametrize("el,box,scatter", [(20, (4, 4, 4), "slots"), (24, (6, 5, 7), "slots"), (8, (31, 63, 63), "slots"),
+                                            (8, (32, 63, 63), "slots"), (8, (64, 63, 127), "slots"),
+                                            (20, (4, 4, 4), "ranges"), (8, (20, 15, 9), "ranges")])
 @pytest.mark.parametrize("precision,every,delta,limit",
                          [("mixed", 0, 0.0, 20000), ("mixed64", 0, 0.1, 20000), ("mixed64", 0, 0.9, 40),
                           ("mixed", 6, 0.1, 60), ("mixed64", 7, 0.1, 61), ("mixed", 5, 0.1, 30), ("mixed64", 1, 0.5, 13)])
-def test_parked_replacements(el, box, precision, every, delta, limit):
+def test_parked_replacements(el, box, scatter, precision, every, delta, limit):
+    if scatter == "ranges" and precision != "mixed":
+        pytest.skip("range-fused products are the mixed solver's")
     if el == 20:
         pr = P.elastic_cube(1, nels_xyz=box, lognormal_e=True)
     elif el == 24:
@@ -304,6 +309,7 @@ def test_parked_replacements(el, box, precision, every, delta, limit):
     kw = dict(stop="relres", precision=precision, refine_delta=delta, refine_every=every)
     with Context(0) as ctx:
         r = P.setup(ctx, pr, store="fp32")
+        ctx.scatter_mode = scatter
         x, res = ctx.pcg_solve(r, limit, 1e-9, **kw)
         ctx.pcg_begin(r, limit, 1e-9, **kw)
         while True:
@@ -312,4 +318,6 @@ def test_parked_replacements(el, box, precision, every, delta, limit):
             if one.converged or one.iters >= limit:
                 break
         assert (res.iters, res.refinements, res.converged) == (one.iters, one.refinements, one.converged)
-        assert res.refinements > 0 and np.array_equal(x, ctx.pcg_x())
+        assert np.array_equal(x, ctx.pcg_x())
+        # (limit 40 may end before the residual has fallen at all)
+        assert res.refinements > 0 or limit == 40
