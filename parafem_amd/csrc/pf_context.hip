@@ -180,13 +180,19 @@ static void reset_problem(pf_ctx *c)
     free_arr(c, c->g_coord, (size_t)c->nod * 3 * c->nels);
     free_arr(c, c->g_g, (size_t)c->ntot * c->nels);
     free_arr(c, c->csr_ptr, (size_t)c->neq + 1);
-    free_arr(c, c->csr_slot, (size_t)c->nnz);
-    free_arr(c, c->csr_slot_t, (size_t)c->nnz);
-    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
+    pf_csr_drop(c);
     free_arr(c, c->utemp, (size_t)c->ntot * c->nels);
     free_arr(c, c->utemp32, (size_t)c->ntot * c->nels);
     c->nod = c->nels = c->ntot = c->neq = 0;
     c->nnz = 0;
+}
+
+// The slot lists (their offsets stay).
+void pf_csr_drop(pf_ctx *c)
+{
+    free_arr(c, c->csr_slot, (size_t)c->nnz);
+    free_arr(c, c->csr_slot_t, (size_t)c->nnz);
+    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
 }
 
 // A new steering of ntot x nels slots and neq equations: the previous
@@ -205,9 +211,7 @@ int pf_steer_install(pf_ctx *c, int ntot, int nels, int neq)
     free_problem_vectors(c);
     free_arr(c, c->g_g, (size_t)c->ntot * c->nels);
     free_arr(c, c->csr_ptr, (size_t)c->neq + 1);
-    free_arr(c, c->csr_slot, (size_t)c->nnz);
-    free_arr(c, c->csr_slot_t, (size_t)c->nnz);
-    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
+    pf_csr_drop(c);
     free_arr(c, c->utemp, (size_t)c->ntot * c->nels);
     free_arr(c, c->utemp32, (size_t)c->ntot * c->nels);
     c->ntot = ntot;
@@ -237,9 +241,7 @@ void pf_steer_drop(pf_ctx *c)
     free_matrices(c);
     free_arr(c, c->g_g, (size_t)c->ntot * c->nels);
     free_arr(c, c->csr_ptr, (size_t)c->neq + 1);
-    free_arr(c, c->csr_slot, (size_t)c->nnz);
-    free_arr(c, c->csr_slot_t, (size_t)c->nnz);
-    free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
+    pf_csr_drop(c);
     free_arr(c, c->utemp, (size_t)c->ntot * c->nels);
     free_arr(c, c->utemp32, (size_t)c->ntot * c->nels);
     c->ntot = c->neq = 0;

@@ -325,6 +325,7 @@ int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const dou
 // Steering set-up (pf_context.hip, pf_setup.hip).
 int pf_steer_install(pf_ctx *c, int ntot, int nels, int neq);
 void pf_steer_drop(pf_ctx *c);
+void pf_csr_drop(pf_ctx *c);
 int pf_csr_build(pf_ctx *c);
 
 // Largest elements-per-lane-group of the single-RHS element product.

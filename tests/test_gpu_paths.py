@@ -321,3 +321,38 @@ def test_parked_replacements(el, box, scatter, precision, every, delta, limit):
         assert np.array_equal(x, ctx.pcg_x())
         # (limit 40 may end before the residual has fallen at all)
         assert res.refinements > 0 or limit == 40
+
+
+# Node freedom tables made on the device and on the host (the rule: 262,144
+# element nodes and freedoms), with rows that a later one overrides.
+@pytest.mark.parametrize("box", [(20, 20, 19), (28, 28, 29), (29, 28, 29), (60, 28, 30)])
+@pytest.mark.parametrize("rows", ["none", "base", "twice"])
+def test_node_freedoms(box, rows):
+    m = M.box_hex8(*box)
+    nod, n = 8, 3 * m.nn
+    rng = np.random.default_rng(m.nn)
+    rest = np.zeros((0, 4), dtype=np.int32)
+    if rows != "none":
+        rest = M.base_fixed_rest(m)
+    if rows == "twice":     # some nodes again, in any order, with other freedoms
+        again = rng.choice(m.nn, m.nn // 3, replace=True) + 1
+        rest = np.concatenate([rest, np.column_stack([again, rng.integers(0, 2, (again.size, 3))])]).astype(np.int32)
+    free = np.ones((m.nn, 3), dtype=bool)
+    for row in rest:
+        free[row[0] - 1] = row[1:] != 0
+    nf = np.where(free.ravel(), np.cumsum(free.ravel()), 0).reshape(m.nn, 3)
+    print(f"[gpu-test] node freedoms {box} {rows} {m.g_num.size + n}", flush=True)
+    with Context(0) as ctx:
+        ctx.mesh_set(m.g_coord())
+        neq, got = ctx.steer_build(m.g_num, rest, m.nn)
+        assert neq == nf.max() and np.array_equal(np.asarray(got).reshape(m.nn, 3), nf)
+        assert np.array_equal(ctx.steer_get().reshape(m.nels, 24), M.g_g_from(nf, m.g_num).reshape(m.nels, 24))
+        # what is refused leaves the steering as it is
+        bad_num = m.g_num.copy()
+        bad_num[-1, -1] = m.nn + 1
+        bad_rest = np.concatenate([rest, np.array([[0, 1, 1, 1]], dtype=np.int32)]).astype(np.int32)
+        every = np.column_stack([np.arange(1, m.nn + 1), np.zeros((m.nn, 3), dtype=int)]).astype(np.int32)
+        for g, rs in ((bad_num, rest), (m.g_num, bad_rest), (m.g_num, every)):
+            with pytest.raises(Exception):
+                ctx.steer_build(g, rs, m.nn)
+            assert np.array_equal(ctx.steer_get().reshape(m.nels, 24), M.g_g_from(nf, m.g_num).reshape(m.nels, 24))
