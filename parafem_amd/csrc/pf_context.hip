@@ -193,6 +193,8 @@ void pf_csr_drop(pf_ctx *c)
     free_arr(c, c->csr_slot, (size_t)c->nnz);
     free_arr(c, c->csr_slot_t, (size_t)c->nnz);
     free_arr(c, c->csr_slot8, (size_t)PF_SLOT8 * c->neq);
+    free_arr(c, c->nl_code, (size_t)c->neq);
+    free_arr(c, c->nl_slot, (size_t)c->nl_n);
 }
 
 // A new steering of ntot x nels slots and neq equations: the previous

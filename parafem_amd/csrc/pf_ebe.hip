@@ -665,6 +665,64 @@ __global__ __launch_bounds__(PF_BLOCK) void k_scatter_pu(const int *__restrict__
     scatter_pu_block<UT>(blockIdx.x, gridDim.x, ptr, slot, utemp, fixstore, p, u, neq, fix_zero, partials);
 }
 
+// k_scatter_pu with the slot lists of nodes: one list for a node's three
+// freedoms, and a code per equation in place of its two offsets.  The scatter
+// is bound by its reads, of which the equations' own lists are more than a
+// third (hex20, FP32 products: 24 of 60 bytes an equation); these are 11.  100^3
+// hex20 mixed 279 -> 272 ms (150 iterations), 71x63x50 438 -> 424 us an
+// iteration, FP64 893 -> 886, 80^3 hex8 elastic mixed 231 -> 222, FP64 441 ->
+// 431.  A wavefront's lists are one contiguous run, staged in LDS; streaming
+// loads of them are slower here (71x63x50 mixed 429).
+template <typename UT>
+__global__ __launch_bounds__(PF_BLOCK) void k_scatter_nl(const unsigned *__restrict__ code,
+                                                        const int *__restrict__ list, const UT *__restrict__ utemp,
+                                                        const double *__restrict__ fixstore,
+                                                        const double *__restrict__ p, double *__restrict__ u,
+                                                        int neq, int fix_zero, double *partials, const pf_state *st)
+{
+    if (skip(st, RUN_LIVE)) return;
+    constexpr int CAP = 64 * 15;
+    __shared__ int sls[PF_BLOCK / 64][CAP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double acc[1] = {0.0};
+    const int stride = gridDim.x * PF_BLOCK;
+    for (int q0 = blockIdx.x * PF_BLOCK + wave * 64; q0 < neq; q0 += stride) {
+        const int q = q0 + lane;
+        const bool live = q < neq;
+        const unsigned cd = live ? __builtin_nontemporal_load(&code[q]) : 0u;
+        const int off = (int)(cd >> 6), n = (int)(cd >> 2) & 15, d = (int)cd & 3;
+        const int a0 = __builtin_amdgcn_readfirstlane(off);
+        const int a1 = __builtin_amdgcn_readlane(off + n, min(63, neq - 1 - q0));
+        for (int k = lane; k < a1 - a0; k += 64) sls[wave][k] = list[a0 + k];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int *sl = &sls[wave][off - a0];
+        int k8[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) k8[j] = j < n ? sl[j] + d : -1;
+        double v[8], s = 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = k8[j] >= 0 ? (double)utemp[k8[j]] : 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (k8[j] >= 0) s = __dadd_rn(s, v[j]);
+        for (int j = 8; j < n; ++j) s = __dadd_rn(s, (double)utemp[sl[j] + d]);
+        __builtin_amdgcn_wave_barrier();   // these reads finish before the next range is written
+        if (live) {
+            const double pq = p[q + 1];
+            if (fixstore) {
+                const double fs = fixstore[q + 1];
+                if (fs != 0.0) s = fix_zero ? 0.0 : __dmul_rn(pq, fs);
+            }
+            u[q + 1] = s;
+            acc[0] = __dadd_rn(acc[0], __dmul_rn(pq, s));
+        }
+    }
+    constexpr int qid[1] = {PF_Q_PU};
+    constexpr bool mx[1] = {false};
+    block_to_partials<1>(acc, qid, mx, partials, blockIdx.x);
+}
+
 __device__ __forceinline__ void fold_alpha_block(const double *partials, int G, pf_state *st)
 {
     constexpr int qid[1] = {PF_Q_PU};
@@ -2280,7 +2338,13 @@ static int run_folds(pf_ctx *c, int n, int G, float *p32, int rm, const int *slo
         if (ranges) {
             rc = pf_ranges_fold(c);
             if (rc) return rc;
-        } else if (mixed)
+        } else if (c->nl_code && mixed)
+            hipLaunchKernelGGL(k_scatter_nl<float>, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->nl_code, c->nl_slot,
+                               c->utemp32, c->fixstore, c->p, c->u, c->neq, c->fix_zero ? 1 : 0, c->partials, c->state);
+        else if (c->nl_code)
+            hipLaunchKernelGGL(k_scatter_nl<double>, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->nl_code, c->nl_slot,
+                               c->utemp, c->fixstore, c->p, c->u, c->neq, c->fix_zero ? 1 : 0, c->partials, c->state);
+        else if (mixed)
             hipLaunchKernelGGL(k_scatter_pu<float>, dim3(G), dim3(PF_BLOCK), 0, c->stream, c->csr_ptr, slot,
                                c->utemp32, c->fixstore, c->p, c->u, c->neq, c->fix_zero ? 1 : 0, c->partials,
                                c->state);

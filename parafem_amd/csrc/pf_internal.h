@@ -218,6 +218,9 @@ struct pf_ctx {
     int *g_g = nullptr;                // (ntot,nels), 1-based, 0 = restrained
     int *csr_ptr = nullptr;            // (neq+1) offsets into csr_slot
     int *csr_slot = nullptr;           // element slots e*ntot+i, ascending
+    unsigned *nl_code = nullptr;       // (neq) node slot lists: offset << 6 | length << 2 | freedom past the leader, or null
+    int *nl_slot = nullptr;            // the leaders' slots
+    int64_t nl_n = 0;
     int *csr_slot8 = nullptr;          // small problems: the list as PF_SLOT8 planes of neq entries, -1 padded
     int *csr_slot_t = nullptr;         // hex8: the same list as i*nels+e (row-major iteration products)
     int64_t nnz = 0;
@@ -325,6 +328,7 @@ int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const dou
 // Steering set-up (pf_context.hip, pf_setup.hip).
 int pf_steer_install(pf_ctx *c, int ntot, int nels, int neq);
 void pf_steer_drop(pf_ctx *c);
+int pf_node_lists_build(pf_ctx *c);   // optional: nothing is kept where they do not fit
 void pf_csr_drop(pf_ctx *c);
 int pf_csr_build(pf_ctx *c);
 

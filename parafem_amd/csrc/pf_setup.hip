@@ -241,6 +241,53 @@ __global__ __launch_bounds__(256) void k_nf_number(const int *__restrict__ ptr, 
         if (nf[k]) nf[k] = ptr[k + 1];
 }
 
+// Freedoms of a node list the same elements: the slots of freedom d are those
+// of freedom 0 plus d.  Equations past their node's first (the leader) whose
+// slots are the leader's plus k, k <= 2; at equation q: k.
+__device__ __forceinline__ int node_follow(const int *__restrict__ ptr, const int *__restrict__ slot, int q)
+{
+    const int d = slot[ptr[q]] % 3;
+    int k = 0;
+    while (k < d && q - k > 0) {
+        const int a = ptr[q - k - 1], b = ptr[q - k], e = ptr[q - k + 1];
+        if (e - b != b - a) break;
+        bool same = true;
+        for (int j = 0; j < e - b; ++j) same &= slot[b + j] == slot[a + j] + 1;
+        if (!same) break;
+        ++k;
+    }
+    return k;
+}
+
+// The leaders' list lengths (0 for the others) and every equation's code but for
+// the offset; *bad where a list is too long for it.
+__global__ __launch_bounds__(256) void k_node_leaders(const int *__restrict__ ptr, const int *__restrict__ slot, int neq,
+                                                     int *__restrict__ cnt, unsigned *__restrict__ code,
+                                                     int *__restrict__ bad)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= neq) return;
+    const int n = ptr[q + 1] - ptr[q], k = node_follow(ptr, slot, q);
+    if (n > 15) *bad = 1;
+    cnt[q] = k ? 0 : n;
+    code[q] = (unsigned)n << 2 | (unsigned)k;
+}
+
+// The offsets into the codes (off[q + 1]: the leaders' entries up to q) and the
+// leaders' slots into the list.
+__global__ __launch_bounds__(256) void k_node_lists(const int *__restrict__ ptr, const int *__restrict__ slot,
+                                                   const int *__restrict__ off, int neq, unsigned *__restrict__ code,
+                                                   int *__restrict__ list)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= neq) return;
+    const unsigned c = code[q];
+    const int k = c & 3, n = c >> 2, o = off[q - k];
+    code[q] = (unsigned)o << 6 | c;
+    if (k == 0)
+        for (int j = 0; j < n; ++j) list[o + j] = slot[ptr[q] + j];
+}
+
 int grid_for_stride(long n) { return (int)std::max<long>(1, std::min<long>((n + 255) / 256, 16384)); }
 
 }  // namespace
@@ -337,7 +384,7 @@ int pf_csr_build(pf_ctx *c)
     if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
     release();
     if (he != hipSuccess) return pf_set_hip_error(he, "transposed steering", __FILE__, __LINE__);
-    return PF_OK;
+    return c->ntot != 8 && !c->csr_slot8 ? pf_node_lists_build(c) : PF_OK;
 }
 
 // The node freedom table and the check of g_num are made on the device from
@@ -389,6 +436,44 @@ static int nf_device(pf_ctx *c, long nslot, int nodof, const int *g_num, int nn,
     pf_free(c, ptr, psz);
     pf_free(c, bsum, bsz);
     return rc;
+}
+
+// The slot lists of nodes, for element nodes of three freedoms.  They only save
+// reads: without the memory, or where a code does not hold a list, none.
+int pf_node_lists_build(pf_ctx *c)
+{
+    const int neq = c->neq;
+    const size_t csz = (size_t)neq * sizeof(int), psz = ((size_t)neq + 1) * sizeof(int);
+    const size_t bsz = ((size_t)pf_scan_blocks(neq) + 1) * sizeof(int);
+    int *cnt = nullptr, *off = nullptr, *bsum = nullptr, *bad = pf_flag_word(c), *total = bad + 1;   // both pinned
+    hipError_t he = hipSuccess;
+    const dim3 grid((neq + 255) / 256), blk(256);
+    bool ok = !pf_alloc(c, (void **)&c->nl_code, csz) && !pf_alloc(c, (void **)&cnt, csz) &&
+              !pf_alloc(c, (void **)&off, psz) && !pf_alloc(c, (void **)&bsum, bsz);
+    if (ok) {
+        hipLaunchKernelGGL(k_node_leaders, grid, blk, 0, c->stream, c->csr_ptr, c->csr_slot, neq, cnt, c->nl_code, bad);
+        he = hipMemsetAsync(off, 0, sizeof(int), c->stream);
+        pf_scan_launch(c, cnt, neq, bsum, off, total, bsum + pf_scan_blocks(neq));   // zero counts: not looked at
+        if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
+        ok = he == hipSuccess && !*bad && *total < 1 << 26;
+    }
+    if (ok) {
+        c->nl_n = *total;
+        ok = !pf_alloc(c, (void **)&c->nl_slot, (size_t)c->nl_n * sizeof(int));
+    }
+    if (ok) {
+        hipLaunchKernelGGL(k_node_lists, grid, blk, 0, c->stream, c->csr_ptr, c->csr_slot, off, neq, c->nl_code,
+                           c->nl_slot);
+        he = hipGetLastError();
+    }
+    if (!ok || he != hipSuccess) {
+        pf_free(c, c->nl_code, csz);
+        c->nl_code = nullptr;
+    }
+    pf_free(c, cnt, csz);   // later users of these blocks follow on the same stream
+    pf_free(c, off, psz);
+    pf_free(c, bsum, bsz);
+    return he == hipSuccess ? PF_OK : pf_set_hip_error(he, "node lists", __FILE__, __LINE__);
 }
 
 extern "C" int pf_steer_build(pf_ctx *c, int nod, int nels, int nodof, const int *g_num, int nn, int nr,

@@ -356,3 +356,41 @@ def test_node_freedoms(box, rows):
             with pytest.raises(Exception):
                 ctx.steer_build(g, rs, m.nn)
             assert np.array_equal(ctx.steer_get().reshape(m.nels, 24), M.g_g_from(nf, m.g_num).reshape(m.nels, 24))
+
+
+# Slot lists of nodes (above 2,048 blocks of three-freedom nodes): freedoms
+# restrained at random (leaders of each freedom, followers behind a gap), tied
+# ones (lists that agree only in part), and a list too long for its code (the
+# equations' own lists then).
+@pytest.mark.parametrize("nf_kind", ["base", "random", "tied", "long"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_node_slot_lists_bitexact(nf_kind, precision):
+    pr = _mesh_problem(24, (2, 2, 20400))
+    rng = np.random.default_rng(3)
+    nf = pr.nf.copy()
+    if nf_kind == "random":
+        nf[rng.random(nf.shape) < 0.03] = 0
+    elif nf_kind == "tied":         # z of every 50th node tied to z of the next
+        a = np.arange(100, pr.mesh.nn - 1, 50)
+        nf[a + 1, 2] = nf[a, 2]
+    elif nf_kind == "long":         # one equation of 40 nodes
+        a = np.arange(1000, 1040)
+        nf[a, 0] = nf[1000, 0]
+    nf = np.unique(nf, return_inverse=True)[1].reshape(nf.shape)   # 0 stays 0, equations consecutive
+    neq = int(nf.max())
+    assert (neq + 255) // 256 > 2048
+    g_g = M.g_g_from(nf.astype(np.int32), pr.mesh.g_num)
+    r = rng.standard_normal(neq)
+    print(f"[gpu-test] node slot lists {nf_kind} {precision} neq={neq}", flush=True)
+    with Context(0) as ctx:
+        ctx.mesh_set(pr.mesh.g_coord())
+        ctx.steer_set(g_g, neq)
+        ctx.assemble_elastic(100.0, 0.3, store="fp64" if precision == "fp64" else "fp32")
+        x, res = ctx.pcg_solve(r, 4, 0.0, stop="relres", precision=precision)
+        K = O.assemble_elastic(pr.mesh.g_coord(), 100.0, 0.3, nthreads=8)
+        xo = O.pcg(g_g, K, r, O.diag(g_g, K, neq), 0.0, 4, stop=O.STOP_RELRES, dot_order=O.DOT_DEVICE)[0]
+        if precision == "fp64":
+            assert np.array_equal(x, xo)
+        else:
+            # FP32 products: 24 terms of 8 elements at 2^-24, four iterations
+            assert np.abs(x - xo).max() <= 4 * 24 * 8 * 2.0 ** -24 * np.abs(xo).max()
