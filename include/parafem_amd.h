@@ -79,7 +79,7 @@ typedef struct {
     double tol;          /* tolerance for the stopping rule                   */
     int    stop_mode;    /* PF_STOP_*                                          */
     int    precision;    /* PF_PREC_*                                          */
-    int    check_every;  /* host polls convergence every n iterations (0=16)  */
+    int    check_every;  /* iterations enqueued at a time (0 or more than 16: 16) */
     int    refine_every; /* mixed: also replace r at least every n iterations
                             (0 = only on the residual-drop trigger)           */
     double refine_delta; /* mixed: replace r when ||r|| falls below delta

@@ -540,7 +540,8 @@ static int form_and_pack(pf_ctx *c, bool colmajor, bool *whole, F form)
     double *stage = nullptr;
     int *bad = pf_flag_word(c);
     if (!rc) rc = pf_alloc(c, (void **)&stage, sb);
-    for (long e0 = 0; !rc && e0 < c->nels; e0 += chunk) {
+    // (ends early where the word is seen: the rest would be packed for nothing)
+    for (long e0 = 0; !rc && e0 < c->nels && !__atomic_load_n(bad, __ATOMIC_RELAXED); e0 += chunk) {
         const long nel = std::min(chunk, (long)c->nels - e0);
         rc = form(stage, e0, nel);
         if (!rc) rc = pf_launch_tri_pack(c, stage, colmajor, e0, nel, bad);
