@@ -1867,11 +1867,17 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
             __builtin_amdgcn_wave_barrier();
         }
         if (!grid_barrier(bar, nb)) return;
-        for (int b = blockIdx.x; b < total_qb; b += nb) bs_scatter_pu<OUT>(T, qst, ns, b);
+        for (int b = blockIdx.x; b < total_qb; b += nb) {
+            bs_scatter_pu<OUT>(T, qst, ns, b);
+            __syncthreads();   // the block's sums are read before the next one's are written
+        }
         if (!grid_barrier(bar, nb)) return;
         for (int s = blockIdx.x; s < ns; s += nb) bs_fold<0>(T, s);
         if (!grid_barrier(bar, nb)) return;
-        for (int b = blockIdx.x; b < total_qb; b += nb) bs_update<CHECON>(T, qst, ns, b);
+        for (int b = blockIdx.x; b < total_qb; b += nb) {
+            bs_update<CHECON>(T, qst, ns, b);
+            __syncthreads();   // the block's sums are read before the next one's are written
+        }
         if (!grid_barrier(bar, nb)) return;
         for (int s = blockIdx.x; s < ns; s += nb) bs_fold<CHECON ? 1 : 2>(T, s);
         if (!grid_barrier(bar, nb)) return;
@@ -1881,7 +1887,10 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
             if (due) {
                 bs_ebe_refine<NT>(T, est + PF_BATCH_MAX, ns, total_ebr, blockIdx.x, nb);
                 if (!grid_barrier(bar, nb)) return;
-                for (int b = blockIdx.x; b < total_qb; b += nb) bs_scatter_res(T, qst, ns, b);
+                for (int b = blockIdx.x; b < total_qb; b += nb) {
+                    bs_scatter_res(T, qst, ns, b);
+                    __syncthreads();   // the block's sums are read before the next one's are written
+                }
                 if (!grid_barrier(bar, nb)) return;
                 for (int s = blockIdx.x; s < ns; s += nb) bs_fold<3>(T, s);
                 if (!grid_barrier(bar, nb)) return;

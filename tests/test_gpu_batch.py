@@ -143,6 +143,42 @@ def test_batch_with_solo_solves_equals_alone(precision, stop, graph, solo):
             c.close()
 
 
+@pytest.mark.parametrize("el,precision,stop", [("hex20", "fp64", "checon"), ("hex20", "mixed64", "relres"),
+                                               ("hex8", "fp64", "relres"), ("hex8", "mixed", "relres"),
+                                               ("hex8", "split", "checon")])
+def test_persistent_with_more_blocks_than_workgroups(el, precision, stop):
+    """Solves of more equation blocks (256 equations) than workgroups are
+    resident (at most 8 a CU, 2,048), so that a workgroup sums one block after
+    another: the iterates of every solve alone, bit for bit."""
+    if el == "hex20":
+        probs = [P.elastic_cube(n) for n in (31, 8, 30, 5)]
+    else:
+        probs = [P.laplace_cube(n, lognormal_k=True, seed=n) for n in (70, 12, 66, 5)]
+    assert sum((pr.neq + 255) // 256 for pr in probs) > 2048
+    store = "fp64" if precision == "fp64" else "fp32"
+    ctxs = [Context(0) for _ in probs]
+    try:
+        rs = [P.setup(c, pr, store=store) for c, pr in zip(ctxs, probs)]
+        say(f"persistent {el} {precision} {stop}: alone")
+        kw = dict(stop=stop, precision=precision)
+        if precision.startswith("mixed"):
+            kw["refine_delta"] = 0.5          # some replacements among the 24 iterations
+        alone = [c.pcg_solve(r, 24, 0.0, **kw) for c, r in zip(ctxs, rs)]
+        for c, r in zip(ctxs, rs):
+            c.pcg_begin(r, 24, 0.0, **kw)
+        say(f"persistent {el} {precision} {stop}: batched")
+        with Batch(0) as b:
+            for _ in range(3):
+                b.run(ctxs, 9, persistent=True)
+            for c, (x, res) in zip(ctxs, alone):
+                got = c.pcg_poll()
+                assert (got.iters, got.refinements) == (res.iters, res.refinements) and res.iters == 24
+                assert np.array_equal(c.pcg_x(), x)
+    finally:
+        for c in ctxs:
+            c.close()
+
+
 def test_batch_rejects_mixed_settings():
     """Solves of one batch share ntot, precision and stopping rule."""
     from parafem_amd import PFError
