@@ -154,11 +154,15 @@ __device__ __forceinline__ void zero_padding(long e, int lane, float *__restrict
 
 // Difference K(i,j) - K(j,i) as an FP16 multiple of the element's unit (inv =
 // 1/unit, a power of two: both scalings are exact), and whether it brings the
-// entry back exactly as the product will form it.
+// entry back exactly as the product will form it, the sign of a zero included:
+// no difference is the zero of the lower entry's sign, which leaves every upper
+// entry but a zero of the other sign as it is.
 __device__ __forceinline__ _Float16 tri_code(double low, double up, double inv, double unit, bool &fail)
 {
-    const _Float16 h = (_Float16)(float)(__dsub_rn(low, up) * inv);
-    fail |= __fma_rn((double)h, unit, up) != low;
+    const double d = __dsub_rn(low, up);
+    const _Float16 h = (_Float16)(float)(d == 0.0 ? copysign(d, low) : d * inv);
+    const double back = __fma_rn((double)h, unit, up);
+    fail |= !(back == low) || signbit(back) != signbit(low);
     return h;
 }
 
@@ -320,7 +324,8 @@ __global__ __launch_bounds__(64, NOD == 20 ? 2 : 4) void k_assemble_elastic(
             const double2 w = lr[s * (NT - 3 - s) + i - 2];
             const double d0 = __dsub_rn(k[2 * s], w.x), d1 = __dsub_rn(k[2 * s + 1], w.y);
             // with the check of the code below: the entry comes back exactly
-            // (an infinite or undefined one does not)
+            // (an infinite or undefined one does not; a sum that started at
+            // +0 is never -0, so that equal entries are the same bits)
             fail |= __dadd_rn(w.x, d0) != k[2 * s] || __dadd_rn(w.y, d1) != k[2 * s + 1];
             k[2 * s] = d0;
             k[2 * s + 1] = d1;

@@ -170,6 +170,28 @@ def test_fp64_storage_bitexact(ntot, box, kind):
             assert np.array_equal(xg, xo)
 
 
+# Zeros with a sign: equal ones on both sides of the diagonal, one only above or
+# only below it (which the triangle cannot tell, so the matrices stay whole).
+@pytest.mark.parametrize("ntot,box", [(60, (11, 11, 10)), (24, (20, 19, 20)), (8, (41, 40, 40))])
+@pytest.mark.parametrize("where", ["both", "above", "below"])
+def test_fp64_storage_keeps_the_sign_of_zeros(ntot, box, where):
+    pr = _mesh_problem(ntot, box)
+    K = _matrices("ulps", pr.nels, ntot)
+    for a, b in ((0, 2), (1, 5), (3, 7), (4, ntot - 1)):        # K[e, column, row]
+        K[:, a, b] = -0.0 if where in ("both", "below") else 0.0
+        K[:, b, a] = -0.0 if where in ("both", "above") else 0.0
+    print(f"[gpu-test] signed zeros {ntot} {where}", flush=True)
+    with Context(0) as ctx:
+        ctx.mesh_set(pr.g_coord())
+        ctx.steer_set(pr.g_g, pr.neq)
+        before = ctx.mem_used()
+        ctx.storkm_set(K)
+        ctx.trim()
+        packed = ctx.mem_used() - before < 0.8 * K.nbytes
+        assert packed == (where != "below")
+        assert np.array_equal(ctx.storkm_get().view(np.uint64), K.view(np.uint64))
+
+
 def test_batch_of_whole_and_packed_matrices():
     """FP64 contexts that hold whole matrices and ones that hold the triangle
     advance in one batch, each as alone."""
