@@ -493,7 +493,7 @@ static int alloc_k64(pf_ctx *c, int store, bool shared = false)
     return pf_alloc(c, (void **)&c->K64, pf_k64_count(c) * sizeof(double));
 }
 
-// FP64 storage as the packed triangle, with or without differences.
+// FP64 storage as the packed triangle, with or (8 freedoms) without differences.
 static int alloc_tri(pf_ctx *c, bool diffs)
 {
     free_matrices(c);

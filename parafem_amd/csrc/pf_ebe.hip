@@ -189,8 +189,9 @@ enum { FORM_NONE = 0, FORM_CHECON = 1, FORM_RELRES = 2 };
 //   KIND_WIDE: packed symmetric (double)hi, FP64 arithmetic on the FP64 p ->
 //             out (double);
 //   KIND_TRI, KIND_TRID: the FP64 packed triangle (K64, with the differences
-//             in Khi and their units in Klo for TRID), the chain of KIND_F64
-//             on the same entries -> out (double).  Lane i loads the column
+//             in Khi and their units in Klo for TRID; without differences
+//             only 8 freedoms' are stored), the chain of KIND_F64 on the same
+//             entries -> out (double).  Lane i loads the column
 //             pairs that hold its row's entries on and right of the diagonal,
 //             and hands its entry (i, j), j beyond its own pair, to lane j
 //             through LDS (row pair t of the triangle, 16 bytes per lane
@@ -224,6 +225,7 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
     // packed layout: Q quads and R more full diagonals, then the half one (d = H)
     constexpr int D = pf_sym_diags(NT), Q = pf_sym_quads(NT), R = pf_sym_rem(NT), H = NT / 2;
     constexpr long PER = pf_sym_per(NT);
+    static_assert(KIND != KIND_TRI || NT == 8, "a triangle without differences has 8 freedoms");
     static_assert(D == 4 * Q + R + 1, "packed layout");
     // Per wave and element slot: p_e (FP64), or p_e twice (packed kinds).
     constexpr bool ONCE = KIND == KIND_F32 || KIND == KIND_TRI || KIND == KIND_TRID;   // (F32: 64 doubles, 128 floats)
@@ -355,9 +357,8 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
                     __builtin_nontemporal_store((OUT)acc, &out[ev[t] * NT + li]);
             }
         }
-    } else if constexpr (KIND == KIND_TRI || KIND == KIND_TRID) {
+    } else if constexpr (KIND == KIND_TRID) {
         static_assert(EPL == 1, "one element per lane group");
-        constexpr bool DIFF = KIND == KIND_TRID;
         constexpr int LOW = H * (H - 1);   // entries (row pair t, lane j > 2t+1): t(NT-3-t) + j-2
         __shared__ __attribute__((aligned(16))) d2_t low[WPB][L::EPW * LOW];
         d2_t kc[H];
@@ -366,14 +367,12 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
 #pragma unroll
         for (int s = 0; s < H; ++s)   // lanes past the pair's rows read its last entry (unused)
             kc[s] = __builtin_nontemporal_load(&Kp[pf_tri_pair(s, i < 2 * s + 1 ? i : 2 * s + 1)]);
-        double unit = 0.0;
-        if constexpr (DIFF) {
-            const unsigned *Dp = reinterpret_cast<const unsigned *>(Khi) + ec[0] * pf_tri_diffs(NT);
+        const unsigned *Dp = reinterpret_cast<const unsigned *>(Khi) + ec[0] * pf_tri_diffs(NT);
 #pragma unroll
-            for (int s = 0; s < H - 1; ++s)
-                df[s] = __builtin_nontemporal_load(&Dp[pf_tri_diff(NT, s, i > 2 * s + 2 ? i : 2 * s + 2)]);
-            unit = __hiloint2double((int)__builtin_nontemporal_load(reinterpret_cast<const unsigned *>(Klo) + ec[0]), 0);
-        }
+        for (int s = 0; s < H - 1; ++s)
+            df[s] = __builtin_nontemporal_load(&Dp[pf_tri_diff(NT, s, i > 2 * s + 2 ? i : 2 * s + 2)]);
+        const double unit =
+            __hiloint2double((int)__builtin_nontemporal_load(reinterpret_cast<const unsigned *>(Klo) + ec[0]), 0);
         if (form()) return;
         ps[wave][0][lane] = entry(0);
         double *lw = reinterpret_cast<double *>(&low[wave][sub * LOW]);
@@ -396,12 +395,10 @@ __device__ __forceinline__ void ebe_block(long lb, const double *__restrict__ K6
             d2_t v = kc[s];
             if (s < H - 1) {
                 d2_t w = lr[s * (NT - 3 - s) + (i > 2 * s + 2 ? i : 2 * s + 2) - 2];
-                if constexpr (DIFF) {
-                    union { unsigned u; _Float16 h[2]; } x;
-                    x.u = df[s];
-                    w.x = __fma_rn((double)x.h[0], unit, w.x);
-                    w.y = __fma_rn((double)x.h[1], unit, w.y);
-                }
+                union { unsigned u; _Float16 h[2]; } x;
+                x.u = df[s];
+                w.x = __fma_rn((double)x.h[0], unit, w.x);
+                w.y = __fma_rn((double)x.h[1], unit, w.y);
                 v.x = i > 2 * s + 1 ? w.x : v.x;
                 v.y = i > 2 * s + 1 ? w.y : v.y;
             }
@@ -1502,7 +1499,8 @@ int launch_ebe_f64(pf_ctx *c, const double *src, double *out, const pf_state *st
 {
     if (!c->T64) return launch_ebe<KIND_F64, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
     if (c->T64d) return launch_ebe<KIND_TRID, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
-    return launch_ebe<KIND_TRI, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
+    if (c->ntot != 8) return PF_ERR_STATE;   // only 8 freedoms' triangles are stored without differences
+    return launch_ebe_nt<8, KIND_TRI, GATHER, double>(c, src, out, st, gate, nullptr, nullptr, rowmajor);
 }
 
 // FP64 element products of the stored matrices (FP64, or hi+lo for FP32
@@ -1642,9 +1640,9 @@ __device__ __forceinline__ void bs_ebe(const pf_bslot *__restrict__ T, const lon
     else if (KIND == KIND_F64 && S.tri == 2)
         ebe_block<NT, KIND_TRID, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
                                                S.kstride, S.rowmajor, stop);
-    else if (KIND == KIND_F64 && S.tri == 1)
-        ebe_block<NT, KIND_TRI, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
-                                              S.kstride, S.rowmajor, stop);
+    else if (NT == 8 && KIND == KIND_F64 && S.tri == 1)
+        ebe_block<NT, NT == 8 && KIND == KIND_F64 ? KIND_TRI : KIND, true, OUT, EPL>(
+            lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels, S.kstride, S.rowmajor, stop);
     else
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
                                             S.kstride, S.rowmajor, stop);
@@ -2209,9 +2207,13 @@ static void launch_form_due(pf_ctx *c, int what, int rm, int G)
     case PF_PREC_MIXED: launch_ebe_form<NT, KIND_F32, float>(c, c->utemp32, rm, G); break;
     case PF_PREC_MIXED64: launch_ebe_form<NT, KIND_WIDE, double>(c, c->utemp, rm, G); break;
     case PF_PREC_SPLIT: launch_ebe_form<NT, KIND_ACC, double>(c, c->utemp, rm, G); break;
-    default:
-        if (!c->T64) launch_ebe_form<NT, KIND_F64, double>(c, c->utemp, rm, G);
-        else launch_ebe_form<NT, KIND_TRI, double>(c, c->utemp, rm, G);
+    default:   // (products of a triangle with differences do not form p: only 8 freedoms' have none)
+        if constexpr (NT == 8)
+            if (c->T64) {
+                launch_ebe_form<NT, KIND_TRI, double>(c, c->utemp, rm, G);
+                break;
+            }
+        launch_ebe_form<NT, KIND_F64, double>(c, c->utemp, rm, G);
         break;
     }
 }
