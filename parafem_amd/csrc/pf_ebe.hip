@@ -534,6 +534,10 @@ constexpr int TRI_WPB = 1, TRI_MINW = 2;
 // 14 KB of LDS each, so that they come one to a workgroup (TRI_WPB)
 template <int NT, int KIND> constexpr int ebe_wpb() { return NT == 60 && KIND >= KIND_TRI ? TRI_WPB : PF_BLOCK / 64; }
 template <int NT, int KIND> constexpr int ebe_minw() { return NT == 60 && KIND >= KIND_TRI ? TRI_MINW : 1; }
+template <int NT, int KIND> constexpr int ebe_epb()   // elements per workgroup
+{
+    return Lanes<NT, KIND>::EPW * Lanes<NT, KIND>::EPL * ebe_wpb<NT, KIND>();
+}
 
 template <int NT, int KIND, bool GATHER, typename OUT, bool LOOP = false, int EPLT = Lanes<NT, KIND>::EPL>
 __global__ __launch_bounds__((64 * ebe_wpb<NT, KIND>()), (ebe_minw<NT, KIND>())) void k_ebe(const double *__restrict__ K64, const float *__restrict__ Khi,
@@ -1608,8 +1612,14 @@ __device__ __forceinline__ pf_bslot slot_of(const pf_bslot *__restrict__ T, int 
     return S;
 }
 
+// Lists of element blocks: the iteration's products (FP64: of whole matrices, or
+// of every solve where one launch or kernel takes any storage), the true-residual
+// products, FP64 triangles with and without differences.
+enum { EST_ITER = 0, EST_REF = 1, EST_TRID = 2, EST_TRI = 3, EST_LISTS = 4 };
+
 // The solve owning block b: the last solve whose first block is <= b (at
-// most 64 solves, one lane each).
+// most 64 solves, one lane each; a solve without blocks in the list starts
+// where the next one does).
 template <typename I>
 __device__ __forceinline__ int bslot_find(const I *__restrict__ start, int ns, long b)
 {
@@ -1622,30 +1632,39 @@ __device__ __forceinline__ int bslot_find(const I *__restrict__ start, int ns, l
 // the launches per kernel and by the persistent kernel).
 // Element products of every solve: the iteration's product of p (gate
 // RUN_LIVE) or, with REF, the true-residual product of x (gate RUN_REFINE).
-template <int NT, int KIND, typename OUT, bool REF>
+// ANY: KIND_F64's solves as each is stored, chosen at run time.
+template <int NT, int KIND, typename OUT, bool REF, bool ANY>
 __device__ __forceinline__ void bs_ebe(const pf_bslot *__restrict__ T, const long *__restrict__ est, int ns, long gb,
                                        int gate)
 {
-    constexpr int EPL = Lanes<NT, KIND>::EPL;
+    constexpr int EPL = Lanes<NT, KIND>::EPL, WPB = ANY || REF ? PF_BLOCK / 64 : ebe_wpb<NT, KIND>();
     const int s = bslot_find(est, ns, gb);
     const pf_bslot S = slot_of(T, s);
     const bool stop = skip(S.st, gate);
     const long lb = gb - est[s];
-    if constexpr (REF)
+    if constexpr (REF) {
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.x, nullptr, (OUT *)S.utemp, S.nels,
                                             S.kstride, S.rowmajor, stop);
-    else if constexpr (KIND == KIND_F32)
+    } else if constexpr (KIND == KIND_F32) {
         ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, S.p32, (OUT *)S.utemp32, S.nels,
                                             S.kstride, S.rowmajor, stop);
-    else if (KIND == KIND_F64 && S.tri == 2)
-        ebe_block<NT, KIND_TRID, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
-                                               S.kstride, S.rowmajor, stop);
-    else if (NT == 8 && KIND == KIND_F64 && S.tri == 1)
-        ebe_block<NT, NT == 8 && KIND == KIND_F64 ? KIND_TRI : KIND, true, OUT, EPL>(
-            lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels, S.kstride, S.rowmajor, stop);
-    else
-        ebe_block<NT, KIND, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp, S.nels,
-                                            S.kstride, S.rowmajor, stop);
+    } else {
+        if constexpr (ANY && KIND == KIND_F64) {
+            if (S.tri == 2) {
+                ebe_block<NT, KIND_TRID, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr, (OUT *)S.utemp,
+                                                         S.nels, S.kstride, S.rowmajor, stop);
+                return;
+            }
+            if constexpr (NT == 8)
+                if (S.tri == 1) {
+                    ebe_block<NT, KIND_TRI, true, OUT, EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr,
+                                                            (OUT *)S.utemp, S.nels, S.kstride, S.rowmajor, stop);
+                    return;
+                }
+        }
+        ebe_block<NT, KIND, true, OUT, EPL, FORM_NONE, WPB>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.p, nullptr,
+                                                            (OUT *)S.utemp, S.nels, S.kstride, S.rowmajor, stop);
+    }
 }
 
 // The true-residual products of the solves due for a replacement, solve by
@@ -1659,7 +1678,7 @@ __device__ __forceinline__ void bs_ebe_refine(const pf_bslot *__restrict__ T, co
         if (skip(as_global(T[s].st), RUN_REFINE)) continue;
         const long end = s + 1 < ns ? est[s + 1] : total;
         for (long gb = est[s] + b0; gb < end; gb += nb) {
-            bs_ebe<NT, KIND_ACC, double, true>(T, est, ns, gb, RUN_REFINE);
+            bs_ebe<NT, KIND_ACC, double, true, false>(T, est, ns, gb, RUN_REFINE);
             __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
         }
     }
@@ -1733,11 +1752,21 @@ __device__ __forceinline__ void bs_fold(const pf_bslot *__restrict__ T, int s)
     else fold_refine_block(S.partials, S.G, S.st);
 }
 
-// One launch per kernel of the iteration.
-template <int NT, int KIND, typename OUT>
-__global__ __launch_bounds__(PF_BLOCK) void kb_ebe(const pf_bslot *__restrict__ T, const long *__restrict__ est, int ns)
+// One launch per kernel of the iteration.  FP64 products of 60 freedoms are one
+// launch per storage that the batch holds, each over the start list of its own
+// solves: with the storage chosen in the kernel (ANY) every FP64 batch has the
+// LDS and registers of the triangle's products, one workgroup a CU, where whole
+// matrices alone have three (us an iteration, ANY / by launch: 16 hex20 solves
+// of n = 6 to 18, both storages, 206 / 162; 8 of 20 to 24, triangles, 483 / 358;
+// 16 of 6 to 10, whole, 71 / 68).  Of 24 and 8 freedoms, whose ANY keeps four
+// and five wavefronts a SIMD, two storages are one launch: 16 hex8 elastic
+// solves of n = 8 to 20 77 / 80.5.
+constexpr bool one_launch(int nt) { return nt != 60; }
+template <int NT, int KIND, typename OUT, bool ANY = false>
+__global__ __launch_bounds__((64 * ebe_wpb<NT, KIND>()), (ebe_minw<NT, KIND>())) void kb_ebe(
+    const pf_bslot *__restrict__ T, const long *__restrict__ est, int ns)
 {
-    bs_ebe<NT, KIND, OUT, false>(T, est, ns, xcd_block(blockIdx.x, gridDim.x), RUN_LIVE);
+    bs_ebe<NT, KIND, OUT, false, ANY>(T, est, ns, xcd_block(blockIdx.x, gridDim.x), RUN_LIVE);
 }
 
 // The true-residual products: few workgroups, dealt to the solves by their
@@ -1861,7 +1890,7 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
         if (!any) break;
         for (long r0 = 0; r0 < total_eb; r0 += nb) {
             const long gb = r0 + lbx;
-            if (gb < total_eb) bs_ebe<NT, KIND, OUT, false>(T, est, ns, gb, RUN_LIVE);
+            if (gb < total_eb) bs_ebe<NT, KIND, OUT, false, true>(T, est, ns, gb, RUN_LIVE);
             __builtin_amdgcn_wave_barrier();
         }
         if (!grid_barrier(bar, nb)) return;
@@ -1883,7 +1912,7 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
             bool due = false;
             for (int s = 0; s < ns; ++s) due |= !skip(as_global(T[s].st), RUN_REFINE);
             if (due) {
-                bs_ebe_refine<NT>(T, est + PF_BATCH_MAX, ns, total_ebr, blockIdx.x, nb);
+                bs_ebe_refine<NT>(T, est + EST_REF * PF_BATCH_MAX, ns, total_ebr, blockIdx.x, nb);
                 if (!grid_barrier(bar, nb)) return;
                 for (int b = blockIdx.x; b < total_qb; b += nb) {
                     bs_scatter_res(T, qst, ns, b);
@@ -2737,20 +2766,21 @@ struct pf_batch {
     hipEvent_t ev_snap = nullptr;
     std::vector<hipEvent_t> ev_ctx;                // one per solve: its context's stream reached the run
     pf_bslot *T = nullptr;                         // device table
-    long *est = nullptr;                           // device: first element block per solve (iteration
-                                                   // kind), then the same for the FP64 hi+lo products
+    long *est = nullptr;                           // device: first element block per solve, a list per
+                                                   // kind of product (EST_*)
     int *qst = nullptr;                            // device: first equation block per solve
     int *rst = nullptr;                            // device: first workgroup per solve of the replacement's products
     pf_bslot *T_host = nullptr;                    // pinned staging of the three (one allocation)
     long *est_host = nullptr;
     int *qst_host = nullptr, *rst_host = nullptr;
     std::vector<pf_bslot> cur;                     // the table on the device
-    std::vector<long> cur_est;                     // iteration-kind starts, then ACC-kind starts
+    std::vector<long> cur_est;
     std::vector<int> cur_qst, cur_rst;
     int ns = 0, ntot = 0, precision = -1, stop = -1;
-    long total_eb = 0, total_ebr = 0;              // element blocks: iteration kind, true-residual kind
+    long total[EST_LISTS] = {};                    // element blocks of each list
     int total_qb = 0, total_rb = 0;
     bool folds = false;   // some batched solve needs the folds' launches
+    bool any = false;     // FP64 products of any storage in EST_ITER
     pf_state *snap = nullptr, *snap_host = nullptr;
     int snap_n = 0;
     bool snap_pending = false;
@@ -2771,7 +2801,7 @@ struct pf_batch {
     bool stale = false;   // the next run rebuilds the table (and drops the graph)
 };
 
-static const size_t kBatchTable = sizeof(pf_bslot) * PF_BATCH_MAX + 2 * sizeof(long) * PF_BATCH_MAX +
+static const size_t kBatchTable = sizeof(pf_bslot) * PF_BATCH_MAX + EST_LISTS * sizeof(long) * PF_BATCH_MAX +
                                   2 * sizeof(int) * PF_BATCH_MAX;
 
 static void batch_graph_drop(pf_batch *b)
@@ -2792,9 +2822,9 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
     const pf_ctx *c0 = ctxs[0];
     if (!c0) return PF_ERR_ARG;
     std::vector<pf_bslot> T(nctx);
-    std::vector<long> est(2 * (size_t)nctx);
+    std::vector<long> est(EST_LISTS * (size_t)nctx);
     std::vector<int> qst(nctx), rst(nctx);
-    long eb = 0;
+    long total[EST_LISTS] = {};
     int qb = 0;
     bool folds = false;
     for (int k = 0; k < nctx; ++k) {
@@ -2838,15 +2868,16 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
         if (!S.solo) qb += S.G;
         if (mixed && !c->utemp32) return PF_ERR_STATE;
     }
-    // elements per logical block of the iteration's product kind and of the
-    // FP64 hi+lo products (the true residual)
-    int EPB = 0, EPBR = 0;
+    // elements per logical block of each list's products
+    int EPB[EST_LISTS];
     const int prec = c0->opts.precision;
     auto epb = [&](auto nt) {
         constexpr int NT = decltype(nt)::value;
-        EPB = prec == PF_PREC_MIXED ? Lanes<NT, KIND_F32>::EPB
-            : prec == PF_PREC_FP64 ? Lanes<NT, KIND_F64>::EPB : Lanes<NT, KIND_ACC>::EPB;
-        EPBR = Lanes<NT, KIND_ACC>::EPB;
+        EPB[EST_ITER] = prec == PF_PREC_MIXED ? Lanes<NT, KIND_F32>::EPB
+                      : prec == PF_PREC_FP64 ? Lanes<NT, KIND_F64>::EPB : Lanes<NT, KIND_ACC>::EPB;
+        EPB[EST_REF] = Lanes<NT, KIND_ACC>::EPB;
+        EPB[EST_TRID] = ebe_epb<NT, KIND_TRID>();
+        EPB[EST_TRI] = ebe_epb<NT, KIND_TRI>();
         static_assert(Lanes<NT, KIND_ACC>::EPB == Lanes<NT, KIND_WIDE>::EPB, "one lane layout");
     };
     switch (c0->ntot) {
@@ -2855,41 +2886,47 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
     case 8: epb(std::integral_constant<int, 8>()); break;
     default: return PF_ERR_ARG;
     }
-    long ebr = 0;
     std::vector<pf_ctx *> solo;
+    bool held[3] = {false, false, false};
+    for (int k = 0; k < nctx; ++k)
+        if (!T[k].solo) held[T[k].tri] = true;
+    const bool any = persistent || (one_launch(c0->ntot) && held[0] + held[1] + held[2] > 1);
     for (int k = 0; k < nctx; ++k) {
-        est[k] = eb;
-        est[nctx + k] = ebr;
+        for (int l = 0; l < EST_LISTS; ++l) est[l * nctx + k] = total[l];
         if (T[k].solo) {
             solo.push_back(ctxs[k]);
             continue;
         }
-        eb += (T[k].nels + EPB - 1) / EPB;
-        ebr += (T[k].nels + EPBR - 1) / EPBR;
+        const int it = any || !T[k].tri ? EST_ITER : T[k].tri == 2 ? EST_TRID : EST_TRI;
+        total[it] += (T[k].nels + EPB[it] - 1) / EPB[it];
+        total[EST_REF] += (T[k].nels + EPB[EST_REF] - 1) / EPB[EST_REF];
     }
     // about 1,024 workgroups for the replacement's products, at least one a solve
     int rb = 0;
     for (int k = 0; k < nctx; ++k) {
         rst[k] = rb;
-        if (!T[k].solo) rb += 1 + (int)(((T[k].nels + EPBR - 1) / EPBR - 1) * std::min<long>(1024, ebr) / ebr);
+        if (!T[k].solo)
+            rb += 1 + (int)(((T[k].nels + EPB[EST_REF] - 1) / EPB[EST_REF] - 1) * std::min<long>(1024, total[EST_REF]) /
+                            total[EST_REF]);
     }
     PF_HIP(hipSetDevice(b->device));
     const bool same = !b->stale && nctx == b->ns &&
                       std::memcmp(T.data(), b->cur.data(), sizeof(pf_bslot) * nctx) == 0 &&
-                      est == b->cur_est && qst == b->cur_qst && rst == b->cur_rst;
+                      est == b->cur_est && qst == b->cur_qst && rst == b->cur_rst && any == b->any &&
+                      std::equal(total, total + EST_LISTS, b->total);
     if (!same) {
         PF_HIP(hipEventSynchronize(b->ev_table));   // the staging buffer is free again
         std::memcpy(b->T_host, T.data(), sizeof(pf_bslot) * nctx);
-        std::memcpy(b->est_host, est.data(), sizeof(long) * nctx);
-        std::memcpy(b->est_host + PF_BATCH_MAX, est.data() + nctx, sizeof(long) * nctx);
+        for (int l = 0; l < EST_LISTS; ++l)
+            std::memcpy(b->est_host + l * PF_BATCH_MAX, est.data() + l * nctx, sizeof(long) * nctx);
         std::memcpy(b->qst_host, qst.data(), sizeof(int) * nctx);
         std::memcpy(b->rst_host, rst.data(), sizeof(int) * nctx);
         PF_HIP(hipMemcpyAsync(b->T, b->T_host, kBatchTable, hipMemcpyHostToDevice, b->stream));
         PF_HIP(hipEventRecord(b->ev_table, b->stream));
         // a captured graph reads the batched solves from the table, but
         // holds the solo solves' launches with their own buffers
-        if (eb != b->total_eb || ebr != b->total_ebr || qb != b->total_qb || rb != b->total_rb ||
-            folds != b->folds || nctx != b->ns || c0->ntot != b->ntot ||
+        if (!std::equal(total, total + EST_LISTS, b->total) || qb != b->total_qb || rb != b->total_rb ||
+            folds != b->folds || any != b->any || nctx != b->ns || c0->ntot != b->ntot ||
             c0->opts.precision != b->precision || c0->opts.stop_mode != b->stop || !solo.empty() ||
             !b->solo.empty() || b->stale)
             batch_graph_drop(b);
@@ -2901,9 +2938,9 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
         b->cur_rst = rst;
         b->total_rb = rb;
         b->folds = folds;
+        b->any = any;
         b->ns = nctx;
-        b->total_eb = eb;
-        b->total_ebr = ebr;
+        std::copy(total, total + EST_LISTS, b->total);
         b->total_qb = qb;
         b->ntot = c0->ntot;
         b->precision = c0->opts.precision;
@@ -2929,21 +2966,27 @@ static int batch_release(pf_batch *b, int nctx, pf_ctx *const *ctxs)
     return PF_OK;
 }
 
-template <int NT, int KIND, typename OUT>
-static void batch_launch_ebe(pf_batch *b)
+template <int NT, int KIND, typename OUT, bool ANY = false>
+static void batch_launch_ebe(pf_batch *b, int list)
 {
-    hipLaunchKernelGGL((kb_ebe<NT, KIND, OUT>), dim3((unsigned)b->total_eb), dim3(PF_BLOCK), 0, b->stream, b->T,
-                       b->est, b->ns);
+    if (!b->total[list]) return;
+    hipLaunchKernelGGL((kb_ebe<NT, KIND, OUT, ANY>), dim3((unsigned)b->total[list]), dim3(64 * ebe_wpb<NT, KIND>()), 0,
+                       b->stream, b->T, b->est + list * PF_BATCH_MAX, b->ns);
 }
 
 template <int NT>
 static void batch_iteration_nt(pf_batch *b)
 {
     const int prec = b->precision;
-    if (prec == PF_PREC_MIXED) batch_launch_ebe<NT, KIND_F32, float>(b);
-    else if (prec == PF_PREC_MIXED64) batch_launch_ebe<NT, KIND_WIDE, double>(b);
-    else if (prec == PF_PREC_SPLIT) batch_launch_ebe<NT, KIND_ACC, double>(b);
-    else batch_launch_ebe<NT, KIND_F64, double>(b);
+    if (prec == PF_PREC_MIXED) batch_launch_ebe<NT, KIND_F32, float>(b, EST_ITER);
+    else if (prec == PF_PREC_MIXED64) batch_launch_ebe<NT, KIND_WIDE, double>(b, EST_ITER);
+    else if (prec == PF_PREC_SPLIT) batch_launch_ebe<NT, KIND_ACC, double>(b, EST_ITER);
+    else if (one_launch(NT) && b->any) batch_launch_ebe<NT, KIND_F64, double, one_launch(NT)>(b, EST_ITER);
+    else {
+        batch_launch_ebe<NT, KIND_F64, double>(b, EST_ITER);
+        batch_launch_ebe<NT, KIND_TRID, double>(b, EST_TRID);
+        if constexpr (NT == 8) batch_launch_ebe<NT, KIND_TRI, double>(b, EST_TRI);
+    }
     const dim3 gq((unsigned)b->total_qb), gs((unsigned)b->ns), blk(PF_BLOCK);
     if (prec == PF_PREC_MIXED)
         hipLaunchKernelGGL(kb_scatter_pu<float>, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
@@ -2978,7 +3021,7 @@ static int batch_launch_persistent(pf_batch *b, int max_iters)
     if (per_cu < 1) return PF_ERR_ARG;
     // every workgroup resident (the cooperative launch refuses otherwise),
     // no more than the largest phase has blocks
-    const long most = std::max<long>(std::max<long>(b->total_eb, b->total_qb), b->ns);
+    const long most = std::max<long>(std::max<long>(b->total[EST_ITER], b->total_qb), b->ns);
     int grid = (int)std::min<long>((long)per_cu * b->cus, most);
     if (grid < 1) grid = 1;
     PF_HIP(hipMemsetAsync(b->bar, 0, sizeof(pf_gbar), b->stream));
@@ -2986,7 +3029,7 @@ static int batch_launch_persistent(pf_batch *b, int max_iters)
     const long *est = b->est;
     const int *qst = b->qst;
     int ns = b->ns, tq = b->total_qb, mi = max_iters;
-    long te = b->total_eb, ter = b->total_ebr;
+    long te = b->total[EST_ITER], ter = b->total[EST_REF];
     pf_gbar *bar = b->bar;
     void *args[] = {(void *)&T, (void *)&est, (void *)&qst, (void *)&ns, (void *)&te, (void *)&ter, (void *)&tq,
                     (void *)&mi, (void *)&bar};
@@ -3026,7 +3069,7 @@ static int batch_iterations(pf_batch *b, int n)
             c->stream = own;
             if (rc) return rc;
         }
-        if (b->total_eb > 0) {
+        if (b->total_qb > 0) {
             switch (b->ntot) {
             case 60: batch_iteration_nt<60>(b); break;
             case 24: batch_iteration_nt<24>(b); break;
@@ -3073,13 +3116,13 @@ int pf_batch_create(int device, pf_batch **out)
     if (dt) {
         b->T = (pf_bslot *)dt;
         b->est = (long *)((char *)dt + sizeof(pf_bslot) * PF_BATCH_MAX);
-        b->qst = (int *)((char *)b->est + 2 * sizeof(long) * PF_BATCH_MAX);
+        b->qst = (int *)((char *)b->est + EST_LISTS * sizeof(long) * PF_BATCH_MAX);
         b->rst = b->qst + PF_BATCH_MAX;
     }
     if (ht) {
         b->T_host = (pf_bslot *)ht;
         b->est_host = (long *)((char *)ht + sizeof(pf_bslot) * PF_BATCH_MAX);
-        b->qst_host = (int *)((char *)b->est_host + 2 * sizeof(long) * PF_BATCH_MAX);
+        b->qst_host = (int *)((char *)b->est_host + EST_LISTS * sizeof(long) * PF_BATCH_MAX);
         b->rst_host = b->qst_host + PF_BATCH_MAX;
     }
     if (e != hipSuccess) {

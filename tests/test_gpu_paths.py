@@ -218,6 +218,59 @@ def test_batch_of_whole_and_packed_matrices():
         ctx.close()
 
 
+# One batch of solves of every storage that a mesh's FP64 matrices can have, each
+# storage's products a launch of their own over its own solves: storages first,
+# last, between and alone in the batch.
+@pytest.mark.parametrize("ntot,small,large", [(60, (5, 4, 3), (11, 11, 10)), (24, (7, 5, 4), (20, 19, 20)),
+                                              (8, (9, 7, 5), (41, 40, 40))])
+@pytest.mark.parametrize("order", ["wdWtD", "DtdwW", "dD", "wW", "t"])
+def test_batch_of_every_storage(ntot, small, large, order):
+    if ntot != 8:
+        order = order.replace("t", "")
+    if not order:
+        pytest.skip("only 8 freedoms have triangles without differences")
+    ctxs, prs, alone = [], [], []
+    print(f"[gpu-test] batch storages {ntot} {order}", flush=True)
+    for k, o in enumerate(order):
+        pr = _mesh_problem(ntot, large if o in "dDW" else small)
+        pr.r0 = np.random.default_rng(k).standard_normal(pr.neq)
+        ctx = Context(0)
+        if o == "t":            # assembled hex8 Laplace: the triangle without differences
+            P.setup(ctx, pr)
+        else:                   # w, W: whole (small; too wide a difference); d, D: with differences
+            ctx.mesh_set(pr.g_coord())
+            ctx.steer_set(pr.g_g, pr.neq)
+            ctx.storkm_set(_matrices("wide" if o == "W" else "ulps", pr.nels, ntot, k))
+        alone.append(ctx.pcg_solve(pr.r0, 9, 0.0, stop="relres")[0])
+        ctxs.append(ctx)
+        prs.append(pr)
+    with Batch(0) as b:
+        for kw in (dict(graph=True), dict(persistent=True), dict(graph=False), dict(graph=True)):
+            for ctx, pr in zip(ctxs, prs):
+                ctx.pcg_begin(pr.r0, 9, 0.0, stop="relres")
+            b.run(ctxs, 5, **kw)
+            b.run(ctxs, 5, **kw)
+            for ctx, x in zip(ctxs, alone):
+                assert ctx.pcg_poll().iters == 9 and np.array_equal(ctx.pcg_x(), x), kw
+    for ctx in ctxs:
+        ctx.close()
+
+
+def test_one_large_solve_persistent_and_by_launches():
+    """A single solve above 2,048 blocks, whose start lists and table are the
+    same for the persistent kernel and for launches, but not its lists' lengths."""
+    pr = P.laplace_cube(81)
+    assert (pr.neq + 255) // 256 > 2048
+    with Context(0) as ctx, Batch(0) as b:
+        r = P.setup(ctx, pr)
+        x = ctx.pcg_solve(r, 9, 0.0, stop="relres")[0]
+        for kw in (dict(persistent=True), dict(graph=False), dict(persistent=True), dict(graph=True), dict(graph=False)):
+            ctx.pcg_begin(r, 9, 0.0, stop="relres")
+            b.run([ctx], 5, **kw)
+            b.run([ctx], 5, **kw)
+            assert ctx.pcg_poll().iters == 9 and np.array_equal(ctx.pcg_x(), x), kw
+
+
 def test_assembly_that_the_triangle_cannot_hold():
     """A degenerate element (zero determinant: undefined entries) is stored
     whole, as the evaluation gives it."""
