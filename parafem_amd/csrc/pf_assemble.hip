@@ -481,8 +481,9 @@ __global__ void k_from_colmajor(const double *__restrict__ src, double *__restri
 
 // FP64 matrices (column pairs, or column-major) -> packed triangle.  One lane
 // group per element (lane = row), the whole matrix in LDS; every entry below
-// the diagonal is reconstructed as the product will and compared.  Bound by
-// the reads of src, which a bounded chunk leaves in the last-level cache.
+// the diagonal is reconstructed as the product will and compared (with T null
+// only that).  Bound by the reads of src, which a bounded chunk leaves in the
+// last-level cache.
 template <int NT, bool COLMAJOR>
 __global__ __launch_bounds__(64) void k_tri_pack(const double *__restrict__ src, double *__restrict__ T,
                                                 unsigned *__restrict__ diff, unsigned *__restrict__ unit, long e0,
@@ -524,18 +525,29 @@ __global__ __launch_bounds__(64) void k_tri_pack(const double *__restrict__ src,
         for (int s = 0; s < H; ++s) {
             const double a = M[i * PITCH + 2 * s], b = M[i * PITCH + 2 * s + 1];
             if (i <= 2 * s + 1) {
-                Te[pf_tri_pair(s, i)] = make_double2(a, b);
+                if (T) Te[pf_tri_pair(s, i)] = make_double2(a, b);
                 continue;
             }
             const double ua = M[2 * s * PITCH + i], ub = M[(2 * s + 1) * PITCH + i];
             union { unsigned u; _Float16 h[2]; } w;
             w.h[0] = tri_code(a, ua, inv, un, fail);
             w.h[1] = tri_code(b, ub, inv, un, fail);
-            De[pf_tri_diff(NT, s, i)] = w.u;
+            if (T) De[pf_tri_diff(NT, s, i)] = w.u;
         }
-        if (i == 0) unit[e] = uh;
+        if (T && i == 0) unit[e] = uh;
     }
     if (fail) *bad = 1;
+}
+
+// Elements 0 .. nel - 1 of the packed triangle -> column pairs.
+__global__ void k_tri_unpack(pf_f64_view V, double *__restrict__ K, int nt, long nel)
+{
+    const long nn = (long)nt * nt, n = nel * nn;
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
+        const long el = q / nn, w = q - el * nn;
+        const int j = (int)(w / nt), i = (int)(w - (long)j * nt);
+        K[pf_idx_pair(el, nt, i, j)] = pf_f64_entry(V, el, nt, i, j);
+    }
 }
 
 // internal layout -> storkm_pp chunk (FP64, or packed symmetric hi + lo).
@@ -647,13 +659,21 @@ static void launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0
 
 int pf_launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad)
 {
-    if (!c->T64 || !c->T64d || !c->T64u) return PF_ERR_STATE;
+    if (c->T64 && (!c->T64d || !c->T64u)) return PF_ERR_STATE;
     switch (c->ntot) {
     case 60: launch_tri_pack<60>(c, src, colmajor, e0, nel, bad); break;
     case 24: launch_tri_pack<24>(c, src, colmajor, e0, nel, bad); break;
     case 8: launch_tri_pack<8>(c, src, colmajor, e0, nel, bad); break;
     default: return PF_ERR_ARG;
     }
+    PF_HIP(hipGetLastError());
+    return PF_OK;
+}
+
+int pf_launch_tri_unpack(pf_ctx *c, double *K, long nel)
+{
+    if (!c->T64) return PF_ERR_STATE;
+    hipLaunchKernelGGL(k_tri_unpack, dim3(8192), dim3(256), 0, c->stream, pf_f64(c), K, c->ntot, nel);
     PF_HIP(hipGetLastError());
     return PF_OK;
 }

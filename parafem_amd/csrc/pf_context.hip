@@ -525,12 +525,12 @@ static long pack_elems(const pf_ctx *c)
 
 }  // extern "C"
 
-// FP64 matrices formed chunk by chunk by form(stage, e0, nel) -- into a
-// bounded staging buffer, as column pairs or column-major -- and packed into
-// the triangle.  *whole is set, and nothing kept, where an entry does not
-// come back exactly: the caller then stores whole matrices.
+// FP64 matrices formed chunk by chunk on the device by form(stage, e0, nel) --
+// into a bounded staging buffer, as column pairs -- and packed into the
+// triangle.  *whole is set, and nothing kept, where an entry does not come back
+// exactly: the caller then forms whole matrices.
 template <class F>
-static int form_and_pack(pf_ctx *c, bool colmajor, bool *whole, F form)
+static int form_and_pack(pf_ctx *c, bool *whole, F form)
 {
     *whole = keep_whole(c);
     if (*whole) return PF_OK;
@@ -544,7 +544,7 @@ static int form_and_pack(pf_ctx *c, bool colmajor, bool *whole, F form)
     for (long e0 = 0; !rc && e0 < c->nels && !__atomic_load_n(bad, __ATOMIC_RELAXED); e0 += chunk) {
         const long nel = std::min(chunk, (long)c->nels - e0);
         rc = form(stage, e0, nel);
-        if (!rc) rc = pf_launch_tri_pack(c, stage, colmajor, e0, nel, bad);
+        if (!rc) rc = pf_launch_tri_pack(c, stage, false, e0, nel, bad);
     }
     const hipError_t he = hipStreamSynchronize(c->stream);
     if (!rc && he != hipSuccess) rc = pf_set_hip_error(he, "packing", __FILE__, __LINE__);
@@ -717,7 +717,7 @@ int pf_assemble_transient(pf_ctx *c, double theta, double dtim, int np_types, co
     };
     bool whole = store == PF_STORE_FP32;   // the hi/lo split reads whole matrices
     if (!rc && !whole)
-        rc = form_and_pack(c, false, &whole, [&](double *Ka, long e0, long nel) {
+        rc = form_and_pack(c, &whole, [&](double *Ka, long e0, long nel) {
             const int r = alloc_b();
             return r ? r : pf_launch_assemble_transient(c, theta, dtim, dprop, dtype, Ka, e0, nel);
         });
@@ -742,6 +742,26 @@ static long staging_elems(const pf_ctx *c)
     return n < c->nels ? n : c->nels;
 }
 
+// Whole matrices in the place of a triangle that holds elements 0 .. done - 1:
+// those unpacked on the device.  *again is set where memory does not hold both:
+// the whole matrices are there, without those elements.
+static int tri_to_whole(pf_ctx *c, long done, bool *again)
+{
+    double *K = nullptr;
+    int rc = pf_alloc(c, (void **)&K, pf_k64_count(c) * sizeof(double));
+    *again = rc == PF_ERR_OOM && done;
+    if (*again) return alloc_k64(c, PF_STORE_FP64);
+    if (!rc && done) {
+        rc = pf_launch_tri_unpack(c, K, done);
+        if (!rc) {
+            free_matrices(c);       // (its blocks are only used again behind the unpacking)
+            pf_cache_release(c);    // a triangle and whole matrices are not kept both
+        }
+    }
+    c->K64 = K;
+    return rc;
+}
+
 int pf_storkm_set(pf_ctx *c, const double *storkm, int store)
 {
     if (!c || !storkm) return PF_ERR_ARG;
@@ -749,27 +769,46 @@ int pf_storkm_set(pf_ctx *c, const double *storkm, int store)
     PF_HIP(hipSetDevice(c->device));
     if (store != PF_STORE_FP64 && store != PF_STORE_FP32) return PF_ERR_ARG;
     const long nn = (long)c->ntot * c->ntot;
-    if (store == PF_STORE_FP64) {
-        bool whole = false;
-        const int rp = form_and_pack(c, true, &whole, [&](double *dst, long e0, long nel) {
-            const hipError_t he = hipMemcpyAsync(dst, storkm + e0 * nn, (size_t)nel * nn * sizeof(double),
-                                                 hipMemcpyHostToDevice, c->stream);
-            return he == hipSuccess ? PF_OK : pf_set_hip_error(he, "storkm upload", __FILE__, __LINE__);
-        });
-        if (rp) return rp;
-        if (!whole) return finish_matrices(c);
+    // The triangle, as long as every entry comes back exactly: the first chunk
+    // is looked at before memory is taken for either storage, and from a chunk
+    // on that the triangle does not hold the matrices are whole.  Every element
+    // is uploaded once: 8,000 hex20 elements without symmetry 7.8 ms (packed,
+    // then uploaded again from the start: 15.6).
+    const bool pack = store == PF_STORE_FP64 && !keep_whole(c);
+    const long chunk = pack ? pack_elems(c) : staging_elems(c);
+    int rc = PF_OK;
+    if (pack) {
+        free_matrices(c);
+        c->store = store;
+        c->k_shared = false;
+    } else {
+        rc = alloc_k64(c, store);
     }
-    int rc = alloc_k64(c, store);
-    if (rc) return rc;
-    const long chunk = staging_elems(c);
     double *stage = nullptr;
-    rc = pf_alloc(c, (void **)&stage, (size_t)chunk * nn * sizeof(double));
+    int *bad = pf_flag_word(c);
+    if (!rc) rc = pf_alloc(c, (void **)&stage, (size_t)chunk * nn * sizeof(double));
     for (long e0 = 0; !rc && e0 < c->nels; e0 += chunk) {
         const long nel = std::min(chunk, (long)c->nels - e0);
         hipError_t he = hipMemcpyAsync(stage, storkm + e0 * nn, (size_t)nel * nn * sizeof(double),
                                        hipMemcpyHostToDevice, c->stream);
         if (he != hipSuccess) rc = pf_set_hip_error(he, "storkm upload", __FILE__, __LINE__);
-        if (!rc) rc = pf_launch_from_colmajor(c, stage, e0, nel);
+        if (!rc && !c->K64) {
+            rc = pf_launch_tri_pack(c, stage, true, e0, nel, bad);   // without a triangle yet: only looked at
+            he = hipStreamSynchronize(c->stream);
+            if (!rc && he != hipSuccess) rc = pf_set_hip_error(he, "packing", __FILE__, __LINE__);
+            if (!rc && *bad) {
+                bool again;
+                rc = tri_to_whole(c, e0, &again);
+                if (again) {
+                    e0 = -chunk;
+                    continue;
+                }
+            } else if (!rc && !c->T64) {
+                rc = alloc_tri(c, true);
+                if (!rc) rc = pf_launch_tri_pack(c, stage, true, e0, nel, bad);
+            }
+        }
+        if (!rc && c->K64) rc = pf_launch_from_colmajor(c, stage, e0, nel);
     }
     (void)hipStreamSynchronize(c->stream);
     pf_free(c, stage, (size_t)chunk * nn * sizeof(double));

@@ -374,9 +374,11 @@ int pf_launch_assemble_elastic(pf_ctx *c, double v2, double vv, double den, doub
                                double *dg, int *bad);
 int pf_launch_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double *k_elem_dev, double *dg);
 // Packs elements e0 .. e0 + nel - 1 (element e0 first in src: column pairs or
-// column-major) into the triangle; *bad is set where an entry does not come
-// back exactly.
+// column-major) into the triangle (none: only looks at them); *bad is set where
+// an entry does not come back exactly.
 int pf_launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad);
+// Elements 0 .. nel - 1 of the triangle into K, as column pairs.
+int pf_launch_tri_unpack(pf_ctx *c, double *K, long nel);
 // Assembled diagonal (leading 0 slot) from element diagonals dg(ntot,nels).
 int pf_launch_diag_elem(pf_ctx *c, const double *dg, double *diag);
 int pf_launch_split_fp32(pf_ctx *c);

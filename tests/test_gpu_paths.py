@@ -218,6 +218,32 @@ def test_batch_of_whole_and_packed_matrices():
         ctx.close()
 
 
+# Matrices that the triangle cannot hold, seen in the first chunk of 128 MB or in
+# the second one (after which the first one's are unpacked again): uploaded
+# once, and no memory kept beyond whole matrices and a chunk.
+@pytest.mark.parametrize("ntot,box", [(60, (11, 11, 10)), (60, (17, 17, 17)), (24, (31, 31, 31)), (8, (64, 64, 65))])
+@pytest.mark.parametrize("kind", ["wide", "general"])
+def test_upload_that_the_triangle_cannot_hold(ntot, box, kind):
+    pr = _mesh_problem(ntot, box)
+    chunk = (128 << 20) // (8 * ntot * ntot)
+    print(f"[gpu-test] upload {ntot} {box} {kind} chunks {pr.nels / chunk:.2f}", flush=True)
+    K = _matrices(kind, pr.nels, ntot)
+    x = np.random.default_rng(3).standard_normal(pr.neq)
+    with Context(0) as ctx:
+        ctx.mesh_set(pr.g_coord())
+        ctx.steer_set(pr.g_g, pr.neq)
+        ctx.trim()
+        before = ctx.mem_used()
+        for _ in range(2):
+            ctx.storkm_set(K)
+            assert ctx.mem_used() - before <= K.nbytes + min(K.nbytes, 128 << 20) + (1 << 20)
+        assert np.array_equal(ctx.storkm_get(), K)
+        assert np.array_equal(ctx.diag_get(), O.diag(pr.g_g, K, pr.neq))
+        assert np.array_equal(ctx.apply(x), O.apply(pr.g_g, K, x))
+        ctx.storkm_set(np.ascontiguousarray((K + K.transpose(0, 2, 1)) / 2))     # and the triangle after it
+        assert np.array_equal(ctx.storkm_get(), (K + K.transpose(0, 2, 1)) / 2)
+
+
 # One batch of solves of every storage that a mesh's FP64 matrices can have, each
 # storage's products a launch of their own over its own solves: storages first,
 # last, between and alone in the batch.
