@@ -2093,14 +2093,13 @@ int pf_checon_par(pf_ctx *c, const double *xnew, double tol, int *converged, dou
     return rc;
 }
 
-// pf_pcg_begin, with x starting at x0 (device, neq) when x0 is given; r0 is
-// read until the stream has passed the copy.
 // Iterations of a solve that parks between two looks for a replacement: three
 // launches every PARK_RUN iterations, against half of PARK_RUN empty iterations
 // at every replacement (four launches of 2.2 to 3.3 us each).  Five
 // replacements in 200 to 3,400 iterations (refine_delta 0.01) or ten in 130 to
-// 1,300 (0.1) are usual; replacements that the caller asks for more often keep
-// their launches in every iteration.  Whole solves, ms, with the launches in
+// 1,300 (0.1) are usual; replacements that the caller asks for more often, by
+// number or by a residual that need not even halve, keep their launches in every
+// iteration.  Whole solves, ms, with the launches in
 // every iteration and parked for runs of 4 / 6 / 8 / 12 iterations: 12^3 hex20
 // mixed 11.8, 10.4 / 9.5 / 9.5 / 9.5, mixed64 7.8, 7.2 / 6.4 / 6.7 / 7.3; 4^3
 // mixed64 (ten in 126) 2.25, 2.16 / 2.08 / 2.2 / 2.2; 31x17x43 mixed 134.8,
@@ -2109,14 +2108,21 @@ int pf_checon_par(pf_ctx *c, const double *xnew, double tol, int *converged, dou
 // gaps: 82^3 Laplace mixed 43.8 -> 42.2, 120^3 147.8 -> 145.2, 40^3 hex20
 // 270 -> 262, range-fused 120x90x75 Laplace 66.6 -> 63.1; 100^3 hex20, where an
 // empty iteration's 250,000 workgroups cost as much as it saves, 280 either way.
+// refine_delta 0.5 / 0.7 / 0.9, launches in every iteration and parked: 4^3 hex20
+// mixed64 2.6, 2.5 / 2.7, 3.8 / 2.9, 5.5; 12^3 15.8, 13.7 / 16.0, 15.0 / 16.6,
+// 19.2; 40^3 Laplace 5.4, 5.5 / 5.6, 6.2 / 6.4, 12.3; 90^3 mixed 55.1, 53.9 /
+// 57.5, 56.9 / 67.1, 70.0.
 constexpr int PARK_RUN = 6;
+constexpr double PARK_DELTA = 0.5;
 static bool solve_parks(const pf_ctx *c, const pf_pcg_opts *o)
 {
     return (o->precision == PF_PREC_MIXED64 || o->precision == PF_PREC_MIXED) && c->dot_order == PF_DOT_TREE &&
-           (o->refine_every == 0 || o->refine_every >= PARK_RUN);
+           (o->refine_every == 0 || o->refine_every >= PARK_RUN) && o->refine_delta <= PARK_DELTA;
 }
 
-// solve: the run is pcg_finish's, which enqueues iterations until it stops.
+// pf_pcg_begin, with x starting at x0 (device, neq) when x0 is given; r0 is
+// read until the stream has passed the copy.  solve: the run is pcg_finish's,
+// which enqueues iterations until it stops.
 static int pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const double *x0, const pf_pcg_opts *opts,
                      bool solve)
 {

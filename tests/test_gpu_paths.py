@@ -424,6 +424,25 @@ def test_parked_replacements(el, box, scatter, precision, every, delta, limit):
         assert res.refinements > 0 or limit == 40
 
 
+# Replacements that nearly every iteration asks for keep their launches in every
+# iteration (as many launches of them as of products); the others are launched
+# once behind each run of iterations.
+@pytest.mark.parametrize("delta,every,parks", [(0.0, 0, True), (0.5, 0, True), (0.5, 6, True), (0.51, 0, False),
+                                               (0.9, 0, False), (0.1, 5, False)])
+@pytest.mark.parametrize("box", [(12, 11, 10), (83, 81, 82)])       # without and with fold launches
+def test_frequent_replacements_do_not_park(box, delta, every, parks):
+    pr = P.laplace_cube(1, nels_xyz=box)
+    print(f"[gpu-test] parks {box} {delta} {every}", flush=True)
+    with Context(0) as ctx:
+        r = P.setup(ctx, pr, store="fp32")
+        ctx.timing_enable()
+        res = ctx.pcg_solve(r, 60, 0.0, stop="relres", precision="mixed64", refine_delta=delta, refine_every=every)[1]
+        t = ctx.timing_get()
+        assert res.iters == 60
+        assert (t["refine"][1] < t["ebe"][1]) == parks
+        assert t["refine"][1] <= t["ebe"][1]
+
+
 # Node freedom tables made on the device and on the host (the rule: 262,144
 # element nodes and freedoms), with rows that a later one overrides.
 @pytest.mark.parametrize("box", [(20, 20, 19), (28, 28, 29), (29, 28, 29), (60, 28, 30)])
