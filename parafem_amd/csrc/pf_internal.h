@@ -228,7 +228,7 @@ struct pf_ctx {
     int store = PF_STORE_FP64;
     double *K64 = nullptr;             // FP64 column pairs (PF_STORE_FP64 where the triangle below does not hold)
     double *T64 = nullptr;             // FP64 packed triangle (PF_STORE_FP64), its differences and their units
-    unsigned *T64d = nullptr, *T64u = nullptr;
+    unsigned *T64d = nullptr, *T64u = nullptr;   // (in the block of T64)
     double *K64b = nullptr;            // p124's second matrix set (storkb_pp), FP64 column pairs
     bool k_shared = false;             // K64 holds one matrix used by every element
     float *K32hi = nullptr;            // packed symmetric FP32, hi = fl32(K)
