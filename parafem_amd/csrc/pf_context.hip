@@ -641,35 +641,27 @@ int pf_assemble_elastic(pf_ctx *c, double e, double v, const double *e_elem, int
     const double v2 = v / (1.0 - v);
     const double vv = (1.0 - 2.0 * v) / (1.0 - v) * 0.5;
     const double den = 2.0 * (1.0 + v) * vv;
-    // the element diagonals go to utemp (ntot*nels doubles, free until the PCG
-    // runs)
-    if (store == PF_STORE_FP32) {
-        rc = alloc_direct32(c);
-        if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp, nullptr);
-    } else {
-        bool whole = keep_whole(c);
-        if (!whole) {
-            rc = alloc_tri(c, true);
-            int *bad = pf_flag_word(c);
-            if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp, bad);
-            if (!rc) {
-                const hipError_t he = hipStreamSynchronize(c->stream);
-                if (he != hipSuccess) rc = pf_set_hip_error(he, "assembly", __FILE__, __LINE__);
-            }
-            whole = !rc && *bad;
-        }
-        if (!rc && whole) {
-            rc = alloc_k64(c, store);
-            if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, nullptr, nullptr);
-        }
+    // The element diagonals go to utemp (ntot*nels doubles, free until the PCG
+    // runs), and the assembled diagonal is formed behind the assembly; whether
+    // the triangle holds the matrices is only known after both.
+    bool whole = store == PF_STORE_FP64 && keep_whole(c);
+    if (!whole) {
+        rc = store == PF_STORE_FP32 ? alloc_direct32(c) : alloc_tri(c, true);
+        int *bad = pf_flag_word(c);
+        if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, c->utemp, bad);
+        if (!rc) rc = finish_direct(c, c->utemp);   // (waits for the stream)
+        whole = !rc && *bad;
+    }
+    if (whole) {
+        rc = alloc_k64(c, store);
+        if (!rc) rc = pf_launch_assemble_elastic(c, v2, vv, den, e, ee, nullptr, nullptr);
+        if (!rc) rc = finish_matrices(c);
     }
     if (ee) {
         (void)hipStreamSynchronize(c->stream);
         pf_free(c, ee, sizeof(double) * c->nels);
     }
-    if (rc) return rc;
-    // the element diagonals are in utemp; whole matrices hold their own
-    return c->K64 ? finish_matrices(c) : finish_direct(c, c->utemp);
+    return rc;
 }
 
 int pf_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double *k_elem, int store)

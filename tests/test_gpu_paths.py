@@ -313,6 +313,24 @@ def test_assembly_that_the_triangle_cannot_hold():
     assert np.array_equal(K[ok], O.assemble_elastic(gc, pr.e, pr.v, nthreads=8)[ok])
 
 
+def test_assembly_kept_whole_is_complete():
+    """Moduli whose differences the triangle has no unit for: after the
+    assembly into the triangle the matrices are formed whole, with their
+    diagonal, and solved with as if they had been so at once."""
+    pr = P.elastic_cube(1, nels_xyz=(11, 11, 10), lognormal_e=True)
+    pr.e_elem = pr.e_elem.copy()
+    pr.e_elem[17] = 1e-300
+    print("[gpu-test] assembly kept whole", flush=True)
+    with Context(0) as ctx:
+        P.setup(ctx, pr)
+        ctx.trim()
+        assert ctx.mem_used() > pr.nels * 28800
+        K = O.assemble_elastic(pr.g_coord(), pr.e, pr.v, pr.e_elem, nthreads=8)
+        assert np.array_equal(ctx.storkm_get(), K)
+        assert np.array_equal(ctx.diag_get(), O.diag(pr.g_g, K, pr.neq))
+        assert np.array_equal(ctx.pcg_solve(pr.r0, 8, 0.0, stop="relres")[0], _oracle_iterates(pr, "relres", 8))
+
+
 @pytest.mark.parametrize("nod,box", [(20, (11, 11, 10)), (8, (20, 19, 20))])
 def test_assembled_triangle_bitexact(nod, box):
     """Distorted elements with moduli of their own, assembled straight into
