@@ -111,19 +111,35 @@ class CubeCache:
         return entry
 
 
+def cube_equations(n: int) -> int:
+    """Equations of the n^3 hex20 cube on a fixed base: three freedoms of its
+    (n+1)^2 (4n+1) nodes but for the base's (n+1)(3n+1)."""
+    return 3 * (n + 1) * ((n + 1) * (4 * n + 1) - (3 * n + 1))
+
+
 def device_bytes(n: int, precision: str) -> int:
-    """Peak device bytes of one request: coordinates (480 B per element),
-    steering (240), transposed steering (240 + 4 per equation), FP64
-    element products (480) and the PCG vectors (12 per equation), plus the
-    element matrices as stored -- FP64 (28,800 B per element where they are
-    kept whole; the packed triangle takes 18,364) or the packed symmetric
-    FP32 hi and lo (2 x 7,328) with FP32 products (240); FP32 storage is
-    assembled straight into hi/lo, with no FP64 copy."""
+    """Peak device bytes of one request.  Per element: coordinates (480),
+    steering (240), transposed steering (240), FP64 element products (480),
+    element nodes during the set-up (80, kept in the context's cache), and
+    the matrices: FP64 28,800 as whole matrices (those above 32 MB are packed
+    into 18,364 where that is exact, which is only known after the assembly)
+    or the packed symmetric FP32 hi and lo (2 x 7,328) with FP32 products
+    (240); FP32 storage is assembled straight into hi/lo, with no FP64 copy.
+    Per equation: nine FP64 vectors (72), the transposed steering's offsets
+    (4), set-up tables (8, cached), and the padded slot table (32) up to 2,048
+    reduction blocks of 256 equations or above them the node lists (4, and 80
+    per element)."""
     nels = n ** 3
-    neq = 3 * ((2 * n + 1) * (n + 1) * (n + 1) + (n + 1) * (n + 1) * n)   # upper bound
-    per_el = 480 + 240 + 240 + 480
+    neq = cube_equations(n)
+    per_el = 480 + 240 + 240 + 480 + 80
     per_el += 28800 if precision == "fp64" else 2 * 7328 + 240
-    return nels * per_el + neq * 8 * 12 + neq * 4 + (16 << 20)
+    per_eq = 72 + 4 + 8
+    if neq <= 2048 * 256:
+        per_eq += 32
+    else:
+        per_eq += 4
+        per_el += 80
+    return nels * per_el + neq * per_eq + (16 << 20)
 
 
 def solve_alone(ctx: Context, cache: CubeCache, req: Request, precision: str, tol: float,

@@ -532,3 +532,21 @@ def test_node_slot_lists_bitexact(nf_kind, precision):
         else:
             # FP32 products: 24 terms of 8 elements at 2^-24, four iterations
             assert np.abs(x - xo).max() <= 4 * 24 * 8 * 2.0 ** -24 * np.abs(xo).max()
+
+
+# What the server admits a request by, on both sides of the padded slot table
+# (2,048 blocks: 34 | 35) and of whole FP64 matrices (32 MB: 10 | 11).
+@pytest.mark.parametrize("n", [1, 10, 11, 34, 35, 50])
+@pytest.mark.parametrize("precision", ["mixed64", "fp64"])
+def test_admission_counts_what_a_request_holds(n, precision):
+    from parafem_amd import serve as S
+    d = S.CubeCache().get(n)
+    print(f"[gpu-test] device bytes {n} {precision}", flush=True)
+    with Context(0) as ctx:
+        ctx.mesh_set(d["g_coord"])
+        ctx.steer_build(d["g_num"], d["rest"], d["nn"])
+        ctx.assemble_elastic(100.0, 0.3, store="fp64" if precision == "fp64" else "fp32")
+        ctx.pcg_begin(d["r_unit"], 10, 0.0, stop="relres", precision=precision)
+        assert ctx.mem_used() <= S.device_bytes(n, precision)
+        ctx.pcg_run(2)
+        assert ctx.pcg_poll().iters == 2

@@ -36,6 +36,13 @@ def test_device_bytes_estimate():
     assert S.device_bytes(80, "fp64") > nels * 28800
 
 
+def test_cube_equations():
+    from parafem_amd import mesh as M
+    for n in (1, 2, 5, 9):
+        m = M.box_hex20(n, n, n, 1.0, 1.0, 1.0)
+        assert S.cube_equations(n) == M.steering(m.nn, 3, M.base_fixed_rest(m))[1]
+
+
 class _Res:
     def __init__(self, iters, converged):
         self.iters, self.converged, self.status, self.refinements = iters, converged, 0, 0
