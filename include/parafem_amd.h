@@ -427,7 +427,7 @@ int pf_block_time_ebe(pf_ctx *ctx, int reps, double *ms);
  * forms its row in the same order whatever the shape.
  *   ebe_epl:   single-RHS products, elements a lane group loads before it
  *              multiplies: 1 or 2 (ntot 60), 1, 2 or 4 (ntot 24), 1, 2, 4
- *              or 8 (ntot 8);
+ *              or 8 (ntot 8); products of one shape (pf_ebe_kernel) ignore it;
  *   blk_waves: block products, elements (wavefronts) per workgroup: 1, 2, 4;
  *   blk_rows:  FP64 block products, 16-row output tiles per pass: 1, 2, 4
  *              (the FP32 block product forms every row tile in one pass).
@@ -439,6 +439,18 @@ typedef struct {
 } pf_tune;
 int pf_tune_set(pf_ctx *ctx, const pf_tune *t);
 int pf_tune_get(pf_ctx *ctx, pf_tune *t);
+/* The element product that an iteration of this precision and stopping rule
+ * runs on the loaded matrices: its kernel's name, the elements a lane group
+ * takes, whether ebe_epl chooses them (products of an FP64 packed triangle,
+ * those that form p and the range-fused ones have one shape), and the bytes of
+ * the stored matrix and the steering it reads per element. */
+typedef struct {
+    char    kernel[64];
+    int     epl;
+    int     tunable;
+    int64_t bytes_per_element;
+} pf_ebe_info;
+int pf_ebe_kernel(pf_ctx *ctx, int precision, int stop_mode, pf_ebe_info *info);
 /* The device's architecture name (gcnArchName, e.g. "gfx950:sramecc+:xnack-")
  * and compute-unit count: the autotuner's cache key. */
 int pf_device_info(pf_ctx *ctx, char *arch, int len, int *cus);

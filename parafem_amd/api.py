@@ -75,6 +75,10 @@ class Tune(C.Structure):
     _fields_ = [("ebe_epl", C.c_int), ("blk_waves", C.c_int), ("blk_rows", C.c_int)]
 
 
+class EbeInfo(C.Structure):
+    _fields_ = [("kernel", C.c_char * 64), ("epl", C.c_int), ("tunable", C.c_int), ("bytes_per_element", C.c_int64)]
+
+
 class BlockResult(C.Structure):
     _fields_ = [("outer", C.c_int), ("inner_iters", C.c_int), ("converged", C.c_int),
                 ("max_relres", C.c_double), ("status", C.c_int)]
@@ -142,6 +146,7 @@ def lib():
         "pf_steer_get": (i32, [vp, pi]),
         "pf_tune_set": (i32, [vp, C.POINTER(Tune)]),
         "pf_tune_get": (i32, [vp, C.POINTER(Tune)]),
+        "pf_ebe_kernel": (i32, [vp, i32, i32, C.POINTER(EbeInfo)]),
         "pf_device_info": (i32, [vp, C.c_char_p, i32, pi]),
         "pf_vec_fill": (i32, [vp, vp, dbl, i64]),
         "pf_vec_waxpy": (i32, [vp, vp, vp, vp, dbl, i64]),
@@ -654,6 +659,15 @@ class Context:
         t = Tune()
         _check(lib().pf_tune_get(self.h, C.byref(t)), "pf_tune_get")
         return {"ebe_epl": t.ebe_epl, "blk_waves": t.blk_waves, "blk_rows": t.blk_rows}
+
+    def ebe_kernel(self, precision: str = "fp64", stop: str = "relres") -> dict:
+        """The iteration's element product on the loaded matrices: kernel
+        name, elements per lane group and whether ``ebe_epl`` chooses them,
+        bytes read per element (stored matrix and steering)."""
+        i = EbeInfo()
+        _check(lib().pf_ebe_kernel(self.h, PREC[precision], STOP[stop], C.byref(i)), "pf_ebe_kernel")
+        return {"kernel": i.kernel.decode(), "epl": i.epl, "tunable": bool(i.tunable),
+                "bytes_per_element": i.bytes_per_element}
 
     def device_info(self):
         """(architecture name, compute units) of the context's device."""

@@ -1450,6 +1450,14 @@ void launch_ebe_epl(pf_ctx *c, const double *src, OUT *out, const pf_state *st, 
                        nlb, rowmajor);
 }
 
+// Elements per lane group of the iteration's product: the tuned shape (an
+// out-of-range value, e.g. from before the mesh changed, keeps the built-in
+// one); the triangle's products have one.
+template <int NT, int KIND> int product_epl(const pf_ctx *c)
+{
+    return KIND < KIND_TRI && c->tune_epl && c->tune_epl <= pf_epl_max(NT) ? c->tune_epl : Lanes<NT, KIND>::EPL;
+}
+
 template <int NT, int KIND, bool GATHER, typename OUT>
 int launch_ebe_nt(pf_ctx *c, const double *src, OUT *out, const pf_state *st, int gate, const double *Kalt,
                   const float *src32, int rowmajor)
@@ -1467,11 +1475,9 @@ int launch_ebe_nt(pf_ctx *c, const double *src, OUT *out, const pf_state *st, in
             return PF_ERR_ARG;   // residual replacements use hi + lo
         }
     } else {
-        // the tuned shape of the iteration's product (an out-of-range value,
-        // e.g. from before the mesh changed, keeps the built-in one)
         constexpr int E0 = Lanes<NT, KIND>::EPL;
-        const int e = GATHER && c->tune_epl <= pf_epl_max(NT) ? c->tune_epl : 0;
-        if constexpr (GATHER && KIND < KIND_TRI) {   // the triangle's products have one shape
+        if constexpr (GATHER && KIND < KIND_TRI) {
+            const int e = product_epl<NT, KIND>(c);
             if (e == 1) launch_ebe_epl<NT, KIND, GATHER, OUT, 1>(c, src, out, st, gate, K64, src32, rowmajor);
             else if (e == 2) launch_ebe_epl<NT, KIND, GATHER, OUT, 2>(c, src, out, st, gate, K64, src32, rowmajor);
             else if (e == 4) launch_ebe_epl<NT, KIND, GATHER, OUT, (NT <= 24 ? 4 : E0)>(c, src, out, st, gate, K64, src32, rowmajor);
@@ -2206,10 +2212,12 @@ int pf_pcg_begin(pf_ctx *c, const double *r0, int r0_on_device, const pf_pcg_opt
 // against eleven of one wavefront (18^3 hex20 35.7 us an iteration with p
 // formed, 33.3 without; 12^3 18.5 either way).
 constexpr int FORM_MAXG = 512;
-static bool forms_p(const pf_ctx *c, int G)
+static bool forms_p(const pf_ctx *c, int precision, int G)
 {
-    return G <= FORM_MAXG && !(c->opts.precision == PF_PREC_FP64 && c->T64d);
+    return G <= FORM_MAXG && !(precision == PF_PREC_FP64 && c->T64d);
 }
+// An iteration without fold launches.
+static bool is_foldless(const pf_ctx *c, bool ranges) { return c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE; }
 
 template <int NT, int KIND, typename OUT>
 static void launch_ebe_form(pf_ctx *c, OUT *out, int rm, int G)
@@ -2294,7 +2302,7 @@ static int run_foldless(pf_ctx *c, int n, int G, float *p32, int rm, const int *
 {
     const bool checon = c->opts.stop_mode == PF_STOP_CHECON, mixed = c->opts.precision == PF_PREC_MIXED;
     const bool refines = !parks && (mixed || c->opts.precision == PF_PREC_MIXED64);
-    const bool form = forms_p(c, G);
+    const bool form = forms_p(c, c->opts.precision, G);
     const dim3 grid(G), blk(PF_BLOCK);
     const int fz = c->fix_zero ? 1 : 0;
     hipEvent_t t0, t1;
@@ -2483,13 +2491,68 @@ static int pcg_run(pf_ctx *c, int n, bool watch)
     const int *slot = rm ? c->csr_slot_t : c->csr_slot;
     const bool ranges = mixed && c->scatter_mode == PF_SCATTER_RANGES;
     if (ranges && !c->rng) return PF_ERR_STATE;   // pf_pcg_begin builds them
-    const bool foldless = c->csr_slot8 && !ranges && c->dot_order == PF_DOT_TREE;
+    const bool foldless = is_foldless(c, ranges);
     const bool parks = watch && solve_parks(c, &c->opts);
     for (int done = 0, m; done < n && !(done && stop_seen(c, watch)); done += m) {
         m = parks ? std::min(PARK_RUN, n - done) : n;
         const int rc = foldless ? run_foldless(c, m, G, p32, rm, slot, watch, parks)
                                 : run_folds(c, m, G, p32, rm, slot, watch, parks, ranges);
         if (rc) return rc;
+    }
+    return PF_OK;
+}
+
+}  // extern "C"
+
+template <int NT, int KIND> static void ebe_info(const pf_ctx *c, int form, pf_ebe_info *o)
+{
+    const char *out = KIND == KIND_F32 ? "float" : "double";
+    const long tri = 2L * pf_tri_pairs(NT) * (long)sizeof(double), sym = (long)pf_sym_per(NT) * (long)sizeof(float);
+    long K = sym;
+    if (KIND == KIND_F64) K = c->k_shared ? 0 : (long)NT * NT * (long)sizeof(double);
+    if (KIND == KIND_ACC) K = 2 * sym;
+    if (KIND == KIND_TRI) K = tri;
+    if (KIND == KIND_TRID) K = tri + (pf_tri_diffs(NT) + 1) * (long)sizeof(unsigned);
+    o->bytes_per_element = K + NT * (long)sizeof(int);
+    o->tunable = !form && KIND < KIND_TRI;
+    o->epl = form ? Lanes<NT, KIND>::EPL : product_epl<NT, KIND>(c);
+    if (form) snprintf(o->kernel, sizeof o->kernel, "k_ebe_form<%d, %d, %s, %d>", NT, KIND, out, form);
+    else snprintf(o->kernel, sizeof o->kernel, "k_ebe<%d, %d, true, %s, false, %d>", NT, KIND, out, o->epl);
+}
+
+template <int NT> static void ebe_info_nt(const pf_ctx *c, int precision, int form, pf_ebe_info *o)
+{
+    if (precision == PF_PREC_MIXED) return ebe_info<NT, KIND_F32>(c, form, o);
+    if (precision == PF_PREC_MIXED64) return ebe_info<NT, KIND_WIDE>(c, form, o);
+    if (precision == PF_PREC_SPLIT) return ebe_info<NT, KIND_ACC>(c, form, o);
+    if (!c->T64) return ebe_info<NT, KIND_F64>(c, form, o);
+    if (c->T64d) return ebe_info<NT, KIND_TRID>(c, form, o);
+    ebe_info<NT, KIND_TRI>(c, form, o);
+}
+
+extern "C" {
+
+int pf_ebe_kernel(pf_ctx *c, int precision, int stop_mode, pf_ebe_info *info)
+{
+    if (!c || !info) return PF_ERR_ARG;
+    if (precision < PF_PREC_FP64 || precision > PF_PREC_SPLIT) return PF_ERR_ARG;
+    if (stop_mode != PF_STOP_CHECON && stop_mode != PF_STOP_RELRES) return PF_ERR_ARG;
+    if (!c->have_K) return PF_ERR_STATE;
+    if (precision == PF_PREC_FP64 ? !pf_has_f64(c) : !c->K32hi) return PF_ERR_ARG;
+    const bool ranges = precision == PF_PREC_MIXED && c->scatter_mode == PF_SCATTER_RANGES;
+    int form = FORM_NONE;
+    if (is_foldless(c, ranges) && forms_p(c, precision, pf_grid_for(c->neq)))
+        form = stop_mode == PF_STOP_CHECON ? FORM_CHECON : FORM_RELRES;
+    switch (c->ntot) {
+    case 60: ebe_info_nt<60>(c, precision, form, info); break;
+    case 24: ebe_info_nt<24>(c, precision, form, info); break;
+    case 8: ebe_info_nt<8>(c, precision, form, info); break;
+    default: return PF_ERR_STATE;
+    }
+    if (ranges) {
+        snprintf(info->kernel, sizeof info->kernel, "k_ebe_range<%d>", c->ntot);
+        info->epl = 1;
+        info->tunable = 0;
     }
     return PF_OK;
 }

@@ -4,7 +4,9 @@ The shapes (C ABI ``pf_tune``):
 
 * single-RHS product ``k_ebe``: ``ebe_epl``, the number of elements a lane
   group loads before it multiplies (more bytes in flight per wavefront
-  against more registers and fewer resident wavefronts);
+  against more registers and fewer resident wavefronts); products of one
+  shape (FP64 packed triangles, products that form p, range-fused ones) are
+  not timed;
 * block products ``k_blk_ebe_sym`` (FP32) and ``k_blk_ebe`` (FP64):
   ``blk_waves``, elements (one wavefront each) per workgroup, tuned on the
   FP32 product; ``blk_rows``, 16-row output tiles per pass of the FP64
@@ -99,6 +101,10 @@ def tune_ebe(ctx, r0, precision: str, reps: int = 20, warm: int = 3, use_cache: 
     if precision == "mixed" and ctx.scatter_mode == "ranges":
         # the range-fused kernel has one shape (an element per lane group)
         return {"ebe_epl": cur["ebe_epl"], "ms": {}, "cached": True}
+    shape = ctx.ebe_kernel(precision, "relres")
+    if not shape["tunable"]:
+        ctx.tune_set(shape["epl"], cur["blk_waves"], cur["blk_rows"])
+        return {"ebe_epl": shape["epl"], "ms": {}, "cached": True}
     key = _key(ctx, "k_ebe", precision, 1)
     hit = lookup(key) if use_cache else None
     if hit is not None:

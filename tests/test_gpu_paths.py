@@ -550,3 +550,29 @@ def test_admission_counts_what_a_request_holds(n, precision):
         assert ctx.mem_used() <= S.device_bytes(n, precision)
         ctx.pcg_run(2)
         assert ctx.pcg_poll().iters == 2
+
+
+# The product that an iteration runs, on both sides of the storage's and the
+# iteration's rules, and the bytes it reads an element.
+@pytest.mark.parametrize("ntot,box,store,precision,stop,want", [
+    (60, (3, 1, 2), "fp64", "fp64", "checon", ("k_ebe_form<60, 0, double, 1>", 1, False, 28800 + 240)),
+    (60, (12, 12, 12), "fp64", "fp64", "relres", ("k_ebe<60, 5, true, double, false, 1>", 1, False, 18364 + 240)),
+    (60, (12, 12, 12), "fp32", "mixed", "relres", ("k_ebe_form<60, 1, float, 2>", 1, False, 7328 + 240)),
+    (60, (24, 24, 24), "fp32", "mixed", "relres", ("k_ebe<60, 1, true, float, false, 1>", 1, True, 7328 + 240)),
+    (60, (24, 24, 24), "fp32", "split", "checon", ("k_ebe<60, 2, true, double, false, 1>", 1, True, 14656 + 240)),
+    (24, (20, 19, 20), "fp64", "fp64", "relres", ("k_ebe<24, 5, true, double, false, 1>", 1, False, 2496 + 532 + 96)),
+    (8, (20, 20, 20), "fp64", "fp64", "relres", ("k_ebe_form<8, 4, double, 2>", 2, False, 320 + 32)),
+    (8, (60, 60, 60), "fp64", "fp64", "relres", ("k_ebe<8, 4, true, double, false, 2>", 2, False, 320 + 32)),
+    (8, (60, 60, 60), "fp32", "mixed64", "relres", ("k_ebe<8, 3, true, double, false, 4>", 4, True, 144 + 32))])
+def test_product_that_an_iteration_runs(ntot, box, store, precision, stop, want):
+    pr = _mesh_problem(ntot, box)
+    print(f"[gpu-test] product {ntot} {box} {precision}", flush=True)
+    with Context(0) as ctx:
+        P.setup(ctx, pr, store=store)
+        got = ctx.ebe_kernel(precision, stop)
+        assert (got["kernel"], got["epl"], got["tunable"], got["bytes_per_element"]) == want
+        if got["tunable"]:
+            ctx.tune_set(ebe_epl=2)
+            assert ctx.ebe_kernel(precision, stop)["epl"] == 2
+        with pytest.raises(Exception):
+            ctx.ebe_kernel("fp64" if store == "fp32" else "mixed", stop)

@@ -77,3 +77,16 @@ def test_unwritable_cache_keeps_results_in_memory(tmp_path, monkeypatch):
     T.tune_block(c)
     c2 = _Ctx()
     assert T.tune_block(c2)["cached"]
+
+
+def test_products_of_one_shape_are_not_timed(tmp_path, monkeypatch):
+    """A product that ebe_epl does not shape: no runs, nothing cached, the
+    shape that it has is reported and set."""
+    monkeypatch.setenv("PARAFEM_AMD_TUNE_CACHE", str(tmp_path / "tune.json"))
+    monkeypatch.setattr(T, "_memory", {})
+    c = _Ctx()
+    c.scatter_mode = "slots"
+    c.ebe_kernel = lambda precision, stop: {"kernel": "k", "epl": 1, "tunable": False, "bytes_per_element": 1}
+    got = T.tune_ebe(c, None, "fp64")          # (the stand-in has no pcg_run to time)
+    assert got == {"ebe_epl": 1, "ms": {}, "cached": True} and c.shape["ebe_epl"] == 1
+    assert T._memory == {} and not (tmp_path / "tune.json").exists()
