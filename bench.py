@@ -45,9 +45,9 @@ def ebe_bytes(ntot, store, precision="mixed"):
     """Algorithmic HBM bytes of one element product: the element matrix once
     (full FP64, or the FP32 hi part packed symmetric: the ntot(ntot+1)/2
     entries of one triangle padded to a multiple of 4, hi and lo for the
-    split precision) and the int32 steering once.  (FP64 matrices are held as
-    a packed triangle where that is exact -- 18,364 bytes a hex20 element --
-    so the FP64 rate by these bytes exceeds what is moved.)"""
+    split precision) and the int32 steering once.  FP64 matrices are read as
+    they are stored, a packed triangle where that is exact (18,364 bytes a
+    hex20 element): the rates reported are by Context.ebe_kernel's bytes."""
     if store == "fp64":
         return ntot * ntot * 8 + ntot * 4
     parts = 2 if precision == "split" else 1
@@ -55,18 +55,10 @@ def ebe_bytes(ntot, store, precision="mixed"):
     return parts * packed * 4 + ntot * 4
 
 
-def iteration_bytes(nels, ntot, neq, store, precision="mixed"):
-    """Per-iteration algorithmic bytes: element matrices + steering + 15 FP64
-    vector streams of length neq."""
-    return nels * ebe_bytes(ntot, store, precision) + 15 * neq * 8
-
-
-def ebe_kernel_name(ntot, precision, epl):
-    """The iteration's element-product kernel as rocprofv3 names it."""
-    if precision == "fp64":              # the packed triangle's products have one shape
-        return f"k_ebe<{ntot}, {4 if ntot == 8 else 5}, true, double, false, {2 if ntot == 8 else 1}>"
-    kind, out = {"mixed": (1, "float"), "split": (2, "double"), "mixed64": (3, "double")}[precision]
-    return f"k_ebe<{ntot}, {kind}, true, {out}, false, {epl}>"
+def iteration_bytes(nels, ntot, neq, store, precision="mixed", per_elem=None):
+    """Per-iteration algorithmic bytes: element matrices + steering (per_elem
+    bytes an element where given) + 15 FP64 vector streams of length neq."""
+    return nels * (per_elem or ebe_bytes(ntot, store, precision)) + 15 * neq * 8
 
 
 def time_iterations(ctx, pr, precision, steps, warmup):
@@ -516,11 +508,12 @@ def main():
         ctx.sync()
         t_setup = time.perf_counter() - t0
         shape = T.tune_ebe(ctx, pr.r0, prec)
-        log(f"{name}: autotuned elements per lane group {shape['ebe_epl']} "
-            f"({'cache' if shape['cached'] else 'timed ' + str(shape['ms'])})")
+        product = ctx.ebe_kernel(prec)
+        log(f"{name}: elements per lane group {product['epl']} "
+            f"({'one shape' if not product['tunable'] else 'cache' if shape['cached'] else 'timed ' + str(shape['ms'])})")
         elapsed, tk, nprof = time_iterations(ctx, pr, prec, args.steps, args.warmup)
         ebe_ms = tk["ebe"][0] / max(tk["ebe"][1], 1)
-        per_elem = ebe_bytes(pr.ntot, store, prec)
+        per_elem = product["bytes_per_element"]
         achieved = pr.nels * per_elem / (ebe_ms * 1e-3) / 1e9
         iter_ms = sum(v[0] for v in tk.values()) / nprof
         paths[name] = {
@@ -532,12 +525,13 @@ def main():
             "ebe_ms": ebe_ms,
             "ebe_gbs": round(achieved, 1),
             "bytes_per_element": per_elem,
-            "iteration_gbs": round(iteration_bytes(pr.nels, pr.ntot, pr.neq, store, prec) / (iter_ms * 1e-3) / 1e9, 1),
+            "iteration_gbs": round(iteration_bytes(pr.nels, pr.ntot, pr.neq, store, prec, per_elem)
+                                   / (iter_ms * 1e-3) / 1e9, 1),
             "setup_assembly_s": round(t_setup, 3),
             "device_gib": round(ctx.mem_used() / 2**30, 2),
-            "tile_shape": {"ebe_epl": shape["ebe_epl"], "source": "autotuner"},
-            "kernel": (f"k_ebe_range<{pr.ntot}> (products and their sums into u, one launch per colour)"
-                       if name == "mixed_ranges" else ebe_kernel_name(pr.ntot, prec, shape["ebe_epl"])),
+            "tile_shape": {"ebe_epl": product["epl"], "source": "autotuner" if product["tunable"] else "one shape"},
+            "kernel": product["kernel"] + (" (products and their sums into u, one launch per colour)"
+                                           if name == "mixed_ranges" else ""),
         }
         log(f"{name}: {paths[name]['iter_per_s']} iter/s, element products {ebe_ms:.3f} ms "
             f"({achieved:.0f} GB/s), kernels " +

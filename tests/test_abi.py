@@ -48,6 +48,15 @@ def test_no_cpu_fallback_without_library(monkeypatch, tmp_path):
         api.Context(0)
 
 
+def test_bench_iteration_bytes_by_the_stored_product():
+    import os
+    import sys
+    sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    import bench
+    assert bench.iteration_bytes(10, 60, 7, "fp64", "fp64", 18604) == 10 * 18604 + 15 * 7 * 8
+    assert bench.iteration_bytes(10, 60, 7, "fp64", "fp64") == 10 * 29040 + 15 * 7 * 8
+
+
 def test_bench_byte_counts_match_the_storage_layouts():
     """bench.py's algorithmic bytes per element: FP64 K_e in full, the packed
     symmetric FP32 layout's ntot(ntot+1)/2 entries padded to a multiple of 4
