@@ -391,15 +391,19 @@ __global__ __launch_bounds__(64 * WAVES) void k_assemble_laplace8(
 // pm - kc*(1-theta)*dtim.  prop(5,np_types) = kx, ky, kz, rho, cp per
 // element type (READ_MATERIAL).  Every product and sum in the reference's
 // order: MATMUL(TRANSPOSE(deriv),kay) has one nonzero term per entry (the
-// others add exact zeros), the weights of SAMPLE are 1.
+// others add exact zeros), the weights of SAMPLE are 1.  TRI: storka as the
+// packed triangle with differences, an entry a lane, the mirrored one read
+// across the wavefront (120^3 bricks, the whole call: whole matrices 2.76 ms,
+// formed whole in chunks and packed from there 3.0, so 2.70).
+template <bool TRI>
 __global__ __launch_bounds__(64 * WAVES) void k_assemble_transient8(
     const double *__restrict__ g_coord, const double *__restrict__ prop, const int *__restrict__ etype,
-    double theta, double dtim, double *__restrict__ Ka, double *__restrict__ Kb, long first, long end)
+    double theta, double dtim, as_out O, double *__restrict__ Kb, int nels)
 {
     __shared__ ElemLds<8> lds[WAVES];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long e = first + (long)blockIdx.x * WAVES + wave;
-    const bool valid = e < end;
+    const long e = (long)blockIdx.x * WAVES + wave;
+    const bool valid = e < nels;
     ElemLds<8> &L = lds[wave];
     element_geometry<8>(L, g_coord + (valid ? e : 0) * 24, lane, valid);
     if (!valid) return;
@@ -428,8 +432,30 @@ __global__ __launch_bounds__(64 * WAVES) void k_assemble_transient8(
         kc = kc + t * det * 1.0;
         pm = pm + fa * fb * det * 1.0 * rho * cp;
     }
-    Ka[pf_idx_pair(e - first, 8, a, b)] = pm + kc * theta * dtim;
     Kb[pf_idx_pair(e, 8, a, b)] = pm - kc * (1.0 - theta) * dtim;
+    const double ka = pm + kc * theta * dtim;
+    if constexpr (TRI) {
+        const double up = __shfl(ka, 8 * a + b, 64);   // entry (b,a)
+        const bool low = a > (b | 1);
+        double dm = low ? fabs(__dsub_rn(ka, up)) : 0.0;
+        dm = wave_max(dm);
+        dm = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(dm)),
+                              __builtin_amdgcn_readfirstlane(__double2loint(dm)));
+        unsigned uh;
+        double unit, inv;
+        bool fail = !tri_unit(dm, uh, unit, inv), code_fails = false;
+        union { unsigned short u; _Float16 h; } c;
+        c.h = tri_code(ka, up, inv, unit, code_fails);
+        fail |= low && code_fails;
+        const unsigned next = __shfl_down((unsigned)c.u, 8, 64);   // column b + 1
+        if (!low) O.K[2 * (e * pf_tri_pairs(8) + pf_tri_pair(b >> 1, a)) + (b & 1)] = ka;
+        else if (!(b & 1)) O.diff[e * pf_tri_diffs(8) + pf_tri_diff(8, b >> 1, a)] = c.u | next << 16;
+        if (a == b) O.dg[e * 8 + a] = ka;
+        if (lane == 0) O.unit[e] = uh;
+        if (fail) *O.bad = 1;
+    } else {
+        O.K[pf_idx_pair(e, 8, a, b)] = ka;
+    }
 }
 
 // hi = fl32(K), lo = fl32(K - hi) in the packed symmetric layout (upper
@@ -479,12 +505,12 @@ __global__ void k_from_colmajor(const double *__restrict__ src, double *__restri
     }
 }
 
-// FP64 matrices (column pairs, or column-major) -> packed triangle.  One lane
+// FP64 matrices (column-major) -> packed triangle.  One lane
 // group per element (lane = row), the whole matrix in LDS; every entry below
 // the diagonal is reconstructed as the product will and compared (with T null
 // only that).  Bound by the reads of src, which a bounded chunk leaves in the
 // last-level cache.
-template <int NT, bool COLMAJOR>
+template <int NT>
 __global__ __launch_bounds__(64) void k_tri_pack(const double *__restrict__ src, double *__restrict__ T,
                                                 unsigned *__restrict__ diff, unsigned *__restrict__ unit, long e0,
                                                 long nel, int *__restrict__ bad)
@@ -499,14 +525,8 @@ __global__ __launch_bounds__(64) void k_tri_pack(const double *__restrict__ src,
     if (on) {
 #pragma unroll
         for (int s = 0; s < H; ++s) {
-            if constexpr (COLMAJOR) {
-                M[i * PITCH + 2 * s] = S[2 * s * NT + i];
-                M[i * PITCH + 2 * s + 1] = S[(2 * s + 1) * NT + i];
-            } else {
-                const double2 v = reinterpret_cast<const double2 *>(S)[s * NT + i];
-                M[i * PITCH + 2 * s] = v.x;
-                M[i * PITCH + 2 * s + 1] = v.y;
-            }
+            M[i * PITCH + 2 * s] = S[2 * s * NT + i];
+            M[i * PITCH + 2 * s + 1] = S[(2 * s + 1) * NT + i];
         }
     }
     __syncthreads();
@@ -647,23 +667,20 @@ int pf_launch_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const
 }
 
 template <int NT>
-static void launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad)
+static void launch_tri_pack(pf_ctx *c, const double *src, long e0, long nel, int *bad)
 {
     constexpr int EPW = NT > 32 ? 1 : (NT > 16 ? 2 : 8);
-    const dim3 grid((unsigned)((nel + EPW - 1) / EPW)), blk(64);
-    if (colmajor)
-        hipLaunchKernelGGL((k_tri_pack<NT, true>), grid, blk, 0, c->stream, src, c->T64, c->T64d, c->T64u, e0, nel, bad);
-    else
-        hipLaunchKernelGGL((k_tri_pack<NT, false>), grid, blk, 0, c->stream, src, c->T64, c->T64d, c->T64u, e0, nel, bad);
+    hipLaunchKernelGGL(k_tri_pack<NT>, dim3((unsigned)((nel + EPW - 1) / EPW)), dim3(64), 0, c->stream, src, c->T64,
+                       c->T64d, c->T64u, e0, nel, bad);
 }
 
-int pf_launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad)
+int pf_launch_tri_pack(pf_ctx *c, const double *src, long e0, long nel, int *bad)
 {
     if (c->T64 && (!c->T64d || !c->T64u)) return PF_ERR_STATE;
     switch (c->ntot) {
-    case 60: launch_tri_pack<60>(c, src, colmajor, e0, nel, bad); break;
-    case 24: launch_tri_pack<24>(c, src, colmajor, e0, nel, bad); break;
-    case 8: launch_tri_pack<8>(c, src, colmajor, e0, nel, bad); break;
+    case 60: launch_tri_pack<60>(c, src, e0, nel, bad); break;
+    case 24: launch_tri_pack<24>(c, src, e0, nel, bad); break;
+    case 8: launch_tri_pack<8>(c, src, e0, nel, bad); break;
     default: return PF_ERR_ARG;
     }
     PF_HIP(hipGetLastError());
@@ -687,11 +704,18 @@ int pf_launch_diag_elem(pf_ctx *c, const double *dg, double *diag)
 }
 
 int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const double *prop, const int *etype,
-                                 double *Ka, long e0, long nel)
+                                 int *bad)
 {
     if (c->nod != 8) return PF_ERR_ARG;
-    hipLaunchKernelGGL(k_assemble_transient8, dim3((unsigned)((nel + WAVES - 1) / WAVES)), dim3(64 * WAVES), 0,
-                       c->stream, c->g_coord, prop, etype, theta, dtim, Ka, c->K64b, e0, e0 + nel);
+    if (!c->K64b || (c->T64 ? !c->T64d || !c->T64u || !bad : !c->K64)) return PF_ERR_STATE;
+    const as_out O{c->T64 ? c->T64 : c->K64, c->T64d, c->T64u, bad, nullptr, nullptr, c->utemp};
+    const dim3 grid((c->nels + WAVES - 1) / WAVES), blk(64 * WAVES);
+    if (c->T64)
+        hipLaunchKernelGGL(k_assemble_transient8<true>, grid, blk, 0, c->stream, c->g_coord, prop, etype, theta, dtim, O,
+                           c->K64b, c->nels);
+    else
+        hipLaunchKernelGGL(k_assemble_transient8<false>, grid, blk, 0, c->stream, c->g_coord, prop, etype, theta, dtim,
+                           O, c->K64b, c->nels);
     PF_HIP(hipGetLastError());
     return PF_OK;
 }

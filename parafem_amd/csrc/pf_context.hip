@@ -519,46 +519,13 @@ static bool keep_whole(const pf_ctx *c)
     return (size_t)c->nels * c->ntot * c->ntot * sizeof(double) <= ((size_t)32 << 20);
 }
 
-// Elements formed and packed at a time: a chunk of whole matrices of 128 MB
-// stays in the last-level cache (256 MB) between the two kernels.
+// Elements uploaded and packed at a time: a chunk of whole matrices of 128 MB
+// stays in the last-level cache (256 MB) between the two.
 static long pack_elems(const pf_ctx *c)
 {
     const long per = (long)c->ntot * c->ntot * (long)sizeof(double), n = (128L << 20) / per;
     return n < c->nels ? n : c->nels;
 }
-
-}  // extern "C"
-
-// FP64 matrices formed chunk by chunk on the device by form(stage, e0, nel) --
-// into a bounded staging buffer, as column pairs -- and packed into the
-// triangle.  *whole is set, and nothing kept, where an entry does not come back
-// exactly: the caller then forms whole matrices.
-template <class F>
-static int form_and_pack(pf_ctx *c, bool *whole, F form)
-{
-    *whole = keep_whole(c);
-    if (*whole) return PF_OK;
-    int rc = alloc_tri(c, true);
-    const long chunk = pack_elems(c);
-    const size_t sb = (size_t)chunk * c->ntot * c->ntot * sizeof(double);
-    double *stage = nullptr;
-    int *bad = pf_flag_word(c);
-    if (!rc) rc = pf_alloc(c, (void **)&stage, sb);
-    // (ends early where the word is seen: the rest would be packed for nothing)
-    for (long e0 = 0; !rc && e0 < c->nels && !__atomic_load_n(bad, __ATOMIC_RELAXED); e0 += chunk) {
-        const long nel = std::min(chunk, (long)c->nels - e0);
-        rc = form(stage, e0, nel);
-        if (!rc) rc = pf_launch_tri_pack(c, stage, false, e0, nel, bad);
-    }
-    const hipError_t he = hipStreamSynchronize(c->stream);
-    if (!rc && he != hipSuccess) rc = pf_set_hip_error(he, "packing", __FILE__, __LINE__);
-    pf_free(c, stage, sb);
-    *whole = !rc && *bad;
-    if (rc || *whole) free_matrices(c);
-    return rc;
-}
-
-extern "C" {
 
 // Storage for an assembly straight into the packed FP32 hi/lo matrices (and
 // the FP32 products' utemp32), with no FP64 copy.
@@ -708,25 +675,28 @@ int pf_assemble_transient(pf_ctx *c, double theta, double dtim, int np_types, co
             he = hipMemcpyAsync(dtype, etype, sizeof(int) * c->nels, hipMemcpyHostToDevice, c->stream);
         if (he != hipSuccess) rc = pf_set_hip_error(he, "transient upload", __FILE__, __LINE__);
     }
-    auto alloc_b = [&]() {
-        return c->K64b ? PF_OK : pf_alloc(c, (void **)&c->K64b, (size_t)64 * c->nels * sizeof(double));
+    auto form = [&](int *bad) {
+        int r = pf_alloc(c, (void **)&c->K64b, (size_t)64 * c->nels * sizeof(double));
+        if (!r) r = pf_launch_assemble_transient(c, theta, dtim, dprop, dtype, bad);
+        if (r) return r;
+        return c->T64 ? finish_direct(c, c->utemp) : finish_matrices(c);   // (both wait for the stream)
     };
-    bool whole = store == PF_STORE_FP32;   // the hi/lo split reads whole matrices
-    if (!rc && !whole)
-        rc = form_and_pack(c, &whole, [&](double *Ka, long e0, long nel) {
-            const int r = alloc_b();
-            return r ? r : pf_launch_assemble_transient(c, theta, dtim, dprop, dtype, Ka, e0, nel);
-        });
+    // (the FP32 hi/lo split reads whole matrices)
+    bool whole = store == PF_STORE_FP32 || keep_whole(c);
+    if (!rc && !whole) {
+        int *bad = pf_flag_word(c);
+        rc = alloc_tri(c, true);
+        if (!rc) rc = form(bad);
+        whole = !rc && *bad;
+    }
     if (!rc && whole) {
         rc = alloc_k64(c, store);
-        if (!rc) rc = alloc_b();
-        if (!rc) rc = pf_launch_assemble_transient(c, theta, dtim, dprop, dtype, c->K64, 0, c->nels);
+        if (!rc) rc = form(nullptr);
     }
     (void)hipStreamSynchronize(c->stream);
     pf_free(c, dprop, sizeof(double) * 5 * np_types);
     pf_free(c, dtype, sizeof(int) * c->nels);
-    if (rc) return rc;
-    return finish_matrices(c);
+    return rc;
 }
 
 // storkm_pp is moved through a bounded staging buffer, chunk by chunk.
@@ -789,7 +759,7 @@ int pf_storkm_set(pf_ctx *c, const double *storkm, int store)
                                        hipMemcpyHostToDevice, c->stream);
         if (he != hipSuccess) rc = pf_set_hip_error(he, "storkm upload", __FILE__, __LINE__);
         if (!rc && !c->K64) {
-            rc = pf_launch_tri_pack(c, stage, true, e0, nel, bad);   // without a triangle yet: only looked at
+            rc = pf_launch_tri_pack(c, stage, e0, nel, bad);   // without a triangle yet: only looked at
             he = hipStreamSynchronize(c->stream);
             if (!rc && he != hipSuccess) rc = pf_set_hip_error(he, "packing", __FILE__, __LINE__);
             if (!rc && *bad) {
@@ -801,7 +771,7 @@ int pf_storkm_set(pf_ctx *c, const double *storkm, int store)
                 }
             } else if (!rc && !c->T64) {
                 rc = alloc_tri(c, true);
-                if (!rc) rc = pf_launch_tri_pack(c, stage, true, e0, nel, bad);
+                if (!rc) rc = pf_launch_tri_pack(c, stage, e0, nel, bad);
             }
         }
         if (!rc && c->K64) rc = pf_launch_from_colmajor(c, stage, e0, nel);

@@ -320,10 +320,11 @@ void pf_node_slots(pf_ctx *c, const int *g_num, int ns, int nn, int *work, int *
 // allocation-free entry points' scratch array (pf_ebe.hip).
 int pf_scratch_init(int device);
 
-// p124's transient element matrices into K64 (storka) and K64b (storkb).
-// Elements e0 .. e0 + nel - 1 of storka into Ka (element e0 first).
+// p124's transient element matrices into T64 or K64 (storka) and K64b (storkb);
+// bad: set where an entry of the triangle does not come back exactly (whose
+// element diagonals go to utemp).
 int pf_launch_assemble_transient(pf_ctx *c, double theta, double dtim, const double *prop, const int *etype,
-                                 double *Ka, long e0, long nel);
+                                 int *bad);
 
 // Steering set-up (pf_context.hip, pf_setup.hip).
 int pf_steer_install(pf_ctx *c, int ntot, int nels, int neq);
@@ -373,10 +374,10 @@ int pf_grid_for(int64_t n);
 int pf_launch_assemble_elastic(pf_ctx *c, double v2, double vv, double den, double e, const double *e_elem_dev,
                                double *dg, int *bad);
 int pf_launch_assemble_laplace(pf_ctx *c, double kx, double ky, double kz, const double *k_elem_dev, double *dg);
-// Packs elements e0 .. e0 + nel - 1 (element e0 first in src: column pairs or
-// column-major) into the triangle (none: only looks at them); *bad is set where
-// an entry does not come back exactly.
-int pf_launch_tri_pack(pf_ctx *c, const double *src, bool colmajor, long e0, long nel, int *bad);
+// Packs elements e0 .. e0 + nel - 1 (element e0 first in src, column-major) into
+// the triangle (none: only looks at them); *bad is set where an entry does not
+// come back exactly.
+int pf_launch_tri_pack(pf_ctx *c, const double *src, long e0, long nel, int *bad);
 // Elements 0 .. nel - 1 of the triangle into K, as column pairs.
 int pf_launch_tri_unpack(pf_ctx *c, double *K, long nel);
 // Assembled diagonal (leading 0 slot) from element diagonals dg(ntot,nels).

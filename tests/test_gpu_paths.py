@@ -331,6 +331,45 @@ def test_assembly_kept_whole_is_complete():
         assert np.array_equal(ctx.pcg_solve(pr.r0, 8, 0.0, stop="relres")[0], _oracle_iterates(pr, "relres", 8))
 
 
+# p124's matrices on both sides of 32 MB (65,536 bricks), in wavefronts of a
+# last workgroup that is partly filled, and with a material whose differences
+# the triangle has no unit for (whole matrices then).
+@pytest.mark.parametrize("box,tiny", [((32, 32, 64), False), ((65537, 1, 1), False), ((41, 40, 41), False),
+                                      ((41, 40, 41), True)])
+def test_transient_storage_bitexact(box, tiny):
+    pr = _mesh_problem(8, box)
+    rng = np.random.default_rng(11)
+    pr.mesh.coords = pr.mesh.coords + rng.uniform(-0.15, 0.15, pr.mesh.coords.shape)
+    gc = pr.mesh.g_coord()
+    prop = np.array([[1.5, 0.7, 2.0, 1.2, 0.8], [0.4, 1.1, 0.3, 2.5, 1.7], [1e-290, 3e-290, 2e-290, 1e-160, 1e-140]])
+    etype = rng.integers(1, 3, pr.nels).astype(np.int32)
+    if tiny:
+        etype[1000] = 3
+    print(f"[gpu-test] transient storage {box} {tiny}", flush=True)
+    KA, KB = O.assemble_transient(gc, prop, etype, 0.5, 0.01, nthreads=8)
+    d = np.abs(KA[1000] - KA[1000].T).max()
+    assert (0 < d < 2.0 ** -1008) == tiny       # a difference, and no unit below it
+    x = rng.standard_normal(pr.neq)
+    with Context(0) as ctx:
+        ctx.mesh_set(gc)
+        ctx.steer_set(pr.g_g, pr.neq)
+        ctx.trim()
+        before = ctx.mem_used()
+        for _ in range(2):
+            ctx.assemble_transient(0.5, 0.01, prop, etype)
+        ctx.trim()
+        # storkb whole; storka whole or as 372 bytes of 512
+        held = ctx.mem_used() - before
+        assert held >= 2 * KA.nbytes if tiny or pr.nels <= 65536 else held < 1.8 * KA.nbytes
+        assert np.array_equal(ctx.storkm_get(), KA)
+        dg = O.diag(pr.g_g, KA, pr.neq)
+        assert np.array_equal(ctx.diag_get(), dg)
+        assert np.array_equal(ctx.apply_raw(0, x), O.apply(pr.g_g, KA, x))
+        assert np.array_equal(ctx.apply_raw(1, x), O.apply(pr.g_g, KB, x))
+        xo = O.pcg(pr.g_g, KA, x, dg, 0.0, 5, stop=O.STOP_RELRES, dot_order=O.DOT_DEVICE, nthreads=8)[0]
+        assert np.array_equal(ctx.pcg_solve(x, 5, 0.0, stop="relres")[0], xo)
+
+
 @pytest.mark.parametrize("nod,box", [(20, (11, 11, 10)), (8, (20, 19, 20))])
 def test_assembled_triangle_bitexact(nod, box):
     """Distorted elements with moduli of their own, assembled straight into
