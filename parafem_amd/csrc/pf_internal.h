@@ -310,9 +310,9 @@ int *pf_flag_word(pf_ctx *c);
 // The (element, element node) slots of every node in ascending order, built on
 // the device from g_num (device, ns entries; entries outside 1..nn are
 // skipped): ptr (nn + 1), slot (ns).  work: pf_node_work(nn) ints.  *many is
-// set to 1 where a node has more than PF_NODE_SORT slots, whose lists are then
-// not sorted.
-constexpr int PF_NODE_SORT = 64;
+// set to 1 where a node has more than PF_NODE_LONG slots, whose lists are then
+// not sorted, and work[0] (device) with it.
+constexpr int PF_NODE_SORT = 16, PF_NODE_LONG = 4096;   // slots a thread sorts; a workgroup
 size_t pf_node_work(int nn);
 void pf_node_slots(pf_ctx *c, const int *g_num, int ns, int nn, int *work, int *ptr, int *slot, int *many);
 

@@ -137,8 +137,9 @@ __global__ __launch_bounds__(128) void k_stress(const double *__restrict__ gc, c
 template <typename SLOT>
 __global__ __launch_bounds__(256) void k_scatter_nodes(const int *__restrict__ ptr, const SLOT *__restrict__ slot,
                                                       const double *__restrict__ contrib, double *__restrict__ out,
-                                                      int nn, int numvar, int flag)
+                                                      int nn, int numvar, int flag, const int *__restrict__ many)
 {
+    if (many && *many) return;   // the host's map will do
     const int node = blockIdx.x * blockDim.x + threadIdx.x;
     if (node >= nn) return;
     const int a = ptr[node], b = ptr[node + 1];
@@ -152,13 +153,15 @@ __global__ __launch_bounds__(256) void k_scatter_nodes(const int *__restrict__ p
 
 }  // namespace
 
-// The node map is built on the device, seven launches of 1 to 20 us.  On the
+// The node map is built on the device, eight launches of 1 to 20 us.  On the
 // host, whose two passes over the slots take about 2 ns a slot, are built the
 // map of few slots and nodes (the line is where both take the same, whole call
 // with three values a node: 42,841 slots and nodes 139 us on the host, 146 on
 // the device; 100,705 292 / 244; 142,576 344 / 210; 795,841 1,968 / 1,304),
-// the map of a node with more elements than the sort takes, and one whose
-// slots an int does not number.
+// the map of a node with more than 4,096 elements, and one whose slots an int
+// does not number.  (A node of 65 elements among 10,000 / 40,000 / 200,000
+// bricks, whole call: host 0.30 / 0.86 / 5.0 ms, device 0.26 / 0.48 / 2.1; of 1,000
+// 0.85 / 1.44 / 5.5 and 0.80 / 1.05 / 2.7.)
 constexpr long NODE_DEVICE = 65536;
 
 extern "C" int pf_scatter_nodes(pf_ctx *c, int nn, int nod, int nels, const int *g_num, int numvar,
@@ -180,6 +183,7 @@ extern "C" int pf_scatter_nodes(pf_ctx *c, int nn, int nod, int nels, const int 
     if (!rc) rc = pf_alloc(c, (void **)&dout, no * sizeof(double));
     hipError_t he = hipSuccess;
     const dim3 grid((nn + 255) / 256), blk(256);
+    bool have_c = false;   // the contributions are on the device
     if (!rc && on_device) {
         int *dnum = nullptr, *dslot = nullptr, *work = nullptr, *many = pf_flag_word(c);
         const size_t wsz = pf_node_work(nn) * sizeof(int);
@@ -193,9 +197,11 @@ extern "C" int pf_scatter_nodes(pf_ctx *c, int nn, int nod, int nels, const int 
                 // the map is built while the contributions travel
                 pf_node_slots(c, dnum, (int)ns, nn, work, dptr, dslot, many);
                 he = hipMemcpyAsync(dc, contrib, (size_t)ns * numvar * sizeof(double), hipMemcpyHostToDevice, c->stream);
+                have_c = he == hipSuccess;
             }
             if (he == hipSuccess) {
-                hipLaunchKernelGGL(k_scatter_nodes<int>, grid, blk, 0, c->stream, dptr, dslot, dc, dout, nn, numvar, flag);
+                hipLaunchKernelGGL(k_scatter_nodes<int>, grid, blk, 0, c->stream, dptr, dslot, dc, dout, nn, numvar, flag,
+                                   work);
                 he = hipGetLastError();
             }
             if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
@@ -222,10 +228,11 @@ extern "C" int pf_scatter_nodes(pf_ctx *c, int nn, int nod, int nels, const int 
         if (!rc) {
             he = hipMemcpyAsync(dptr, ptr.data(), psz, hipMemcpyHostToDevice, c->stream);
             if (he == hipSuccess) he = hipMemcpyAsync(dslot, slot.data(), ssz, hipMemcpyHostToDevice, c->stream);
-            if (he == hipSuccess && ns)
+            if (he == hipSuccess && ns && !have_c)
                 he = hipMemcpyAsync(dc, contrib, (size_t)ns * numvar * sizeof(double), hipMemcpyHostToDevice, c->stream);
             if (he == hipSuccess) {
-                hipLaunchKernelGGL(k_scatter_nodes<long>, grid, blk, 0, c->stream, dptr, dslot, dc, dout, nn, numvar, flag);
+                hipLaunchKernelGGL(k_scatter_nodes<long>, grid, blk, 0, c->stream, dptr, dslot, dc, dout, nn, numvar, flag,
+                                   nullptr);
                 he = hipGetLastError();
             }
             (void)hipStreamSynchronize(c->stream);

@@ -172,13 +172,15 @@ __global__ __launch_bounds__(256) void k_steer_gather(const int *__restrict__ g_
     }
 }
 
-// Slots per node; *many is set where a node has more than the sort takes.
+// Slots per node; *many and its copy on the device are set where a node has more
+// than the sorts take.
 __global__ __launch_bounds__(256) void k_node_count(const int *__restrict__ g_num, int ns, int nn,
-                                                   int *__restrict__ cnt, int *__restrict__ many)
+                                                   int *__restrict__ cnt, int *__restrict__ many,
+                                                   int *__restrict__ dmany)
 {
     for (long s = (long)blockIdx.x * blockDim.x + threadIdx.x; s < ns; s += (long)gridDim.x * blockDim.x) {
         const int g = g_num[s];
-        if (g >= 1 && g <= nn && atomicAdd(&cnt[g - 1], 1) == PF_NODE_SORT) *many = 1;
+        if (g >= 1 && g <= nn && atomicAdd(&cnt[g - 1], 1) == PF_NODE_LONG) *many = *dmany = 1;
     }
 }
 
@@ -193,13 +195,39 @@ __global__ __launch_bounds__(256) void k_node_fill(const int *__restrict__ g_num
     }
 }
 
-// Ascending order of the lists the sort takes (it is quadratic in the length).
-__global__ __launch_bounds__(256) void k_node_sort(const int *__restrict__ ptr, int *__restrict__ slot, int nn)
+// Ascending order of the short lists, a thread each (quadratic in the length);
+// the nodes of the longer ones are noted.
+__global__ __launch_bounds__(256) void k_node_sort(const int *__restrict__ ptr, int *__restrict__ slot, int nn,
+                                                  int *__restrict__ longs, int *__restrict__ nlong)
 {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= nn) return;
     const int a = ptr[n], b = ptr[n + 1];
     if (b - a <= PF_NODE_SORT) sort_slots(slot, a, b);
+    else if (b - a <= PF_NODE_LONG) longs[atomicAdd(nlong, 1)] = n;
+}
+
+// Ascending order of the longer lists, a workgroup each: every slot to the place
+// that the number of smaller ones gives.
+constexpr int LONG_T = 1024;
+__global__ __launch_bounds__(LONG_T) void k_node_sort_long(const int *__restrict__ ptr, int *__restrict__ slot,
+                                                       const int *__restrict__ longs, const int *__restrict__ nlong)
+{
+    __shared__ int s[PF_NODE_LONG];
+    const int nl = *nlong;
+    for (int l = blockIdx.x; l < nl; l += gridDim.x) {
+        const int a = ptr[longs[l]], n = ptr[longs[l] + 1] - a;
+        for (int i = threadIdx.x; i < n; i += LONG_T) s[i] = slot[a + i];
+        __syncthreads();
+        for (int i = threadIdx.x; i < n; i += LONG_T) {
+            const int v = s[i];
+            int rank = 0;
+#pragma unroll 8
+            for (int j = 0; j < n; ++j) rank += s[j] < v;
+            slot[a + rank] = v;
+        }
+        __syncthreads();   // the list is read before the next one is written
+    }
 }
 
 // *bad is set where an entry of g_num is not a node.
@@ -302,19 +330,22 @@ void pf_scan_launch(pf_ctx *c, const int *cnt, int n, int *bsum, int *ptr, int *
     hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, c->stream, cnt, n, bsum, ptr, zero_flag);
 }
 
-// work: nn counts, the block sums of the scan, its total and its flags (unused)
-size_t pf_node_work(int nn) { return (size_t)nn + pf_scan_blocks(nn) + 2; }
+// work: the device's copy of many, the number of longer lists, nn counts (then
+// the nodes of the longer lists), the block sums of the scan, its total and its
+// flags (unused)
+size_t pf_node_work(int nn) { return 2 + (size_t)nn + pf_scan_blocks(nn) + 2; }
 
 void pf_node_slots(pf_ctx *c, const int *g_num, int ns, int nn, int *work, int *ptr, int *slot, int *many)
 {
-    int *cnt = work, *bsum = cnt + nn, *total = bsum + pf_scan_blocks(nn);
-    (void)hipMemsetAsync(cnt, 0, (size_t)nn * sizeof(int), c->stream);
+    int *nlong = work + 1, *cnt = work + 2, *bsum = cnt + nn, *total = bsum + pf_scan_blocks(nn);
+    (void)hipMemsetAsync(work, 0, ((size_t)nn + 2) * sizeof(int), c->stream);
     (void)hipMemsetAsync(ptr, 0, sizeof(int), c->stream);
     const dim3 gs(grid_for_stride(ns));
-    hipLaunchKernelGGL(k_node_count, gs, dim3(256), 0, c->stream, g_num, ns, nn, cnt, many);
+    hipLaunchKernelGGL(k_node_count, gs, dim3(256), 0, c->stream, g_num, ns, nn, cnt, many, work);
     pf_scan_launch(c, cnt, nn, bsum, ptr, total, total + 1);
     hipLaunchKernelGGL(k_node_fill, gs, dim3(256), 0, c->stream, g_num, ns, nn, ptr, cnt, slot);
-    hipLaunchKernelGGL(k_node_sort, dim3((nn + 255) / 256), dim3(256), 0, c->stream, ptr, slot, nn);
+    hipLaunchKernelGGL(k_node_sort, dim3((nn + 255) / 256), dim3(256), 0, c->stream, ptr, slot, nn, cnt, nlong);
+    hipLaunchKernelGGL(k_node_sort_long, dim3(64), dim3(LONG_T), 0, c->stream, ptr, slot, cnt, nlong);
 }
 
 // Transposed steering of c->g_g (already on the device, c->neq and c->ntot,

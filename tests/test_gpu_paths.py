@@ -414,6 +414,24 @@ def test_node_maps(nels, star):
             assert np.array_equal(ctx.scatter_nodes(g, c, nn, flag), O.scatter_nodes(g, c, nn, flag), equal_nan=True)
 
 
+# Lists that a thread sorts (16 slots) and that a workgroup does (17 to 4,096),
+# more of them than workgroups, and one that is left to the host (4,097).
+@pytest.mark.parametrize("length,count", [(16, 5), (17, 5), (255, 3), (256, 3), (257, 200), (4096, 2), (4097, 1)])
+def test_node_maps_with_long_lists(length, count):
+    rng = np.random.default_rng(length)
+    nels, nod, nn = 20000, 8, 30000
+    g = rng.permutation(np.resize(np.arange(1000, nn) + 1, nels * nod)).astype(np.int32)   # 5 or 6 each
+    where = rng.choice(g.size, length * count, replace=False).reshape(count, length)
+    for k in range(count):
+        g[where[k]] = 1 + 3 * k
+    g = g.reshape(nels, nod)
+    print(f"[gpu-test] node lists {length} {count}", flush=True)
+    with Context(0) as ctx:
+        for numvar, flag in ((1, 1), (3, 0)):
+            c = rng.standard_normal((nels, nod, numvar))
+            assert np.array_equal(ctx.scatter_nodes(g, c, nn, flag), O.scatter_nodes(g, c, nn, flag), equal_nan=True)
+
+
 # Elements of p122's stress update around the eight of a wavefront.
 @pytest.mark.parametrize("nels", [1, 7, 8, 9, 67])
 @pytest.mark.parametrize("phi", [0.0, 20.0])
