@@ -669,11 +669,14 @@ __global__ __launch_bounds__(PF_BLOCK) void k_scatter_pu(const int *__restrict__
 // k_scatter_pu with the slot lists of nodes: one list for a node's three
 // freedoms, and a code per equation in place of its two offsets.  The scatter
 // is bound by its reads, of which the equations' own lists are more than a
-// third (hex20, FP32 products: 24 of 60 bytes an equation); these are 11.  100^3
-// hex20 mixed 279 -> 272 ms (150 iterations), 71x63x50 438 -> 424 us an
-// iteration, FP64 893 -> 886, 80^3 hex8 elastic mixed 231 -> 222, FP64 441 ->
-// 431.  A wavefront's lists are one contiguous run, staged in LDS; streaming
-// loads of them are slower here (71x63x50 mixed 429).
+// third (hex20, FP32 products: 24 of 60 bytes an equation); these are 11.  The
+// kernel, us with a list per equation / with these: 100^3 hex20, FP32 products
+// 262 / 210 (1.66 / 1.48 GB by the counters), FP64 293 / 265; 40^3 hex20 26.9 /
+// 22.7 and 26.7 / 24.3; 62^3 hex8 elastic 30.6 / 25.7 and 35.4 / 33.0; where the
+// equations are numbered so that no node's follow each other, the same (40^3
+// freedom by freedom 44.4 / 41.8 and 40.8 / 40.6).  A wavefront's lists are one
+// contiguous run, staged in LDS; streaming loads of them are slower here
+// (71x63x50 mixed 429 us an iteration against 424).
 template <typename UT>
 __global__ __launch_bounds__(PF_BLOCK) void k_scatter_nl(const unsigned *__restrict__ code,
                                                         const int *__restrict__ list, const UT *__restrict__ utemp,

@@ -191,7 +191,7 @@ struct pf_ranges {
     std::vector<int> cstart;           // (ncol+1) colour offsets into cdesc
 };
 
-// The pinned words of a context, in one allocation (each costs about 40 us).
+// The pinned words of a context, in one allocation (each costs about 24 us).
 struct pf_pinned {
     pf_state state, query;
     alignas(64) double scalar[64];
