@@ -1693,7 +1693,9 @@ __device__ __forceinline__ void bs_ebe_refine(const pf_bslot *__restrict__ T, co
     }
 }
 
-template <typename UT>
+// PERS: of the persistent kernel, whose solves all fold in phases of their own
+// (no slot8).
+template <typename UT, bool PERS>
 __device__ __forceinline__ void bs_scatter_pu(const pf_bslot *__restrict__ T, const int *__restrict__ qst, int ns,
                                               int b)
 {
@@ -1702,7 +1704,7 @@ __device__ __forceinline__ void bs_scatter_pu(const pf_bslot *__restrict__ T, co
     const UT *ut;
     if constexpr (sizeof(UT) == 4) ut = (const UT *)S.utemp32;
     else ut = (const UT *)S.utemp;
-    if (S.slot8) {
+    if (!PERS && S.slot8) {
         scatter_copy_block<UT>(b - qst[s], S.slot8, ut, S.fixstore, S.p, S.u, S.neq, S.fix_zero, S.partials, S.st,
                                nullptr, S.rowmajor, S.nels);
         return;
@@ -1712,12 +1714,12 @@ __device__ __forceinline__ void bs_scatter_pu(const pf_bslot *__restrict__ T, co
                          S.partials);
 }
 
-template <bool CHECON>
+template <bool CHECON, bool PERS>
 __device__ __forceinline__ void bs_update(const pf_bslot *__restrict__ T, const int *__restrict__ qst, int ns, int b)
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
-    if (S.slot8) {
+    if (!PERS && S.slot8) {
         update_fold_block<CHECON>(b - qst[s], S.G, S.x, S.r, S.d, S.p, S.u, S.dinv, S.neq, S.partials, S.st);
         return;
     }
@@ -1725,22 +1727,23 @@ __device__ __forceinline__ void bs_update(const pf_bslot *__restrict__ T, const 
     update_block<CHECON>(b - qst[s], S.G, S.x, S.r, S.d, S.p, S.u, S.dinv, S.neq, S.partials, S.st);
 }
 
+template <bool PERS>
 __device__ __forceinline__ void bs_scatter_res(const pf_bslot *__restrict__ T, const int *__restrict__ qst, int ns,
                                                int b)
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
-    if (S.slot8 ? stopped(S.st + 1) || !S.st[1].refine : skip(S.st, RUN_REFINE)) return;
+    if (!PERS && S.slot8 ? stopped(S.st + 1) || !S.st[1].refine : skip(S.st, RUN_REFINE)) return;
     scatter_res_block(b - qst[s], S.G, S.csr_ptr, S.slot, S.utemp, S.fixstore, S.x, S.f, S.r, S.d, S.dinv, S.neq,
-                      S.partials, S.slot8 != nullptr);
+                      S.partials, !PERS && S.slot8);
 }
 
-template <bool CHECON>
+template <bool CHECON, bool PERS>
 __device__ __forceinline__ void bs_pupdate(const pf_bslot *__restrict__ T, const int *__restrict__ qst, int ns, int b)
 {
     const int s = bslot_find(qst, ns, b);
     const pf_bslot S = slot_of(T, s);
-    if (S.slot8) {
+    if (!PERS && S.slot8) {
         pupdate_fold_block<CHECON>(b - qst[s], S.G, S.p, S.p32, S.d, S.neq, S.partials, S.st);
         return;
     }
@@ -1804,27 +1807,27 @@ template <typename UT>
 __global__ __launch_bounds__(PF_BLOCK) void kb_scatter_pu(const pf_bslot *__restrict__ T, const int *__restrict__ qst,
                                                          int ns)
 {
-    bs_scatter_pu<UT>(T, qst, ns, blockIdx.x);
+    bs_scatter_pu<UT, false>(T, qst, ns, blockIdx.x);
 }
 
 template <bool CHECON>
 __global__ __launch_bounds__(PF_BLOCK) void kb_update(const pf_bslot *__restrict__ T, const int *__restrict__ qst,
                                                      int ns)
 {
-    bs_update<CHECON>(T, qst, ns, blockIdx.x);
+    bs_update<CHECON, false>(T, qst, ns, blockIdx.x);
 }
 
 __global__ __launch_bounds__(PF_BLOCK) void kb_scatter_res(const pf_bslot *__restrict__ T, const int *__restrict__ qst,
                                                           int ns)
 {
-    bs_scatter_res(T, qst, ns, blockIdx.x);
+    bs_scatter_res<false>(T, qst, ns, blockIdx.x);
 }
 
 template <bool CHECON>
 __global__ __launch_bounds__(PF_BLOCK) void kb_pupdate(const pf_bslot *__restrict__ T, const int *__restrict__ qst,
                                                       int ns)
 {
-    bs_pupdate<CHECON>(T, qst, ns, blockIdx.x);
+    bs_pupdate<CHECON, false>(T, qst, ns, blockIdx.x);
 }
 
 template <int WHICH>
@@ -1904,14 +1907,14 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
         }
         if (!grid_barrier(bar, nb)) return;
         for (int b = blockIdx.x; b < total_qb; b += nb) {
-            bs_scatter_pu<OUT>(T, qst, ns, b);
+            bs_scatter_pu<OUT, true>(T, qst, ns, b);
             __syncthreads();   // the block's sums are read before the next one's are written
         }
         if (!grid_barrier(bar, nb)) return;
         for (int s = blockIdx.x; s < ns; s += nb) bs_fold<0>(T, s);
         if (!grid_barrier(bar, nb)) return;
         for (int b = blockIdx.x; b < total_qb; b += nb) {
-            bs_update<CHECON>(T, qst, ns, b);
+            bs_update<CHECON, true>(T, qst, ns, b);
             __syncthreads();   // the block's sums are read before the next one's are written
         }
         if (!grid_barrier(bar, nb)) return;
@@ -1924,7 +1927,7 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
                 bs_ebe_refine<NT>(T, est + EST_REF * PF_BATCH_MAX, ns, total_ebr, blockIdx.x, nb);
                 if (!grid_barrier(bar, nb)) return;
                 for (int b = blockIdx.x; b < total_qb; b += nb) {
-                    bs_scatter_res(T, qst, ns, b);
+                    bs_scatter_res<true>(T, qst, ns, b);
                     __syncthreads();   // the block's sums are read before the next one's are written
                 }
                 if (!grid_barrier(bar, nb)) return;
@@ -1932,7 +1935,7 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_persistent(const pf_bslot *__rest
                 if (!grid_barrier(bar, nb)) return;
             }
         }
-        for (int b = blockIdx.x; b < total_qb; b += nb) bs_pupdate<CHECON>(T, qst, ns, b);
+        for (int b = blockIdx.x; b < total_qb; b += nb) bs_pupdate<CHECON, true>(T, qst, ns, b);
         if (!grid_barrier(bar, nb)) return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) bar->iters = it;
