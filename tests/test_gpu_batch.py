@@ -179,6 +179,35 @@ def test_persistent_with_more_blocks_than_workgroups(el, precision, stop):
             c.close()
 
 
+@pytest.mark.parametrize("precision", ["mixed64", "mixed"])
+def test_batch_replacements_in_turn(precision):
+    """Solves of very different sizes whose residuals are replaced in the same
+    and in different iterations, more blocks of products than workgroups:
+    every solve as alone, replacements counted alike."""
+    probs = [P.elastic_cube(18, e=37.0, v=0.22), P.elastic_cube(2), P.elastic_cube(9, lognormal_e=True),
+             P.elastic_cube(18, e=74.0, v=0.22), P.elastic_cube(5, v=0.4)]
+    ctxs = [Context(0) for _ in probs]
+    try:
+        rs = [P.setup(c, pr, store="fp32") for c, pr in zip(ctxs, probs)]
+        say(f"batch replacements {precision}")
+        kw = dict(stop="relres", precision=precision, refine_delta=0.5)
+        alone = [c.pcg_solve(r, 90, 0.0, **kw) for c, r in zip(ctxs, rs)]
+        assert min(res.refinements for _, res in alone) > 0
+        with Batch(0) as b:
+            for graph in (True, False):
+                for c, r in zip(ctxs, rs):
+                    c.pcg_begin(r, 90, 0.0, **kw)
+                for _ in range(6):
+                    b.run(ctxs, 16, graph=graph)
+                for c, (x, res) in zip(ctxs, alone):
+                    got = c.pcg_poll()
+                    assert (got.iters, got.refinements) == (res.iters, res.refinements)
+                    assert np.array_equal(c.pcg_x(), x)
+    finally:
+        for c in ctxs:
+            c.close()
+
+
 def test_batch_rejects_mixed_settings():
     """Solves of one batch share ntot, precision and stopping rule."""
     from parafem_amd import PFError
