@@ -2959,6 +2959,15 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
         if (!S.solo) qb += S.G;
         if (mixed && !c->utemp32) return PF_ERR_STATE;
     }
+    // Where some solve needs the folds' launches, all take them: an iteration
+    // has them anyway, and the others would only add their own folds and
+    // kb_due to it (ms to convergence in mixed64, each as it can / all alike:
+    // 16 hex20 solves of n = 20 to 35 774 / 754, 16 of 10 to 40 846 / 832, 8 of
+    // 30 to 44 1,083 / 1,069).
+    if (folds && due) {
+        due = false;
+        for (pf_bslot &S : T) S.slot8 = nullptr;
+    }
     // elements per logical block of each list's products
     int EPB[EST_LISTS];
     const int prec = c0->opts.precision;

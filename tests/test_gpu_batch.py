@@ -208,6 +208,39 @@ def test_batch_replacements_in_turn(precision):
             c.close()
 
 
+@pytest.mark.parametrize("precision,stop", [("fp64", "checon"), ("mixed64", "relres"), ("mixed", "relres")])
+def test_batch_of_solves_with_and_without_folds(precision, stop):
+    """A solve above 2,048 reduction blocks joins and leaves a batch of solves
+    below (which then fold by launches, or for themselves): the iterates of
+    every solve alone, whichever way each run took."""
+    probs = [P.laplace_cube(n, lognormal_k=True, seed=n) for n in (12, 81, 30, 5)]
+    assert (probs[1].neq + 255) // 256 > 2048 >= (probs[2].neq + 255) // 256
+    ctxs = [Context(0) for _ in probs]
+    try:
+        rs = [P.setup(c, pr, store="fp64" if precision == "fp64" else "fp32") for c, pr in zip(ctxs, probs)]
+        say(f"batch with and without folds {precision}")
+        kw = dict(stop=stop, precision=precision)
+        if precision != "fp64":
+            kw["refine_delta"] = 0.5
+        alone = [c.pcg_solve(r, 30, 0.0, **kw) for c, r in zip(ctxs, rs)]
+        small = [ctxs[0], ctxs[2], ctxs[3]]
+        with Batch(0) as b:
+            for graph in (True, False):
+                for c, r in zip(ctxs, rs):
+                    c.pcg_begin(r, 30, 0.0, **kw)
+                b.run(small, 7, graph=graph)
+                b.run(ctxs, 11, graph=graph)
+                b.run(small, 5, graph=graph)
+                b.run(ctxs, 30, graph=graph)
+                for c, (x, res) in zip(ctxs, alone):
+                    got = c.pcg_poll()
+                    assert (got.iters, got.refinements) == (res.iters, res.refinements) and res.iters == 30
+                    assert np.array_equal(c.pcg_x(), x)
+    finally:
+        for c in ctxs:
+            c.close()
+
+
 def test_batch_rejects_mixed_settings():
     """Solves of one batch share ntot, precision and stopping rule."""
     from parafem_amd import PFError
