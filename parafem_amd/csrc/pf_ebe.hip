@@ -1576,7 +1576,7 @@ int reduce_prim(pf_ctx *c, const double *a, double *b, int64_t n, int mode, doub
 // for bit.  Solves with a padded slot table fold for themselves (as in
 // iterations without fold launches, p formed by kb_pupdate); the folds are
 // launched only for the others, so a batch of small solves runs 4 launches an
-// iteration (mixed: 7) instead of 6 (9): sixteen solves of n = 6 to 18 in
+// iteration (mixed: 6 or 7) instead of 6 (9): sixteen solves of n = 6 to 18 in
 // mixed64 83 -> 64 ms.
 struct pf_bslot {
     const double *K64;
@@ -1781,6 +1781,19 @@ __global__ __launch_bounds__((64 * ebe_wpb<NT, KIND>()), (ebe_minw<NT, KIND>()))
     bs_ebe<NT, KIND, OUT, false, ANY>(T, est, ns, xcd_block(blockIdx.x, gridDim.x), RUN_LIVE);
 }
 
+// The true-residual products of solve S: blocks b0, b0 + nb, ...
+template <int NT>
+__device__ __forceinline__ void bs_refine_products(const pf_bslot &S, long b0, long nb)
+{
+    constexpr int EPB = Lanes<NT, KIND_ACC>::EPB;
+    const long nlb = (S.nels + EPB - 1) / EPB;
+    for (long lb = b0; lb < nlb; lb += nb) {
+        ebe_block<NT, KIND_ACC, true, double, Lanes<NT, KIND_ACC>::EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.x, nullptr,
+                                                                       S.utemp, S.nels, S.kstride, S.rowmajor, false);
+        __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
+    }
+}
+
 // Whether a replacement is due, for the solves that fold for themselves: a
 // workgroup a solve, which notes it in the working state.
 __global__ __launch_bounds__(PF_BLOCK) void kb_due(const pf_bslot *__restrict__ T)
@@ -1791,11 +1804,7 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_due(const pf_bslot *__restrict__ 
 
 // The true-residual products of the solves that a replacement is due for, every
 // workgroup on each of them in turn: a lane looks at a solve's state, and on
-// most iterations none is due.  (Workgroups dealt to the solves by their size,
-// each folding to find out, left most of the device idle while a few solves
-// were replaced; ms to convergence in mixed64, so / now: 32 hex20 solves of
-// n = 16 to 24 399 / 374, 32 of n = 24 735 / 712, 16 of 6 to 18 60.3 / 60.2.
-// 512 to 2,048 workgroups the same.)
+// most iterations none is due.
 template <int NT>
 __global__ __launch_bounds__(PF_BLOCK) void kb_ebe_refine(const pf_bslot *__restrict__ T, int ns)
 {
@@ -1806,17 +1815,27 @@ __global__ __launch_bounds__(PF_BLOCK) void kb_ebe_refine(const pf_bslot *__rest
         const pf_state *st = as_global(R.st);
         due = !R.solo && (R.slot8 ? !stopped(st + 1) && st[1].refine : !skip(st, RUN_REFINE));
     }
-    constexpr int EPB = Lanes<NT, KIND_ACC>::EPB;
-    for (unsigned long long m = __ballot(due); m; m &= m - 1) {
-        const pf_bslot S = slot_of(T, __ffsll(m) - 1);
-        const long nlb = (S.nels + EPB - 1) / EPB;
-        for (long lb = blockIdx.x; lb < nlb; lb += gridDim.x) {
-            ebe_block<NT, KIND_ACC, true, double, Lanes<NT, KIND_ACC>::EPL>(lb, S.K64, S.Khi, S.Klo, S.g_g, S.x, nullptr,
-                                                                           S.utemp, S.nels, S.kstride, S.rowmajor,
-                                                                           false);
-            __builtin_amdgcn_wave_barrier();   // this wave's LDS reads finish before the next block's writes
-        }
-    }
+    for (unsigned long long m = __ballot(due); m; m &= m - 1)
+        bs_refine_products<NT>(slot_of(T, __ffsll(m) - 1), blockIdx.x, gridDim.x);
+}
+
+// The same where every solve folds for itself and the matrices are few: the
+// workgroups dealt to the solves by their size (rst: first workgroup of each
+// solve, total in all), each folding to find out, without kb_due's launch.
+// While a few solves are replaced the others' workgroups stand idle, which large
+// matrices feel.  ms to convergence in mixed64, dealt / in turn, by GB of hi and
+// lo: 2 hex20 solves of n = 12 (0.05) 13.5 / 14.5, 16 of 6 to 18 (0.48) 57.6 /
+// 61.1, 16 of 14 to 20 (1.14) 118.8 / 120.3, 32 of 10 to 18 (1.33) 128 / 124, 32 of 16
+// to 24 (3.9) 399 / 374.  512 to 2,048 workgroups in turn the same.
+constexpr size_t REFINE_DEALT = (size_t)1 << 30;
+template <int NT>
+__global__ __launch_bounds__(PF_BLOCK) void kb_ebe_refine_dealt(const pf_bslot *__restrict__ T,
+                                                               const int *__restrict__ rst, int ns, int total)
+{
+    const int b = blockIdx.x, s = bslot_find(rst, ns, b);
+    const pf_bslot S = slot_of(T, s);
+    const int b0 = b - rst[s], nb = (s + 1 < ns ? rst[s + 1] : total) - rst[s];
+    if (refine_due(S.partials, S.G, S.st + 1, b0 == 0)) bs_refine_products<NT>(S, b0, nb);
 }
 
 template <typename UT>
@@ -2860,15 +2879,16 @@ struct pf_batch {
     long *est = nullptr;                           // device: first element block per solve, a list per
                                                    // kind of product (EST_*)
     int *qst = nullptr;                            // device: first equation block per solve
+    int *rst = nullptr;                            // device: first workgroup per solve of the replacement's products
     pf_bslot *T_host = nullptr;                    // pinned staging of the three (one allocation)
     long *est_host = nullptr;
-    int *qst_host = nullptr;
+    int *qst_host = nullptr, *rst_host = nullptr;
     std::vector<pf_bslot> cur;                     // the table on the device
     std::vector<long> cur_est;
-    std::vector<int> cur_qst;
+    std::vector<int> cur_qst, cur_rst;
     int ns = 0, ntot = 0, precision = -1, stop = -1;
     long total[EST_LISTS] = {};                    // element blocks of each list
-    int total_qb = 0;
+    int total_qb = 0, total_rb = 0;                // total_rb 0: every workgroup takes each solve
     bool folds = false;   // some batched solve needs the folds' launches
     bool due = false;     // some folds for itself
     bool any = false;     // FP64 products of any storage in EST_ITER
@@ -2893,7 +2913,7 @@ struct pf_batch {
 };
 
 static const size_t kBatchTable = sizeof(pf_bslot) * PF_BATCH_MAX + EST_LISTS * sizeof(long) * PF_BATCH_MAX +
-                                  sizeof(int) * PF_BATCH_MAX;
+                                  2 * sizeof(int) * PF_BATCH_MAX;
 
 static void batch_graph_drop(pf_batch *b)
 {
@@ -2914,7 +2934,7 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
     if (!c0) return PF_ERR_ARG;
     std::vector<pf_bslot> T(nctx);
     std::vector<long> est(EST_LISTS * (size_t)nctx);
-    std::vector<int> qst(nctx);
+    std::vector<int> qst(nctx), rst(nctx);
     long total[EST_LISTS] = {};
     int qb = 0;
     bool folds = false, due = false;
@@ -3001,10 +3021,21 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
         total[it] += (T[k].nels + EPB[it] - 1) / EPB[it];
         total[EST_REF] += (T[k].nels + EPB[EST_REF] - 1) / EPB[EST_REF];
     }
+    // the replacement's products dealt by size: about 1,024 workgroups, at least
+    // one a solve
+    int rb = 0;
+    const size_t hilo = (size_t)total[EST_REF] * EPB[EST_REF] * 2 * pf_sym_per(c0->ntot) * sizeof(float);
+    if (due && hilo <= REFINE_DEALT)
+        for (int k = 0; k < nctx; ++k) {
+            rst[k] = rb;
+            if (!T[k].solo)
+                rb += 1 + (int)(((T[k].nels + EPB[EST_REF] - 1) / EPB[EST_REF] - 1) *
+                                std::min<long>(1024, total[EST_REF]) / total[EST_REF]);
+        }
     PF_HIP(hipSetDevice(b->device));
     const bool same = !b->stale && nctx == b->ns &&
                       std::memcmp(T.data(), b->cur.data(), sizeof(pf_bslot) * nctx) == 0 &&
-                      est == b->cur_est && qst == b->cur_qst && any == b->any &&
+                      est == b->cur_est && qst == b->cur_qst && rst == b->cur_rst && any == b->any &&
                       std::equal(total, total + EST_LISTS, b->total);
     if (!same) {
         PF_HIP(hipEventSynchronize(b->ev_table));   // the staging buffer is free again
@@ -3012,11 +3043,12 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
         for (int l = 0; l < EST_LISTS; ++l)
             std::memcpy(b->est_host + l * PF_BATCH_MAX, est.data() + l * nctx, sizeof(long) * nctx);
         std::memcpy(b->qst_host, qst.data(), sizeof(int) * nctx);
+        std::memcpy(b->rst_host, rst.data(), sizeof(int) * nctx);
         PF_HIP(hipMemcpyAsync(b->T, b->T_host, kBatchTable, hipMemcpyHostToDevice, b->stream));
         PF_HIP(hipEventRecord(b->ev_table, b->stream));
         // a captured graph reads the batched solves from the table, but
         // holds the solo solves' launches with their own buffers
-        if (!std::equal(total, total + EST_LISTS, b->total) || qb != b->total_qb ||
+        if (!std::equal(total, total + EST_LISTS, b->total) || qb != b->total_qb || rb != b->total_rb ||
             folds != b->folds || due != b->due || any != b->any || nctx != b->ns || c0->ntot != b->ntot ||
             c0->opts.precision != b->precision || c0->opts.stop_mode != b->stop || !solo.empty() ||
             !b->solo.empty() || b->stale)
@@ -3026,6 +3058,8 @@ static int batch_prepare(pf_batch *b, int nctx, pf_ctx *const *ctxs, bool persis
         b->cur = T;
         b->cur_est = est;
         b->cur_qst = qst;
+        b->cur_rst = rst;
+        b->total_rb = rb;
         b->folds = folds;
         b->due = due;
         b->any = any;
@@ -3092,9 +3126,14 @@ static void batch_iteration_nt(pf_batch *b)
         if (b->folds) hipLaunchKernelGGL(kb_fold<2>, gs, blk, 0, b->stream, b->T);
     }
     if (prec == PF_PREC_MIXED || prec == PF_PREC_MIXED64) {
-        if (b->due) hipLaunchKernelGGL(kb_due, gs, blk, 0, b->stream, b->T);
-        hipLaunchKernelGGL(kb_ebe_refine<NT>, dim3((unsigned)std::min<long>(b->total[EST_REF], REFINE_GRID)), blk, 0,
-                           b->stream, b->T, b->ns);
+        if (b->total_rb) {
+            hipLaunchKernelGGL(kb_ebe_refine_dealt<NT>, dim3((unsigned)b->total_rb), blk, 0, b->stream, b->T, b->rst,
+                               b->ns, b->total_rb);
+        } else {
+            if (b->due) hipLaunchKernelGGL(kb_due, gs, blk, 0, b->stream, b->T);
+            hipLaunchKernelGGL(kb_ebe_refine<NT>, dim3((unsigned)std::min<long>(b->total[EST_REF], REFINE_GRID)), blk,
+                               0, b->stream, b->T, b->ns);
+        }
         hipLaunchKernelGGL(kb_scatter_res, gq, blk, 0, b->stream, b->T, b->qst, b->ns);
         if (b->folds) hipLaunchKernelGGL(kb_fold<3>, gs, blk, 0, b->stream, b->T);
     }
@@ -3209,11 +3248,13 @@ int pf_batch_create(int device, pf_batch **out)
         b->T = (pf_bslot *)dt;
         b->est = (long *)((char *)dt + sizeof(pf_bslot) * PF_BATCH_MAX);
         b->qst = (int *)((char *)b->est + EST_LISTS * sizeof(long) * PF_BATCH_MAX);
+        b->rst = b->qst + PF_BATCH_MAX;
     }
     if (ht) {
         b->T_host = (pf_bslot *)ht;
         b->est_host = (long *)((char *)ht + sizeof(pf_bslot) * PF_BATCH_MAX);
         b->qst_host = (int *)((char *)b->est_host + EST_LISTS * sizeof(long) * PF_BATCH_MAX);
+        b->rst_host = b->qst_host + PF_BATCH_MAX;
     }
     if (e != hipSuccess) {
         const int rc = pf_set_hip_error(e, "pf_batch_create", __FILE__, __LINE__);

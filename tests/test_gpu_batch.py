@@ -179,18 +179,21 @@ def test_persistent_with_more_blocks_than_workgroups(el, precision, stop):
             c.close()
 
 
-@pytest.mark.parametrize("precision", ["mixed64", "mixed"])
-def test_batch_replacements_in_turn(precision):
+@pytest.mark.parametrize("precision,n", [("mixed64", 18), ("mixed", 18), ("mixed64", 34), ("mixed", 34)])
+def test_batch_replacements(precision, n):
     """Solves of very different sizes whose residuals are replaced in the same
-    and in different iterations, more blocks of products than workgroups:
-    every solve as alone, replacements counted alike."""
-    probs = [P.elastic_cube(18, e=37.0, v=0.22), P.elastic_cube(2), P.elastic_cube(9, lognormal_e=True),
-             P.elastic_cube(18, e=74.0, v=0.22), P.elastic_cube(5, v=0.4)]
+    and in different iterations, more blocks of products than workgroups; below
+    1 GiB of matrices (dealt to the solves) and above (every workgroup on each
+    solve in turn): every solve as alone, replacements counted alike."""
+    probs = [P.elastic_cube(n, e=37.0, v=0.22), P.elastic_cube(2), P.elastic_cube(9, lognormal_e=True),
+             P.elastic_cube(n, e=74.0, v=0.22), P.elastic_cube(5, v=0.4)]
+    assert (sum(pr.nels for pr in probs) * 14656 > 1 << 30) == (n == 34) and (probs[0].neq + 255) // 256 <= 2048
     ctxs = [Context(0) for _ in probs]
     try:
         rs = [P.setup(c, pr, store="fp32") for c, pr in zip(ctxs, probs)]
-        say(f"batch replacements {precision}")
-        kw = dict(stop="relres", precision=precision, refine_delta=0.5)
+        say(f"batch replacements {precision} {n}")
+        # (the residuals of the large solves have not fallen yet: every 40 iterations)
+        kw = dict(stop="relres", precision=precision, refine_delta=0.5, refine_every=40)
         alone = [c.pcg_solve(r, 90, 0.0, **kw) for c, r in zip(ctxs, rs)]
         assert min(res.refinements for _, res in alone) > 0
         with Batch(0) as b:
